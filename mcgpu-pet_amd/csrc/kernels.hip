@@ -1183,18 +1183,21 @@ __device__ __forceinline__ int after_photon(const KParams& P, int photon_no, boo
 // wq[1]) lives in LDS
 // (a single global counter updated once per stream was the limit of short runs). The range
 // is read by every lane and written by the lowest one; volatile keeps each access an LDS
-// operation in program order, which a wave executes in order.
+// operation in program order, which a wave executes in order. Dealt thinly (shares > 0), the
+// queue counts shares: one atomic claims the streams share, share + shares, ... of `lanes` lanes.
 #define K_CHUNK 64
 // Index (from the queue's origin) of the next stream for every calling lane. Not inlined:
 // inlined into the state machine it raised the register pressure of every phase (32 more
 // spilled VGPRs); as a call it costs a few register saves at each claim.
-__device__ __attribute__((noinline)) long long claim_stream(unsigned long long* queue, volatile K_LDS long long* wq)
+__device__ __attribute__((noinline)) long long claim_stream(unsigned long long* queue, volatile K_LDS long long* wq, int lanes,
+                                                               int shares)
 {
   // the lanes here all need a stream: rank among them, claim a new chunk if short
   // (the range is wave-uniform: read into scalar registers)
   const unsigned long long need = __ballot(1);
   const int cnt = __popcll(need);
   const int rank = __popcll(need & ((1ull << __lane_id()) - 1ull));
+  const int step = shares ? shares : 1;
   const long long q0 = wq[0];
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)q0);
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)((unsigned long long)q0 >> 32));
@@ -1202,21 +1205,22 @@ __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* 
   const int avail = __builtin_amdgcn_readfirstlane((int)wq[1]);
   long long idx;
   if (avail >= cnt) {
-    idx = qn + rank;
+    idx = qn + rank * step;
     if (rank == 0) {
-      wq[0] = qn + cnt;
+      wq[0] = qn + cnt * step;
       wq[1] = avail - cnt;
     }
   } else {
     unsigned long long base = 0;
-    if (rank == 0) base = gatomic_add(queue, (unsigned long long)K_CHUNK);
+    if (rank == 0) base = gatomic_add(queue, shares ? 1ull : (unsigned long long)K_CHUNK);
     const unsigned blo = __builtin_amdgcn_readfirstlane((unsigned)base);
     const unsigned bhi = __builtin_amdgcn_readfirstlane((unsigned)(base >> 32));
-    const long long b = (long long)(((unsigned long long)bhi << 32) | blo);
-    idx = rank < avail ? qn + rank : b + (rank - avail);
+    long long b = (long long)(((unsigned long long)bhi << 32) | blo);
+    if (shares && b >= shares) b = 1ll << 62;   // no share is left
+    idx = rank < avail ? qn + rank * step : b + (rank - avail) * step;
     if (rank == 0) {
-      wq[0] = b + (cnt - avail);
-      wq[1] = K_CHUNK - (cnt - avail);
+      wq[0] = b + (cnt - avail) * step;
+      wq[1] = lanes - (cnt - avail);
     }
   }
   return idx;
@@ -1237,7 +1241,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
   bool have = false;
   bool prompt = false;           // the current decay still has its prompt gamma to emit
   int photon_no = 1;
-  int state = LS_DECAY;
+  int state = (int)__lane_id() < P.lanes ? LS_DECAY : LS_DONE;
   for (;;) {
     int best = -1;
     if (P.sm_policy == 0) {
@@ -1338,7 +1342,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
     if (run_decay && state == LS_DECAY) {
       for (;;) {
         if (!have) {
-          const long long idx = claim_stream(P.queue, wq);
+          const long long idx = claim_stream(P.queue, wq, P.lanes, P.shares);
           const long long sid = P.stream_base + (P.stream_stride > 1 ? idx * P.stream_stride : idx);
           if (sid >= P.n_streams) {
             state = LS_DONE;

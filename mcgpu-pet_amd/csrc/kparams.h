@@ -61,6 +61,11 @@ struct KParams {
   long long stream_base;
   int tpb;
   unsigned long long* queue;   // persistent kernel: next stream index
+  // persistent kernel: lanes of each wave that run streams, and, where streams are dealt thinly
+  // (few streams for the device), the number of shares they are dealt to: share k is the streams
+  // k, k + shares, ... of one wave's lanes, so that neighbouring (equally long) streams go to
+  // different waves. shares 0: 64 lanes, streams in queue order.
+  int lanes, shares;
   // source
   int seed;
   int bg_mode;

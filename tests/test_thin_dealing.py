@@ -1,0 +1,21 @@
+"""Streams dealt thinly to the persistent kernel's waves (few streams for the device): the same
+tallies as the oracle's at the edges of the dealing."""
+import pytest
+
+import mcpet
+from harness import assert_tallies_equal, water_cube_scenario
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tpb,kw", [
+    (1, {}),                                          # 729 streams: one lane per wave, fewer waves than resident
+    (7, {}),                                          # 5103 streams: two lanes, a short last row
+    (7, dict(block_size=64, blocks_per_cu=1)),        # fewer waves than shares: waves come back for more
+    (359, {}),                                        # 261711 streams: 64 lanes, still dealt
+    (360, {}),                                        # 262440 streams: full waves, in queue order
+])
+def test_thinly_dealt_streams_give_the_oracles_tallies(tpb, kw):
+    print(f"thin dealing: water cube, tpb {tpb}, {kw}", flush=True)
+    sc = water_cube_scenario(n_decays=3e4, tpb=tpb, material_dose=True)
+    o = sc.run_oracle("fmath")
+    assert_tallies_equal(sc.run_gpu(kernel=mcpet.KERNEL_PERSISTENT, count_events=False, **kw), o, counters="lite")
