@@ -94,6 +94,68 @@ struct Rng {
   int x, y;
 };
 
+// Skip-ahead in digits of 11 bits: y[j][d] = (a1, a2)^(L d 2^(11 j)) mod (m1, m2), L = 555555 x
+// 256, for the three digits of a stream number below 2^33 (built by the compiler, 48 KB, read
+// through L2). A stream's start is then the product of three entries and the seed; with one
+// factor per set bit, a DECAY phase in which three or four of thirty lanes took a new stream
+// spent more than a third of its instructions there (head, 1e8 decays: 41.6 -> 39.7 ms;
+// eight phantoms of 3e7 decays in all in one launch: 14.0 -> 12.0 ms).
+struct JumpDigits {
+  static constexpr int kBits = 11, kDigits = 3;
+  alignas(8) unsigned y[kDigits << kBits][2];
+};
+constexpr JumpDigits jump_digits()
+{
+  JumpDigits t{};
+  const unsigned long long a[2] = {MCR_A1, MCR_A2}, m[2] = {MCR_M1, MCR_M2};
+  for (int g = 0; g < 2; g++) {
+    unsigned long long base = 1, sq = a[g];
+    for (unsigned long long e = (unsigned long long)MCR_HIST_PER_THREAD * MCR_LEAP_DISTANCE; e; e >>= 1) {
+      if (e & 1) base = base * sq % m[g];
+      sq = sq * sq % m[g];
+    }
+    for (int j = 0; j < JumpDigits::kDigits; j++) {   // base = a^(L 2^(11 j))
+      unsigned long long v = 1;
+      for (int d = 0; d < (1 << JumpDigits::kBits); d++) {
+        t.y[(j << JumpDigits::kBits) + d][g] = (unsigned)v;
+        v = v * base % m[g];
+      }
+      base = v;
+    }
+  }
+  return t;
+}
+__device__ const JumpDigits k_jump = jump_digits();
+
+// mcr_init_stream (ranecu.h) with the digit table; j1, j2: the bit tables for the bits above it.
+__device__ __forceinline__ void init_stream_seeds(long long id, int seed, const uint32_t* j1, const uint32_t* j2, int* sx, int* sy)
+{
+  constexpr uint32_t c1 = 0x80000000u - (uint32_t)MCR_M1, c2 = 0x80000000u - (uint32_t)MCR_M2;
+  constexpr int B = JumpDigits::kBits;
+  const unsigned long long n = (unsigned long long)(id + 1);
+  uint32_t y1 = 0, y2 = 0;
+#pragma unroll
+  for (int j = 0; j < JumpDigits::kDigits; j++) {
+    const unsigned d = (j << B) + ((unsigned)(n >> (B * j)) & ((1u << B) - 1u));
+    const unsigned long long e = gld(reinterpret_cast<const unsigned long long*>(k_jump.y), d);
+    y1 = j ? mcr_mulmod_pm(y1, (uint32_t)e, c1) : (uint32_t)e;
+    y2 = j ? mcr_mulmod_pm(y2, (uint32_t)(e >> 32), c2) : (uint32_t)(e >> 32);
+  }
+  int k = B * JumpDigits::kDigits;
+  for (unsigned long long h = n >> k; h && k < MCR_JUMP_BITS; k++, h >>= 1)
+    if (h & 1ull) {
+      y1 = mcr_mulmod_pm(y1, j1[k], c1);
+      y2 = mcr_mulmod_pm(y2, j2[k], c2);
+    }
+  if (seed > 0 && seed < MCR_M2) {
+    *sx = (int)mcr_mulmod_pm((uint32_t)seed, y1, c1);
+    *sy = (int)mcr_mulmod_pm((uint32_t)seed, y2, c2);
+  } else {
+    *sx = mcr_abmodm(MCR_M1, seed, (int)y1);
+    *sy = mcr_abmodm(MCR_M2, seed, (int)y2);
+  }
+}
+
 // Event counters, a compile-time policy of every device function below.
 // FullCounters (instrumented instantiation): every event count, per lane in registers,
 // flushed once per lane. LiteCounters (production): only decays, streams, tallied pairs
@@ -986,7 +1048,7 @@ __device__ __forceinline__ void stream_init(const KParams& P, long long s, Strea
   }
   st.absvox = gld(P.active_vox, k);
   const float act = gld(P.active_act, k);
-  mcr_init_stream(tid, P.seed, P.j1, P.j2, &st.r.x, &st.r.y);
+  init_stream_seeds(tid, P.seed, P.j1, P.j2, &st.r.x, &st.r.y);
   st.event = (unsigned long long)tid << 32;
   st.remaining = P.acq_ps;
   st.inv_act = ((double)per_voxel / (double)act);
@@ -1505,7 +1567,7 @@ __global__ void k_selftest_ranecu(int seed, const long long* ids, int nstreams, 
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nstreams) return;
   int sx, sy;
-  mcr_init_stream(ids[i], seed, j1, j2, &sx, &sy);
+  init_stream_seeds(ids[i], seed, j1, j2, &sx, &sy);
   for (int k = 0; k < n; k++) {
     if (as_double) out_d[(size_t)i * n + k] = mcr_ranecu_double(&sx, &sy);
     else out[(size_t)i * n + k] = mcr_ranecu(&sx, &sy);
