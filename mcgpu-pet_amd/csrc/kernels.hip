@@ -28,6 +28,7 @@
 #include <climits>
 
 #include "devutil.h"
+#include "fastmath.h"
 #include "fmath.h"
 #include "kparams.h"
 
@@ -222,17 +223,18 @@ __device__ __forceinline__ void rotate_double(float* d, double costh, double phi
 {
   double DXY, NORM, cosphi, sinphi, SDT;
   DXY = (double)(d[0] * d[0] + d[1] * d[1]);
-  mcf_sincos(phi, &sinphi, &cosphi);
+  sincos_n(phi, &sinphi, &cosphi);   // 0 <= phi < 2 pi
   NORM = DXY + (double)(d[2] * d[2]);
   if (fabs(NORM - 1.0) > 1.0e-14) {
-    NORM = 1.0 / sqrt(NORM);
+    NORM = div_n(1.0, sqrt_n(NORM));   // a unit vector up to rounding
     d[0] = (float)(NORM * d[0]);
     d[1] = (float)(NORM * d[1]);
     d[2] = (float)(NORM * d[2]);
     DXY = (double)(d[0] * d[0] + d[1] * d[1]);
   }
   if (DXY > 1.0e-28) {
-    SDT = sqrt((1.0 - costh * costh) / DXY);
+    const double sin2 = 1.0 - costh * costh;   // zero or above 2^-53; DXY lies in (1e-28, 1]
+    SDT = sin2 > 0.0 ? sqrt_n(div_n(sin2, DXY)) : 0.0;
     float xin = d[0];
     float yz = d[1] * d[2];
     float xz = xin * d[2];
@@ -323,26 +325,18 @@ __device__ __forceinline__ float shell_term(const mcpet_compton_table& cg, int m
   float pzomc;
   if (!use_cdt) {
     float aux = energy * (energy - temp) * 2.f;
-    pzomc = cg.fj0[mat + i * K_MAXMAT] * (aux - temp * 510998.918f) / (sqrtf(aux + aux + temp * temp) * 510998.918f);
-    if (pzomc > 0.0f)
-      temp = (0.707106781186545f + pzomc * 1.4142135623731f) * (0.707106781186545f + pzomc * 1.4142135623731f);
-    else
-      temp = (0.707106781186545f - pzomc * 1.4142135623731f) * (0.707106781186545f - pzomc * 1.4142135623731f);
-    temp = 0.5f * mcf_expf(0.5f - temp);
+    pzomc = div_n(cg.fj0[mat + i * K_MAXMAT] * (aux - temp * 510998.918f), sqrt_nz(aux + aux + temp * temp) * 510998.918f);
+    const float m = (pzomc > 0.0f) ? 0.707106781186545f + pzomc * 1.4142135623731f : 0.707106781186545f - pzomc * 1.4142135623731f;
+    temp = 0.5f * exp_n(0.5f - m * m);
     if (pzomc > 0.0f) temp = 1.0f - temp;
     return temp;
   }
   float aux = (energy) * (energy - temp) * cdtf;
-  if ((aux > 1.0e-12f) || (temp > 1.0e-12f))
-    pzomc = cg.fj0[mat + i * K_MAXMAT] * (aux - temp * 510998.918f) / (sqrtf(aux + aux + temp * temp) * 510998.918f);
-  else
-    pzomc = 0.002f;
+  pzomc = div_n(cg.fj0[mat + i * K_MAXMAT] * (aux - temp * 510998.918f), sqrt_nz(aux + aux + temp * temp) * 510998.918f);
+  if (!((aux > 1.0e-12f) || (temp > 1.0e-12f))) pzomc = 0.002f;
   temp = pzomc * 1.4142135623731f;
-  if (pzomc > 0.0f)
-    temp = 0.5f - (temp + 0.70710678118654502f) * (temp + 0.70710678118654502f);
-  else
-    temp = 0.5f - (0.70710678118654502f - temp) * (0.70710678118654502f - temp);
-  temp = 0.5f * mcf_expf(temp);
+  const float m = (pzomc > 0.0f) ? temp + 0.70710678118654502f : 0.70710678118654502f - temp;
+  temp = 0.5f * exp_n(0.5f - m * m);
   if (pzomc > 0.0f) temp = 1.0f - temp;
   return temp;
 }
@@ -368,8 +362,8 @@ __device__ __forceinline__ void gcoa_init(float E, int mat, const mcpet_compton_
   const int my_noscco = cg.noscco[mat];
   const float ek = E * 1.956951306108245e-6f;
   const float ek2 = ek * 2.f + 1.f;
-  cs.taumin = 1.f / ek2;
-  cs.a1 = mcf_logf(ek2);
+  cs.taumin = div_n(1.f, ek2);
+  cs.a1 = log_n(ek2);
   float s0 = 0.0f;
   for (int i = 0; i < my_noscco; i++) {
     if (cg.uico[mat + i * K_MAXMAT] < E) s0 += cg.fco[mat + i * K_MAXMAT] * shell_term(cg, mat, i, E, 0.0f, false);
@@ -390,10 +384,10 @@ __device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, 
   const float taumin = cs.taumin, a1 = cs.a1;
   float tau;
   if (rn(r, C) * (a1 + 2. * ek * (ek + 1.f) * taumin * taumin) < a1)
-    tau = mcf_powf(taumin, rn(r, C));
+    tau = exp_n(rn(r, C) * log_n(taumin));   // taumin^u: 0 < taumin < 1, u > 0
   else
-    tau = sqrtf(1.f + rn(r, C) * (taumin * taumin - 1.f));
-  double cdt1 = (double)(1.f - tau) / (((double)tau) * ((double)E) * 1.956951306108245e-6);
+    tau = sqrt_nz(1.f + rn(r, C) * (taumin * taumin - 1.f));
+  double cdt1 = div_n((double)(1.f - tau), ((double)tau) * ((double)E) * 1.956951306108245e-6);
   if (cdt1 > 2.0) cdt1 = 1.99999999;
   const float cdtf = (float)cdt1;
   float s = 0.0f;
@@ -418,7 +412,7 @@ __device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, 
   cs.rc2 = rc2;
   cs.rc3 = rc3;
   const bool reject =
-      (rn(r, C) * cs.s0) > (s * (1.0f + tau * ((ek3 - ek2 - 1.0f) + tau * (ek2 + tau * ek3))) / (ek3 * tau * (tau * tau + 1.0f)));
+      (rn(r, C) * cs.s0) > div_n(s * (1.0f + tau * ((ek3 - ek2 - 1.0f) + tau * (ek2 + tau * ek3))), ek3 * tau * (tau * tau + 1.0f));
   if (!reject) return true;
   return ++cs.trials >= K_MAX_TRIALS;
 }
@@ -449,17 +443,20 @@ __device__ __forceinline__ bool gcoa_pz_trial(float E, int mat, Rng& r, CN& C, c
   }
   temp = rn(r, C) * gcoa_rnv(E, mat, cg, cs, ishell);
   const float fj = cg.fj0[mat + ishell * K_MAXMAT];
-  float pzomc;
-  if (temp < 0.5f)
-    pzomc = (0.70710678118654502f - sqrtf(0.5f - mcf_logf(temp + temp))) / (fj * 1.4142135623731f);
-  else
-    pzomc = (sqrtf(0.5f - mcf_logf(2.0f - 2.0f * temp)) - 0.70710678118654502f) / (fj * 1.4142135623731f);
+  // both halves of the profile through one logarithm and root; its argument is below 1, and zero
+  // (pzomc = -infinity) or subnormal only where the profile term underflows (lower half)
+  const bool low = temp < 0.5f;
+  const float y = low ? temp + temp : 2.0f - 2.0f * temp;
+  const float root = sqrt_nz(0.5f - (y < 0x1p-126f ? mcf_logf(y) : log_n(y)));
+  const float dev = root - 0.70710678118654502f;
+  float pzomc = div_n(low ? -dev : dev, fj * 1.4142135623731f);
+  if (y == 0.0f) pzomc = -MCF_INFF;
   cs.pzomc = pzomc;
   if (!(pzomc < -1.0f)) {
     float af;
     temp = (float)(tau * (tau - costh * 2.f) + 1.f);
     if (temp > 1.0e-20f)
-      af = sqrtf(temp) * (tau * (tau - ((float)costh)) / temp + 1.f);
+      af = sqrt_nz(temp) * (div_n(tau * (tau - ((float)costh)), temp) + 1.f);
     else
       af = 0.00200f;
     if (af > 0.0f) temp = af * 0.2f + 1.f;
@@ -537,14 +534,15 @@ K_RARE void tally_sinogram(const KParams& P, float energy, float energyFirst, co
   if (ibin < 0) return;
   float randno1 = rn(st.r, C);
   float randno2 = rn(st.r, C);
-  float g1 = sqrtf((float)(-2.0 * (double)mcf_logf(randno1 + 1e-8f))) * mcf_cosf((float)(2.0f * K_PI * (double)randno2));
+  // -2 log(u) is zero or above 1e-7; the doubling is exact
+  float g1 = sqrt_nz(-2.0f * log_n(randno1 + 1e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno2));
   float randno3 = rn(st.r, C);
   float randno4 = rn(st.r, C);
-  float g2 = sqrtf((float)(-2.0 * (double)mcf_logf(randno3 + 1.0e-8f))) * mcf_cosf((float)(2.0f * K_PI * (double)randno4));
+  float g2 = sqrt_nz(-2.0f * log_n(randno3 + 1.0e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno4));
   float Energia1 = energy + ((P.e_resol) / 2.35f) * energy * g1;
   float Energia2 = energyFirst + ((P.e_resol) / 2.35f) * energyFirst * g2;
-  int iE1 = f2i_rd(Energia1 / 1000.0f);
-  int iE2 = f2i_rd(Energia2 / 1000.0f);
+  int iE1 = floor_i32(div_r(Energia1, 1000.0f, 1.0f / 1000.0f));
+  int iE2 = floor_i32(div_r(Energia2, 1000.0f, 1.0f / 1000.0f));
   if ((iE1 < P.ne) && (iE1 >= 0)) spectrum_add(P, s_spec, iE1);
   if ((iE2 < P.ne) && (iE2 >= 0)) spectrum_add(P, s_spec, iE2);
   C.inc(KC_PAIRS);
@@ -608,10 +606,10 @@ K_RARE void tally_psf(const KParams& P, float energy, float energyFirst, const f
   positionFirst[2] = (posf_in[2] - P.cz) + dist * dirf[2];
   float randno1 = rn(st.r, C);
   float randno2 = rn(st.r, C);
-  float g1 = sqrtf(-2.0f * mcf_logf(randno1 + 1e-8f)) * mcf_cosf((float)(2.0f * K_PI * (double)randno2));
+  float g1 = sqrt_nz(-2.0f * log_n(randno1 + 1e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno2));
   float randno3 = rn(st.r, C);
   float randno4 = rn(st.r, C);
-  float g2 = sqrtf(-2.0f * mcf_logf(randno3 + 1.0e-8f)) * mcf_cosf((float)(2.0f * K_PI * (double)randno4));
+  float g2 = sqrt_nz(-2.0f * log_n(randno3 + 1.0e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno4));
   float Energia1 = energy + ((P.e_resol) * (1.0f / 2.35f)) * energy * g1;
   float Energia2 = energyFirst + ((P.e_resol) * (1.0f / 2.35f)) * energyFirst * g2;
   if (fabsf(positionFirst[2]) < 0.5f * P.height && (Energia1 > P.e_low) && (Energia1 < P.e_high) && (Energia2 > P.e_low) &&
@@ -654,9 +652,9 @@ __device__ __forceinline__ void record_single(const KParams& P, const float* pos
   if (!(fabsf(z) < 0.5f * P.height)) return;
   const float randno1 = rn(st.r, C);
   const float randno2 = rn(st.r, C);
-  const float g = sqrtf(-2.0f * mcf_logf(randno1 + 1e-8f)) * mcf_cosf((float)(2.0f * K_PI * (double)randno2));
+  const float g = sqrt_nz(-2.0f * log_n(randno1 + 1e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno2));
   const float e = energy + ((P.e_resol) * (1.0f / 2.35f)) * energy * g;
-  const int iE = f2i_rd(e / 1000.0f);
+  const int iE = floor_i32(div_r(e, 1000.0f, 1.0f / 1000.0f));
   if ((iE < P.ne) && (iE >= 0)) spectrum_add(P, s_spec, iE);
   if (!(e > P.e_low && e < P.e_high)) return;
   const float phi = mcf_atan2f(y0 + dist * dir[1], x0 + dist * dir[0]);
@@ -678,9 +676,9 @@ __device__ __forceinline__ void tally_dose(const KParams& P, float Edep, int mat
     atomicAdd(&s_mat[2 * mat + 1], f2ull_rn(Edep * Edep));
   }
   if (P.voxel_dose) {
-    short vx = (short)f2i_rd(pos[0] * P.ivx);
-    short vy = (short)f2i_rd(pos[1] * P.ivy);
-    short vz = (short)f2i_rd(pos[2] * P.ivz);
+    short vx = (short)floor_i32(pos[0] * P.ivx);
+    short vy = (short)floor_i32(pos[1] * P.ivy);
+    short vz = (short)floor_i32(pos[2] * P.ivz);
     if ((vx < P.roi[0]) || (vx > P.roi[1]) || (vy < P.roi[2]) || (vy > P.roi[3]) || (vz < P.roi[4]) || (vz > P.roi[5])) return;
     int DX = 1 + (int)(P.roi[1] - P.roi[0]);
     int num = (int)(vx - P.roi[0]) + ((int)(vy - P.roi[2])) * DX + ((int)(vz - P.roi[4])) * DX * (1 + (int)(P.roi[3] - P.roi[2]));
@@ -709,7 +707,7 @@ __device__ __forceinline__ void photon_start(const KParams& P, Photon& ph, float
   ph.E = energy;
   ph.ss = 0;
   ph.travel = 0.0f;
-  ph.index = f2i_rd((ph.E - P.e0) * P.ide);
+  ph.index = floor_i32((ph.E - P.e0) * P.ide);
   const float2 w = gld(P.woodcock, ph.index);
   ph.mfpW = w.x + ph.E * w.y;
   ph.mat_old = -1;
@@ -748,7 +746,7 @@ __device__ __forceinline__ float2 voxel_word(const KParams& P, int absvox)
 template <class CN>
 __device__ __forceinline__ int woodcock_step(const KParams& P, Photon& ph, Rng& r, CN& C)
 {
-  const float step = -(ph.mfpW)*mcf_logf(rn(r, C));
+  const float step = -(ph.mfpW)*log_n(rn(r, C));
   C.inc(KC_WOODCOCK);
   ph.travel += step;
   ph.pos[0] += step * ph.dir[0];
@@ -820,7 +818,7 @@ __device__ __forceinline__ bool compton_end(const KParams& P, Photon& ph, Rng& r
   const double costh_Compton = gcoa_finish(&ph.E, cs);
   rotate_double(ph.dir, costh_Compton, 6.28318530717958647693 * rnd(r, C));
   const float randno = ph.E - e_before;
-  ph.index = f2i_rd((ph.E - P.e0) * P.ide);
+  ph.index = floor_i32((ph.E - P.e0) * P.ide);
   if (ph.index > -1) {
     const float2 w = gld(P.woodcock, ph.index);
     ph.mfpW = w.x + ph.E * w.y;
@@ -888,9 +886,9 @@ __device__ __forceinline__ void source_first(const KParams& P, Stream& st, CN& C
 {
   dir[2] = 1.0f - 2.0f * rn(st.r, C);
   float phi_sampled = 6.28318530716f * rn(st.r, C);
-  float sin_theta = sqrtf(1.0f - dir[2] * dir[2]);
+  float sin_theta = sqrt_nz(1.0f - dir[2] * dir[2]);
   float sp, cp;
-  mcf_sincosf(phi_sampled, &sp, &cp);
+  sincos_n(phi_sampled, &sp, &cp);
   dir[1] = sin_theta * sp;
   dir[0] = sin_theta * cp;
   float r1 = rn(st.r, C);
@@ -912,9 +910,9 @@ __device__ __forceinline__ void isotropic_dir(Stream& st, CN& C, float* dir)
 {
   dir[2] = 1.0f - 2.0f * rn(st.r, C);
   float phi_sampled = 6.28318530716f * rn(st.r, C);
-  float sin_theta = sqrtf(1.0f - dir[2] * dir[2]);
+  float sin_theta = sqrt_nz(1.0f - dir[2] * dir[2]);
   float sp, cp;
-  mcf_sincosf(phi_sampled, &sp, &cp);
+  sincos_n(phi_sampled, &sp, &cp);
   dir[1] = sin_theta * sp;
   dir[0] = sin_theta * cp;
 }
@@ -930,14 +928,14 @@ __device__ __forceinline__ void source_second(const KParams& P, Stream& st, CN& 
   float theta_sampled2 = (float)(K_PI - (double)mcf_acosf(dir1[2]));
   float V1 = rn(st.r, C);
   float V2 = rn(st.r, C);
-  float THETA_NC = (float)((2.0 * 0.21276 * K_PI / 180.0) * (double)sqrtf(-2.0f * mcf_logf(V2 + 1e-8f)) *
-                           (double)mcf_cosf((float)((2.0 * K_PI) * (double)V1)));
+  float THETA_NC = (float)((2.0 * 0.21276 * K_PI / 180.0) * (double)sqrt_nz(-2.0f * log_n(V2 + 1e-8f)) *
+                           (double)cos_n((float)((2.0 * K_PI) * (double)V1)));
   float PHI_NC = (float)((2.0 * K_PI) * (double)rn(st.r, C));
   float ST, CT, CP, SP, ST1, CT1, CP1, SP1;
-  mcf_sincosf(THETA_NC, &ST, &CT);
-  mcf_sincosf(PHI_NC, &SP, &CP);
-  mcf_sincosf(theta_sampled2, &ST1, &CT1);
-  mcf_sincosf(phi_sampled2, &SP1, &CP1);
+  sincos_n(THETA_NC, &ST, &CT);
+  sincos_n(PHI_NC, &SP, &CP);
+  sincos_n(theta_sampled2, &ST1, &CT1);
+  sincos_n(phi_sampled2, &SP1, &CP1);
   float GX = CP * ST;
   float GY = SP * ST;
   float GZ = CT;
@@ -951,13 +949,13 @@ __device__ __forceinline__ void source_second(const KParams& P, Stream& st, CN& 
 template <class CN>
 __device__ __forceinline__ bool decay_time(const KParams& P, Stream& st, CN& C)
 {
-  const double Dt = -mcf_log(rnd(st.r, C)) * st.inv_act;
+  const double Dt = -log_n(rnd(st.r, C)) * st.inv_act;
   const unsigned long long Dt_ps = d2ull_rn(Dt * 1e12);
   if (!(Dt_ps < st.remaining)) return false;
   st.remaining -= Dt_ps;
   st.event++;
   C.inc(KC_DECAYS);              // 2 photon histories per decay (K:282)
-  st.inv_act = st.inv_act * mcf_exp(Dt * P.inv_mean_life);
+  st.inv_act = st.inv_act * exp_nonneg(Dt * P.inv_mean_life);
   return true;
 }
 
