@@ -31,6 +31,14 @@ static __device__ __forceinline__ float4 gld(const float4* p, size_t i)
   const v4 v = ((const DU_GLOBAL v4*)p)[i];
   return make_float4(v.x, v.y, v.z, v.w);
 }
+// Element i of a table below 4 GiB: a 32-bit byte offset beside the scalar base, instead of a
+// 64-bit address computed per lane.
+template <class T>
+static __device__ __forceinline__ T gld32(const T* p, unsigned i)
+{
+  const char* b = reinterpret_cast<const char*>(p);
+  return gld(reinterpret_cast<const T*>(b + (unsigned)(i * (unsigned)sizeof(T))), 0);
+}
 template <class T>
 static __device__ __forceinline__ T gatomic_add(T* p, T v)
 {

@@ -202,20 +202,26 @@ __device__ __forceinline__ double rnd(Rng& r, CN& C)
   return mcr_ranecu_double(&r.x, &r.y);
 }
 
+// Voxel index x + nx (y + ny z).
+__device__ __forceinline__ int voxel_index(const StepParams& P, int x, int y, int z)
+{
+  if (P.index24) return (int)(__umul24(__umul24(z, P.ny) + y, P.nx) + x);
+  return x + P.nx * (y + P.ny * z);
+}
+
 // locate_voxel (K:1097-1124). NaN positions count as outside and indices are clamped
 // to the grid (the reference would read out of bounds in both cases). Evaluated without
-// branches: the six bound tests (a NaN coordinate fails them) combine into one select, and
-// inside the box every floor(p * inverse size) lies in [0, n], so it converts directly after
-// clamping to [0, n - 1]; the same index as the reference's early returns and
+// branches: positive floats order as their bits, so one unsigned comparison per axis tests both
+// bounds, and fails for negative numbers and NaN; inside the box floor(p * inverse size) lies in
+// [0, n], so only n is clamped. The same index as the reference's early returns and
 // __float2int_rd.
-__device__ __forceinline__ int locate(const KParams& P, const float* p)
+__device__ __forceinline__ int locate(const StepParams& P, const float* p)
 {
-  const bool inside = (p[1] >= K_EPS) & (p[1] <= (P.by - K_EPS)) & (p[0] >= K_EPS) & (p[0] <= (P.bx - K_EPS)) &
-                      (p[2] >= K_EPS) & (p[2] <= (P.bz - K_EPS));
-  const int vx = (int)fminf(fmaxf(floorf(p[0] * P.ivx), 0.0f), (float)(P.nx - 1));
-  const int vy = (int)fminf(fmaxf(floorf(p[1] * P.ivy), 0.0f), (float)(P.ny - 1));
-  const int vz = (int)fminf(fmaxf(floorf(p[2] * P.ivz), 0.0f), (float)(P.nz - 1));
-  return inside ? (vx + vy * (P.nx) + vz * (P.nx) * (P.ny)) : -100;
+  const bool inside = (__float_as_uint(p[0]) - P.box_lo <= P.box_span[0]) & (__float_as_uint(p[1]) - P.box_lo <= P.box_span[1]) &
+                      (__float_as_uint(p[2]) - P.box_lo <= P.box_span[2]);
+  const int vx = min(floor_i32(p[0] * P.ivx), P.nx - 1), vy = min(floor_i32(p[1] * P.ivy), P.ny - 1),
+            vz = min(floor_i32(p[2] * P.ivz), P.nz - 1);
+  return inside ? voxel_index(P, vx, vy, vz) : -100;
 }
 
 // rotate_double (K:1159-1200): PENELOPE DIRECT in double precision on a float vector.
@@ -708,7 +714,7 @@ __device__ __forceinline__ void photon_start(const KParams& P, Photon& ph, float
   ph.ss = 0;
   ph.travel = 0.0f;
   ph.index = floor_i32((ph.E - P.e0) * P.ide);
-  const float2 w = gld(P.woodcock, ph.index);
+  const float2 w = gld32(P.woodcock, ph.index);
   ph.mfpW = w.x + ph.E * w.y;
   ph.mat_old = -1;
 }
@@ -722,29 +728,27 @@ __shared__ float2 k_palette[256];
 // copied to LDS per workgroup: unscattered photons (most Woodcock steps) reload (a, b) from
 // here on a table change instead of from global memory. The same values as P.tot's row.
 __shared__ float2 k_tot511[K_MAXMAT];
-__shared__ int k_idx511;
 
-// Fill k_tot511 / k_idx511 (all lanes of the workgroup; a barrier must follow).
+// Fill k_tot511 (all lanes of the workgroup; a barrier must follow).
 __device__ __forceinline__ void load_tot511(const KParams& P)
 {
   const int idx = f2i_rd((K_E511 - P.e0) * P.ide);
   if (threadIdx.x < K_MAXMAT) k_tot511[threadIdx.x] = gld(P.tot, idx * K_MAXMAT + threadIdx.x);
-  if (threadIdx.x == 0) k_idx511 = P.lds_xs511 ? idx : -1;   // -1: no energy bin matches, rows from global memory
 }
 
 // The (density, material) word of voxel absvox in the device layout chosen at set-up.
-__device__ __forceinline__ float2 voxel_word(const KParams& P, int absvox)
+__device__ __forceinline__ float2 voxel_word(const StepParams& P, int absvox)
 {
   if (P.vox_fmt == 1) {
-    const unsigned i = gld(P.vox8, absvox);
-    return P.lds_palette ? k_palette[i] : gld(P.palette, i);
+    const unsigned i = gld32(P.vox8, absvox);
+    return P.lds_palette ? k_palette[i] : gld32(P.palette, i);
   }
-  if (P.vox_fmt == 2) return gld(P.palette, gld(P.vox16, absvox));
+  if (P.vox_fmt == 2) return gld32(P.palette, gld32(P.vox16, absvox));
   return gld(P.vox, absvox);
 }
 
 template <class CN>
-__device__ __forceinline__ int woodcock_step(const KParams& P, Photon& ph, Rng& r, CN& C)
+__device__ __forceinline__ int woodcock_step(const StepParams& P, Photon& ph, Rng& r, CN& C)
 {
   const float step = -(ph.mfpW)*log_n(rn(r, C));
   C.inc(KC_WOODCOCK);
@@ -762,7 +766,7 @@ __device__ __forceinline__ int woodcock_step(const KParams& P, Photon& ph, Rng& 
   ph.mat0 = w & 0xff;
   if (w != ph.mat_old) {
     if (ph.mat_old < 0 || (w >> 8) != (ph.mat_old >> 8))
-      ph.tab = ph.index == k_idx511 ? k_tot511[ph.mat0] : gld(P.tot, ph.index * K_MAXMAT + ph.mat0);
+      ph.tab = ph.index == P.idx511 ? k_tot511[ph.mat0] : gld32(P.tot, ph.index * K_MAXMAT + ph.mat0);
     ph.mat_old = w;
     C.inc(KC_MATCHANGE);
   }
@@ -782,7 +786,7 @@ template <class CN>
 __device__ __forceinline__ int interaction_begin(const KParams& P, Photon& ph, Rng& r, CN& C,
                                                  const mcpet_compton_table& cg, ComptonState& cs, unsigned long long* s_mat)
 {
-  const float4 cr = gld(P.cr, ph.index * K_MAXMAT + ph.mat0);
+  const float4 cr = gld32(P.cr, ph.index * K_MAXMAT + ph.mat0);
   float prob = ph.prob + ph.mfp_density * (cr.x + ph.E * cr.y);
   const float randno = ph.randno;
   if (randno < prob) {
@@ -820,7 +824,7 @@ __device__ __forceinline__ bool compton_end(const KParams& P, Photon& ph, Rng& r
   const float randno = ph.E - e_before;
   ph.index = floor_i32((ph.E - P.e0) * P.ide);
   if (ph.index > -1) {
-    const float2 w = gld(P.woodcock, ph.index);
+    const float2 w = gld32(P.woodcock, ph.index);
     ph.mfpW = w.x + ph.E * w.y;
     ph.mat_old = -2;
     ph.ss = (ph.ss == 0) ? 1 : 3;
@@ -850,8 +854,8 @@ template <class CN>
 __device__ __forceinline__ void transport_photon(const KParams& P, Photon& ph, Stream& st, CN& C,
                                                  const mcpet_compton_table& cg, unsigned long long* s_mat)
 {
+  if (locate(P, ph.pos) < 0) return;   // an interaction leaves the photon inside the box
   for (;;) {
-    if (locate(P, ph.pos) < 0) return;
     int o;
     do {
       o = woodcock_step(P, ph, st.r, C);
@@ -899,9 +903,9 @@ __device__ __forceinline__ void source_first(const KParams& P, Stream& st, CN& C
   r3 = (K_EPS > r3 - K_EPS) ? K_EPS : r3 - K_EPS;
   int ix, iy, iz;
   voxel_coords(P, st.absvox, ix, iy, iz);
-  pos[0] = ((float)ix + r1) / P.ivx;
-  pos[1] = ((float)iy + r2) / P.ivy;
-  pos[2] = ((float)iz + r3) / P.ivz;
+  pos[0] = div_r((float)ix + r1, P.ivx, P.rvx);
+  pos[1] = div_r((float)iy + r2, P.ivy, P.rvy);
+  pos[2] = div_r((float)iz + r3, P.ivz, P.rvz);
 }
 
 // Isotropic direction (K:711-720, the BG-mode second photon).
@@ -1354,7 +1358,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
       if (o == IA_COMPTON) {
         cs_store(L, cs);
         state = LS_CTAU;
-      } else if (o == IA_ABSORBED || locate(P, ph.pos) < 0) {
+      } else if (o == IA_ABSORBED) {
         state = after_photon(P, photon_no, prompt, ph, L);
       } else {
         state = LS_STEP;
@@ -1385,7 +1389,8 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
         ok = gcoa_pz_trial(ph.E, ph.mat0, st.r, C, s_cmp, cs);
       } while (!ok && ++k < MCPET_TRIALS_PER_PHASE);
       if (ok) {
-        if (!compton_end(P, ph, st.r, C, cs, s_mat) || locate(P, ph.pos) < 0) state = after_photon(P, photon_no, prompt, ph, L);
+        // (the photon is where its last step found it inside the box)
+        if (!compton_end(P, ph, st.r, C, cs, s_mat)) state = after_photon(P, photon_no, prompt, ph, L);
         else state = LS_STEP;
       } else {
         L[CS_TRIALS] = __int_as_float(cs.trials);
@@ -1471,9 +1476,10 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
     const bool run_step = best == LS_STEP || ((MCPET_CHAIN & 4) && run_pz) ||
                           ((MCPET_CHAIN & 8) && (run_decay || run_src2 || run_src3));
     if (run_step && state == LS_STEP) {
+      const StepParams S = P;   // one block of scalar loads
       int o, k = 0;
       do {
-        o = woodcock_step(P, ph, st.r, C);
+        o = woodcock_step(S, ph, st.r, C);
       } while (o == STEP_VIRTUAL && ++k < MCPET_STEPS_PER_PHASE);
       if (o == STEP_ESCAPED) {
         state = after_photon(P, photon_no, prompt, ph, L);

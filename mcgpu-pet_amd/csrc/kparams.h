@@ -31,19 +31,33 @@ enum KCounter {
   KC_N = 16 + 3 * MCPET_NPHASES
 };
 
-struct KParams {
+// What a Woodcock step reads, together in 64 bytes (and the less used pointers behind them): the
+// step loads them as one block of scalars, since a lone lane's chain waits for every separate load.
+struct alignas(64) StepParams {
+  // the box test on the bits of positive floats: a coordinate p is inside iff
+  // bits(p) - box_lo <= box_span (unsigned), box_lo the bits of the margin EPS
+  unsigned box_lo, box_span[3];
+  float ivx, ivy, ivz;         // inverse voxel size
+  int nx, ny, nz;
+  int index24;                 // ny nz and nx below 2^24: voxel indices by 24-bit multiplies
   // phantom, x fastest. vox_fmt 0: one packed word (density, material index 0..14 as int
   // bits) per voxel; 1: u8 index into a palette of such words (palette copied to LDS);
   // 2: u16 index into the palette (read from global memory).
-  const float2* vox;
+  int vox_fmt;
+  int lds_palette;             // 1: u8 palette copied to LDS (single-phantom kernels)
+  int idx511;                  // energy bin of 511 keV whose total cross sections are read from LDS (-1: none)
   const uint8_t* vox8;
-  const uint16_t* vox16;
   const float2* palette;
-  int vox_fmt, n_palette;
-  int nx, ny, nz;
+  const uint16_t* vox16;
+  const float2* vox;
+  const float2* tot;           // [N][15]      (a_total, b_total)
+};
+
+struct KParams : StepParams {
+  int n_palette;
   double inv_nx, inv_ny;       // 1 / nx, 1 / ny: voxel coordinates by multiplication (src_coords)
-  float ivx, ivy, ivz;         // inverse voxel size
   float bx, by, bz;            // bounding box size
+  float rvx, rvy, rvz;         // 1 / inverse voxel size
   // decay streams: stream s -> emitting voxel active_vox[s / tpb], lane s % tpb; with a
   // balanced layout (stream_start != null) voxel k owns streams [stream_start[k],
   // stream_start[k + 1]) whose random-number stream ids start at stream_id[k]
@@ -75,7 +89,6 @@ struct KParams {
   uint32_t j2[MCR_JUMP_BITS];
   // interaction tables
   const float2* woodcock;      // [N]          (a, b)
-  const float2* tot;           // [N][15]      (a_total, b_total)
   const float4* cr;            // [N][15]      (a_compton, b_compton, a_rayleigh, b_rayleigh)
   const mcpet_rayleigh_table* ray;
   const mcpet_compton_table* cmp;
@@ -111,7 +124,6 @@ struct KParams {
   int* final_seed;
   long long last_thread_id;      // reference thread id whose final seed is stored (K:454-455)
   int lds_spectrum;              // 1: privatise the spectrum in LDS
-  int lds_palette;               // 1: u8 palette copied to LDS (single-phantom kernels)
   int lds_xs511;                 // 1: the 511 keV total-cross-section row read from LDS
   long long stream_stride;       // > 1: the k-th claimed stream is stream_base + k * stride (sampling)
   // Decay branching (drawn per decay only when active) and the singles list.

@@ -607,6 +607,25 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   P.bx = ph->size_bbox[0];
   P.by = ph->size_bbox[1];
   P.bz = ph->size_bbox[2];
+  {
+    const float lo = 0.00015f, hi[3] = {P.bx - lo, P.by - lo, P.bz - lo};   // locate_voxel's margins (K:1099-1104)
+    bool some = true;
+    std::memcpy(&P.box_lo, &lo, 4);
+    for (int k = 0; k < 3; k++) {
+      uint32_t b;
+      std::memcpy(&b, &hi[k], 4);
+      P.box_span[k] = b - P.box_lo;
+      some = some && hi[k] >= lo;
+    }
+    if (!some) {   // a box thinner than its margins: no coordinate is inside (only this NaN would be)
+      P.box_lo = 0xffffffffu;
+      P.box_span[0] = P.box_span[1] = P.box_span[2] = 0;
+    }
+  }
+  P.index24 = (long long)ph->ny * ph->nz < (1LL << 24) && ph->nx < (1 << 24) ? 1 : 0;
+  P.rvx = 1.0f / P.ivx;
+  P.rvy = 1.0f / P.ivy;
+  P.rvz = 1.0f / P.ivz;
   P.active_vox = c->d_active_vox;
   P.active_act = c->d_active_act;
   P.tpb = cfg->threads_per_block;
@@ -678,6 +697,7 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   P.lds_spectrum = (cfg->ne > 0 && cfg->ne <= 8192) ? 1 : 0;
   P.lds_palette = 1;
   P.lds_xs511 = 1;
+  P.idx511 = (int)std::floor((510998.95f - P.e0) * P.ide);
   P.stream_stride = 1;
   P.lanes = 64;
   *out = c;
@@ -749,6 +769,7 @@ extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
     P.lds_palette = (lds & MCPET_LDS_PALETTE) ? 1 : 0;
     P.lds_spectrum = (lds & MCPET_LDS_SPECTRUM) && c->P.lds_spectrum ? 1 : 0;   // only where the spectrum fits
     P.lds_xs511 = (lds & MCPET_LDS_XS511) ? 1 : 0;
+    if (!P.lds_xs511) P.idx511 = -1;   // no energy bin matches: the rows come from global memory
   }
   P.sm_policy = (p.phase_policy == 2) ? 1 : 0;
   static const int default_cost[MCPET_NPHASES] = {4, 6, 1, 3, 6, 3, 2, 4, 4, 1};
