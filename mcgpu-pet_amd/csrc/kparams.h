@@ -10,6 +10,10 @@
 #include "mcpet.h"
 #include "ranecu.h"
 
+// Records of a wave's staging buffer (KParams::stage): fewer than 64 left over and at most 128
+// (a pair per lane) of one pass through the phases.
+#define K_STAGE_RECORDS 192
+
 // Event counters accumulated by the kernels (order of mcpet_stats after the two times).
 enum KCounter {
   KC_DECAYS = 0,
@@ -126,6 +130,10 @@ struct KParams : StepParams {
   int lds_spectrum;              // 1: privatise the spectrum in LDS
   int lds_xs511;                 // 1: the 511 keV total-cross-section row read from LDS
   long long stream_stride;       // > 1: the k-th claimed stream is stream_base + k * stride (sampling)
+  // staging of the phase-space or singles records of every wave of the launch (null: each record
+  // takes its place in the list by itself): stage_stride bytes per wave
+  char* stage;
+  int stage_stride;
   // Decay branching (drawn per decay only when active) and the singles list.
   float positron_frac;           // < 1: a decay emits the annihilation pair with this probability
   float prompt_frac;             // > 0: a decay emits a prompt gamma with this probability

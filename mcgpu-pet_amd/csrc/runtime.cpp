@@ -63,6 +63,8 @@ struct mcpet_ctx {
   int* d_spectrum = nullptr;
   mcpet_psf_record* d_psf = nullptr;
   int* d_psf_index = nullptr;
+  char* d_stage = nullptr;       // the waves' staging of appended records (allocated at the first run that uses it)
+  size_t stage_bytes = 0;
   unsigned long long* d_voxel_edep = nullptr;
   unsigned long long* d_mat_edep = nullptr;
   unsigned long long* d_counters = nullptr;  // KC_N counters + stream queue
@@ -148,7 +150,7 @@ mcpet_status dalloc(mcpet_ctx* c, T** p, size_t n)
 void free_all(mcpet_ctx* c)
 {
   void* ptrs[] = {c->d_vox, c->d_vox8, c->d_vox16, c->d_palette, c->d_active_vox, c->d_active_act, c->d_stream_start, c->d_stream_id, c->d_stream_hint, c->d_rbt, c->d_rbt_plane, c->d_woodcock, c->d_tot, c->d_cr, c->d_ray, c->d_cmp,
-                  c->d_trues, c->d_scatter, c->d_img_t, c->d_img_sc, c->d_spectrum, c->d_psf, c->d_psf_index,
+                  c->d_trues, c->d_scatter, c->d_img_t, c->d_img_sc, c->d_spectrum, c->d_psf, c->d_psf_index, c->d_stage,
                   c->d_voxel_edep, c->d_mat_edep, c->d_counters, c->d_final_seed, c->d_singles, c->d_singles_n,
                   c->d_keys[0], c->d_keys[1], c->d_vals[0], c->d_vals[1], c->d_hist, c->d_randoms, c->d_spurious,
                   c->d_coinc, c->d_rb_off, c->d_rb_sino, c->d_rb_out, c->d_pj_params, c->d_pj_out};
@@ -812,6 +814,19 @@ extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
   } else {
     blocks = std::max(1LL, (P.n_streams + bs - 1) / bs);
     if (blocks > 0x7fffffffLL) return set_err(c, MCPET_E_RANGE, "mcpet_run: too many streams for one launch");
+  }
+  if (kind == MCPET_KERNEL_PERSISTENT && P.mode != 2) {   // a phase-space file or a singles list
+    P.stage_stride = K_STAGE_RECORDS * (int)(c->singles_mode ? sizeof(mcpet_single) : sizeof(mcpet_psf_record));
+    const size_t need = (size_t)blocks * (bs / 64) * P.stage_stride;
+    if (need > c->stage_bytes) {   // this run waits for the context's last one above
+      if (c->d_stage) (void)hipFree(c->d_stage);
+      c->dev_bytes -= c->stage_bytes;
+      c->d_stage = nullptr;
+      c->stage_bytes = 0;
+      if (dalloc(c, &c->d_stage, need) == MCPET_OK) c->stage_bytes = need;   // else every record appends by itself
+      else (void)hipGetLastError();
+    }
+    P.stage = c->d_stage;
   }
   // the rebinned tallies hold the sinograms' counts only if every run since the last clear added to them
   c->rbt_ran = P.rb_trues != nullptr && (p.zero_tallies || c->rbt_ran);
@@ -1629,7 +1644,7 @@ mcpet_status mcpet_run_contexts(const CtxRun* runs, int n, hipStream_t stream, K
     P.sm_policy = 0;
     P.lds_spectrum = 0;
     P.lds_palette = 0;
-    ext = ext || P.prompt_frac > 0.0f;
+    ext = ext || P.prompt_frac > 0.0f || P.mode != 2;
     h_params[k] = P;
     c->rbt_ran = P.rb_trues != nullptr && (runs[k].clear != 0 || c->rbt_ran);
     mcpet_status st = clear_buffers(c, stream, runs[k].clear != 0, runs[k].clear != 0);
@@ -1758,7 +1773,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
     for (int i = 0; i < MCPET_NPHASES; i++) P.sm_cost[i] = p.phase_cost[i] > 0 ? p.phase_cost[i] : default_cost[i];
     P.lds_spectrum = 0;   // per phantom: global atomics
     P.lds_palette = 0;
-    ext = ext || P.prompt_frac > 0.0f;
+    ext = ext || P.prompt_frac > 0.0f || P.mode != 2;
     b->h_params[k] = P;
   }
   const int bs = p.block_size > 0 ? p.block_size : (b->tuned_bs > 0 ? b->tuned_bs : 256);
