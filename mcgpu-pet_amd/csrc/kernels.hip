@@ -45,10 +45,12 @@
 // corrupt input. The CPU checker applies the same bound.
 #define K_MAX_TRIALS (1 << 20)
 
-// Occupancy target of the transport kernels (waves per SIMD; 0 leaves it to the compiler).
-// The persistent kernel is bound by the latency of dependent gathers and transcendental
-// chains; 4 waves per SIMD (128 VGPRs, ~10 dwords of spill) hides more of it than 3 (+17%
-// on the head workload) or 5 (spills grow), and than the compiler's own 2.
+// Occupancy target of the persistent transport kernels (waves per SIMD; 0 leaves it to the
+// compiler). They wait on dependent gathers and on chains of dependent operations, so waves pay
+// up to the last one that fits without spilling: 5 (96 VGPRs, 28 KB of LDS per workgroup with
+// the shells and the palette at the phantom's own sizes) against 4: head, 1e8 decays, 31.6 ->
+// 29.0 ms; 4e7 torso decays with singles 38.1 -> 36.3 ms; eight phantoms in one launch 10.75 ->
+// 10.2 ms.
 // Woodcock steps a lane may take in one STEP phase while its steps stay virtual, and GCOa
 // rejection trials (tau loop, p_z loop) in one CTAU / CPZ phase: the phase selection's ballots
 // are paid once for several. 3 and 2 measured best on the head workload (1-4 steps, 1-3
@@ -68,7 +70,7 @@
 #define MCPET_CHAIN 31
 #endif
 #ifndef MCPET_WAVES_PER_EU
-#define MCPET_WAVES_PER_EU 4
+#define MCPET_WAVES_PER_EU 5
 #endif
 #if MCPET_WAVES_PER_EU > 0
 #define K_OCCUPANCY __attribute__((amdgpu_waves_per_eu(MCPET_WAVES_PER_EU, 8)))
@@ -322,23 +324,34 @@ K_RARE void graa(float energy, double* costh, int mat, float pmax_current, Rng& 
   }
 }
 
+// Compton shells in LDS: the shells of every distinct material file in turn, each (ionisation
+// energy U, occupation f, profile J0, U x 510998.918) in one 16-byte read, and per material slot
+// (first shell << 8) | number of shells.
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+struct Shells {
+  const K_LDS v4f* table;
+  const K_LDS unsigned* of;
+  const K_LDS v2f* pal;        // the u8 voxel palette (density, material word), where it is in LDS
+};
+
 // Compton profile term of shell i at momentum transfer factor `cdtf` (the inner body of
 // the incoherent-scattering-function loops, K:1407-1449); 0 for inaccessible shells.
-__device__ __forceinline__ float shell_term(const mcpet_compton_table& cg, int mat, int i, float energy, float cdtf, bool use_cdt)
+__device__ __forceinline__ float shell_term(v4f sh, float energy, float cdtf, bool use_cdt)
 {
-  float temp = cg.uico[mat + i * K_MAXMAT];
+  float temp = sh.x;
   if (!(temp < energy)) return 0.0f;
   float pzomc;
   if (!use_cdt) {
     float aux = energy * (energy - temp) * 2.f;
-    pzomc = div_n(cg.fj0[mat + i * K_MAXMAT] * (aux - temp * 510998.918f), sqrt_nz(aux + aux + temp * temp) * 510998.918f);
+    pzomc = div_n(sh.z * (aux - sh.w), sqrt_nz(aux + aux + temp * temp) * 510998.918f);
     const float m = (pzomc > 0.0f) ? 0.707106781186545f + pzomc * 1.4142135623731f : 0.707106781186545f - pzomc * 1.4142135623731f;
     temp = 0.5f * exp_n(0.5f - m * m);
     if (pzomc > 0.0f) temp = 1.0f - temp;
     return temp;
   }
   float aux = (energy) * (energy - temp) * cdtf;
-  pzomc = div_n(cg.fj0[mat + i * K_MAXMAT] * (aux - temp * 510998.918f), sqrt_nz(aux + aux + temp * temp) * 510998.918f);
+  pzomc = div_n(sh.z * (aux - sh.w), sqrt_nz(aux + aux + temp * temp) * 510998.918f);
   if (!((aux > 1.0e-12f) || (temp > 1.0e-12f))) pzomc = 0.002f;
   temp = pzomc * 1.4142135623731f;
   const float m = (pzomc > 0.0f) ? temp + 0.70710678118654502f : 0.70710678118654502f - temp;
@@ -356,23 +369,26 @@ __device__ __forceinline__ float shell_term(const mcpet_compton_table& cg, int m
 // and recomputed for later shells instead of a 30-entry array (same values).
 struct ComptonState {
   float a1, s0, taumin;            // set by gcoa_init
-  float tau, s, cdtf;              // accepted tau trial
+  float tau, s;                    // accepted tau trial
   float rc0, rc1, rc2, rc3;        // its profile terms of shells 0..3
   float pzomc;
   double cdt1;
   int trials;
 };
 
-__device__ __forceinline__ void gcoa_init(float E, int mat, const mcpet_compton_table& cg, ComptonState& cs)
+__device__ __forceinline__ void gcoa_init(float E, int mat, const Shells& cg, ComptonState& cs)
 {
-  const int my_noscco = cg.noscco[mat];
+  const unsigned of = cg.of[mat];
+  const K_LDS v4f* table = cg.table + (of >> 8);
+  const int my_noscco = of & 0xff;
   const float ek = E * 1.956951306108245e-6f;
   const float ek2 = ek * 2.f + 1.f;
   cs.taumin = div_n(1.f, ek2);
   cs.a1 = log_n(ek2);
   float s0 = 0.0f;
   for (int i = 0; i < my_noscco; i++) {
-    if (cg.uico[mat + i * K_MAXMAT] < E) s0 += cg.fco[mat + i * K_MAXMAT] * shell_term(cg, mat, i, E, 0.0f, false);
+    const v4f sh = table[i];
+    if (sh.x < E) s0 += sh.y * shell_term(sh, E, 0.0f, false);
   }
   cs.s0 = s0;
   cs.trials = 0;
@@ -380,10 +396,12 @@ __device__ __forceinline__ void gcoa_init(float E, int mat, const mcpet_compton_
 
 // One trial of the tau loop; true when the loop is over (accepted or trial cap).
 template <class CN>
-__device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, const mcpet_compton_table& cg,
+__device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, const Shells& cg,
                                                ComptonState& cs)
 {
-  const int my_noscco = cg.noscco[mat];
+  const unsigned of = cg.of[mat];
+  const K_LDS v4f* table = cg.table + (of >> 8);
+  const int my_noscco = of & 0xff;
   const float ek = E * 1.956951306108245e-6f;
   const float ek2 = ek * 2.f + 1.f;
   const float ek3 = ek * ek;
@@ -400,9 +418,10 @@ __device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, 
   C.add(KC_SHELLEVAL, (unsigned)my_noscco);
   float rc0 = 0.0f, rc1 = 0.0f, rc2 = 0.0f, rc3 = 0.0f;
   for (int i = 0; i < my_noscco; i++) {
-    if (cg.uico[mat + i * K_MAXMAT] < E) {
-      const float t = shell_term(cg, mat, i, E, cdtf, true);
-      s += cg.fco[mat + i * K_MAXMAT] * t;
+    const v4f sh = table[i];
+    if (sh.x < E) {
+      const float t = shell_term(sh, E, cdtf, true);
+      s += sh.y * t;
       rc0 = (i == 0) ? t : rc0;
       rc1 = (i == 1) ? t : rc1;
       rc2 = (i == 2) ? t : rc2;
@@ -411,7 +430,6 @@ __device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, 
   }
   cs.tau = tau;
   cs.cdt1 = cdt1;
-  cs.cdtf = cdtf;
   cs.s = s;
   cs.rc0 = rc0;
   cs.rc1 = rc1;
@@ -423,32 +441,34 @@ __device__ __forceinline__ bool gcoa_tau_trial(float E, int mat, Rng& r, CN& C, 
   return ++cs.trials >= K_MAX_TRIALS;
 }
 
-__device__ __forceinline__ float gcoa_rnv(float E, int mat, const mcpet_compton_table& cg, const ComptonState& cs, int i)
+__device__ __forceinline__ float gcoa_rnv(float E, const K_LDS v4f* table, const ComptonState& cs, int i)
 {
   if (i < 4) return i == 0 ? cs.rc0 : i == 1 ? cs.rc1 : i == 2 ? cs.rc2 : cs.rc3;
-  return shell_term(cg, mat, i, E, cs.cdtf, true);
+  return shell_term(table[i], E, (float)cs.cdt1, true);
 }
 
 // One trial of the p_z loop; true when the loop is over (accepted or trial cap).
 template <class CN>
-__device__ __forceinline__ bool gcoa_pz_trial(float E, int mat, Rng& r, CN& C, const mcpet_compton_table& cg,
+__device__ __forceinline__ bool gcoa_pz_trial(float E, int mat, Rng& r, CN& C, const Shells& cg,
                                               ComptonState& cs)
 {
-  const int my_noscco = cg.noscco[mat];
+  const unsigned of = cg.of[mat];
+  const K_LDS v4f* table = cg.table + (of >> 8);
+  const int my_noscco = of & 0xff;
   const double costh = 1.0 - cs.cdt1;
   const float tau = cs.tau;
   float temp = cs.s * rn(r, C);
   float pac = 0.0f;
   int ishell = my_noscco - 1;
   for (int i = 0; i < (my_noscco - 1); i++) {
-    pac += cg.fco[mat + i * K_MAXMAT] * gcoa_rnv(E, mat, cg, cs, i);
+    pac += table[i].y * gcoa_rnv(E, table, cs, i);
     if (pac > temp) {
       ishell = i;
       break;
     }
   }
-  temp = rn(r, C) * gcoa_rnv(E, mat, cg, cs, ishell);
-  const float fj = cg.fj0[mat + ishell * K_MAXMAT];
+  temp = rn(r, C) * gcoa_rnv(E, table, cs, ishell);
+  const float fj = table[ishell].z;
   // both halves of the profile through one logarithm and root; its argument is below 1, and zero
   // (pzomc = -infinity) or subnormal only where the profile term underflows (lower half)
   const bool low = temp < 0.5f;
@@ -780,9 +800,6 @@ __device__ __forceinline__ void photon_start(const KParams& P, Photon& ph, float
 
 enum StepOutcome { STEP_ESCAPED = 0, STEP_VIRTUAL = 1, STEP_REAL = 2 };
 
-// Palette of (density, material) words for u8-indexed phantoms, filled by each
-// workgroup's prologue.
-__shared__ float2 k_palette[256];
 // The total-cross-section row (a, b) of every material slot at the annihilation energy's bin,
 // copied to LDS per workgroup: unscattered photons (most Woodcock steps) reload (a, b) from
 // here on a table change instead of from global memory. The same values as P.tot's row.
@@ -796,18 +813,20 @@ __device__ __forceinline__ void load_tot511(const KParams& P)
 }
 
 // The (density, material) word of voxel absvox in the device layout chosen at set-up.
-__device__ __forceinline__ float2 voxel_word(const StepParams& P, int absvox)
+__device__ __forceinline__ float2 voxel_word(const StepParams& P, const K_LDS v2f* pal, int absvox)
 {
   if (P.vox_fmt == 1) {
     const unsigned i = gld32(P.vox8, absvox);
-    return P.lds_palette ? k_palette[i] : gld32(P.palette, i);
+    if (!P.lds_palette) return gld32(P.palette, i);
+    const v2f v = pal[i];
+    return make_float2(v.x, v.y);
   }
   if (P.vox_fmt == 2) return gld32(P.palette, gld32(P.vox16, absvox));
   return gld(P.vox, absvox);
 }
 
 template <class CN>
-__device__ __forceinline__ int woodcock_step(const StepParams& P, Photon& ph, Rng& r, CN& C)
+__device__ __forceinline__ int woodcock_step(const StepParams& P, const K_LDS v2f* pal, Photon& ph, Rng& r, CN& C)
 {
   const float step = -(ph.mfpW)*log_n(rn(r, C));
   C.inc(KC_WOODCOCK);
@@ -817,7 +836,7 @@ __device__ __forceinline__ int woodcock_step(const StepParams& P, Photon& ph, Rn
   ph.pos[2] += step * ph.dir[2];
   const int absvox = locate(P, ph.pos);
   if (absvox < 0) return STEP_ESCAPED;
-  const float2 md = voxel_word(P, absvox);
+  const float2 md = voxel_word(P, pal, absvox);
   // material word: slot (bits 0-7) | id of its total cross-section table (bits 8-15); slots
   // whose tables are bitwise identical share an id, so a change between them (a material
   // change of the reference, K:331-336) keeps the (a, b) already loaded: the same values
@@ -843,7 +862,7 @@ enum InteractionOutcome { IA_ALIVE = 0, IA_ABSORBED = 1, IA_COMPTON = 2 };
 
 template <class CN>
 __device__ __forceinline__ int interaction_begin(const KParams& P, Photon& ph, Rng& r, CN& C,
-                                                 const mcpet_compton_table& cg, ComptonState& cs, unsigned long long* s_mat)
+                                                 const Shells& cg, ComptonState& cs, unsigned long long* s_mat)
 {
   const float4 cr = gld32(P.cr, ph.index * K_MAXMAT + ph.mat0);
   float prob = ph.prob + ph.mfp_density * (cr.x + ph.E * cr.y);
@@ -894,7 +913,7 @@ __device__ __forceinline__ bool compton_end(const KParams& P, Photon& ph, Rng& r
 
 // Whole real event, nested form. False when the photon is absorbed.
 template <class CN>
-__device__ __forceinline__ bool real_interaction(const KParams& P, Photon& ph, Rng& r, CN& C, const mcpet_compton_table& cg,
+__device__ __forceinline__ bool real_interaction(const KParams& P, Photon& ph, Rng& r, CN& C, const Shells& cg,
                                                  unsigned long long* s_mat)
 {
   ComptonState cs;
@@ -911,13 +930,13 @@ __device__ __forceinline__ bool real_interaction(const KParams& P, Photon& ph, R
 // Whole photon (K:297-415), nested loops: escape or absorption.
 template <class CN>
 __device__ __forceinline__ void transport_photon(const KParams& P, Photon& ph, Stream& st, CN& C,
-                                                 const mcpet_compton_table& cg, unsigned long long* s_mat)
+                                                 const Shells& cg, unsigned long long* s_mat)
 {
   if (locate(P, ph.pos) < 0) return;   // an interaction leaves the photon inside the box
   for (;;) {
     int o;
     do {
-      o = woodcock_step(P, ph, st.r, C);
+      o = woodcock_step(P, cg.pal, ph, st.r, C);
     } while (o == STEP_VIRTUAL);
     if (o == STEP_ESCAPED) return;
     if (!real_interaction(P, ph, st.r, C, cg, s_mat)) return;
@@ -1059,7 +1078,7 @@ __device__ __forceinline__ void keep_first(Pair& pr, const Photon& ph)
 
 // One annihilation, both photons, nested loops (reference main loop body, K:259-449).
 template <class CN>
-__device__ bool decay(const KParams& P, Stream& st, CN& C, const mcpet_compton_table& cg, int* s_spec,
+__device__ bool decay(const KParams& P, Stream& st, CN& C, const Shells& cg, int* s_spec,
                       unsigned long long* s_mat)
 {
   if (!decay_time(P, st, C)) return false;
@@ -1123,25 +1142,35 @@ __device__ __forceinline__ void stream_finish(const KParams& P, const Stream& st
 
 // Workgroup prologue/epilogue shared by the kernels: Compton table, spectrum, material
 // dose and workgroup counters in LDS; counters flushed once per lane / per workgroup.
+// Dynamic LDS of the single-phantom kernels: the shells, the palette and the spectrum (the last
+// two where the layout keeps them in LDS), of the sizes this phantom needs.
 #define K_PROLOGUE(CN)                                                                           \
-  __shared__ mcpet_compton_table s_cmp;                                                          \
+  __shared__ unsigned s_shell_of[K_MAXMAT];                                                      \
   __shared__ unsigned long long s_mat[2 * K_MAXMAT];                                             \
   __shared__ unsigned s_cnt[KC_N];                                                               \
-  extern __shared__ int s_spec[];                                                                \
+  extern __shared__ v4f s_dyn[];                                                                 \
+  const bool use_pal = P.vox_fmt == 1 && P.lds_palette;                                          \
+  v2f* const s_pal = (v2f*)(s_dyn + P.n_shells);                                                 \
+  int* const s_spec = (int*)(s_pal + (use_pal ? P.n_palette : 0));                               \
   {                                                                                              \
-    const int* src = reinterpret_cast<const int*>(P.cmp);                                        \
-    int* dst = reinterpret_cast<int*>(&s_cmp);                                                   \
-    for (int i = threadIdx.x; i < (int)(sizeof(mcpet_compton_table) / 4); i += blockDim.x)       \
-      dst[i] = gld(src, i);                                                                      \
+    for (int i = threadIdx.x; i < P.n_shells; i += blockDim.x) {                                 \
+      const float4 v = gld(P.shells, i);                                                         \
+      s_dyn[i] = v4f{v.x, v.y, v.z, v.w};                                                        \
+    }                                                                                            \
+    if (threadIdx.x < K_MAXMAT) s_shell_of[threadIdx.x] = P.shell_of[threadIdx.x];               \
     if (threadIdx.x < 2 * K_MAXMAT) s_mat[threadIdx.x] = 0ull;                                   \
     if (threadIdx.x < KC_N) s_cnt[threadIdx.x] = 0u;                                             \
-    if (P.vox_fmt == 1 && P.lds_palette)                                                         \
-      for (int i = threadIdx.x; i < P.n_palette; i += blockDim.x) k_palette[i] = gld(P.palette, i); \
+    if (use_pal)                                                                                 \
+      for (int i = threadIdx.x; i < P.n_palette; i += blockDim.x) {                              \
+        const float2 v = gld(P.palette, i);                                                      \
+        s_pal[i] = v2f{v.x, v.y};                                                                \
+      }                                                                                          \
     load_tot511(P);                                                                              \
     if (P.lds_spectrum)                                                                          \
       for (int i = threadIdx.x; i < P.ne; i += blockDim.x) s_spec[i] = 0;                        \
   }                                                                                              \
   __syncthreads();                                                                               \
+  const Shells s_cmp{(const K_LDS v4f*)s_dyn, (const K_LDS unsigned*)s_shell_of, (const K_LDS v2f*)s_pal}; \
   CN C;                                                                                          \
   C.init(s_cnt);
 
@@ -1156,7 +1185,10 @@ __device__ __forceinline__ void stream_finish(const KParams& P, const Stream& st
   if (threadIdx.x < 2 * K_MAXMAT && s_mat[threadIdx.x]) gatomic_add(&P.mat_edep[threadIdx.x], s_mat[threadIdx.x]);
 
 // Plain kernel: lane i of the grid runs stream i to the end (nested loops, no queue).
-__global__ __launch_bounds__(256) K_OCCUPANCY void k_transport_plain(KParams P)
+#ifndef MCPET_PLAIN_WAVES
+#define MCPET_PLAIN_WAVES 4
+#endif
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MCPET_PLAIN_WAVES, 8))) void k_transport_plain(KParams P)
 {
   K_PROLOGUE(FullCounters)
   const long long sid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1198,12 +1230,16 @@ enum LaneState {
 // (structure of arrays, slot k of lane i at [k][i]: consecutive lanes, consecutive banks):
 // the pair kept between the two photons (15 words) and the Compton sampler's state
 // between its rejection trials (14 words). Only the stream and the current photon stay
-// in registers across iterations, which keeps the kernel at 3 waves per SIMD.
+// in registers across iterations.
 #define K_BLOCK 256
-enum PairSlot { PS_P1 = 0, PS_D1 = 3, PS_EF = 6, PS_TRAVELF = 7, PS_POSF = 8, PS_DIRF = 11, PS_SSF = 14, PS_N = 15 };
+// Slots whose contents are never needed together share a place: photon 1's direction waits for
+// photon 2's emission where the pair's first hit goes later, and moves to the Compton sampler's
+// slots when photon 1 has ended.
+enum PairSlot { PS_P1 = 0, PS_POSF = 3, PS_DIRF = 6, PS_EF = 9, PS_SSF = 10, PS_TRAVELF = 11, PS_N = 12, PS_D1 = PS_POSF };
 enum ComptonSlot {
-  CS_A1 = PS_N, CS_S0, CS_TAUMIN, CS_TAU, CS_S, CS_CDTF, CS_RC0, CS_RC1, CS_RC2, CS_RC3, CS_PZOMC, CS_CDT1_LO, CS_CDT1_HI,
-  CS_TRIALS, LANE_SLOTS
+  CS_A1 = PS_N, CS_S0, CS_TAUMIN, CS_TAU, CS_S, CS_RC0, CS_RC1, CS_RC2, CS_RC3, CS_CDT1_LO, CS_CDT1_HI, CS_TRIALS, LANE_SLOTS,
+  CS_PROB = CS_A1, CS_MFPD, CS_RANDNO,   // a real interaction's inputs until GCOa starts
+  PS_D1_LATER = CS_A1                    // photon 1's direction between the two photons
 };
 
 struct LaneSlots {
@@ -1219,26 +1255,25 @@ __device__ __forceinline__ void pair_store_source(const LaneSlots& L, const Pair
   }
   L[PS_EF] = pr.EF;
 }
+__device__ __forceinline__ void pair_keep_d1(const LaneSlots& L)
+{
+  for (int k = 0; k < 3; k++) L[PS_D1_LATER + k] = L[PS_D1 + k];
+}
 __device__ __forceinline__ void pair_store_first(const LaneSlots& L, const Photon& ph)
 {
-  Pair pr;
-  pr.EF = L[PS_EF];
-  keep_first(pr, ph);
-  if (ph.index > -1) {
-    L[PS_EF] = pr.EF;
-    L[PS_TRAVELF] = pr.travelF;
-    L[PS_SSF] = __int_as_float(pr.ssF);
+  if (ph.index > -1) {   // as keep_first
+    L[PS_EF] = ph.E;
+    L[PS_TRAVELF] = ph.travel;
+    L[PS_SSF] = __int_as_float(ph.ss);
     for (int k = 0; k < 3; k++) {
-      L[PS_POSF + k] = pr.posF[k];
-      L[PS_DIRF + k] = pr.dirF[k];
+      L[PS_POSF + k] = ph.pos[k];
+      L[PS_DIRF + k] = ph.dir[k];
     }
   }
 }
 __device__ __forceinline__ void pair_load(const LaneSlots& L, Pair& pr)
 {
   for (int k = 0; k < 3; k++) {
-    pr.p1[k] = L[PS_P1 + k];
-    pr.d1[k] = L[PS_D1 + k];
     pr.posF[k] = L[PS_POSF + k];
     pr.dirF[k] = L[PS_DIRF + k];
   }
@@ -1253,12 +1288,10 @@ __device__ __forceinline__ void cs_store(const LaneSlots& L, const ComptonState&
   L[CS_TAUMIN] = cs.taumin;
   L[CS_TAU] = cs.tau;
   L[CS_S] = cs.s;
-  L[CS_CDTF] = cs.cdtf;
   L[CS_RC0] = cs.rc0;
   L[CS_RC1] = cs.rc1;
   L[CS_RC2] = cs.rc2;
   L[CS_RC3] = cs.rc3;
-  L[CS_PZOMC] = cs.pzomc;
   const unsigned long long b = (unsigned long long)__double_as_longlong(cs.cdt1);
   L[CS_CDT1_LO] = __uint_as_float((unsigned)b);
   L[CS_CDT1_HI] = __uint_as_float((unsigned)(b >> 32));
@@ -1271,12 +1304,10 @@ __device__ __forceinline__ void cs_load(const LaneSlots& L, ComptonState& cs)
   cs.taumin = L[CS_TAUMIN];
   cs.tau = L[CS_TAU];
   cs.s = L[CS_S];
-  cs.cdtf = L[CS_CDTF];
   cs.rc0 = L[CS_RC0];
   cs.rc1 = L[CS_RC1];
   cs.rc2 = L[CS_RC2];
   cs.rc3 = L[CS_RC3];
-  cs.pzomc = L[CS_PZOMC];
   const unsigned long long b = (unsigned long long)__float_as_uint(L[CS_CDT1_LO]) |
                                ((unsigned long long)__float_as_uint(L[CS_CDT1_HI]) << 32);
   cs.cdt1 = __longlong_as_double((long long)b);
@@ -1288,6 +1319,7 @@ __device__ __forceinline__ void cs_load(const LaneSlots& L, ComptonState& cs)
 // photon in DETECT instead of pairing them here.
 __device__ __forceinline__ int after_photon(const KParams& P, bool singles, int photon_no, bool prompt, const Photon& ph, const LaneSlots& L)
 {
+  if (photon_no == 1) pair_keep_d1(L);
   if (singles) return LS_DETECT;
   if (photon_no == 1) {
     pair_store_first(L, ph);
@@ -1351,7 +1383,7 @@ __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* 
 }
 
 template <class CN, bool kExt>
-__device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_compton_table& s_cmp, int* s_spec,
+__device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& s_cmp, int* s_spec,
                                          unsigned long long* s_mat, const LaneSlots& L, volatile K_LDS long long* wq)
 {
   constexpr int kPhases = kExt ? LS_N : LS_CPZ + 1;
@@ -1421,9 +1453,9 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
     const bool run_int = best == LS_INTERACT;
     if (run_int && state == LS_INTERACT) {
       ComptonState cs;
-      ph.prob = L[CS_TAU];
-      ph.mfp_density = L[CS_S];
-      ph.randno = L[CS_CDTF];
+      ph.prob = L[CS_PROB];
+      ph.mfp_density = L[CS_MFPD];
+      ph.randno = L[CS_RANDNO];
       const int o = interaction_begin(P, ph, st.r, C, s_cmp, cs, s_mat);
       if (o == IA_COMPTON) {
         cs_store(L, cs);
@@ -1521,7 +1553,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
       float p1[3], d1[3];
       for (int k = 0; k < 3; k++) {
         p1[k] = L[PS_P1 + k];
-        d1[k] = L[PS_D1 + k];
+        d1[k] = L[PS_D1_LATER + k];
       }
       source_second(P, st, C, d1, ph.dir);
       for (int k = 0; k < 3; k++) ph.pos[k] = p1[k];
@@ -1549,15 +1581,15 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const mcpet_co
       const StepParams S = P;   // one block of scalar loads
       int o, k = 0;
       do {
-        o = woodcock_step(S, ph, st.r, C);
+        o = woodcock_step(S, s_cmp.pal, ph, st.r, C);
       } while (o == STEP_VIRTUAL && ++k < MCPET_STEPS_PER_PHASE);
       if (o == STEP_ESCAPED) {
         state = after_photon(P, singles, photon_no, prompt, ph, L);
       } else if (o == STEP_REAL) {
         // the interaction's inputs wait in LDS (Compton slots, free until GCOa starts)
-        L[CS_TAU] = ph.prob;
-        L[CS_S] = ph.mfp_density;
-        L[CS_CDTF] = ph.randno;
+        L[CS_PROB] = ph.prob;
+        L[CS_MFPD] = ph.mfp_density;
+        L[CS_RANDNO] = ph.randno;
         state = LS_INTERACT;
       }
     }
@@ -1596,15 +1628,18 @@ __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_sm(const KPar
 template <class CN, bool kExt>
 __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_batch(const KParams* __restrict__ Ps, int n)
 {
-  __shared__ mcpet_compton_table s_cmp;
+  __shared__ unsigned s_shell_of[K_MAXMAT];
+  extern __shared__ v4f s_dyn[];
   __shared__ unsigned long long s_matw[K_BLOCK / 64][2 * K_MAXMAT];
   __shared__ unsigned s_cntw[K_BLOCK / 64][KC_N];
   __shared__ float s_slots[LANE_SLOTS][K_BLOCK];
   __shared__ long long s_wq[K_BLOCK / 64][3];
   {
-    const int* src = reinterpret_cast<const int*>(Ps[0].cmp);
-    int* dst = reinterpret_cast<int*>(&s_cmp);
-    for (int i = threadIdx.x; i < (int)(sizeof(mcpet_compton_table) / 4); i += blockDim.x) dst[i] = gld(src, i);
+    for (int i = threadIdx.x; i < Ps[0].n_shells; i += blockDim.x) {
+      const float4 v = gld(Ps[0].shells, i);
+      s_dyn[i] = v4f{v.x, v.y, v.z, v.w};
+    }
+    if (threadIdx.x < K_MAXMAT) s_shell_of[threadIdx.x] = Ps[0].shell_of[threadIdx.x];
     for (int i = threadIdx.x; i < (K_BLOCK / 64) * 2 * K_MAXMAT; i += blockDim.x) (&s_matw[0][0])[i] = 0ull;
     for (int i = threadIdx.x; i < (K_BLOCK / 64) * KC_N; i += blockDim.x) (&s_cntw[0][0])[i] = 0u;
     load_tot511(Ps[0]);   // the phantoms of a batch share their interaction tables
@@ -1612,6 +1647,7 @@ __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_batch(const K
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const LaneSlots L{&s_slots[0][threadIdx.x]};
+  const Shells s_cmp{(const K_LDS v4f*)s_dyn, (const K_LDS unsigned*)s_shell_of, nullptr};
   const int first = (int)(((long long)blockIdx.x * (blockDim.x >> 6) + wave) % n);
   for (int j = 0; j < n; j++) {
     const int k = __builtin_amdgcn_readfirstlane((first + j) % n);
@@ -1714,11 +1750,17 @@ __global__ void k_copy(const uint4* __restrict__ src, uint4* __restrict__ dst, s
 
 }  // namespace
 
+size_t mcpet_transport_dyn_lds(const KParams& P)
+{
+  return 16 * (size_t)P.n_shells + (P.vox_fmt == 1 && P.lds_palette ? 8 * (size_t)P.n_palette : 0) +
+         (P.lds_spectrum ? 4 * (size_t)P.ne : 0);
+}
+
 hipError_t mcpet_launch_transport(const KParams& P, const KParams* d_P, int kind, int count_events, int blocks, int block_size,
                                   hipStream_t stream)
 {
   if (block_size > K_BLOCK || block_size % 64 != 0) return hipErrorInvalidValue;
-  size_t lds = P.lds_spectrum ? (size_t)P.ne * sizeof(int) : 0;
+  const size_t lds = mcpet_transport_dyn_lds(P);
   const bool ext = P.mode != 2 || P.prompt_frac > 0.0f;   // lists or prompt gammas
   if (kind == MCPET_KERNEL_PERSISTENT && count_events && ext)
     hipLaunchKernelGGL((k_transport_sm<FullCounters, true>), dim3(blocks), dim3(block_size), lds, stream, d_P);
@@ -1733,18 +1775,18 @@ hipError_t mcpet_launch_transport(const KParams& P, const KParams* d_P, int kind
   return hipGetLastError();
 }
 
-hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, bool ext, int count_events, int blocks, int block_size,
-                                        hipStream_t stream)
+hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, int n_shells, bool ext, int count_events, int blocks,
+                                        int block_size, hipStream_t stream)
 {
   if (block_size > K_BLOCK || block_size % 64 != 0 || n < 1) return hipErrorInvalidValue;
   if (count_events && ext)
-    hipLaunchKernelGGL((k_transport_batch<FullCounters, true>), dim3(blocks), dim3(block_size), 0, stream, d_params, n);
+    hipLaunchKernelGGL((k_transport_batch<FullCounters, true>), dim3(blocks), dim3(block_size), 16 * (size_t)n_shells, stream, d_params, n);
   else if (count_events)
-    hipLaunchKernelGGL((k_transport_batch<FullCounters, false>), dim3(blocks), dim3(block_size), 0, stream, d_params, n);
+    hipLaunchKernelGGL((k_transport_batch<FullCounters, false>), dim3(blocks), dim3(block_size), 16 * (size_t)n_shells, stream, d_params, n);
   else if (ext)
-    hipLaunchKernelGGL((k_transport_batch<LiteCounters, true>), dim3(blocks), dim3(block_size), 0, stream, d_params, n);
+    hipLaunchKernelGGL((k_transport_batch<LiteCounters, true>), dim3(blocks), dim3(block_size), 16 * (size_t)n_shells, stream, d_params, n);
   else
-    hipLaunchKernelGGL((k_transport_batch<LiteCounters, false>), dim3(blocks), dim3(block_size), 0, stream, d_params, n);
+    hipLaunchKernelGGL((k_transport_batch<LiteCounters, false>), dim3(blocks), dim3(block_size), 16 * (size_t)n_shells, stream, d_params, n);
   return hipGetLastError();
 }
 

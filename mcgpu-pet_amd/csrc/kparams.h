@@ -95,7 +95,9 @@ struct KParams : StepParams {
   const float2* woodcock;      // [N]          (a, b)
   const float4* cr;            // [N][15]      (a_compton, b_compton, a_rayleigh, b_rayleigh)
   const mcpet_rayleigh_table* ray;
-  const mcpet_compton_table* cmp;
+  const float4* shells;        // Compton shells (U, f, J0, U x 510998.918) of the distinct material files
+  int n_shells;
+  unsigned shell_of[MCPET_MAX_MATERIALS];   // per slot: (first shell << 8) | number of shells
   int num_values;
   float e0, ide;
   // detector
@@ -155,8 +157,10 @@ struct KParams : StepParams {
 // Launchers implemented in kernels.hip.
 hipError_t mcpet_launch_transport(const KParams& P, const KParams* d_P, int kind, int count_events, int blocks, int block_size,
                                   hipStream_t stream);
-hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, bool ext, int count_events, int blocks, int block_size,
-                                        hipStream_t stream);
+// dynamic LDS of a single-phantom launch (bytes)
+size_t mcpet_transport_dyn_lds(const KParams& P);
+hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, int n_shells, bool ext, int count_events, int blocks,
+                                        int block_size, hipStream_t stream);
 hipError_t mcpet_launch_fill_u32(void* p, size_t n_words, hipStream_t stream);
 // zero n regions of n_words[i] 4-byte words at p[i], K_FILL_MAX regions per launch
 #define K_FILL_MAX 16

@@ -55,7 +55,7 @@ struct mcpet_ctx {
   float2* d_tot = nullptr;
   float4* d_cr = nullptr;
   mcpet_rayleigh_table* d_ray = nullptr;
-  mcpet_compton_table* d_cmp = nullptr;
+  float4* d_shells = nullptr;
   int* d_trues = nullptr;
   int* d_scatter = nullptr;
   int* d_img_t = nullptr;
@@ -149,7 +149,7 @@ mcpet_status dalloc(mcpet_ctx* c, T** p, size_t n)
 
 void free_all(mcpet_ctx* c)
 {
-  void* ptrs[] = {c->d_vox, c->d_vox8, c->d_vox16, c->d_palette, c->d_active_vox, c->d_active_act, c->d_stream_start, c->d_stream_id, c->d_stream_hint, c->d_rbt, c->d_rbt_plane, c->d_woodcock, c->d_tot, c->d_cr, c->d_ray, c->d_cmp,
+  void* ptrs[] = {c->d_vox, c->d_vox8, c->d_vox16, c->d_palette, c->d_active_vox, c->d_active_act, c->d_stream_start, c->d_stream_id, c->d_stream_hint, c->d_rbt, c->d_rbt_plane, c->d_woodcock, c->d_tot, c->d_cr, c->d_ray, c->d_shells,
                   c->d_trues, c->d_scatter, c->d_img_t, c->d_img_sc, c->d_spectrum, c->d_psf, c->d_psf_index, c->d_stage,
                   c->d_voxel_edep, c->d_mat_edep, c->d_counters, c->d_final_seed, c->d_singles, c->d_singles_n,
                   c->d_keys[0], c->d_keys[1], c->d_vals[0], c->d_vals[1], c->d_hist, c->d_randoms, c->d_spurious,
@@ -499,6 +499,27 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
     hcr[b] = make_float4(a[1], s[1], a[2], s[2]);
   }
 
+  // Compton shells, once per distinct material (slots of one file hold the same shells).
+  std::vector<float4> hsh;
+  unsigned shell_of[MCPET_MAX_MATERIALS];
+  for (int m = 0; m < MCPET_MAX_MATERIALS; m++) {
+    const mcpet_compton_table& ct = *tab->compton;
+    const int n = std::min(std::max(ct.noscco[m], 0), MCPET_MAX_SHELLS);
+    std::vector<float4> sh((size_t)n);
+    for (int i = 0; i < n; i++) {
+      const int k = m + i * MCPET_MAX_MATERIALS;
+      sh[(size_t)i] = make_float4(ct.uico[k], ct.fco[k], ct.fj0[k], ct.uico[k] * 510998.918f);
+    }
+    size_t first = hsh.size();
+    for (int m2 = 0; m2 < m && n > 0; m2++)
+      if ((int)(shell_of[m2] & 0xff) == n && std::memcmp(&hsh[shell_of[m2] >> 8], sh.data(), sizeof(float4) * (size_t)n) == 0) {
+        first = shell_of[m2] >> 8;
+        break;
+      }
+    if (first == hsh.size()) hsh.insert(hsh.end(), sh.begin(), sh.end());
+    shell_of[m] = (unsigned)(first << 8) | (unsigned)n;
+  }
+
   // ROI (dose) size.
   const bool voxel_dose = cfg->voxel_dose && cfg->roi_x_max > -1;
   if (voxel_dose) {   // inside the phantom (checked above)
@@ -527,7 +548,7 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   CK(dalloc(c, &c->d_tot, htot.size()));
   CK(dalloc(c, &c->d_cr, hcr.size()));
   CK(dalloc(c, &c->d_ray, 1));
-  CK(dalloc(c, &c->d_cmp, 1));
+  CK(dalloc(c, &c->d_shells, hsh.size()));
   CK(dalloc(c, &c->d_trues, (size_t)cfg->nbins));
   CK(dalloc(c, &c->d_scatter, (size_t)cfg->nbins));
   CK(dalloc(c, &c->d_img_t, (size_t)c->nvox));
@@ -583,7 +604,7 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   HK(hipMemcpy(c->d_tot, htot.data(), htot.size() * sizeof(float2), hipMemcpyHostToDevice));
   HK(hipMemcpy(c->d_cr, hcr.data(), hcr.size() * sizeof(float4), hipMemcpyHostToDevice));
   HK(hipMemcpy(c->d_ray, tab->rayleigh, sizeof(mcpet_rayleigh_table), hipMemcpyHostToDevice));
-  HK(hipMemcpy(c->d_cmp, tab->compton, sizeof(mcpet_compton_table), hipMemcpyHostToDevice));
+  if (!hsh.empty()) HK(hipMemcpy(c->d_shells, hsh.data(), sizeof(float4) * hsh.size(), hipMemcpyHostToDevice));
 
   KParams& P = c->P;
   P.positron_frac = (cfg->positron_fraction > 0.0f && cfg->positron_fraction < 1.0f) ? cfg->positron_fraction : 1.0f;
@@ -650,7 +671,9 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   P.tot = c->d_tot;
   P.cr = c->d_cr;
   P.ray = c->d_ray;
-  P.cmp = c->d_cmp;
+  P.shells = c->d_shells;
+  P.n_shells = (int)hsh.size();
+  std::memcpy(P.shell_of, shell_of, sizeof P.shell_of);
   P.num_values = N;
   P.e0 = tab->e0;
   P.ide = tab->ide;
@@ -802,10 +825,10 @@ extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
     if (blocks > need) blocks = std::max(1LL, need);
     // Few streams for the device: deal them thinly. A stream is a serial chain (a decay of a lone
     // lane takes 16 us, 38 us with 64 lanes of its wave in other phases), and the longest streams
-    // come first, so each resident wave (16 per CU) takes one share of them. Above 64 streams per
+    // come first, so each resident wave (20 per CU) takes one share of them. Above 64 streams per
     // wave every lane is needed. 1e5 / 1e6 decays of the 9 x 9 x 9 cube (23 328 streams, three
     // voxels at 100 times the activity): 13.1 / 118 ms with full waves, 6.0 / 60 ms dealt.
-    const long long waves = 16LL * c->num_cus;
+    const long long waves = 20LL * c->num_cus;
     if (P.n_streams > 0 && P.n_streams < 64 * waves && P.stream_stride == 1) {
       P.lanes = (int)((P.n_streams + waves - 1) / waves);
       P.shares = (int)((P.n_streams + P.lanes - 1) / P.lanes);
@@ -1654,7 +1677,7 @@ mcpet_status mcpet_run_contexts(const CtxRun* runs, int n, hipStream_t stream, K
     c->ran = true;
   }
   hipError_t e = hipMemcpyAsync(d_params, h_params, sizeof(KParams) * (size_t)n, hipMemcpyHostToDevice, stream);
-  if (e == hipSuccess) e = mcpet_launch_transport_batch(d_params, n, ext, 0, blocks, block_size, stream);
+  if (e == hipSuccess) e = mcpet_launch_transport_batch(d_params, n, h_params[0].n_shells, ext, 0, blocks, block_size, stream);
   for (int k = 0; k < n && e == hipSuccess; k++) e = hipEventRecord(runs[k].c->ev_done, stream);
   if (e != hipSuccess) return fail(MCPET_E_HIP, std::string("batched launch: ") + hipGetErrorString(e));
   return MCPET_OK;
@@ -1792,7 +1815,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
       mcpet_status st = MCPET_OK;
       for (int k = 0; k < n && st == MCPET_OK; k++) st = clear_buffers(b->ctx[k], b->stream, p.zero_tallies != 0, true);
       hipError_t e = hipSuccess;
-      if (st == MCPET_OK) e = mcpet_launch_transport_batch(b->d_params, n, ext, p.count_events, blocks, bs, b->stream);
+      if (st == MCPET_OK) e = mcpet_launch_transport_batch(b->d_params, n, b->h_params[0].n_shells, ext, p.count_events, blocks, bs, b->stream);
       hipGraph_t g = nullptr;
       hipError_t e2 = hipStreamEndCapture(b->stream, &g);
       if ((st != MCPET_OK || e != hipSuccess || e2 != hipSuccess) && g) (void)hipGraphDestroy(g);
@@ -1812,7 +1835,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
       if (st != MCPET_OK) return st;
     }
     BHIP(b, hipEventRecord(b->ev0, b->stream));
-    hipError_t e = mcpet_launch_transport_batch(b->d_params, n, ext, p.count_events, blocks, bs, b->stream);
+    hipError_t e = mcpet_launch_transport_batch(b->d_params, n, b->h_params[0].n_shells, ext, p.count_events, blocks, bs, b->stream);
     if (e != hipSuccess) return bset_err(b, MCPET_E_HIP, std::string("batch launch failed: ") + hipGetErrorString(e));
     BHIP(b, hipEventRecord(b->ev1, b->stream));
   }

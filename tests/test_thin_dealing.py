@@ -11,8 +11,8 @@ from harness import assert_tallies_equal, water_cube_scenario
     (1, {}),                                          # 729 streams: one lane per wave, fewer waves than resident
     (7, {}),                                          # 5103 streams: two lanes, a short last row
     (7, dict(block_size=64, blocks_per_cu=1)),        # fewer waves than shares: waves come back for more
-    (359, {}),                                        # 261711 streams: 64 lanes, still dealt
-    (360, {}),                                        # 262440 streams: full waves, in queue order
+    (449, {}),                                        # 327321 streams: 64 lanes, still dealt
+    (450, {}),                                        # 328050 streams: full waves, in queue order
 ])
 def test_thinly_dealt_streams_give_the_oracles_tallies(tpb, kw):
     print(f"thin dealing: water cube, tpb {tpb}, {kw}", flush=True)
