@@ -45,12 +45,12 @@
 // corrupt input. The CPU checker applies the same bound.
 #define K_MAX_TRIALS (1 << 20)
 
-// Occupancy target of the persistent transport kernels (waves per SIMD; 0 leaves it to the
-// compiler). They wait on dependent gathers and on chains of dependent operations, so waves pay
-// up to the last one that fits without spilling: 5 (96 VGPRs, 28 KB of LDS per workgroup with
-// the shells and the palette at the phantom's own sizes) against 4: head, 1e8 decays, 31.6 ->
-// 29.0 ms; 4e7 torso decays with singles 38.1 -> 36.3 ms; eight phantoms in one launch 10.75 ->
-// 10.2 ms.
+// Occupancy targets of the persistent transport kernels (waves per SIMD). They wait on dependent
+// gathers and on chains of dependent operations, so waves pay up to the last one that fits: 6 (80
+// VGPRs, one spilled; 26.4 KB of LDS per workgroup with the shells and the palette at the phantom's
+// own sizes) where only sinograms are tallied (head, 1e8 decays, at 4 / 5 / 6 waves: 31.6 / 29.0 /
+// 27.8 ms; eight phantoms in one launch 10.75 / 10.2 / 10.1 ms), 5 (96 VGPRs) with lists or
+// prompt gammas (4e7 torso decays with singles, 4 / 5 / 6 waves: 38.1 / 36.3 / 36.8 ms).
 // Woodcock steps a lane may take in one STEP phase while its steps stay virtual, and GCOa
 // rejection trials (tau loop, p_z loop) in one CTAU / CPZ phase: the phase selection's ballots
 // are paid once for several. 3 and 2 measured best on the head workload (1-4 steps, 1-3
@@ -70,13 +70,12 @@
 #define MCPET_CHAIN 31
 #endif
 #ifndef MCPET_WAVES_PER_EU
-#define MCPET_WAVES_PER_EU 5
+#define MCPET_WAVES_PER_EU 6
 #endif
-#if MCPET_WAVES_PER_EU > 0
-#define K_OCCUPANCY __attribute__((amdgpu_waves_per_eu(MCPET_WAVES_PER_EU, 8)))
-#else
-#define K_OCCUPANCY
+#ifndef MCPET_WAVES_PER_EU_EXT
+#define MCPET_WAVES_PER_EU_EXT 5
 #endif
+#define K_OCCUPANCY(ext) __attribute__((amdgpu_waves_per_eu((ext) ? MCPET_WAVES_PER_EU_EXT : MCPET_WAVES_PER_EU, 8)))
 // Per-phase execution statistics of the persistent kernel (diagnostic builds only).
 #ifndef MCPET_SM_STATS
 #define MCPET_SM_STATS 0
@@ -1123,7 +1122,8 @@ __device__ __forceinline__ void stream_init(const KParams& P, long long s, Strea
     per_voxel = gld(P.stream_start, k + 1) - s0;
     tid = gld(P.stream_id, k) + (s - s0);
   } else {
-    k = (int)(s / P.tpb);
+    k = (int)((double)s * P.inv_tpb);   // s / tpb: exact, or one too small where tpb divides s
+    if ((long long)(k + 1) * P.tpb <= s) k++;
     per_voxel = P.tpb;
     tid = (long long)gld(P.active_vox, k) * P.tpb + (s - (long long)k * P.tpb);
   }
@@ -1132,7 +1132,7 @@ __device__ __forceinline__ void stream_init(const KParams& P, long long s, Strea
   init_stream_seeds(tid, P.seed, P.j1, P.j2, &st.r.x, &st.r.y);
   st.event = (unsigned long long)tid << 32;
   st.remaining = P.acq_ps;
-  st.inv_act = ((double)per_voxel / (double)act);
+  st.inv_act = div_n((double)per_voxel, (double)act);
 }
 
 __device__ __forceinline__ void stream_finish(const KParams& P, const Stream& st)
@@ -1235,11 +1235,12 @@ enum LaneState {
 // Slots whose contents are never needed together share a place: photon 1's direction waits for
 // photon 2's emission where the pair's first hit goes later, and moves to the Compton sampler's
 // slots when photon 1 has ended.
-enum PairSlot { PS_P1 = 0, PS_POSF = 3, PS_DIRF = 6, PS_EF = 9, PS_SSF = 10, PS_TRAVELF = 11, PS_N = 12, PS_D1 = PS_POSF };
+enum PairSlot { PS_P1 = 0, PS_POSF = 3, PS_DIRF = 6, PS_EF = 9, PS_SSF = 10, PS_N = 11, PS_D1 = PS_POSF };
 enum ComptonSlot {
-  CS_A1 = PS_N, CS_S0, CS_TAUMIN, CS_TAU, CS_S, CS_RC0, CS_RC1, CS_RC2, CS_RC3, CS_CDT1_LO, CS_CDT1_HI, CS_TRIALS, LANE_SLOTS,
+  CS_A1 = PS_N, CS_S0, CS_TAUMIN, CS_TAU, CS_S, CS_RC0, CS_RC1, CS_RC2, CS_RC3, CS_CDT1_LO, CS_CDT1_HI, LANE_SLOTS,
   CS_PROB = CS_A1, CS_MFPD, CS_RANDNO,   // a real interaction's inputs until GCOa starts
-  PS_D1_LATER = CS_A1                    // photon 1's direction between the two photons
+  PS_D1_LATER = CS_A1,                   // photon 1's direction between the two photons
+  PS_TRAVELF = LANE_SLOTS, LANE_SLOTS_EXT   // photon 1's path, only where records are listed
 };
 
 struct LaneSlots {
@@ -1259,11 +1260,12 @@ __device__ __forceinline__ void pair_keep_d1(const LaneSlots& L)
 {
   for (int k = 0; k < 3; k++) L[PS_D1_LATER + k] = L[PS_D1 + k];
 }
+template <bool kExt>
 __device__ __forceinline__ void pair_store_first(const LaneSlots& L, const Photon& ph)
 {
   if (ph.index > -1) {   // as keep_first
     L[PS_EF] = ph.E;
-    L[PS_TRAVELF] = ph.travel;
+    if (kExt) L[PS_TRAVELF] = ph.travel;
     L[PS_SSF] = __int_as_float(ph.ss);
     for (int k = 0; k < 3; k++) {
       L[PS_POSF + k] = ph.pos[k];
@@ -1271,6 +1273,7 @@ __device__ __forceinline__ void pair_store_first(const LaneSlots& L, const Photo
     }
   }
 }
+template <bool kExt>
 __device__ __forceinline__ void pair_load(const LaneSlots& L, Pair& pr)
 {
   for (int k = 0; k < 3; k++) {
@@ -1278,7 +1281,7 @@ __device__ __forceinline__ void pair_load(const LaneSlots& L, Pair& pr)
     pr.dirF[k] = L[PS_DIRF + k];
   }
   pr.EF = L[PS_EF];
-  pr.travelF = L[PS_TRAVELF];
+  pr.travelF = kExt ? L[PS_TRAVELF] : 0.0f;
   pr.ssF = __float_as_int(L[PS_SSF]);
 }
 __device__ __forceinline__ void cs_store(const LaneSlots& L, const ComptonState& cs)
@@ -1295,7 +1298,6 @@ __device__ __forceinline__ void cs_store(const LaneSlots& L, const ComptonState&
   const unsigned long long b = (unsigned long long)__double_as_longlong(cs.cdt1);
   L[CS_CDT1_LO] = __uint_as_float((unsigned)b);
   L[CS_CDT1_HI] = __uint_as_float((unsigned)(b >> 32));
-  L[CS_TRIALS] = __int_as_float(cs.trials);
 }
 __device__ __forceinline__ void cs_load(const LaneSlots& L, ComptonState& cs)
 {
@@ -1311,18 +1313,18 @@ __device__ __forceinline__ void cs_load(const LaneSlots& L, ComptonState& cs)
   const unsigned long long b = (unsigned long long)__float_as_uint(L[CS_CDT1_LO]) |
                                ((unsigned long long)__float_as_uint(L[CS_CDT1_HI]) << 32);
   cs.cdt1 = __longlong_as_double((long long)b);
-  cs.trials = __float_as_int(L[CS_TRIALS]);
 }
 
 // Next state once the current photon has escaped or was absorbed (K:418-442). Photons are
 // numbered 1, 2 (annihilation pair) and 3 (prompt gamma); the singles pipeline records every
 // photon in DETECT instead of pairing them here.
+template <bool kExt>
 __device__ __forceinline__ int after_photon(const KParams& P, bool singles, int photon_no, bool prompt, const Photon& ph, const LaneSlots& L)
 {
   if (photon_no == 1) pair_keep_d1(L);
   if (singles) return LS_DETECT;
   if (photon_no == 1) {
-    pair_store_first(L, ph);
+    pair_store_first<kExt>(L, ph);
     return LS_SOURCE2;
   }
   if (photon_no == 2 && ph.index > -1 && L[PS_EF] > -0.5f && pair_selected(P, ph.ss, __float_as_int(L[PS_SSF])))
@@ -1334,19 +1336,21 @@ __device__ __forceinline__ int after_photon(const KParams& P, bool singles, int 
 // and every lane of the wave has finished its stream. kExt: a phase-space file, the singles list
 // or prompt gammas are in use (staged records, phases DETECT and SOURCE3 exist); otherwise the
 // wave only ballots over the seven phases of the sinogram's pair tallies.
-// Streams are claimed from the queue by the wave, K_CHUNK indices per atomic, and handed to
+// Streams are claimed from the queue by the wave, many indices per atomic, and handed to
 // the lanes that need one in lane order; the wave's unused range (next index wq[0], count
 // wq[1]) lives in LDS
 // (a single global counter updated once per stream was the limit of short runs). The range
 // is read by every lane and written by the lowest one; volatile keeps each access an LDS
 // operation in program order, which a wave executes in order. Dealt thinly (shares > 0), the
 // queue counts shares: one atomic claims the streams share, share + shares, ... of `lanes` lanes.
-#define K_CHUNK 64
+// A wave's first chunk (share) is that of its own number, without an atomic (`first` chunks are
+// given out that way; the queue counts the others).
 // Index (from the queue's origin) of the next stream for every calling lane. Not inlined:
 // inlined into the state machine it raised the register pressure of every phase (32 more
 // spilled VGPRs); as a call it costs a few register saves at each claim.
 __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* queue, volatile K_LDS long long* wq, int lanes,
-                                                               int shares)
+                                                               int shares, int first, int chunk0, int chunk_min, int shift,
+                                                               long long n)
 {
   // the lanes here all need a stream: rank among them, claim a new chunk if short
   // (the range is wave-uniform: read into scalar registers)
@@ -1368,15 +1372,17 @@ __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* 
     }
   } else {
     unsigned long long base = 0;
-    if (rank == 0) base = gatomic_add(queue, shares ? 1ull : (unsigned long long)K_CHUNK);
+    // a part of the rest as far as this wave knows it (from its last claim)
+    const int more = shares ? lanes : max(cnt - avail, (int)min(512ll, max((long long)chunk_min, (n - qn) >> shift)));
+    if (rank == 0) base = gatomic_add(queue, shares ? 1ull : (unsigned long long)more);
     const unsigned blo = __builtin_amdgcn_readfirstlane((unsigned)base);
     const unsigned bhi = __builtin_amdgcn_readfirstlane((unsigned)(base >> 32));
-    long long b = (long long)(((unsigned long long)bhi << 32) | blo);
+    long long b = (long long)(((unsigned long long)bhi << 32) | blo) + (long long)first * chunk0;
     if (shares && b >= shares) b = 1ll << 62;   // no share is left
     idx = rank < avail ? qn + rank * step : b + (rank - avail) * step;
     if (rank == 0) {
       wq[0] = b + (cnt - avail) * step;
-      wq[1] = lanes - (cnt - avail);
+      wq[1] = more - (cnt - avail);
     }
   }
   return idx;
@@ -1384,12 +1390,14 @@ __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* 
 
 template <class CN, bool kExt>
 __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& s_cmp, int* s_spec,
-                                         unsigned long long* s_mat, const LaneSlots& L, volatile K_LDS long long* wq)
+                                         unsigned long long* s_mat, const LaneSlots& L, volatile K_LDS long long* wq, int wave = 0,
+                                         int first = 0)
 {
   constexpr int kPhases = kExt ? LS_N : LS_CPZ + 1;
   if (__lane_id() == 0) {
-    wq[0] = 0;
-    wq[1] = 0;
+    // the wave's own first chunk, where chunks are given out that way
+    wq[0] = first ? (long long)wave * P.chunk0 : 0;
+    wq[1] = first ? P.chunk0 : 0;
     wq[2] = 0;
   }
   __builtin_amdgcn_wave_barrier();
@@ -1400,6 +1408,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
   bool have = false;
   bool prompt = false;           // the current decay still has its prompt gamma to emit
   int photon_no = 1;
+  int trials = 0;                // of the current GCOa loop
   int state = (int)__lane_id() < P.lanes ? LS_DECAY : LS_DONE;
   for (;;) {
     int best = -1;
@@ -1459,9 +1468,10 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
       const int o = interaction_begin(P, ph, st.r, C, s_cmp, cs, s_mat);
       if (o == IA_COMPTON) {
         cs_store(L, cs);
+        trials = 0;
         state = LS_CTAU;
       } else if (o == IA_ABSORBED) {
-        state = after_photon(P, singles, photon_no, prompt, ph, L);
+        state = after_photon<kExt>(P, singles, photon_no, prompt, ph, L);
       } else {
         state = LS_STEP;
       }
@@ -1470,13 +1480,15 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
     if (run_tau && state == LS_CTAU) {
       ComptonState cs;
       cs_load(L, cs);
+      cs.trials = trials;
       bool ok;
       int k = 0;
       do {
         ok = gcoa_tau_trial(ph.E, ph.mat0, st.r, C, s_cmp, cs);
       } while (!ok && ++k < MCPET_TRIALS_PER_PHASE);
+      trials = cs.trials;
       if (ok) {
-        cs.trials = 0;
+        trials = 0;
         state = LS_CPZ;
       }
       cs_store(L, cs);
@@ -1485,6 +1497,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
     if (run_pz && state == LS_CPZ) {
       ComptonState cs;
       cs_load(L, cs);
+      cs.trials = trials;
       bool ok;
       int k = 0;
       do {
@@ -1492,16 +1505,16 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
       } while (!ok && ++k < MCPET_TRIALS_PER_PHASE);
       if (ok) {
         // (the photon is where its last step found it inside the box)
-        if (!compton_end(P, ph, st.r, C, cs, s_mat)) state = after_photon(P, singles, photon_no, prompt, ph, L);
+        if (!compton_end(P, ph, st.r, C, cs, s_mat)) state = after_photon<kExt>(P, singles, photon_no, prompt, ph, L);
         else state = LS_STEP;
       } else {
-        L[CS_TRIALS] = __int_as_float(cs.trials);
+        trials = cs.trials;
       }
     }
     const bool run_tally = best == LS_TALLY;
     if (run_tally && state == LS_TALLY) {
       Pair pr;
-      pair_load(L, pr);
+      pair_load<kExt>(L, pr);
       tally_pair<CN, kExt>(P, ph, pr, st, C, s_spec, stage, wq);
       state = prompt ? LS_SOURCE3 : LS_DECAY;
     }
@@ -1509,7 +1522,8 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
     if (run_decay && state == LS_DECAY) {
       for (;;) {
         if (!have) {
-          const long long idx = claim_stream(P.queue, wq, P.lanes, P.shares);
+          const long long idx = claim_stream(P.queue, wq, P.lanes, P.shares, first, P.chunk0, P.chunk_min, P.chunk_shift,
+                                             P.n_claims);
           const long long sid = P.stream_base + (P.stream_stride > 1 ? idx * P.stream_stride : idx);
           if (sid >= P.n_streams) {
             state = LS_DONE;
@@ -1542,7 +1556,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
           }
           photon_start(P, ph);
           photon_no = 1;
-          state = (locate(P, ph.pos) < 0) ? after_photon(P, singles, 1, prompt, ph, L) : LS_STEP;
+          state = (locate(P, ph.pos) < 0) ? after_photon<kExt>(P, singles, 1, prompt, ph, L) : LS_STEP;
         } else {
           state = prompt ? LS_SOURCE3 : LS_DECAY;
         }
@@ -1559,7 +1573,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
       for (int k = 0; k < 3; k++) ph.pos[k] = p1[k];
       photon_start(P, ph);
       photon_no = 2;
-      state = (locate(P, ph.pos) < 0) ? after_photon(P, singles, 2, prompt, ph, L) : LS_STEP;
+      state = (locate(P, ph.pos) < 0) ? after_photon<kExt>(P, singles, 2, prompt, ph, L) : LS_STEP;
     }
     const bool run_det = kExt && best == LS_DETECT;
     if (run_det && state == LS_DETECT) {
@@ -1573,7 +1587,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
       photon_start(P, ph, P.prompt_energy);
       photon_no = 3;
       prompt = false;
-      state = (locate(P, ph.pos) < 0) ? after_photon(P, singles, 3, false, ph, L) : LS_STEP;
+      state = (locate(P, ph.pos) < 0) ? after_photon<kExt>(P, singles, 3, false, ph, L) : LS_STEP;
     }
     const bool run_step = best == LS_STEP || ((MCPET_CHAIN & 4) && run_pz) ||
                           ((MCPET_CHAIN & 8) && (run_decay || run_src2 || run_src3));
@@ -1584,7 +1598,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
         o = woodcock_step(S, s_cmp.pal, ph, st.r, C);
       } while (o == STEP_VIRTUAL && ++k < MCPET_STEPS_PER_PHASE);
       if (o == STEP_ESCAPED) {
-        state = after_photon(P, singles, photon_no, prompt, ph, L);
+        state = after_photon<kExt>(P, singles, photon_no, prompt, ph, L);
       } else if (o == STEP_REAL) {
         // the interaction's inputs wait in LDS (Compton slots, free until GCOa starts)
         L[CS_PROB] = ph.prob;
@@ -1604,14 +1618,16 @@ template <class CN, bool kExt>
 // Parameters are read through a pointer to device memory: only the fields a phase uses are
 // loaded (as scalars), instead of a by-value block that would be kept in scalar registers
 // (and spilled) or copied to private memory.
-__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_sm(const KParams* __restrict__ Pd)
+__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_sm(const KParams* __restrict__ Pd)
 {
   const KParams& P = *Pd;
   K_PROLOGUE(CN)
-  __shared__ float s_slots[LANE_SLOTS][K_BLOCK];
+  __shared__ float s_slots[kExt ? LANE_SLOTS_EXT : LANE_SLOTS][K_BLOCK];
   __shared__ long long s_wq[K_BLOCK / 64][3];
   const LaneSlots L{&s_slots[0][threadIdx.x]};
-  sm_waves<CN, kExt>(P, C, s_cmp, s_spec, s_mat, L, (volatile K_LDS long long*)s_wq[threadIdx.x >> 6]);
+  const int waves = (int)(blockDim.x >> 6), wave = (int)(threadIdx.x >> 6);
+  sm_waves<CN, kExt>(P, C, s_cmp, s_spec, s_mat, L, (volatile K_LDS long long*)s_wq[wave], (int)blockIdx.x * waves + wave,
+                     P.chunk0 ? (int)gridDim.x * waves : 0);
   K_EPILOGUE
 }
 
@@ -1626,13 +1642,13 @@ __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_sm(const KPar
 // memory (both are per phantom). Per phantom, streams and random numbers are those of a
 // single-phantom run, so each phantom's tallies equal its own run's bit for bit.
 template <class CN, bool kExt>
-__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_batch(const KParams* __restrict__ Ps, int n)
+__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_batch(const KParams* __restrict__ Ps, int n)
 {
   __shared__ unsigned s_shell_of[K_MAXMAT];
   extern __shared__ v4f s_dyn[];
   __shared__ unsigned long long s_matw[K_BLOCK / 64][2 * K_MAXMAT];
   __shared__ unsigned s_cntw[K_BLOCK / 64][KC_N];
-  __shared__ float s_slots[LANE_SLOTS][K_BLOCK];
+  __shared__ float s_slots[kExt ? LANE_SLOTS_EXT : LANE_SLOTS][K_BLOCK];
   __shared__ long long s_wq[K_BLOCK / 64][3];
   {
     for (int i = threadIdx.x; i < Ps[0].n_shells; i += blockDim.x) {
@@ -1754,6 +1770,17 @@ size_t mcpet_transport_dyn_lds(const KParams& P)
 {
   return 16 * (size_t)P.n_shells + (P.vox_fmt == 1 && P.lds_palette ? 8 * (size_t)P.n_palette : 0) +
          (P.lds_spectrum ? 4 * (size_t)P.ne : 0);
+}
+
+// Workgroups of the persistent kernel that a CU holds at once.
+int mcpet_transport_resident(const KParams& P, int count_events, int block_size)
+{
+  const bool ext = P.mode != 2 || P.prompt_frac > 0.0f;
+  const void* f = count_events ? (ext ? (const void*)k_transport_sm<FullCounters, true> : (const void*)k_transport_sm<FullCounters, false>)
+                               : (ext ? (const void*)k_transport_sm<LiteCounters, true> : (const void*)k_transport_sm<LiteCounters, false>);
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, block_size, mcpet_transport_dyn_lds(P)) != hipSuccess || n < 1) return 1;
+  return n;
 }
 
 hipError_t mcpet_launch_transport(const KParams& P, const KParams* d_P, int kind, int count_events, int blocks, int block_size,

@@ -78,12 +78,17 @@ struct KParams : StepParams {
   long long n_streams;           // streams [stream_base, n_streams) are simulated by a launch
   long long stream_base;
   int tpb;
+  double inv_tpb;              // 1 / tpb
   unsigned long long* queue;   // persistent kernel: next stream index
   // persistent kernel: lanes of each wave that run streams, and, where streams are dealt thinly
   // (few streams for the device), the number of shares they are dealt to: share k is the streams
   // k, k + shares, ... of one wave's lanes, so that neighbouring (equally long) streams go to
   // different waves. shares 0: 64 lanes, streams in queue order.
   int lanes, shares;
+  // streams of a wave's first claim, taken by its number (0: every claim goes through the queue);
+  // later claims: the rest of the queue >> shift
+  int chunk0, chunk_min, chunk_shift;
+  long long n_claims;          // indices of the queue
   // source
   int seed;
   int bg_mode;
@@ -157,6 +162,7 @@ struct KParams : StepParams {
 // Launchers implemented in kernels.hip.
 hipError_t mcpet_launch_transport(const KParams& P, const KParams* d_P, int kind, int count_events, int blocks, int block_size,
                                   hipStream_t stream);
+int mcpet_transport_resident(const KParams& P, int count_events, int block_size);
 // dynamic LDS of a single-phantom launch (bytes)
 size_t mcpet_transport_dyn_lds(const KParams& P);
 hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, int n_shells, bool ext, int count_events, int blocks,

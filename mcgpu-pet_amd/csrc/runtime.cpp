@@ -34,6 +34,7 @@ struct mcpet_ctx {
   int nx = 0, ny = 0, nz = 0;
   long long nvox = 0;
   long long n_active = 0;
+  double expected_rate = 0.0;    // decays per second at the start: the sum of the activities
   long long n_roi = 0;
   KParams P{};
   // device allocations
@@ -304,11 +305,12 @@ static int stream_hints(const std::vector<long long>& start, std::vector<int>& h
   return g;
 }
 
-static double effective_time(const mcpet_config* cfg)
+static double effective_seconds(float mean_life, uint64_t acquisition_ps)
 {
-  const double tau = (double)cfg->mean_life, T = (double)cfg->acquisition_time_ps * 1.0e-12;
+  const double tau = (double)mean_life, T = (double)acquisition_ps * 1.0e-12;
   return tau * (1.0 - std::exp(-T / tau));
 }
+static double effective_time(const mcpet_config* cfg) { return effective_seconds(cfg->mean_life, cfg->acquisition_time_ps); }
 
 extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phantom* ph, const mcpet_tables* tab, mcpet_ctx** out)
 {
@@ -467,6 +469,7 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   std::vector<float> act_val(act_idx.size());
   for (size_t i = 0; i < act_idx.size(); i++) act_val[i] = ph->voxel_mat_dens[3 * (size_t)act_idx[i] + 2];
   c->n_active = (long long)act_idx.size();
+  for (float a : act_val) c->expected_rate += (double)a;
   // Balanced stream layout: voxel v gets max(1, ceil(E_v / stream_decays)) streams (E_v: its
   // expected decays over the acquisition); random-number stream ids count the streams in voxel
   // order, the device processes the voxels hottest first.
@@ -652,6 +655,7 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
   P.active_vox = c->d_active_vox;
   P.active_act = c->d_active_act;
   P.tpb = cfg->threads_per_block;
+  P.inv_tpb = 1.0 / (double)P.tpb;
   P.stream_start = c->d_stream_start;
   P.stream_id = c->d_stream_id;
   P.stream_hint = c->d_stream_hint;
@@ -770,6 +774,24 @@ static mcpet_status clear_buffers(mcpet_ctx* c, hipStream_t stream, bool tallies
   return MCPET_OK;
 }
 
+// How the waves of a launch claim streams from the queue: an eighth of their part of the rest at
+// a time (a wave knows the queue's position from its last claim, so half of it, 512 streams at
+// once, left the last waves too much: head, 1e8 decays, 27.7 -> 33.2 ms), down to chunks worth
+// about 64 decays, since a claim costs the device about 6 ns and one address serves them all:
+// 16-64 streams. own: the first claim is the wave's by its number, without an atomic (only if
+// every wave is resident from the start). 5e6 decays at 4 a stream: fixed chunks of 64, 1.79 ms,
+// now 1.62; 4e7 torso decays 36.4 -> 33.8 ms.
+static void set_claims(KParams& P, double expected_decays, long long n_waves, bool own)
+{
+  P.n_claims = std::max(0LL, (P.n_streams - P.stream_base + P.stream_stride - 1) / std::max(1LL, P.stream_stride));
+  int shift = 1;
+  while (shift < 40 && (1LL << shift) < 8 * n_waves) shift++;
+  P.chunk_shift = shift;
+  const double per_stream = expected_decays / (double)std::max(1LL, P.n_streams);
+  P.chunk_min = per_stream >= 4.0 ? 16 : per_stream >= 2.0 ? 32 : 64;
+  P.chunk0 = own && !P.shares ? (int)std::min(512LL, std::max(1LL, P.n_claims >> shift)) : 0;
+}
+
 extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
 {
   if (!c) return set_err(nullptr, MCPET_E_ARG, "mcpet_run: null context");
@@ -819,21 +841,29 @@ extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
   HIPCHK(c, hipEventRecord(c->ev_k0, c->stream));
   long long blocks;
   if (kind == MCPET_KERNEL_PERSISTENT) {
-    int per_cu = p.blocks_per_cu > 0 ? p.blocks_per_cu : 8;
+    const int resident = mcpet_transport_resident(P, p.count_events, bs);
+    // Short runs end with lanes waiting for the last streams, the longer the more lanes share the
+    // device: about 16 decays a lane, from four workgroups per CU up (4e6 decays: 6 / 5 / 4
+    // workgroups 1.10 / 1.04 / 1.00 ms, 5e6: 1.67 / 1.62 / 1.66 ms; 2e7: 6 are best).
+    const double decays = c->expected_rate * effective_seconds(c->cfg.mean_life, P.acq_ps);
+    const int wanted = (int)std::min((double)resident, std::ceil(decays / (16.0 * c->num_cus * bs)));
+    const int per_cu = p.blocks_per_cu > 0 ? p.blocks_per_cu : std::min(resident, std::max(4, wanted));
     blocks = (long long)c->num_cus * per_cu;
     long long need = (P.n_streams + bs - 1) / bs;
     if (blocks > need) blocks = std::max(1LL, need);
     // Few streams for the device: deal them thinly. A stream is a serial chain (a decay of a lone
-    // lane takes 16 us, 38 us with 64 lanes of its wave in other phases), and the longest streams
-    // come first, so each resident wave (20 per CU) takes one share of them. Above 64 streams per
-    // wave every lane is needed. 1e5 / 1e6 decays of the 9 x 9 x 9 cube (23 328 streams, three
-    // voxels at 100 times the activity): 13.1 / 118 ms with full waves, 6.0 / 60 ms dealt.
-    const long long waves = 20LL * c->num_cus;
+    // lane took 16 us, 38 us with 64 lanes of its wave in other phases), and the longest streams
+    // come first, so each resident wave takes one share of them. Above 64 streams per wave every
+    // lane is needed. 1e5 / 1e6 decays of the 9 x 9 x 9 cube (23 328 streams, three voxels at 100
+    // times the activity): 13.1 / 118 ms with full waves, 6.0 / 60 ms dealt.
+    const long long full = (long long)c->num_cus * (p.blocks_per_cu > 0 ? p.blocks_per_cu : resident), waves = full * (bs / 64);
     if (P.n_streams > 0 && P.n_streams < 64 * waves && P.stream_stride == 1) {
       P.lanes = (int)((P.n_streams + waves - 1) / waves);
       P.shares = (int)((P.n_streams + P.lanes - 1) / P.lanes);
-      blocks = std::min((long long)c->num_cus * per_cu, (P.shares + bs / 64 - 1LL) / (bs / 64));
+      blocks = std::min(full, (P.shares + bs / 64 - 1LL) / (bs / 64));
     }
+    const long long n_waves = blocks * (bs / 64);
+    set_claims(P, decays, n_waves, blocks <= (long long)c->num_cus * resident);
   } else {
     blocks = std::max(1LL, (P.n_streams + bs - 1) / bs);
     if (blocks > 0x7fffffffLL) return set_err(c, MCPET_E_RANGE, "mcpet_run: too many streams for one launch");
@@ -1667,6 +1697,8 @@ mcpet_status mcpet_run_contexts(const CtxRun* runs, int n, hipStream_t stream, K
     P.sm_policy = 0;
     P.lds_spectrum = 0;
     P.lds_palette = 0;
+    set_claims(P, c->expected_rate * effective_seconds(c->cfg.mean_life, P.acq_ps) * (double)(P.n_streams - P.stream_base) /
+                      (double)std::max(1LL, c->P.n_streams), (long long)blocks * (block_size / 64), false);
     ext = ext || P.prompt_frac > 0.0f || P.mode != 2;
     h_params[k] = P;
     c->rbt_ran = P.rb_trues != nullptr && (runs[k].clear != 0 || c->rbt_ran);
@@ -1803,6 +1835,11 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
   if (bs % 64 != 0 || bs > 256) return bset_err(b, MCPET_E_RANGE, "mcpet_batch_run: block_size must be a multiple of 64, <= 256");
   const int per_cu = p.blocks_per_cu > 0 ? p.blocks_per_cu : (b->tuned_per_cu > 0 ? b->tuned_per_cu : 8);
   const int blocks = b->num_cus * per_cu;
+  for (int k = 0; k < n; k++) {
+    const mcpet_ctx* c = b->ctx[k];
+    set_claims(b->h_params[k], c->expected_rate * effective_seconds(c->cfg.mean_life, b->h_params[k].acq_ps), (long long)blocks * (bs / 64),
+               false);
+  }
   BHIP(b, hipMemcpyAsync(b->d_params, b->h_params, sizeof(KParams) * (size_t)n, hipMemcpyHostToDevice, b->stream));
   if (p.use_graph) {
     const int key[3] = {bs, blocks, p.count_events ? 1 : 0};

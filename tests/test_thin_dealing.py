@@ -9,10 +9,11 @@ from harness import assert_tallies_equal, water_cube_scenario
 @pytest.mark.gpu
 @pytest.mark.parametrize("tpb,kw", [
     (1, {}),                                          # 729 streams: one lane per wave, fewer waves than resident
-    (7, {}),                                          # 5103 streams: two lanes, a short last row
-    (7, dict(block_size=64, blocks_per_cu=1)),        # fewer waves than shares: waves come back for more
-    (449, {}),                                        # 327321 streams: 64 lanes, still dealt
-    (450, {}),                                        # 328050 streams: full waves, in queue order
+    (9, {}),                                          # 6561 streams: two lanes, a short last row
+    (7, dict(block_size=64, blocks_per_cu=1)),        # 5103 streams on 256 waves: 20 lanes
+    (539, {}),                                        # 392931 streams: 64 lanes, still dealt
+    (540, {}),                                        # 393660 streams: full waves, in queue order
+    (540, dict(blocks_per_cu=12)),                    # more waves than are resident: no chunk by number
 ])
 def test_thinly_dealt_streams_give_the_oracles_tallies(tpb, kw):
     print(f"thin dealing: water cube, tpb {tpb}, {kw}", flush=True)
