@@ -1377,7 +1377,7 @@ __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* 
     if (rank == 0) base = gatomic_add(queue, shares ? 1ull : (unsigned long long)more);
     const unsigned blo = __builtin_amdgcn_readfirstlane((unsigned)base);
     const unsigned bhi = __builtin_amdgcn_readfirstlane((unsigned)(base >> 32));
-    long long b = (long long)(((unsigned long long)bhi << 32) | blo) + (long long)first * chunk0;
+    long long b = (long long)(((unsigned long long)bhi << 32) | blo) + (long long)first * (shares ? 1 : chunk0);
     if (shares && b >= shares) b = 1ll << 62;   // no share is left
     idx = rank < avail ? qn + rank * step : b + (rank - avail) * step;
     if (rank == 0) {
@@ -1396,8 +1396,16 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
   constexpr int kPhases = kExt ? LS_N : LS_CPZ + 1;
   if (__lane_id() == 0) {
     // the wave's own first chunk, where chunks are given out that way
-    wq[0] = first ? (long long)wave * P.chunk0 : 0;
-    wq[1] = first ? P.chunk0 : 0;
+    // (dealt thinly: the first share; the waves of one workgroup take shares far apart, so that the
+    // longest streams run on different CUs)
+    if (first && P.shares) {
+      const int share = (wave % (int)(blockDim.x >> 6)) * (int)gridDim.x + (int)blockIdx.x;
+      wq[0] = share < P.shares ? (long long)share : 1ll << 62;
+      wq[1] = P.lanes;
+    } else {
+      wq[0] = first ? (long long)wave * P.chunk0 : 0;
+      wq[1] = first ? P.chunk0 : 0;
+    }
     wq[2] = 0;
   }
   __builtin_amdgcn_wave_barrier();

@@ -789,7 +789,7 @@ static void set_claims(KParams& P, double expected_decays, long long n_waves, bo
   P.chunk_shift = shift;
   const double per_stream = expected_decays / (double)std::max(1LL, P.n_streams);
   P.chunk_min = per_stream >= 4.0 ? 16 : per_stream >= 2.0 ? 32 : 64;
-  P.chunk0 = own && !P.shares ? (int)std::min(512LL, std::max(1LL, P.n_claims >> shift)) : 0;
+  P.chunk0 = own ? (int)std::min(512LL, std::max(1LL, P.n_claims >> shift)) : 0;
 }
 
 extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
