@@ -108,15 +108,13 @@ hipError_t gemm(AOp A, BOp B, float* C, int M, int N, int K, int ldc, const floa
 //   FWD   : Y[co][p]        = act(sum_k Wf[co][k] X[c][s p + d_t] + b[co])    m = co, n = output voxel
 //   BDATA : dX[ci][p]      (+)= mask(sum_k Wb[ci][k] dY[c][q], s q + d_t = p)  m = ci, n = input voxel
 //   BWGT  : G[co][ci T + t] += sum_q dY[co][q] X[ci][s q + d_t]              m = co, n = t Cin + ci, k = q
-// Wf, Wb: BF16 copies of the FP32 weights in those layouts (zero padded). FWD and BDATA read
-// their B tensor from a channels-last BF16 copy ([voxel][Cp], padding zero), so a lane's 8
-// channels are one 16-byte load; their epilogues write such copies of what they produce (for
-// the next product) beside the FP32 channel-first tensor (which BWGT, the bias gradients and
-// the ReLU masks read). A workgroup is four waves on one 16 MT x 16 output tile that split the
-// k-steps between them and reduce through LDS; BWGT also splits its (voxel) reduction over
-// workgroups and adds with atomics.
+// Wf, Wb: BF16 copies of the FP32 weights in those layouts (zero padded, in MFMA fragment order). FWD
+// and BDATA read their B tensor from a channels-last BF16 copy ([voxel][Cp], padding zero), so a
+// lane's 8 channels are one 16-byte load; their epilogues write such copies of what they produce
+// (for the next product) beside the FP32 channel-first tensor (which BWGT, the bias gradients and
+// the ReLU masks read). BWGT splits its (voxel) reduction over workgroups.
 
-enum { FWD = 0, BDATA = 1, BWGT = 2 };
+enum { FWD = 0, BDATA = 1 };
 
 // Where an epilogue writes a channels-last BF16 copy of its output: element (m, n) at
 // p[n * ld + off + m] (p null: no copy).
@@ -126,7 +124,7 @@ struct ClOut {
 };
 
 struct ConvK {
-  const __bf16* A;     // FWD, BDATA: BF16 weights [rows][Kp]
+  const __bf16* A;     // FWD, BDATA: BF16 weights [Kp / 32][nrb][64 lanes][8] (k_derive)
   const float* Ad;     // BWGT: dY [M][K]
   const float* X;      // BWGT: input activations [Cin][D][H][W]
   const __bf16* Xl;    // FWD: input activations [D][H][W][Cbp]; BDATA: dY [oD][oH][oW][Cbp] (channels-last BF16)
@@ -135,7 +133,8 @@ struct ConvK {
   const float* bias;   // FWD
   const float* mask;   // BDATA: the layer input (gradient zero where it is <= 0: the ReLU before it); may be null
   int relu, beta;      // FWD: ReLU on the output; BDATA: add to C
-  int M, N, K, Kp;     // GEMM sizes; Kp: row length of A
+  int M, N, K, Kp;     // GEMM sizes; Kp: K padded to whole k-steps
+  int nrb;             // 16-row blocks of A
   int Cb, Cbp;         // channels of the B tensor (FWD, BWGT: Cin; BDATA: Cout) and Cb rounded up to 8
   int D, H, W, oD, oH, oW, ks, stride, T;
   int k_per_split;     // BWGT: voxels per workgroup
@@ -153,22 +152,10 @@ __device__ __forceinline__ void tap3(int t, int ks, int& dz, int& dy, int& dx)
   }
 }
 
-// q with s q + d = p (stride 1 or 2); false if none
-__device__ __forceinline__ bool src_of(int p, int d, int s, int n, int& q)
-{
-  const int v = p - d;
-  if (v < 0) return false;
-  if (s == 2) {
-    if (v & 1) return false;
-    q = v >> 1;
-  } else {
-    q = v;
-  }
-  return q < n;
-}
-
-template <int MODE, int MT>
-__global__ __launch_bounds__(256) void k_conv(ConvK a)
+// Weight-gradient product of the layers without the tiled form: four waves split a slab of voxels
+// (the K range of the workgroup) and reduce through LDS, workgroups add with atomics.
+template <int MT>
+__global__ __launch_bounds__(256) void k_conv_bwgt(ConvK a)
 {
   __shared__ floatx4 red[4][MT][64];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -176,299 +163,297 @@ __global__ __launch_bounds__(256) void k_conv(ConvK a)
   const int m0 = blockIdx.y * (16 * MT);
   const int n = blockIdx.x * 16 + r;                 // this lane's B column
   const bool nvalid = n < a.N;
-  const size_t vin = (size_t)a.D * a.H * a.W, vout = (size_t)a.oD * a.oH * a.oW;
+  const size_t vin = (size_t)a.D * a.H * a.W;
   floatx4 acc[MT];
 #pragma unroll
   for (int i = 0; i < MT; i++) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-  // per-lane column coordinates
-  int cz = 0, cy = 0, cx = 0, bt = 0, bci = 0;
-  if (MODE == FWD) {
-    cx = n % a.oW;
-    cy = (n / a.oW) % a.oH;
-    cz = n / (a.oW * a.oH);
-  } else if (MODE == BDATA) {
-    cx = n % a.W;
-    cy = (n / a.W) % a.H;
-    cz = n / (a.W * a.H);
-  } else {
-    bt = n / a.Cb;
-    bci = n - bt * a.Cb;
-  }
-  int kb = 0, ke = a.K;
-  if (MODE == BWGT) {
-    kb = blockIdx.z * a.k_per_split;
-    ke = min(a.K, kb + a.k_per_split);
-  }
-  if constexpr (MODE == FWD || MODE == BDATA) {
-    // The lane's k = k0 + 8 kg advances by 128 per step: its tap t and channel c0 (k = t Cbp +
-    // c0) are carried forward (one division before the loop), the tap's offsets come from two
-    // multiplications (exact for t < 27: t / 9 = (7282 t) >> 16, t / 3 = (21846 t) >> 16), the
-    // voxel index is 32-bit and the weight rows' addresses are fixed.
-    const int Cbp = a.Cbp, dt = 128 / Cbp, dc = 128 - dt * Cbp;
-    int k = wave * 32 + kg * 8;
-    int t = k / Cbp, c0 = k - t * Cbp;
-    const __bf16* arow[MT];
-#pragma unroll
-    for (int i = 0; i < MT; i++) arow[i] = a.A + (size_t)(m0 + 16 * i + r) * a.Kp;
-    bf16x8 zero;
-#pragma unroll
-    for (int e = 0; e < 8; e++) zero[e] = to_bf16(0.0f);
-    for (int k0 = wave * 32; k0 < ke; k0 += 128, k += 128) {
-      int dz = -1, dy = -1, dx = -1;   // kernel size 1: tap 0, no offset
-      if (a.ks == 3) {
-        const int q9 = (t * 7282) >> 16, q3 = (t * 21846) >> 16;
-        dz += q9;
-        dy += q3 - 3 * q9;
-        dx += t - 3 * q3;
-      } else {
-        dz = dy = dx = 0;
-      }
-      bool in = nvalid && k < ke;
-      int vox = 0;
-      if (MODE == FWD) {
-        const int z = cz * a.stride + dz, y = cy * a.stride + dy, x = cx * a.stride + dx;
-        in = in && z >= 0 && y >= 0 && x >= 0 && z < a.D && y < a.H && x < a.W;
-        vox = (z * a.H + y) * a.W + x;
-      } else {
-        int qz = 0, qy = 0, qx = 0;
-        in = in && src_of(cz, dz, a.stride, a.oD, qz) && src_of(cy, dy, a.stride, a.oH, qy) && src_of(cx, dx, a.stride, a.oW, qx);
-        vox = (qz * a.oH + qy) * a.oW + qx;
-      }
-      bf16x8 b = zero;
-      if (in) b = *(const bf16x8*)(a.Xl + (size_t)vox * Cbp + c0);
-#pragma unroll
-      for (int i = 0; i < MT; i++) {
-        const bf16x8 av = *(const bf16x8*)(arow[i] + k);
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b, acc[i], 0, 0, 0);
-      }
-      c0 += dc;
-      t += dt;
-      if (c0 >= Cbp) {
-        c0 -= Cbp;
-        t++;
-      }
-    }
-  } else
+  const int bt = n / a.Cb, bci = n - bt * a.Cb;
+  const int kb = blockIdx.z * a.k_per_split, ke = min(a.K, kb + a.k_per_split);
   for (int k0 = kb + wave * 32; k0 < ke; k0 += 128) {
     const int k = k0 + kg * 8;
     bf16x8 b;
-    {
-      // B: X[ci][s q + d_t] for q = k .. k + 7
-      int dz, dy, dx;
-      tap3(bt, a.ks, dz, dy, dx);
-      int ox = k % a.oW, oy = (k / a.oW) % a.oH, oz = k / (a.oW * a.oH);
-      const float* xc = a.X + (size_t)bci * vin;
+    // B: X[ci][s q + d_t] for q = k .. k + 7
+    int dz, dy, dx;
+    tap3(bt, a.ks, dz, dy, dx);
+    int ox = k % a.oW, oy = (k / a.oW) % a.oH, oz = k / (a.oW * a.oH);
+    const float* xc = a.X + (size_t)bci * vin;
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int z = oz * a.stride + dz, y = oy * a.stride + dy, x = ox * a.stride + dx;
-        const bool in = nvalid && k + e < ke && z >= 0 && y >= 0 && x >= 0 && z < a.D && y < a.H && x < a.W;
-        b[e] = to_bf16(in ? xc[((size_t)z * a.H + y) * a.W + x] : 0.0f);
-        if (++ox == a.oW) {
-          ox = 0;
-          if (++oy == a.oH) {
-            oy = 0;
-            ++oz;
-          }
+    for (int e = 0; e < 8; e++) {
+      const int z = oz * a.stride + dz, y = oy * a.stride + dy, x = ox * a.stride + dx;
+      const bool in = nvalid && k + e < ke && z >= 0 && y >= 0 && x >= 0 && z < a.D && y < a.H && x < a.W;
+      b[e] = to_bf16(in ? xc[((size_t)z * a.H + y) * a.W + x] : 0.0f);
+      if (++ox == a.oW) {
+        ox = 0;
+        if (++oy == a.oH) {
+          oy = 0;
+          ++oz;
         }
       }
+    }
 #pragma unroll
-      for (int i = 0; i < MT; i++) {
-        const int m = m0 + 16 * i + r;
-        bf16x8 av;
-        if (m < a.M && a.vec && k + 8 <= ke) {
-          const float4* p4 = (const float4*)(a.Ad + (size_t)m * a.K + k);
-          const float4 u = p4[0], w = p4[1];
-          av[0] = to_bf16(u.x); av[1] = to_bf16(u.y); av[2] = to_bf16(u.z); av[3] = to_bf16(u.w);
-          av[4] = to_bf16(w.x); av[5] = to_bf16(w.y); av[6] = to_bf16(w.z); av[7] = to_bf16(w.w);
-        } else {
+    for (int i = 0; i < MT; i++) {
+      const int m = m0 + 16 * i + r;
+      bf16x8 av;
+      if (m < a.M && a.vec && k + 8 <= ke) {
+        const float4* p4 = (const float4*)(a.Ad + (size_t)m * a.K + k);
+        const float4 u = p4[0], w = p4[1];
+        av[0] = to_bf16(u.x); av[1] = to_bf16(u.y); av[2] = to_bf16(u.z); av[3] = to_bf16(u.w);
+        av[4] = to_bf16(w.x); av[5] = to_bf16(w.y); av[6] = to_bf16(w.z); av[7] = to_bf16(w.w);
+      } else {
 #pragma unroll
-          for (int e = 0; e < 8; e++) av[e] = to_bf16((m < a.M && k + e < ke) ? a.Ad[(size_t)m * a.K + k + e] : 0.0f);
-        }
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b, acc[i], 0, 0, 0);
+        for (int e = 0; e < 8; e++) av[e] = to_bf16((m < a.M && k + e < ke) ? a.Ad[(size_t)m * a.K + k + e] : 0.0f);
       }
+      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b, acc[i], 0, 0, 0);
     }
   }
 #pragma unroll
   for (int i = 0; i < MT; i++) red[wave][i][lane] = acc[i];
   __syncthreads();
-  // epilogue: wave w finishes the row blocks i = w, w + 4, ...
-  for (int i = wave; i < MT; i += 4) {
+  for (int i = wave; i < MT; i += 4) {   // wave w finishes the row blocks w, w + 4, ...
     const floatx4 s = red[0][i][lane] + red[1][i][lane] + red[2][i][lane] + red[3][i][lane];
     const int row0 = m0 + 16 * i + kg * 4;   // this lane's four rows row0 .. row0 + 3
     if (!nvalid) continue;
-    if (MODE == FWD || MODE == BDATA) {
-      float ov[4];
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int row = row0 + v;
-        ov[v] = 0.0f;
-        if (row >= a.M) continue;
-        const size_t idx = (size_t)row * a.N + n;
-        float o;
-        if (MODE == FWD) {
-          o = s[v] + a.bias[row];
-          if (a.relu) o = fmaxf(o, 0.0f);
-          if (a.C) a.C[idx] = o;   // null: no FP32 copy (inference)
-        } else {
-          o = s[v] + (a.beta ? a.C[idx] : 0.0f);
-          if (a.mask && !(a.mask[idx] > 0.0f)) o = 0.0f;
-          a.C[idx] = o;
-        }
-        ov[v] = o;
-      }
-      // channels-last copies: the four channels in one 8-byte store when they all exist
-      const ClOut* outs[2] = {&a.o1, &a.o2};
+    for (int v = 0; v < 4; v++)
+      if (row0 + v < a.M) atomicAdd(&a.C[((size_t)(row0 + v) * a.Cb + bci) * a.T + bt], s[v]);
+  }
+}
+
+// One output tile's four rows row0 .. row0 + 3 of column n (FWD: bias, ReLU; BDATA: add, mask) and
+// their channels-last copies.
+template <int MODE>
+__device__ __forceinline__ void conv_out(const ConvK& a, const floatx4& s, int row0, int n)
+{
+  float ov[4];
 #pragma unroll
-      for (int j = 0; j < 2; j++) {
-        const ClOut& o = *outs[j];
-        if (!o.p) continue;
-        __bf16* dst = o.p + (size_t)n * o.ld + o.off + row0;
-        if (row0 + 3 < a.M && ((o.ld | o.off) & 3) == 0) {
-          bf16x4 q;
+  for (int v = 0; v < 4; v++) {
+    const int row = row0 + v;
+    ov[v] = 0.0f;
+    if (row >= a.M) continue;
+    const size_t idx = (size_t)row * a.N + n;
+    float o;
+    if (MODE == FWD) {
+      o = s[v] + a.bias[row];
+      if (a.relu) o = fmaxf(o, 0.0f);
+      if (a.C) a.C[idx] = o;   // null: no FP32 copy (inference)
+    } else {
+      o = s[v] + (a.beta ? a.C[idx] : 0.0f);
+      if (a.mask && !(a.mask[idx] > 0.0f)) o = 0.0f;
+      a.C[idx] = o;
+    }
+    ov[v] = o;
+  }
+  // the four channels in one 8-byte store when they all exist
+  const ClOut* outs[2] = {&a.o1, &a.o2};
 #pragma unroll
-          for (int v = 0; v < 4; v++) q[v] = to_bf16(ov[v]);
-          *(bf16x4*)dst = q;
-        } else {
+  for (int j = 0; j < 2; j++) {
+    const ClOut& o = *outs[j];
+    if (!o.p) continue;
+    __bf16* dst = o.p + (size_t)n * o.ld + o.off + row0;
+    if (row0 + 3 < a.M && ((o.ld | o.off) & 3) == 0) {
+      bf16x4 q;
 #pragma unroll
-          for (int v = 0; v < 4; v++)
-            if (row0 + v < a.M) dst[v] = to_bf16(ov[v]);
-        }
-      }
+      for (int v = 0; v < 4; v++) q[v] = to_bf16(ov[v]);
+      *(bf16x4*)dst = q;
     } else {
 #pragma unroll
       for (int v = 0; v < 4; v++)
-        if (row0 + v < a.M) atomicAdd(&a.C[((size_t)(row0 + v) * a.Cb + bci) * a.T + bt], s[v]);
+        if (row0 + v < a.M) dst[v] = to_bf16(ov[v]);
     }
   }
 }
 
-// Forward and input-gradient products as k_conv's, with NC 16-voxel column tiles per workgroup:
-// each wave's weight fragments (MT per k-step) serve the NC tiles, so the weights stream from
-// L2 once per 16 NC voxels; the four waves still split the k-steps and reduce through LDS.
-#ifndef MCPET_CONV_COLS
-#define MCPET_CONV_COLS 2
-#endif
-template <int MODE, int MT, int NC>
+// what a lane reads as its 8 channels outside the volume
+__device__ __attribute__((aligned(16))) const unsigned k_zeros[4] = {0u, 0u, 0u, 0u};
+
+// bits t of the taps t = 9 (dz + 1) + 3 (dy + 1) + (dx + 1) whose three bits are all set
+__device__ __forceinline__ unsigned tap_mask(unsigned vz, unsigned vy, unsigned vx)
+{
+  const unsigned row = (vy & 1 ? vx : 0u) | (vy & 2 ? vx << 3 : 0u) | (vy & 4 ? vx << 6 : 0u);
+  return (vz & 1 ? row : 0u) | (vz & 2 ? row << 9 : 0u) | (vz & 4 ? row << 18 : 0u);
+}
+
+// Forward and input-gradient products on NC tiles of 16 voxels and MT blocks of 16 channels per
+// workgroup; the four waves split the k-steps (wave w: steps w, w + 4, ...) and their sums are
+// added in wave order through LDS. A lane's taps inside the volume are one bit mask and its input
+// voxel is linear in the tap, so a k-step is the tap's offset, MT + NC 16-byte loads (weights 1 KB
+// contiguous) and MT NC MFMAs; the loads of CONV_PF steps are in flight (one workgroup or two per CU
+// at the coarse levels, where a k-step without prefetch took 1.2 to 1.5 us). Width 16 on 16 x 28 x 28
+// voxels, all products of a forward: 95 -> 61 us; 192 -> 64 channels on 16 x 28 x 28: 61 -> 40 us.
+// Stride-2 input gradients: output voxels are taken parity class by parity class (D, H, W even),
+// so a tile's voxels share their 1 to 8 taps and the other k-steps are skipped (64 -> 32 channels on
+// 32 x 56 x 56: 60 -> 29 us).
+#define CONV_PF 4
+template <int MODE, int MT, int NC, bool kSkip>
 __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
 {
   static_assert(MODE == FWD || MODE == BDATA, "forward and input-gradient products only");
   __shared__ floatx4 red[4][NC * MT][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4;
-  const int m0 = blockIdx.y * (16 * MT);
-  int nn[NC], cz[NC], cy[NC], cx[NC];
-  bool nvalid[NC];
+  const int rb0 = blockIdx.y * MT;
+  int nn[NC], base[NC];
+  unsigned mask[NC];
+  // the tap's step in the B tensor: rows and planes of that tensor
+  const int bW = MODE == FWD ? a.W : a.oW, bH = MODE == FWD ? a.H : a.oH;
 #pragma unroll
   for (int j = 0; j < NC; j++) {
-    const int n = (blockIdx.x * NC + j) * 16 + r;   // this lane's column in tile j
+    int n = (blockIdx.x * NC + j) * 16 + r;   // this lane's column in tile j
+    const int w = MODE == FWD ? a.oW : a.W, h = MODE == FWD ? a.oH : a.H, d = MODE == FWD ? a.oD : a.D;
+    int x, y, z;
+    if (kSkip) {
+      const int per = a.N >> 3, cls = n / per, i = n - cls * per, w2 = w >> 1, h2 = h >> 1;
+      x = 2 * (i % w2) + (cls & 1);
+      y = 2 * ((i / w2) % h2) + ((cls >> 1) & 1);
+      z = 2 * (i / (w2 * h2)) + (cls >> 2);
+      const bool ok = n < a.N;
+      n = ok ? (z * h + y) * w + x : a.N;
+    } else {
+      x = n % w;
+      y = (n / w) % h;
+      z = n / (w * h);
+    }
     nn[j] = n;
-    nvalid[j] = n < a.N;
-    const int w = MODE == FWD ? a.oW : a.W, h = MODE == FWD ? a.oH : a.H;
-    cx[j] = n % w;
-    cy[j] = (n / w) % h;
-    cz[j] = n / (w * h);
+    unsigned vx = 7, vy = 7, vz = 7;
+    if (MODE == FWD) {
+      x *= a.stride;
+      y *= a.stride;
+      z *= a.stride;
+      if (x == 0) vx &= ~1u;
+      if (y == 0) vy &= ~1u;
+      if (z == 0) vz &= ~1u;
+      if (x + 1 >= a.W) vx &= ~4u;
+      if (y + 1 >= a.H) vy &= ~4u;
+      if (z + 1 >= a.D) vz &= ~4u;
+      base[j] = (z * a.H + y) * a.W + x;
+    } else if (kSkip) {   // 2 q + d = p: p even d = 0, p odd d = -1 (q = (p + 1) / 2) and +1 (q one less)
+      vx = x & 1 ? 5u : 2u;
+      vy = y & 1 ? 5u : 2u;
+      vz = z & 1 ? 5u : 2u;
+      x = (x + 1) >> 1;
+      y = (y + 1) >> 1;
+      z = (z + 1) >> 1;
+      if (x >= a.oW) vx &= ~3u;
+      if (y >= a.oH) vy &= ~3u;
+      if (z >= a.oD) vz &= ~3u;
+      base[j] = (z * a.oH + y) * a.oW + x;
+    } else {                      // q = p - d
+      if (x == 0) vx &= ~4u;
+      if (y == 0) vy &= ~4u;
+      if (z == 0) vz &= ~4u;
+      if (x + 1 >= w) vx &= ~1u;
+      if (y + 1 >= h) vy &= ~1u;
+      if (z + 1 >= d) vz &= ~1u;
+      base[j] = (z * h + y) * w + x;
+    }
+    mask[j] = n < a.N ? (a.ks == 3 ? tap_mask(vz, vy, vx) : 1u) : 0u;
   }
   floatx4 acc[NC][MT];
 #pragma unroll
   for (int j = 0; j < NC; j++)
 #pragma unroll
     for (int i = 0; i < MT; i++) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // tap and channel carried across k-steps as in k_conv
-  const int Cbp = a.Cbp, dt = 128 / Cbp, dc = 128 - dt * Cbp, ke = a.K;
-  int k = wave * 32 + kg * 8;
-  int t = k / Cbp, c0 = k - t * Cbp;
-  const __bf16* arow[MT];
-#pragma unroll
-  for (int i = 0; i < MT; i++) arow[i] = a.A + (size_t)(m0 + 16 * i + r) * a.Kp;
-  bf16x8 zero;
-#pragma unroll
-  for (int e = 0; e < 8; e++) zero[e] = to_bf16(0.0f);
-  for (int k0 = wave * 32; k0 < ke; k0 += 128, k += 128) {
-    int dz = 0, dy = 0, dx = 0;
-    if (a.ks == 3) {
-      const int q9 = (t * 7282) >> 16, q3 = (t * 21846) >> 16;
-      dz = q9 - 1;
-      dy = q3 - 3 * q9 - 1;
-      dx = t - 3 * q3 - 1;
-    }
-    bf16x8 av[MT];
-#pragma unroll
-    for (int i = 0; i < MT; i++) av[i] = *(const bf16x8*)(arow[i] + k);
-#pragma unroll
-    for (int j = 0; j < NC; j++) {
-      bool in = nvalid[j] && k < ke;
-      int vox = 0;
-      if (MODE == FWD) {
-        const int z = cz[j] * a.stride + dz, y = cy[j] * a.stride + dy, x = cx[j] * a.stride + dx;
-        in = in && z >= 0 && y >= 0 && x >= 0 && z < a.D && y < a.H && x < a.W;
-        vox = (z * a.H + y) * a.W + x;
-      } else {
-        int qz = 0, qy = 0, qx = 0;
-        in = in && src_of(cz[j], dz, a.stride, a.oD, qz) && src_of(cy[j], dy, a.stride, a.oH, qy) &&
-             src_of(cx[j], dx, a.stride, a.oW, qx);
-        vox = (qz * a.oH + qy) * a.oW + qx;
-      }
-      bf16x8 b = zero;
-      if (in) b = *(const bf16x8*)(a.Xl + (size_t)vox * Cbp + c0);
-#pragma unroll
-      for (int i = 0; i < MT; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], b, acc[j][i], 0, 0, 0);
-    }
+  // the lane's tap t and channel c0 of k = t Cbp + c0 are carried from step to step
+  const int Cbp = a.Cbp, dt = 128 / Cbp, dc = 128 - dt * Cbp;
+  const int n_steps = (a.K + 31) >> 5, n_mine = (n_steps - wave + 3) >> 2;
+  int t, c0, step = wave;
+  {
+    const int k = wave * 32 + kg * 8;
+    t = k / Cbp;
+    c0 = k - t * Cbp;
+  }
+  const __bf16* ap = a.A + ((size_t)wave * a.nrb + rb0) * 512 + lane * 8;
+  const size_t astep = (size_t)a.nrb * 2048;
+  bf16x8 av[CONV_PF][MT], bv[CONV_PF][NC];
+  auto advance = [&]() {
+    step += 4;
+    ap += astep;
     c0 += dc;
     t += dt;
     if (c0 >= Cbp) {
       c0 -= Cbp;
       t++;
     }
+  };
+  auto fetch = [&](bf16x8* fa, bf16x8* fb) {   // step `step`, then on to the wave's next one
+    int off = 0;
+    if (a.ks == 3) {   // t / 9 = (7282 t) >> 16 and t / 3 = (21846 t) >> 16, exact for t < 32
+      const int q9 = (t * 7282) >> 16, q3 = (t * 21846) >> 16;
+      const int uz = q9, uy = q3 - 3 * q9, ux = t - 3 * q3;   // d + 1
+      if (kSkip) off = -(((uz >> 1) * bH + (uy >> 1)) * bW + (ux >> 1));
+      else {
+        off = ((uz - 1) * bH + (uy - 1)) * bW + (ux - 1);
+        if (MODE == BDATA) off = -off;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; i++) fa[i] = *(const bf16x8*)(ap + i * 512);
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+      const bool in = t < 32 && ((mask[j] >> t) & 1u);
+      const __bf16* p = a.Xl + ((size_t)(unsigned)(base[j] + off) * (unsigned)Cbp + (unsigned)c0);
+      fb[j] = *(const bf16x8*)(in ? p : (const __bf16*)k_zeros);
+    }
+    advance();
+  };
+  auto mult = [&](const bf16x8* fa, const bf16x8* fb) {
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+#pragma unroll
+      for (int i = 0; i < MT; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[j][i], 0, 0, 0);
+  };
+  if constexpr (kSkip) {
+    unsigned any = 0;
+#pragma unroll
+    for (int j = 0; j < NC; j++) any |= mask[j];
+    auto live = [&]() {   // on to the next step with a tap of one of the tiles
+      while (step < n_steps && !__any(t < 32 && ((any >> t) & 1u))) advance();
+      return step < n_steps;
+    };
+    while (live()) {
+      fetch(av[0], bv[0]);
+      const bool two = live();
+      if (two) fetch(av[1], bv[1]);
+      mult(av[0], bv[0]);
+      if (two) mult(av[1], bv[1]);
+    }
+  } else if (n_mine > 0) {
+    int left = n_mine;
+#pragma unroll
+    for (int p = 0; p < CONV_PF; p++) {
+      if (left > 0) fetch(av[p], bv[p]);
+      left--;
+    }
+    int i = 0;
+    for (; i + 2 * CONV_PF <= n_mine; i += CONV_PF) {
+#pragma unroll
+      for (int p = 0; p < CONV_PF; p++) {
+        mult(av[p], bv[p]);
+        fetch(av[p], bv[p]);
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < CONV_PF; p++) {
+      if (i + p < n_mine) mult(av[p], bv[p]);
+      if (i + p + CONV_PF < n_mine) fetch(av[p], bv[p]);
+    }
+    i += CONV_PF;
+#pragma unroll
+    for (int p = 0; p < CONV_PF; p++)
+      if (i + p < n_mine) mult(av[p], bv[p]);
   }
 #pragma unroll
   for (int j = 0; j < NC; j++)
 #pragma unroll
     for (int i = 0; i < MT; i++) red[wave][j * MT + i][lane] = acc[j][i];
   __syncthreads();
-  // epilogue (as k_conv's): wave w finishes the (tile, row block) pairs w, w + 4, ...
-  for (int q = wave; q < NC * MT; q += 4) {
-    const int j = q / MT, i = q - (q / MT) * MT;
+  // wave w finishes the (tile, row block) pairs w, w + 4, ...
+#pragma unroll
+  for (int q = 0; q < NC * MT; q++) {
+    if ((q & 3) != wave) continue;
     const floatx4 s = red[0][q][lane] + red[1][q][lane] + red[2][q][lane] + red[3][q][lane];
-    const int row0 = m0 + 16 * i + kg * 4;
-    const int n = nn[j];
-    if (!nvalid[j]) continue;
-    float ov[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      const int row = row0 + v;
-      ov[v] = 0.0f;
-      if (row >= a.M) continue;
-      const size_t idx = (size_t)row * a.N + n;
-      float o;
-      if (MODE == FWD) {
-        o = s[v] + a.bias[row];
-        if (a.relu) o = fmaxf(o, 0.0f);
-        if (a.C) a.C[idx] = o;
-      } else {
-        o = s[v] + (a.beta ? a.C[idx] : 0.0f);
-        if (a.mask && !(a.mask[idx] > 0.0f)) o = 0.0f;
-        a.C[idx] = o;
-      }
-      ov[v] = o;
-    }
-    const ClOut* outs[2] = {&a.o1, &a.o2};
-#pragma unroll
-    for (int jj = 0; jj < 2; jj++) {
-      const ClOut& o = *outs[jj];
-      if (!o.p) continue;
-      __bf16* dst = o.p + (size_t)n * o.ld + o.off + row0;
-      if (row0 + 3 < a.M && ((o.ld | o.off) & 3) == 0) {
-        bf16x4 qv;
-#pragma unroll
-        for (int v = 0; v < 4; v++) qv[v] = to_bf16(ov[v]);
-        *(bf16x4*)dst = qv;
-      } else {
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-          if (row0 + v < a.M) dst[v] = to_bf16(ov[v]);
-      }
-    }
+    const int j = q / MT, i = q % MT;
+    if (nn[j] < a.N) conv_out<MODE>(a, s, (rb0 + i) * 16 + kg * 4, nn[j]);
   }
 }
 
@@ -503,19 +488,18 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
   b /= tiles_x;
   const int y0 = (b % tiles_y) * FT_Y;
   const int z = b / tiles_y;
-  const int m0 = blockIdx.y * (16 * MT);
+  const int rb0 = blockIdx.y * MT;
   floatx4 acc[FT_R][MT];
 #pragma unroll
   for (int j = 0; j < FT_R; j++)
 #pragma unroll
     for (int i = 0; i < MT; i++) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const __bf16* arow[MT];
-#pragma unroll
-  for (int i = 0; i < MT; i++) arow[i] = a.A + (size_t)(m0 + 16 * i + r) * a.Kp + kg * 8;
+  const __bf16* ap = a.A + (size_t)rb0 * 512 + lane * 8;
+  const size_t atap = (size_t)(a.Cbp >> 5) * a.nrb * 512;   // weights of the next tap
   bf16x8 zero;
 #pragma unroll
   for (int e = 0; e < 8; e++) zero[e] = to_bf16(0.0f);
-  for (int c0 = 0; c0 < a.Cbp; c0 += 32) {
+  for (int c0 = 0; c0 < a.Cbp; c0 += 32, ap += (size_t)a.nrb * 512) {
     for (int i = threadIdx.x; i < FT_HALO * 4; i += 256) {
       const int hv = i >> 2, q = i & 3;
       const int hx = hv % FT_HX, hy = (hv / FT_HX) % FT_HY, hz = hv / (FT_HX * FT_HY);
@@ -531,10 +515,9 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
       const int dz = MODE == FWD ? t / 9 : 2 - t / 9;            // halo coordinates of p + d_t or p - d_t
       const int dy = MODE == FWD ? (t / 3) % 3 : 2 - (t / 3) % 3;
       const int dx = MODE == FWD ? t % 3 : 2 - t % 3;
-      const int k = t * a.Cbp + c0;
       bf16x8 av[MT];
 #pragma unroll
-      for (int i = 0; i < MT; i++) av[i] = *(const bf16x8*)(arow[i] + k);
+      for (int i = 0; i < MT; i++) av[i] = *(const bf16x8*)(ap + t * atap + i * 512);
 #pragma unroll
       for (int j = 0; j < FT_R; j++) {
         const bf16x8 bv = s_halo[((dz * FT_HY + FT_R * wave + j + dy) * FT_HX + r + dx) * 4 + kg];
@@ -544,7 +527,7 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
     }
     __syncthreads();
   }
-  // epilogue (as k_conv's): this lane's columns are voxels (z, y0 + FT_R wave + j, x0 + r)
+  // this lane's columns are voxels (z, y0 + FT_R wave + j, x0 + r)
   const int x = x0 + r;
 #pragma unroll
   for (int j = 0; j < FT_R; j++) {
@@ -552,45 +535,7 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
     if (x >= a.W || y >= a.H) continue;
     const int n = (z * a.H + y) * a.W + x;
 #pragma unroll
-    for (int i = 0; i < MT; i++) {
-      const int row0 = m0 + 16 * i + kg * 4;
-      float ov[4];
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int row = row0 + v;
-        ov[v] = 0.0f;
-        if (row >= a.M) continue;
-        const size_t idx = (size_t)row * a.N + n;
-        float o;
-        if (MODE == FWD) {
-          o = acc[j][i][v] + a.bias[row];
-          if (a.relu) o = fmaxf(o, 0.0f);
-          if (a.C) a.C[idx] = o;
-        } else {
-          o = acc[j][i][v] + (a.beta ? a.C[idx] : 0.0f);
-          if (a.mask && !(a.mask[idx] > 0.0f)) o = 0.0f;
-          a.C[idx] = o;
-        }
-        ov[v] = o;
-      }
-      const ClOut* outs[2] = {&a.o1, &a.o2};
-#pragma unroll
-      for (int jj = 0; jj < 2; jj++) {
-        const ClOut& o = *outs[jj];
-        if (!o.p) continue;
-        __bf16* dst = o.p + (size_t)n * o.ld + o.off + row0;
-        if (row0 + 3 < a.M && ((o.ld | o.off) & 3) == 0) {
-          bf16x4 q;
-#pragma unroll
-          for (int v = 0; v < 4; v++) q[v] = to_bf16(ov[v]);
-          *(bf16x4*)dst = q;
-        } else {
-#pragma unroll
-          for (int v = 0; v < 4; v++)
-            if (row0 + v < a.M) dst[v] = to_bf16(ov[v]);
-        }
-      }
-    }
+    for (int i = 0; i < MT; i++) conv_out<MODE>(a, acc[j][i], (rb0 + i) * 16 + kg * 4, n);
   }
 }
 
@@ -609,38 +554,61 @@ inline int rows_for(int M)
 }
 inline int rup(int x, int m) { return (x + m - 1) / m * m; }
 
+template <int MODE, int NC, bool kSkip>
+void launch_cols(const ConvK& a, int mt, hipStream_t st)
+{
+  const dim3 g((a.N + 16 * NC - 1) / (16 * NC), a.nrb / mt, 1);
+  switch (mt) {
+    case 1: hipLaunchKernelGGL((k_conv_cols<MODE, 1, NC, kSkip>), g, dim3(256), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((k_conv_cols<MODE, 2, NC, kSkip>), g, dim3(256), 0, st, a); break;
+    case 3: hipLaunchKernelGGL((k_conv_cols<MODE, 3, NC, kSkip>), g, dim3(256), 0, st, a); break;
+    default: hipLaunchKernelGGL((k_conv_cols<MODE, 4, NC, kSkip>), g, dim3(256), 0, st, a); break;
+  }
+}
+
+// Forward and input-gradient products outside the tiled form. The tile of a workgroup does not
+// change the order of any sum: it is the largest of the list that still gives COLS_WGS workgroups
+// (two per CU), the smallest where none does.
+#ifndef COLS_WGS
+#define COLS_WGS 512
+#endif
 template <int MODE>
 hipError_t launch_conv(const ConvK& a, hipStream_t st)
 {
-  const int mt = mt_for(a.M);
-  if constexpr (MODE != BWGT && MCPET_CONV_COLS > 1) {
-    constexpr int NC = MCPET_CONV_COLS;
-    dim3 g((a.N + 16 * NC - 1) / (16 * NC), (a.M + 16 * mt - 1) / (16 * mt), 1);
-    switch (mt) {
-      case 1: hipLaunchKernelGGL((k_conv_cols<MODE, 1, NC>), g, dim3(256), 0, st, a); break;
-      case 2: hipLaunchKernelGGL((k_conv_cols<MODE, 2, NC>), g, dim3(256), 0, st, a); break;
-      case 3: hipLaunchKernelGGL((k_conv_cols<MODE, 3, NC>), g, dim3(256), 0, st, a); break;
-      default: hipLaunchKernelGGL((k_conv_cols<MODE, 4, NC>), g, dim3(256), 0, st, a); break;
-    }
-    return hipGetLastError();
+  int mt = mt_for(a.M), nc = 2;
+  auto wgs = [&](int m, int c) { return (long long)(a.nrb / m) * ((a.N + 16 * c - 1) / (16 * c)); };
+  if (wgs(mt, nc) < COLS_WGS) {
+    nc = 1;
+    while (mt > 1 && wgs(mt, nc) < COLS_WGS) mt = mt % 2 == 0 ? mt / 2 : 1;
   }
+  if (MODE == BDATA && a.stride == 2) {
+    if (a.ks != 3 || a.D % 2 || a.H % 2 || a.W % 2) return hipErrorInvalidValue;
+    if (nc == 2) launch_cols<BDATA, 2, true>(a, mt, st);
+    else launch_cols<BDATA, 1, true>(a, mt, st);
+  } else {
+    if (nc == 2) launch_cols<MODE, 2, false>(a, mt, st);
+    else launch_cols<MODE, 1, false>(a, mt, st);
+  }
+  return hipGetLastError();
+}
+
+// Weight gradients outside the tiled form: about 2048 workgroups, of at least 256 voxels.
+hipError_t launch_bwgt(const ConvK& a, hipStream_t st)
+{
+  const int mt = mt_for(a.M);
   dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt), 1);
   ConvK b = a;
-  if (MODE == BWGT) {
-    const long long xy = (long long)grid.x * grid.y;
-    int split = (int)std::max<long long>(1, std::min<long long>(2048 / std::max<long long>(1, xy), (a.K + 255) / 256));
-    int kps = (a.K + split - 1) / split;
-    kps = rup(kps, 128);
-    split = (a.K + kps - 1) / kps;
-    grid.z = split;
-    b.k_per_split = kps;
-    b.vec = (a.K % 4 == 0) ? 1 : 0;
-  }
+  const long long xy = (long long)grid.x * grid.y;
+  int split = (int)std::max<long long>(1, std::min<long long>(2048 / std::max<long long>(1, xy), (a.K + 255) / 256));
+  const int kps = rup((a.K + split - 1) / split, 128);
+  grid.z = (a.K + kps - 1) / kps;
+  b.k_per_split = kps;
+  b.vec = (a.K % 4 == 0) ? 1 : 0;
   switch (mt) {
-    case 1: hipLaunchKernelGGL((k_conv<MODE, 1>), grid, dim3(256), 0, st, b); break;
-    case 2: hipLaunchKernelGGL((k_conv<MODE, 2>), grid, dim3(256), 0, st, b); break;
-    case 3: hipLaunchKernelGGL((k_conv<MODE, 3>), grid, dim3(256), 0, st, b); break;
-    default: hipLaunchKernelGGL((k_conv<MODE, 4>), grid, dim3(256), 0, st, b); break;
+    case 1: hipLaunchKernelGGL(k_conv_bwgt<1>, grid, dim3(256), 0, st, b); break;
+    case 2: hipLaunchKernelGGL(k_conv_bwgt<2>, grid, dim3(256), 0, st, b); break;
+    case 3: hipLaunchKernelGGL(k_conv_bwgt<3>, grid, dim3(256), 0, st, b); break;
+    default: hipLaunchKernelGGL(k_conv_bwgt<4>, grid, dim3(256), 0, st, b); break;
   }
   return hipGetLastError();
 }
@@ -932,14 +900,18 @@ hipError_t launch_bwgt_tiled(int stride, const __bf16* xl, int ldx, const __bf16
   return hipGetLastError();
 }
 
-// BF16 weight copies: out[m][t * Cp + c] = W[co][ci][t] with (co, ci) = (m, c) (forward) or
-// (c, m) (transposed, for the input gradient); zero outside the real channels.
+// BF16 weight copies in the order in which the MFMA fragments read them: k-step s = k / 32, then
+// the 16-row block, then the lane (row m % 16, k-group (k % 32) / 8) and its 8 k, so that a fragment
+// is one contiguous 1 KB load (row by row it was 16 segments of 64 bytes). Element (m, k = t Cp + c)
+// is W[co][ci][t] with (co, ci) = (m, c) (forward) or (c, m) (transposed, for the input gradient);
+// zero outside the real channels.
 __global__ void k_derive(const float* __restrict__ w, __bf16* __restrict__ out, int rows, int Kp, int Cout, int Cin, int T, int Cp,
                          int transpose)
 {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (size_t)rows * Kp) return;
-  const int m = (int)(i / Kp), k = (int)(i % Kp);
+  const int step = (int)(i / ((size_t)rows * 32)), q = (int)(i % ((size_t)rows * 32)), l = (q & 511) >> 3;
+  const int m = (q >> 9) * 16 + (l & 15), k = step * 32 + (l >> 4) * 8 + (q & 7);
   const int t = k / Cp, c = k - t * Cp;
   const int co = transpose ? c : m, ci = transpose ? m : c;
   const bool ok = t < T && co < Cout && ci < Cin;
@@ -1248,6 +1220,7 @@ hipError_t conv_fwd(mcpet_surrogate* s, const Conv& l, const Vol& vin, const __b
   a.Cbp = rup(l.cin, 8);
   a.K = a.T * a.Cbp;
   a.Kp = l.kp_f;
+  a.nrb = l.rows_f / 16;
   s->flops_fwd += 2.0 * l.cout * (double)l.cin * a.T * a.N;
   if (use_tiled(a)) return launch_conv_tiled<FWD>(a, s->st);
   return launch_conv<FWD>(a, s->st);
@@ -1270,6 +1243,7 @@ hipError_t conv_bwd_data(mcpet_surrogate* s, const Conv& l, const Vol& vin, cons
   a.Cbp = rup(l.cout, 8);
   a.K = a.T * a.Cbp;
   a.Kp = l.kp_b;
+  a.nrb = l.rows_b / 16;
   if (use_tiled(a)) return launch_conv_tiled<BDATA>(a, s->st);
   return launch_conv<BDATA>(a, s->st);
 }
@@ -1297,7 +1271,7 @@ hipError_t conv_bwd_weights(mcpet_surrogate* s, const Conv& l, const Vol& vin, c
   a.K = (int)vout.vox();
   a.Cb = l.cin;
   a.Cbp = l.cin;
-  hipError_t e = launch_conv<BWGT>(a, s->st);
+  hipError_t e = launch_bwgt(a, s->st);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per), dim3(256), 0, s->st, gy, s->g + l.b, vox, per);
   return hipGetLastError();
