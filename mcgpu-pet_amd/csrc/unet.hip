@@ -137,7 +137,9 @@ struct ConvK {
   int nrb;             // 16-row blocks of A
   int Cb, Cbp;         // channels of the B tensor (FWD, BWGT: Cin; BDATA: Cout) and Cb rounded up to 8
   int D, H, W, oD, oH, oW, ks, stride, T;
-  int k_per_split;     // BWGT: voxels per workgroup
+  size_t sX, sC;       // from one sample to the next (blockIdx.z): B tensor; C and mask (BWGT: X; Ad)
+  int samples;
+  int k_per_split, splits;   // BWGT: voxels per workgroup, workgroups per sample
   int vec;             // BWGT: K % 4 == 0 (dY rows are float4-aligned)
 };
 
@@ -168,7 +170,9 @@ __global__ __launch_bounds__(256) void k_conv_bwgt(ConvK a)
 #pragma unroll
   for (int i = 0; i < MT; i++) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
   const int bt = n / a.Cb, bci = n - bt * a.Cb;
-  const int kb = blockIdx.z * a.k_per_split, ke = min(a.K, kb + a.k_per_split);
+  const int smp = blockIdx.z / a.splits, kb = (blockIdx.z - smp * a.splits) * a.k_per_split, ke = min(a.K, kb + a.k_per_split);
+  a.X += smp * a.sX;
+  a.Ad += smp * a.sC;
   for (int k0 = kb + wave * 32; k0 < ke; k0 += 128) {
     const int k = k0 + kg * 8;
     bf16x8 b;
@@ -217,6 +221,17 @@ __global__ __launch_bounds__(256) void k_conv_bwgt(ConvK a)
     for (int v = 0; v < 4; v++)
       if (row0 + v < a.M) atomicAdd(&a.C[((size_t)(row0 + v) * a.Cb + bci) * a.T + bt], s[v]);
   }
+}
+
+// the tensors of sample blockIdx.z
+__device__ __forceinline__ void to_sample(ConvK& a)
+{
+  const size_t z = blockIdx.z;
+  a.Xl += z * a.sX;
+  if (a.C) a.C += z * a.sC;
+  if (a.mask) a.mask += z * a.sC;
+  if (a.o1.p) a.o1.p += z * a.N * a.o1.ld;
+  if (a.o2.p) a.o2.p += z * a.N * a.o2.ld;
 }
 
 // One output tile's four rows row0 .. row0 + 3 of column n (FWD: bias, ReLU; BDATA: add, mask) and
@@ -292,6 +307,7 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4;
   const int rb0 = blockIdx.y * MT;
+  to_sample(a);
   int nn[NC], base[NC];
   unsigned mask[NC];
   // the tap's step in the B tensor: rows and planes of that tensor
@@ -489,6 +505,7 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
   const int y0 = (b % tiles_y) * FT_Y;
   const int z = b / tiles_y;
   const int rb0 = blockIdx.y * MT;
+  to_sample(a);
   floatx4 acc[FT_R][MT];
 #pragma unroll
   for (int j = 0; j < FT_R; j++)
@@ -557,7 +574,7 @@ inline int rup(int x, int m) { return (x + m - 1) / m * m; }
 template <int MODE, int NC, bool kSkip>
 void launch_cols(const ConvK& a, int mt, hipStream_t st)
 {
-  const dim3 g((a.N + 16 * NC - 1) / (16 * NC), a.nrb / mt, 1);
+  const dim3 g((a.N + 16 * NC - 1) / (16 * NC), a.nrb / mt, a.samples);
   switch (mt) {
     case 1: hipLaunchKernelGGL((k_conv_cols<MODE, 1, NC, kSkip>), g, dim3(256), 0, st, a); break;
     case 2: hipLaunchKernelGGL((k_conv_cols<MODE, 2, NC, kSkip>), g, dim3(256), 0, st, a); break;
@@ -576,7 +593,7 @@ template <int MODE>
 hipError_t launch_conv(const ConvK& a, hipStream_t st)
 {
   int mt = mt_for(a.M), nc = 2;
-  auto wgs = [&](int m, int c) { return (long long)(a.nrb / m) * ((a.N + 16 * c - 1) / (16 * c)); };
+  auto wgs = [&](int m, int c) { return (long long)a.samples * (a.nrb / m) * ((a.N + 16 * c - 1) / (16 * c)); };
   if (wgs(mt, nc) < COLS_WGS) {
     nc = 1;
     while (mt > 1 && wgs(mt, nc) < COLS_WGS) mt = mt % 2 == 0 ? mt / 2 : 1;
@@ -598,10 +615,11 @@ hipError_t launch_bwgt(const ConvK& a, hipStream_t st)
   const int mt = mt_for(a.M);
   dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt), 1);
   ConvK b = a;
-  const long long xy = (long long)grid.x * grid.y;
+  const long long xy = (long long)grid.x * grid.y * a.samples;
   int split = (int)std::max<long long>(1, std::min<long long>(2048 / std::max<long long>(1, xy), (a.K + 255) / 256));
   const int kps = rup((a.K + split - 1) / split, 128);
-  grid.z = (a.K + kps - 1) / kps;
+  b.splits = (a.K + kps - 1) / kps;
+  grid.z = b.splits * a.samples;
   b.k_per_split = kps;
   b.vec = (a.K % 4 == 0) ? 1 : 0;
   switch (mt) {
@@ -637,7 +655,7 @@ hipError_t launch_conv_tiled(const ConvK& a, hipStream_t st)
   if (a.ks != 3 || a.stride != 1 || a.D != a.oD || a.H != a.oH || a.W != a.oW || a.Cbp % 32 != 0 || a.Kp < 27 * a.Cbp ||
       tiles > 0x7fffffffLL)
     return hipErrorInvalidValue;
-  dim3 grid((unsigned)tiles, (a.M + 16 * mt - 1) / (16 * mt), 1);
+  dim3 grid((unsigned)tiles, (a.M + 16 * mt - 1) / (16 * mt), a.samples);
   switch (mt) {
     case 1: hipLaunchKernelGGL((k_conv_tiled<MODE, 1>), grid, dim3(256), 0, st, a); break;
     case 2: hipLaunchKernelGGL((k_conv_tiled<MODE, 2>), grid, dim3(256), 0, st, a); break;
@@ -671,7 +689,8 @@ struct BwK {
   const __bf16* Gl;   // output gradient, channels-last [ovox][ldg]
   float* part;        // [n_slabs][27][32 cob][32 cib]
   int ldx, ldg, Cin, Cout, D, H, W, oD, oH, oW;
-  int tiles_x, tiles_y, n_tiles, per_slab, cob, cib;
+  int tiles_x, tiles_y, n_tiles, per_slab, cob, cib;   // n_tiles: of all samples
+  size_t sX, sG;                                       // from one sample to the next
 };
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -727,7 +746,10 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
     const int x0 = (b % a.tiles_x) * BW_X;
     b /= a.tiles_x;
     const int y0 = (b % a.tiles_y) * BW_Y;
-    const int z0 = b / a.tiles_y;
+    b /= a.tiles_y;
+    const int z0 = b % a.oD, smp = b / a.oD;
+    const __bf16* const Xl = a.Xl + smp * a.sX;
+    const __bf16* const Gl = a.Gl + smp * a.sG;
     // input region: voxel (S z0 - 1 + hz, S y0 - 1 + hy, S x0 - 1 + hx), 4 groups of 8 channels
     for (int i = threadIdx.x; i < 3 * HY * HX * 4; i += BW_THREADS) {
       const int q = i & 3, hv = i >> 2;
@@ -736,7 +758,7 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
       const int c = ci0 + q * 8;
       bf16x8 v = zero;
       if (gz >= 0 && gz < a.D && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W && c < a.ldx)
-        v = *(const bf16x8*)(a.Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.ldx + c);
+        v = *(const bf16x8*)(Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.ldx + c);
       if constexpr (S == 1) {
 #pragma unroll
         for (int e = 0; e < 8; e++) L.x[q * 8 + e][hz][hy][hx + 7] = v[e];
@@ -755,7 +777,7 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
       const int c = co0 + q4 * 8;
       bf16x8 v = zero;
       if (gy < a.oH && gx < a.oW && c < a.ldg)
-        v = *(const bf16x8*)(a.Gl + (((size_t)z0 * a.oH + gy) * a.oW + gx) * a.ldg + c);
+        v = *(const bf16x8*)(Gl + (((size_t)z0 * a.oH + gy) * a.oW + gx) * a.ldg + c);
 #pragma unroll
       for (int e = 0; e < 8; e++) gs[q4 * 8 + e][qv] = v[e];
     }
@@ -847,11 +869,11 @@ __global__ __launch_bounds__(256) void k_bwgt_reduce(const float* __restrict__ p
 #ifndef BW_WGS
 #define BW_WGS 512
 #endif
-inline void bwgt_shape(int oD, int oH, int oW, int Cin, int Cout, BwK& b, int& n_slabs)
+inline void bwgt_shape(int samples, int oD, int oH, int oW, int Cin, int Cout, BwK& b, int& n_slabs)
 {
   b.tiles_x = (oW + BW_X - 1) / BW_X;
   b.tiles_y = (oH + BW_Y - 1) / BW_Y;
-  b.n_tiles = b.tiles_x * b.tiles_y * oD;
+  b.n_tiles = b.tiles_x * b.tiles_y * oD * samples;
   b.cob = (Cout + 31) / 32;
   b.cib = (Cin + 31) / 32;
   n_slabs = std::max(1, std::min(b.n_tiles, BW_WGS / (b.cob * b.cib)));
@@ -861,21 +883,21 @@ inline void bwgt_shape(int oD, int oH, int oW, int Cin, int Cout, BwK& b, int& n
 constexpr size_t kBwPartFloats = (size_t)BW_WGS * 27 * 1024;
 
 // true when the tiled weight gradient takes this layer (its slab sums fit the buffer)
-inline bool bwgt_fits(int oD, int oH, int oW, int Cin, int Cout)
+inline bool bwgt_fits(int samples, int oD, int oH, int oW, int Cin, int Cout)
 {
   BwK b{};
   int n_slabs = 0;
-  bwgt_shape(oD, oH, oW, Cin, Cout, b, n_slabs);
+  bwgt_shape(samples, oD, oH, oW, Cin, Cout, b, n_slabs);
   return (size_t)n_slabs * 27 * (32 * b.cob) * (32 * b.cib) <= kBwPartFloats;
 }
 
 // stride 1 (input and output volumes equal) or 2 (output (D/2, H/2, W/2) rounded down or up)
-hipError_t launch_bwgt_tiled(int stride, const __bf16* xl, int ldx, const __bf16* gyl, int ldg, int Cin, int Cout, int D, int H,
+hipError_t launch_bwgt_tiled(int samples, int stride, const __bf16* xl, int ldx, const __bf16* gyl, int ldg, int Cin, int Cout, int D, int H,
                              int W, int oD, int oH, int oW, float* part, float* G, hipStream_t st)
 {
   BwK b{};
   int n_slabs = 0;
-  bwgt_shape(oD, oH, oW, Cin, Cout, b, n_slabs);
+  bwgt_shape(samples, oD, oH, oW, Cin, Cout, b, n_slabs);
   if ((size_t)n_slabs * 27 * (32 * b.cob) * (32 * b.cib) > kBwPartFloats || ldx % 8 != 0 || ldg % 8 != 0 ||
       (stride != 1 && stride != 2))
     return hipErrorInvalidValue;
@@ -883,6 +905,8 @@ hipError_t launch_bwgt_tiled(int stride, const __bf16* xl, int ldx, const __bf16
   b.Gl = gyl;
   b.part = part;
   b.ldx = ldx;
+  b.sX = (size_t)D * H * W * ldx;
+  b.sG = (size_t)oD * oH * oW * ldg;
   b.ldg = ldg;
   b.Cin = Cin;
   b.Cout = Cout;
@@ -920,9 +944,14 @@ __global__ void k_derive(const float* __restrict__ w, __bf16* __restrict__ out, 
 
 // ------------------------------------------------------------------ elementwise kernels
 
+// Elementwise kernels take sample blockIdx.y; a tensor that is part of a larger one comes with its
+// step from sample to sample.
 // nearest x2 upsampling of [C][d][h][w] into [C][2d][2h][2w] (and its channels-last copy o)
-__global__ void k_upsample(const float* __restrict__ x, float* __restrict__ y, int C, int d, int h, int w, ClOut o)
+__global__ void k_upsample(const float* __restrict__ x, float* __restrict__ y, size_t sy, int C, int d, int h, int w, ClOut o)
 {
+  x += blockIdx.y * ((size_t)C * d * h * w);
+  if (y) y += blockIdx.y * sy;
+  if (o.p) o.p += blockIdx.y * ((size_t)8 * d * h * w) * o.ld;
   const size_t n = (size_t)C * 8 * d * h * w;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -937,8 +966,11 @@ __global__ void k_upsample(const float* __restrict__ x, float* __restrict__ y, i
 // k_upsample with each thread on 8 channels of one output voxel: the FP32 stores stay
 // coalesced across threads (consecutive voxels), and the channels-last copy of the 8 channels
 // is one 16-byte store (C % 8 == 0, o.ld and o.off multiples of 8).
-__global__ void k_upsample8(const float* __restrict__ x, float* __restrict__ y, int C, int d, int h, int w, ClOut o)
+__global__ void k_upsample8(const float* __restrict__ x, float* __restrict__ y, size_t sy, int C, int d, int h, int w, ClOut o)
 {
+  x += blockIdx.y * ((size_t)C * d * h * w);
+  if (y) y += blockIdx.y * sy;
+  if (o.p) o.p += blockIdx.y * ((size_t)8 * d * h * w) * o.ld;
   const int W2 = 2 * w, H2 = 2 * h, D2 = 2 * d;
   const size_t vox2 = (size_t)W2 * H2 * D2;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -961,10 +993,13 @@ __global__ void k_to_cl(const float* __restrict__ x, int C, size_t vox, ClOut o)
 {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (size_t)C * vox) return;
-  o.p[(i % vox) * o.ld + o.off + i / vox] = to_bf16(x[i]);
+  o.p[(blockIdx.y * vox + i % vox) * o.ld + o.off + i / vox] = to_bf16(x[blockIdx.y * (C * vox) + i]);
 }
-__global__ void k_upsample_bwd(const float* __restrict__ gy, float* __restrict__ gx, int C, int d, int h, int w, ClOut o)
+__global__ void k_upsample_bwd(const float* __restrict__ gy, size_t sy, float* __restrict__ gx, int C, int d, int h, int w, ClOut o)
 {
+  gy += blockIdx.y * sy;
+  gx += blockIdx.y * ((size_t)C * d * h * w);
+  if (o.p) o.p += blockIdx.y * ((size_t)d * h * w) * o.ld;
   const size_t n = (size_t)C * d * h * w;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -978,11 +1013,11 @@ __global__ void k_upsample_bwd(const float* __restrict__ gy, float* __restrict__
   gx[i] = s;
   if (o.p) o.p[(i % ((size_t)w * h * d)) * o.ld + o.off + c] = to_bf16(s);
 }
-// per-channel sum (bias gradient): workgroups (channel, chunk of `per` voxels), added atomically
-__global__ void k_channel_sum(const float* __restrict__ g, float* __restrict__ out, int vox, int per)
+// per-channel sum (bias gradient): workgroups (channel, chunk of `per` voxels, sample), added atomically
+__global__ void k_channel_sum(const float* __restrict__ g, size_t sg, float* __restrict__ out, int vox, int per)
 {
   __shared__ float sh[256];
-  const float* p = g + (size_t)blockIdx.x * vox;
+  const float* p = g + blockIdx.z * sg + (size_t)blockIdx.x * vox;
   const int b = blockIdx.y * per, e = min(vox, b + per);
   float s = 0.0f;
   for (int i = b + threadIdx.x; i < e; i += blockDim.x) s += p[i];
@@ -995,20 +1030,21 @@ __global__ void k_channel_sum(const float* __restrict__ g, float* __restrict__ o
   if (threadIdx.x == 0) atomicAdd(&out[blockIdx.x], sh[0]);
 }
 // out = x0 + r (residual output) and, with a target, the loss gradient and squared error
-__global__ void k_output(const float* __restrict__ x0, const float* __restrict__ r, float* __restrict__ out,
+__global__ void k_output(const float* __restrict__ x0, size_t sx, const float* __restrict__ r, float* __restrict__ out,
                          const float* __restrict__ target, float* __restrict__ g, float scale, float* __restrict__ sse, int n,
                          ClOut gl)
 {
   __shared__ float sh[256];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int v = blockIdx.x * blockDim.x + threadIdx.x;
+  const size_t i = blockIdx.y * (size_t)n + v;
   float e2 = 0.0f;
-  if (i < n) {
-    const float o = x0[i] + r[i];
+  if (v < n) {
+    const float o = x0[blockIdx.y * sx + v] + r[i];
     out[i] = o;
     if (target) {
       const float d = o - target[i];
       g[i] = 2.0f * d * scale;
-      if (gl.p) gl.p[(size_t)i * gl.ld] = to_bf16(g[i]);
+      if (gl.p) gl.p[i * gl.ld] = to_bf16(g[i]);
       e2 = d * d;
     }
   }
@@ -1129,6 +1165,7 @@ struct mcpet_surrogate {
   __bf16 *grl = nullptr, *ge1l = nullptr, *ge2l = nullptr, *gb3l = nullptr, *gd2l = nullptr, *gb2l = nullptr, *gd1l = nullptr,
          *gb1l = nullptr;
   float *raw_s = nullptr, *raw_t = nullptr, *est = nullptr;   // the fused estimate's buffers
+  int slots = 0;                                                // samples that the tensors above have room for
   double* sums = nullptr;                                       // 256 partial totals + the total
   float* bw_part = nullptr;                                     // slab sums of the tiled weight gradient
   long long t_adam = 0;
@@ -1137,7 +1174,7 @@ struct mcpet_surrogate {
   hipEvent_t ev_f0 = nullptr, ev_f1 = nullptr;   // around the last forward of mcpet_surrogate_forward
   float* h_stage = nullptr;   // pinned host staging of the fused estimate's two outputs (2 x voxels)
   unsigned long long* h_decays = nullptr;   // pinned: the estimated run's decays
-  bool fwd_timed = false;
+  int fwd_timed = 0;   // samples between the two events
   std::vector<void*> allocs;
   std::string err;
   double flops_fwd = 0.0;
@@ -1203,8 +1240,8 @@ ConvK conv_args(const Conv& l, const Vol& vin, const Vol& vout)
 const ClOut kNoCl{nullptr, 0, 0};
 
 // y = act(conv(x) + b); x read from its channels-last copy xl; o1, o2: copies of y to write
-hipError_t conv_fwd(mcpet_surrogate* s, const Conv& l, const Vol& vin, const __bf16* xl, const Vol& vout, float* y, bool relu,
-                    ClOut o1, ClOut o2 = kNoCl)
+hipError_t conv_fwd(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, const __bf16* xl, const Vol& vout, float* y,
+                    size_t sy, bool relu, ClOut o1, ClOut o2 = kNoCl)
 {
   ConvK a = conv_args(l, vin, vout);
   a.A = s->wbf + l.wf;
@@ -1218,6 +1255,9 @@ hipError_t conv_fwd(mcpet_surrogate* s, const Conv& l, const Vol& vin, const __b
   a.N = (int)vout.vox();
   a.Cb = l.cin;
   a.Cbp = rup(l.cin, 8);
+  a.samples = ns;
+  a.sX = vin.vox() * a.Cbp;
+  a.sC = sy;
   a.K = a.T * a.Cbp;
   a.Kp = l.kp_f;
   a.nrb = l.rows_f / 16;
@@ -1226,8 +1266,8 @@ hipError_t conv_fwd(mcpet_surrogate* s, const Conv& l, const Vol& vin, const __b
   return launch_conv<FWD>(a, s->st);
 }
 // gx (+)= dL/dx of the layer input, zeroed where mask <= 0; gy read from its channels-last copy
-hipError_t conv_bwd_data(mcpet_surrogate* s, const Conv& l, const Vol& vin, const Vol& vout, const __bf16* gyl, float* gx,
-                         const float* mask, bool add, ClOut o1)
+hipError_t conv_bwd_data(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, const Vol& vout, const __bf16* gyl, float* gx,
+                         size_t sx, const float* mask, bool add, ClOut o1)
 {
   ConvK a = conv_args(l, vin, vout);
   a.A = s->wbf + l.wb;
@@ -1241,6 +1281,9 @@ hipError_t conv_bwd_data(mcpet_surrogate* s, const Conv& l, const Vol& vin, cons
   a.N = (int)vin.vox();
   a.Cb = l.cout;
   a.Cbp = rup(l.cout, 8);
+  a.samples = ns;
+  a.sX = vout.vox() * a.Cbp;
+  a.sC = sx;
   a.K = a.T * a.Cbp;
   a.Kp = l.kp_b;
   a.nrb = l.rows_b / 16;
@@ -1250,16 +1293,16 @@ hipError_t conv_bwd_data(mcpet_surrogate* s, const Conv& l, const Vol& vin, cons
 // weight and bias gradients accumulated from gy (dL/d pre-activation) and the layer input x;
 // xl, gyl: their channels-last BF16 copies (ClOut ld = row length) or null. 3x3x3 layers with
 // both copies take the LDS-tiled product, the others k_conv's.
-hipError_t conv_bwd_weights(mcpet_surrogate* s, const Conv& l, const Vol& vin, const float* x, const Vol& vout, const float* gy,
-                            ClOut xl = ClOut{nullptr, 0, 0}, ClOut gyl = ClOut{nullptr, 0, 0})
+hipError_t conv_bwd_weights(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, const float* x, const Vol& vout,
+                            const float* gy, size_t sg, ClOut xl = ClOut{nullptr, 0, 0}, ClOut gyl = ClOut{nullptr, 0, 0})
 {
   const int vox = (int)vout.vox(), per = 4096;
   if (l.ks == 3 && (l.stride == 1 || l.stride == 2) && xl.p && gyl.p && xl.off == 0 && gyl.off == 0 && xl.ld % 8 == 0 &&
-      gyl.ld % 8 == 0 && bwgt_fits(vout.D, vout.H, vout.W, l.cin, l.cout)) {
-    hipError_t e = launch_bwgt_tiled(l.stride, xl.p, xl.ld, gyl.p, gyl.ld, l.cin, l.cout, vin.D, vin.H, vin.W, vout.D, vout.H,
+      gyl.ld % 8 == 0 && bwgt_fits(ns, vout.D, vout.H, vout.W, l.cin, l.cout)) {
+    hipError_t e = launch_bwgt_tiled(ns, l.stride, xl.p, xl.ld, gyl.p, gyl.ld, l.cin, l.cout, vin.D, vin.H, vin.W, vout.D, vout.H,
                                      vout.W, s->bw_part, s->g + l.w, s->st);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per), dim3(256), 0, s->st, gy, s->g + l.b, vox, per);
+    hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per, ns), dim3(256), 0, s->st, gy, sg, s->g + l.b, vox, per);
     return hipGetLastError();
   }
   ConvK a = conv_args(l, vin, vout);
@@ -1271,94 +1314,175 @@ hipError_t conv_bwd_weights(mcpet_surrogate* s, const Conv& l, const Vol& vin, c
   a.K = (int)vout.vox();
   a.Cb = l.cin;
   a.Cbp = l.cin;
+  a.samples = ns;
+  a.sX = vin.size();
+  a.sC = sg;
   hipError_t e = launch_bwgt(a, s->st);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per), dim3(256), 0, s->st, gy, s->g + l.b, vox, per);
+  hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per, ns), dim3(256), 0, s->st, gy, sg, s->g + l.b, vox, per);
   return hipGetLastError();
 }
-hipError_t upsample(mcpet_surrogate* s, const Vol& v, const float* x, float* y, ClOut o)
+hipError_t upsample(mcpet_surrogate* s, int ns, const Vol& v, const float* x, float* y, size_t sy, ClOut o)
 {
   if (v.C % 8 == 0 && (!o.p || (o.ld % 8 == 0 && o.off % 8 == 0)))
-    hipLaunchKernelGGL(k_upsample8, dim3(blocks_for(v.size())), dim3(256), 0, s->st, x, y, v.C, v.D, v.H, v.W, o);
+    hipLaunchKernelGGL(k_upsample8, dim3(blocks_for(v.size()), ns), dim3(256), 0, s->st, x, y, sy, v.C, v.D, v.H, v.W, o);
   else
-    hipLaunchKernelGGL(k_upsample, dim3(blocks_for(v.size() * 8)), dim3(256), 0, s->st, x, y, v.C, v.D, v.H, v.W, o);
+    hipLaunchKernelGGL(k_upsample, dim3(blocks_for(v.size() * 8), ns), dim3(256), 0, s->st, x, y, sy, v.C, v.D, v.H, v.W, o);
   return hipGetLastError();
 }
-hipError_t upsample_bwd(mcpet_surrogate* s, const Vol& v, const float* gy, float* gx, ClOut o)
+hipError_t upsample_bwd(mcpet_surrogate* s, int ns, const Vol& v, const float* gy, size_t sy, float* gx, ClOut o)
 {
-  hipLaunchKernelGGL(k_upsample_bwd, dim3(blocks_for(v.size())), dim3(256), 0, s->st, gy, gx, v.C, v.D, v.H, v.W, o);
+  hipLaunchKernelGGL(k_upsample_bwd, dim3(blocks_for(v.size()), ns), dim3(256), 0, s->st, gy, sy, gx, v.C, v.D, v.H, v.W, o);
   return hipGetLastError();
 }
 ClOut cl(__bf16* p, int channels, int off = 0) { return ClOut{p, rup(channels, 8), off}; }
 
-// Forward of one sample already in s->x0 (r = the residual). keep: write the FP32 copy of every
+// Forward of the ns samples already in s->x0 (r = the residuals). keep: write the FP32 copy of every
 // activation (training reads them); without it only the tensors the forward itself reads in
 // FP32 (the upsampling inputs b3 and e2, the residual r) are written, the layers passing their
 // outputs to the next one through the channels-last BF16 copies alone.
-hipError_t forward(mcpet_surrogate* s, bool keep)
+hipError_t forward(mcpet_surrogate* s, int ns, bool keep)
 {
   hipError_t e = hipSuccess;
   const int c = s->c;
   const Vol vb1{c, s->D, s->H, s->W}, vb2{2 * c, s->D / 2, s->H / 2, s->W / 2};
+  const size_t s1 = s->vcat1.size(), s2 = s->vcat2.size();
   float* b1 = s->cat1 + (size_t)2 * c * vb1.vox();   // enc1 output lives in the concat buffer
   float* b2 = s->cat2 + (size_t)4 * c * vb2.vox();
   s->flops_fwd = 0.0;
-  hipLaunchKernelGGL(k_to_cl, dim3(blocks_for(s->vx.size())), dim3(256), 0, s->st, s->x0, s->cin, s->vx.vox(), cl(s->x0l, s->cin));
+  hipLaunchKernelGGL(k_to_cl, dim3(blocks_for(s->vx.size()), ns), dim3(256), 0, s->st, s->x0, s->cin, s->vx.vox(),
+                     cl(s->x0l, s->cin));
   e = hipGetLastError();
 #define STEP(x) \
   if (e == hipSuccess) e = (x)
   auto k = [keep](float* p) { return keep ? p : nullptr; };
-  STEP(conv_fwd(s, s->L[0], s->vx, s->x0l, s->va1, k(s->a1), true, cl(s->a1l, c)));
-  STEP(conv_fwd(s, s->L[1], s->va1, s->a1l, vb1, k(b1), true, cl(s->b1l, c), cl(s->cat1l, 3 * c, 2 * c)));
-  STEP(conv_fwd(s, s->L[2], vb1, s->b1l, s->vd1, k(s->d1), true, cl(s->d1l, 2 * c)));
-  STEP(conv_fwd(s, s->L[3], s->vd1, s->d1l, vb2, k(b2), true, cl(s->b2l, 2 * c), cl(s->cat2l, 6 * c, 4 * c)));
-  STEP(conv_fwd(s, s->L[4], vb2, s->b2l, s->vd2, k(s->d2), true, cl(s->d2l, 4 * c)));
-  STEP(conv_fwd(s, s->L[5], s->vd2, s->d2l, s->vb3, s->b3, true, kNoCl));
-  STEP(upsample(s, s->vb3, s->b3, k(s->cat2), cl(s->cat2l, 6 * c)));    // first 4c channels of cat2
-  STEP(conv_fwd(s, s->L[6], s->vcat2, s->cat2l, s->ve2, s->e2, true, kNoCl));
-  STEP(upsample(s, s->ve2, s->e2, k(s->cat1), cl(s->cat1l, 3 * c)));    // first 2c channels of cat1
-  STEP(conv_fwd(s, s->L[7], s->vcat1, s->cat1l, s->ve1, k(s->e1), true, cl(s->e1l, c)));
-  STEP(conv_fwd(s, s->L[8], s->ve1, s->e1l, s->vr, s->r, false, kNoCl));
+  STEP(conv_fwd(s, ns, s->L[0], s->vx, s->x0l, s->va1, k(s->a1), s->va1.size(), true, cl(s->a1l, c)));
+  STEP(conv_fwd(s, ns, s->L[1], s->va1, s->a1l, vb1, k(b1), s1, true, cl(s->b1l, c), cl(s->cat1l, 3 * c, 2 * c)));
+  STEP(conv_fwd(s, ns, s->L[2], vb1, s->b1l, s->vd1, k(s->d1), s->vd1.size(), true, cl(s->d1l, 2 * c)));
+  STEP(conv_fwd(s, ns, s->L[3], s->vd1, s->d1l, vb2, k(b2), s2, true, cl(s->b2l, 2 * c), cl(s->cat2l, 6 * c, 4 * c)));
+  STEP(conv_fwd(s, ns, s->L[4], vb2, s->b2l, s->vd2, k(s->d2), s->vd2.size(), true, cl(s->d2l, 4 * c)));
+  STEP(conv_fwd(s, ns, s->L[5], s->vd2, s->d2l, s->vb3, s->b3, s->vb3.size(), true, kNoCl));
+  STEP(upsample(s, ns, s->vb3, s->b3, k(s->cat2), s2, cl(s->cat2l, 6 * c)));    // first 4c channels of cat2
+  STEP(conv_fwd(s, ns, s->L[6], s->vcat2, s->cat2l, s->ve2, s->e2, s->ve2.size(), true, kNoCl));
+  STEP(upsample(s, ns, s->ve2, s->e2, k(s->cat1), s1, cl(s->cat1l, 3 * c)));    // first 2c channels of cat1
+  STEP(conv_fwd(s, ns, s->L[7], s->vcat1, s->cat1l, s->ve1, k(s->e1), s->ve1.size(), true, cl(s->e1l, c)));
+  STEP(conv_fwd(s, ns, s->L[8], s->ve1, s->e1l, s->vr, s->r, s->vr.size(), false, kNoCl));
 #undef STEP
   return e;
 }
 
-// Backward of one sample from gr (= dL/dr, with its channels-last copy); accumulates the
+// Backward of ns samples from gr (= dL/dr, with its channels-last copy); accumulates the
 // parameter gradients. The ReLU derivative is applied where each gradient is produced (mask =
 // the post-ReLU activation; the upsampled and concatenated copies carry the same sign as their
 // sources). A gradient's channels-last copy is written by the product that completes it.
-hipError_t backward(mcpet_surrogate* s)
+hipError_t backward(mcpet_surrogate* s, int ns)
 {
   hipError_t e = hipSuccess;
   const int c = s->c;
   const Vol vb1{c, s->D, s->H, s->W}, vb2{2 * c, s->D / 2, s->H / 2, s->W / 2};
+  const size_t s1 = s->vcat1.size(), s2 = s->vcat2.size();
   const float* b1 = s->cat1 + (size_t)2 * c * vb1.vox();
   const float* b2 = s->cat2 + (size_t)4 * c * vb2.vox();
   float* gb1 = s->gcat1 + (size_t)2 * c * vb1.vox();
   float* gb2 = s->gcat2 + (size_t)4 * c * vb2.vox();
 #define STEP(x) \
   if (e == hipSuccess) e = (x)
-  STEP(conv_bwd_weights(s, s->L[8], s->ve1, s->e1, s->vr, s->gr));
-  STEP(conv_bwd_data(s, s->L[8], s->ve1, s->vr, s->grl, s->ge1, s->e1, false, cl(s->ge1l, c)));
-  STEP(conv_bwd_weights(s, s->L[7], s->vcat1, s->cat1, s->ve1, s->ge1, cl(s->cat1l, 3 * c), cl(s->ge1l, c)));
-  STEP(conv_bwd_data(s, s->L[7], s->vcat1, s->ve1, s->ge1l, s->gcat1, s->cat1, false, kNoCl));   // g(up1), g(b1 skip)
-  STEP(upsample_bwd(s, s->ve2, s->gcat1, s->ge2, cl(s->ge2l, 2 * c)));
-  STEP(conv_bwd_weights(s, s->L[6], s->vcat2, s->cat2, s->ve2, s->ge2, cl(s->cat2l, 6 * c), cl(s->ge2l, 2 * c)));
-  STEP(conv_bwd_data(s, s->L[6], s->vcat2, s->ve2, s->ge2l, s->gcat2, s->cat2, false, kNoCl));   // g(up2), g(b2 skip)
-  STEP(upsample_bwd(s, s->vb3, s->gcat2, s->gb3, cl(s->gb3l, 4 * c)));
-  STEP(conv_bwd_weights(s, s->L[5], s->vd2, s->d2, s->vb3, s->gb3, cl(s->d2l, 4 * c), cl(s->gb3l, 4 * c)));
-  STEP(conv_bwd_data(s, s->L[5], s->vd2, s->vb3, s->gb3l, s->gd2, s->d2, false, cl(s->gd2l, 4 * c)));
-  STEP(conv_bwd_weights(s, s->L[4], vb2, b2, s->vd2, s->gd2, cl(s->b2l, 2 * c), cl(s->gd2l, 4 * c)));
-  STEP(conv_bwd_data(s, s->L[4], vb2, s->vd2, s->gd2l, gb2, b2, true, cl(s->gb2l, 2 * c)));   // + the skip's gradient
-  STEP(conv_bwd_weights(s, s->L[3], s->vd1, s->d1, vb2, gb2, cl(s->d1l, 2 * c), cl(s->gb2l, 2 * c)));
-  STEP(conv_bwd_data(s, s->L[3], s->vd1, vb2, s->gb2l, s->gd1, s->d1, false, cl(s->gd1l, 2 * c)));
-  STEP(conv_bwd_weights(s, s->L[2], vb1, b1, s->vd1, s->gd1, cl(s->b1l, c), cl(s->gd1l, 2 * c)));
-  STEP(conv_bwd_data(s, s->L[2], vb1, s->vd1, s->gd1l, gb1, b1, true, cl(s->gb1l, c)));       // + the skip's gradient
-  STEP(conv_bwd_weights(s, s->L[1], s->va1, s->a1, vb1, gb1, cl(s->a1l, c), cl(s->gb1l, c)));
-  STEP(conv_bwd_data(s, s->L[1], s->va1, vb1, s->gb1l, s->ga1, s->a1, false, kNoCl));
-  STEP(conv_bwd_weights(s, s->L[0], s->vx, s->x0, s->va1, s->ga1));
+#define WGT(l, vin, x, vout, gy, sg, ...) STEP(conv_bwd_weights(s, ns, s->L[l], vin, x, vout, gy, sg, ##__VA_ARGS__))
+#define DATA(l, vin, vout, gyl, gx, sx, mask, add, o1) STEP(conv_bwd_data(s, ns, s->L[l], vin, vout, gyl, gx, sx, mask, add, o1))
+  WGT(8, s->ve1, s->e1, s->vr, s->gr, s->vr.size());
+  DATA(8, s->ve1, s->vr, s->grl, s->ge1, s->ve1.size(), s->e1, false, cl(s->ge1l, c));
+  WGT(7, s->vcat1, s->cat1, s->ve1, s->ge1, s->ve1.size(), cl(s->cat1l, 3 * c), cl(s->ge1l, c));
+  DATA(7, s->vcat1, s->ve1, s->ge1l, s->gcat1, s1, s->cat1, false, kNoCl);   // g(up1), g(b1 skip)
+  STEP(upsample_bwd(s, ns, s->ve2, s->gcat1, s1, s->ge2, cl(s->ge2l, 2 * c)));
+  WGT(6, s->vcat2, s->cat2, s->ve2, s->ge2, s->ve2.size(), cl(s->cat2l, 6 * c), cl(s->ge2l, 2 * c));
+  DATA(6, s->vcat2, s->ve2, s->ge2l, s->gcat2, s2, s->cat2, false, kNoCl);   // g(up2), g(b2 skip)
+  STEP(upsample_bwd(s, ns, s->vb3, s->gcat2, s2, s->gb3, cl(s->gb3l, 4 * c)));
+  WGT(5, s->vd2, s->d2, s->vb3, s->gb3, s->vb3.size(), cl(s->d2l, 4 * c), cl(s->gb3l, 4 * c));
+  DATA(5, s->vd2, s->vb3, s->gb3l, s->gd2, s->vd2.size(), s->d2, false, cl(s->gd2l, 4 * c));
+  WGT(4, vb2, b2, s->vd2, s->gd2, s->vd2.size(), cl(s->b2l, 2 * c), cl(s->gd2l, 4 * c));
+  DATA(4, vb2, s->vd2, s->gd2l, gb2, s2, b2, true, cl(s->gb2l, 2 * c));      // + the skip's gradient
+  WGT(3, s->vd1, s->d1, vb2, gb2, s2, cl(s->d1l, 2 * c), cl(s->gb2l, 2 * c));
+  DATA(3, s->vd1, vb2, s->gb2l, s->gd1, s->vd1.size(), s->d1, false, cl(s->gd1l, 2 * c));
+  WGT(2, vb1, b1, s->vd1, s->gd1, s->vd1.size(), cl(s->b1l, c), cl(s->gd1l, 2 * c));
+  DATA(2, vb1, s->vd1, s->gd1l, gb1, s1, b1, true, cl(s->gb1l, c));          // + the skip's gradient
+  WGT(1, s->va1, s->a1, vb1, gb1, s1, cl(s->a1l, c), cl(s->gb1l, c));
+  DATA(1, s->va1, vb1, s->gb1l, s->ga1, s->va1.size(), s->a1, false, kNoCl);
+  WGT(0, s->vx, s->x0, s->va1, s->ga1, s->va1.size());
+#undef WGT
+#undef DATA
 #undef STEP
   return e;
+}
+
+// The tensors held per sample.
+struct Slot {
+  void** p;
+  size_t bytes;   // of one sample
+  bool zero;
+};
+
+std::vector<Slot> sample_tensors(mcpet_surrogate* s)
+{
+  const int c = s->c, ci = s->cin;
+  const size_t v0 = s->vx.vox(), v1 = s->vd1.vox(), v2 = s->vd2.vox();
+  std::vector<Slot> t;
+  auto f = [&](float** p, const Vol& v) { t.push_back({(void**)p, sizeof(float) * v.size(), false}); };
+  auto h = [&](__bf16** p, size_t vox, int ch) { t.push_back({(void**)p, sizeof(__bf16) * vox * rup(ch, 8), true}); };
+  f(&s->x0, s->vx), f(&s->b3, s->vb3), f(&s->e2, s->ve2), f(&s->r, s->vr), f(&s->out, s->vr);
+  f(&s->a1, s->va1), f(&s->cat1, s->vcat1), f(&s->d1, s->vd1), f(&s->cat2, s->vcat2);
+  f(&s->d2, s->vd2), f(&s->e1, s->ve1), f(&s->tgt, s->vr);
+  f(&s->ga1, s->va1), f(&s->gcat1, s->vcat1), f(&s->gd1, s->vd1), f(&s->gcat2, s->vcat2);
+  f(&s->gd2, s->vd2), f(&s->gb3, s->vb3), f(&s->ge2, s->ve2), f(&s->ge1, s->ve1), f(&s->gr, s->vr);
+  h(&s->x0l, v0, ci), h(&s->a1l, v0, c), h(&s->b1l, v0, c), h(&s->cat1l, v0, 3 * c);
+  h(&s->d1l, v1, 2 * c), h(&s->b2l, v1, 2 * c), h(&s->cat2l, v1, 6 * c), h(&s->d2l, v2, 4 * c);
+  h(&s->e1l, v0, c);
+  h(&s->grl, v0, 8), h(&s->ge1l, v0, c), h(&s->ge2l, v1, 2 * c), h(&s->gb3l, v2, 4 * c);
+  h(&s->gd2l, v2, 4 * c), h(&s->gb2l, v1, 2 * c), h(&s->gd1l, v1, 2 * c), h(&s->gb1l, v0, c);
+  return t;
+}
+
+// Samples that go through the network together: one launch per layer serves them all, so the
+// coarse levels and the short launches fill the device. About 2^19 voxels are enough, and at most
+// 1 GiB is held for them. Four samples of 32 x 56 x 56 on width 32: 1.09 ms of device time one by
+// one, 0.56 together; eight of 16 x 28 x 28 on width 16: 0.77 and 0.11.
+hipError_t hold_samples(mcpet_surrogate* s)
+{
+  const std::vector<Slot> t = sample_tensors(s);
+  size_t per = 0;
+  for (const Slot& b : t) per += b.bytes;
+  const size_t by_vox = (((size_t)1 << 19) + s->vr.vox() - 1) / s->vr.vox(), by_mem = ((size_t)1 << 30) / per;
+  s->slots = (int)std::max<size_t>(1, std::min(std::min<size_t>(by_vox, 64), by_mem));
+  // one allocation, the BF16 copies first: zeroed, their padding channels stay zero
+  auto room = [s](const Slot& b) { return (b.bytes * s->slots + 255) / 256 * 256; };
+  size_t zeroed = 0, plain = 0;
+  auto total = [&]() {
+    zeroed = plain = 0;
+    for (const Slot& b : t) (b.zero ? zeroed : plain) += room(b);
+    return zeroed + plain;
+  };
+  char* q = nullptr;
+  hipError_t e = hipMalloc((void**)&q, total());
+  if (e != hipSuccess && s->slots > 1) {
+    (void)hipGetLastError();
+    s->slots = 1;
+    e = hipMalloc((void**)&q, total());
+  }
+  if (e != hipSuccess) return e;
+  s->allocs.push_back(q);
+  char *z = q, *p = q + zeroed;
+  for (const Slot& b : t) {
+    char*& at = b.zero ? z : p;
+    *b.p = at;
+    at += room(b);
+  }
+  return hipMemsetAsync(q, 0, zeroed, s->st);
+}
+
+// samples per pass of a batch: equal groups of at most s->slots
+int sample_group(const mcpet_surrogate* s, int batch)
+{
+  const int groups = (batch + s->slots - 1) / s->slots;
+  return (batch + groups - 1) / groups;
 }
 
 }  // namespace
@@ -1424,32 +1548,13 @@ extern "C" mcpet_status mcpet_surrogate_create(int32_t D, int32_t H, int32_t W, 
     float** p;
     size_t n;
   } al[] = {{&s->p, off},          {&s->g, off},          {&s->m, off},           {&s->v, off},
-            {&s->x0, s->vx.size()}, {&s->a1, s->va1.size()}, {&s->cat1, s->vcat1.size()}, {&s->d1, s->vd1.size()},
-            {&s->cat2, s->vcat2.size()}, {&s->d2, s->vd2.size()}, {&s->b3, s->vb3.size()}, {&s->e2, s->ve2.size()},
-            {&s->e1, s->ve1.size()}, {&s->r, s->vr.size()}, {&s->out, s->vr.size()}, {&s->tgt, s->vr.size()},
-            {&s->ga1, s->va1.size()}, {&s->gcat1, s->vcat1.size()}, {&s->gd1, s->vd1.size()}, {&s->gcat2, s->vcat2.size()},
-            {&s->gd2, s->vd2.size()}, {&s->gb3, s->vb3.size()}, {&s->ge2, s->ve2.size()}, {&s->ge1, s->ve1.size()},
-            {&s->gr, s->vr.size()}, {&s->sse, 1}, {&s->raw_s, s->vr.size()}, {&s->raw_t, s->vr.size()},
-            {&s->est, s->vr.size()}};
+            {&s->sse, 1}, {&s->raw_s, s->vr.size()}, {&s->raw_t, s->vr.size()}, {&s->est, s->vr.size()}};
   for (auto& a : al)
     if (e == hipSuccess) e = dalloc_t(s, a.p, a.n);
   if (e == hipSuccess) e = dalloc_t(s, &s->wbf, s->n_bf16);
   if (e == hipSuccess) e = dalloc_t(s, &s->sums, 257);
   if (e == hipSuccess) e = dalloc_t(s, &s->bw_part, kBwPartFloats);
-  {
-    const size_t v0 = s->vx.vox(), v1 = s->vd1.vox(), v2 = s->vd2.vox();
-    struct B {
-      __bf16** p;
-      size_t n;
-    } bl[] = {{&s->x0l, v0 * rup(in_channels, 8)}, {&s->a1l, v0 * rup(c, 8)},      {&s->b1l, v0 * rup(c, 8)},
-              {&s->cat1l, v0 * rup(3 * c, 8)},      {&s->d1l, v1 * rup(2 * c, 8)}, {&s->b2l, v1 * rup(2 * c, 8)},
-              {&s->cat2l, v1 * rup(6 * c, 8)},      {&s->d2l, v2 * rup(4 * c, 8)}, {&s->e1l, v0 * rup(c, 8)},
-              {&s->grl, v0 * 8},                    {&s->ge1l, v0 * rup(c, 8)},    {&s->ge2l, v1 * rup(2 * c, 8)},
-              {&s->gb3l, v2 * rup(4 * c, 8)},       {&s->gd2l, v2 * rup(4 * c, 8)}, {&s->gb2l, v1 * rup(2 * c, 8)},
-              {&s->gd1l, v1 * rup(2 * c, 8)},       {&s->gb1l, v0 * rup(c, 8)}};
-    for (auto& x : bl)
-      if (e == hipSuccess) e = dalloc_t(s, x.p, x.n);
-  }
+  if (e == hipSuccess) e = hold_samples(s);
   if (e != hipSuccess) {
     std::string m = std::string("mcpet_surrogate_create: ") + hipGetErrorString(e);
     mcpet_surrogate_destroy(s);
@@ -1509,32 +1614,35 @@ extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float*
 {
   if (!s || !x || !y || batch < 1) return serr(s, MCPET_E_ARG, "mcpet_surrogate_forward: bad arguments");
   const size_t nx = s->vx.size(), nv = s->vr.size();
-  for (int b = 0; b < batch; b++) {
-    SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx, hipMemcpyHostToDevice, s->st));
-    const bool last = b == batch - 1;
+  const int group = sample_group(s, batch);
+  for (int b = 0; b < batch; b += group) {
+    const int n = std::min(group, batch - b);
+    SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx * n, hipMemcpyHostToDevice, s->st));
+    const bool last = b + n == batch;
     if (last) SHIP(s, hipEventRecord(s->ev_f0, s->st));
-    SHIP(s, forward(s, false));
-    hipLaunchKernelGGL(k_output, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->x0, s->r, s->out, (const float*)nullptr,
+    SHIP(s, forward(s, n, false));
+    hipLaunchKernelGGL(k_output, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->x0, nx, s->r, s->out, (const float*)nullptr,
                        (float*)nullptr, 0.0f, (float*)nullptr, (int)nv, kNoCl);
     SHIP(s, hipGetLastError());
     if (last) SHIP(s, hipEventRecord(s->ev_f1, s->st));
-    SHIP(s, hipMemcpyAsync(y + b * nv, s->out, sizeof(float) * nv, hipMemcpyDeviceToHost, s->st));
+    SHIP(s, hipMemcpyAsync(y + b * nv, s->out, sizeof(float) * nv * n, hipMemcpyDeviceToHost, s->st));
   }
   SHIP(s, hipStreamSynchronize(s->st));
-  s->fwd_timed = true;
+  s->fwd_timed = batch - (batch - 1) / group * group;
   if (gflop) *gflop = s->flops_fwd * 1e-9;
   return MCPET_OK;
 }
 
-// Device time of the network in the last mcpet_surrogate_forward (its last sample: every kernel
-// from the input conversion to the output, HIP events on the network's stream).
+// Device time per sample of the network in the last mcpet_surrogate_forward (its last samples that
+// went through together: every kernel from the input conversion to the output, HIP events on the
+// network's stream).
 extern "C" mcpet_status mcpet_surrogate_forward_ms(mcpet_surrogate* s, double* ms)
 {
   if (!s || !ms) return serr(s, MCPET_E_ARG, "mcpet_surrogate_forward_ms: null argument");
   if (!s->fwd_timed) return serr(s, MCPET_E_STATE, "mcpet_surrogate_forward_ms: no forward yet");
   float t = 0.0f;
   SHIP(s, hipEventElapsedTime(&t, s->ev_f0, s->ev_f1));
-  *ms = t;
+  *ms = t / s->fwd_timed;
   return MCPET_OK;
 }
 
@@ -1572,8 +1680,8 @@ extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* 
   hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, s->st, s->sums, 256, s->sums + 256);
   hipLaunchKernelGGL(k_normalize, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->raw_s, s->raw_t, s->x0, nv, s->sums + 256);
   SHIP(s, hipGetLastError());
-  SHIP(s, forward(s, false));
-  hipLaunchKernelGGL(k_output, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->x0, s->r, s->out, (const float*)nullptr,
+  SHIP(s, forward(s, 1, false));
+  hipLaunchKernelGGL(k_output, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->x0, s->vx.size(), s->r, s->out, (const float*)nullptr,
                      (float*)nullptr, 0.0f, (float*)nullptr, (int)nv, kNoCl);
   hipLaunchKernelGGL(k_estimate, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->out, s->est, nv, s->sums + 256, d_decays);
   SHIP(s, hipGetLastError());
@@ -1597,14 +1705,16 @@ static mcpet_status batch_gradients(mcpet_surrogate* s, const float* x, const fl
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, s->st, s->sse, (size_t)1);
   SHIP(s, hipGetLastError());
   const float scale = 1.0f / ((float)nv * (float)batch);
-  for (int b = 0; b < batch; b++) {
-    SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx, hipMemcpyHostToDevice, s->st));
-    SHIP(s, hipMemcpyAsync(s->tgt, target + b * nv, sizeof(float) * nv, hipMemcpyHostToDevice, s->st));
-    SHIP(s, forward(s, true));
-    hipLaunchKernelGGL(k_output, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->x0, s->r, s->out, s->tgt, s->gr, scale, s->sse,
-                       (int)nv, ClOut{s->grl, 8, 0});
+  const int group = sample_group(s, batch);
+  for (int b = 0; b < batch; b += group) {
+    const int n = std::min(group, batch - b);
+    SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx * n, hipMemcpyHostToDevice, s->st));
+    SHIP(s, hipMemcpyAsync(s->tgt, target + b * nv, sizeof(float) * nv * n, hipMemcpyHostToDevice, s->st));
+    SHIP(s, forward(s, n, true));
+    hipLaunchKernelGGL(k_output, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->x0, nx, s->r, s->out, s->tgt, s->gr, scale,
+                       s->sse, (int)nv, ClOut{s->grl, 8, 0});
     SHIP(s, hipGetLastError());
-    SHIP(s, backward(s));
+    SHIP(s, backward(s, n));
   }
   float sse = 0.0f;
   SHIP(s, hipMemcpyAsync(&sse, s->sse, sizeof(float), hipMemcpyDeviceToHost, s->st));

@@ -923,7 +923,7 @@ class Surrogate:
         return y
 
     def forward_ms(self):
-        """Device time (ms) of the network in the last forward() call (its last sample)."""
+        """Device time (ms) per sample of the network in the last forward() call (its last group of samples)."""
         ms = C.c_double()
         self._check(lib().mcpet_surrogate_forward_ms(self.s, C.byref(ms)))
         return ms.value

@@ -1,0 +1,37 @@
+"""Samples of a batch go through the network together, in equal groups: every sample's output has
+the same bits as alone, and the gradients are the mean of the samples' own ones."""
+import numpy as np
+import pytest
+
+import mcpet
+
+
+def _network(grid, cin, c, rng):
+    net = mcpet.Surrogate(grid, in_channels=cin, width=c, seed=11)
+    p = net.params()
+    p[-(c + 1):] = rng.normal(0, 0.1, c + 1)   # a residual that is not zero
+    net.set_params(p.astype(np.float32))
+    return net
+
+
+# one group, a full one, two unequal ones of 64 at most (35 + 34); widths with and without whole
+# 32-channel slices; volumes below and above one tile; one whose group is bounded by its voxels
+@pytest.mark.gpu
+@pytest.mark.parametrize("grid,cin,c,batch", [((4, 4, 4), 1, 3, 69), ((4, 8, 20), 2, 16, 5), ((8, 12, 16), 4, 32, 3),
+                                              ((12, 36, 36), 2, 32, 7), ((32, 68, 64), 2, 8, 5)])
+def test_batch_equals_its_samples(grid, cin, c, batch):
+    rng = np.random.default_rng(5)
+    net = _network(grid, cin, c, rng)
+    x = rng.random((batch, cin) + grid).astype(np.float32)
+    y = rng.random((batch,) + grid).astype(np.float32)
+    together = net.forward(x)
+    alone = np.concatenate([net.forward(x[i:i + 1]) for i in range(batch)])
+    assert np.array_equal(together, alone)
+    loss, grad = net.gradients(x, y)
+    each = [net.gradients(x[i:i + 1], y[i:i + 1]) for i in range(batch)]
+    mean = np.mean([g.astype(np.float64) for _, g in each], axis=0)
+    # the loss gradient of a sample is scaled by 1 / batch before its BF16 rounding, which moves each
+    # product's operands by up to 2^-9: the norm of the difference is bounded by that of the parts
+    size = np.mean([np.linalg.norm(g.astype(np.float64)) for _, g in each])
+    assert np.linalg.norm(grad - mean) <= 2.0 ** -8 * size
+    assert abs(loss - np.mean([l for l, _ in each])) <= 1e-5 * abs(loss)
