@@ -281,6 +281,13 @@ __device__ __forceinline__ void conv_out(const ConvK& a, const floatx4& s, int r
 // what a lane reads as its 8 channels outside the volume
 __device__ __attribute__((aligned(16))) const unsigned k_zeros[4] = {0u, 0u, 0u, 0u};
 
+// 8 channels of a voxel, or zeros; a global load (a pointer chosen between the two is a generic one,
+// whose loads also count as LDS accesses)
+__device__ __forceinline__ bf16x8 load_cl(const __bf16* p, bool in)
+{
+  return *(const __attribute__((address_space(1))) bf16x8*)(in ? (unsigned long long)p : (unsigned long long)k_zeros);
+}
+
 // bits t of the taps t = 9 (dz + 1) + 3 (dy + 1) + (dx + 1) whose three bits are all set
 __device__ __forceinline__ unsigned tap_mask(unsigned vz, unsigned vy, unsigned vx)
 {
@@ -408,7 +415,7 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
     for (int j = 0; j < NC; j++) {
       const bool in = t < 32 && ((mask[j] >> t) & 1u);
       const __bf16* p = a.Xl + ((size_t)(unsigned)(base[j] + off) * (unsigned)Cbp + (unsigned)c0);
-      fb[j] = *(const bf16x8*)(in ? p : (const __bf16*)k_zeros);
+      fb[j] = load_cl(p, in);
     }
     advance();
   };
@@ -446,6 +453,7 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
       for (int p = 0; p < CONV_PF; p++) {
         mult(av[p], bv[p]);
         fetch(av[p], bv[p]);
+        __builtin_amdgcn_sched_barrier(0);   // the loads are issued here, CONV_PF steps ahead of their use
       }
     }
 #pragma unroll
@@ -473,86 +481,243 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
   }
 }
 
-// Forward and input-gradient products of a stride-1 3x3x3 convolution whose B tensor (the
-// input, or the output gradient) has a multiple of 32 (padded) channels, on a tile of 4 FT_R
-// rows x 16 voxels of one z-plane per workgroup (wave w: rows y0 + FT_R w .. + FT_R - 1, the 16
-// voxels of each as its MFMA columns). The B tile with its one-voxel halo (3 x (4 FT_R + 2) x 18
-// voxels) is staged in LDS 32 channels at a time, zero outside the volume, so a k-step is one
-// LDS read per row at a compile-time offset per tap (no tap decode, no bounds test, no global
-// gather) and MT MFMAs per row; each weight fragment, read as in k_conv, serves the wave's FT_R
-// rows (the weights stream from L2 once per FT_R rows). FWD reads voxel p + d_t for tap t, BDATA
-// (stride 1: q = p - d_t) voxel p - d_t; the epilogues are k_conv's.
-#ifndef MCPET_TILED_ROWS
-#define MCPET_TILED_ROWS 2
-#endif
-#define FT_R MCPET_TILED_ROWS
-#define FT_Y (4 * FT_R)
+// Forward and input-gradient products of a stride-1 3x3x3 convolution whose B tensor (the input, or
+// the output gradient) has a multiple of 32 (padded) channels, in tiles of 16 x 8 x 2 voxels per
+// workgroup: wave w has the 16 x 4 voxels from row 4 (w % 2) of plane w / 2, one row per MFMA column
+// tile. The B tile with its one-voxel halo (18 x 10 x 4 voxels) is staged in LDS 32 channels at a time,
+// zero outside the volume, as [channel group of 8][voxel] (a fragment read is 16 consecutive voxels:
+// no bank conflict); the six rows x three shifts that a tap plane's nine taps read are read once, and
+// each weight fragment serves the wave's four rows. FWD reads voxel p + d_t for tap t, BDATA
+// (q = p - d_t) voxel p - d_t. Waiting for loads bounds it: the compiler sinks them to their use, so
+// they are pinned FT_PF taps ahead, and a thread's halo loads are all issued before the first store.
+// 96 -> 32 channels on four volumes of 32 x 56 x 56 (66.6 GFLOP): 169 us with 128-voxel tiles and
+// loads at their use, 136 with the larger tile and batched halo loads, 93 with pinned loads.
 #define FT_X 16
-#define FT_HY (FT_Y + 2)
+#define FT_Y 8
+#define FT_Z 2
 #define FT_HX (FT_X + 2)
-#define FT_HALO (3 * FT_HY * FT_HX)
+#define FT_HY (FT_Y + 2)
+#define FT_HALO ((FT_Z + 2) * FT_HY * FT_HX)
+#define FT_HP (FT_HALO + 2)   // voxels per channel group, padded: the four groups of a voxel on different banks
 
+// Workgroups are dealt to the eight XCDs in turn: number b of n, such that each XCD (and its L2) gets
+// consecutive tiles, which share their halos.
+__device__ __forceinline__ int xcd_order(int b, int n)
+{
+  const int per = n >> 3;
+  return b < per * 8 ? (b & 7) * per + (b >> 3) : b;
+}
+
+#define FT_PF 3
 template <int MODE, int MT>
 __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
 {
-  __shared__ bf16x8 s_halo[FT_HALO * 4];              // [halo voxel][channel group of 8]
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ bf16x8 s_halo[4 * FT_HP];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4;
   const int tiles_x = (a.W + FT_X - 1) / FT_X, tiles_y = (a.H + FT_Y - 1) / FT_Y;
-  int b = blockIdx.x;
+  int b = xcd_order(blockIdx.x, gridDim.x);
   const int x0 = (b % tiles_x) * FT_X;
   b /= tiles_x;
   const int y0 = (b % tiles_y) * FT_Y;
-  const int z = b / tiles_y;
+  const int z0 = (b / tiles_y) * FT_Z;
   const int rb0 = blockIdx.y * MT;
   to_sample(a);
-  floatx4 acc[FT_R][MT];
+  floatx4 acc[4][MT];
 #pragma unroll
-  for (int j = 0; j < FT_R; j++)
+  for (int j = 0; j < 4; j++)
 #pragma unroll
     for (int i = 0; i < MT; i++) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
   const __bf16* ap = a.A + (size_t)rb0 * 512 + lane * 8;
   const size_t atap = (size_t)(a.Cbp >> 5) * a.nrb * 512;   // weights of the next tap
-  bf16x8 zero;
-#pragma unroll
-  for (int e = 0; e < 8; e++) zero[e] = to_bf16(0.0f);
+  const bf16x8* const hp = s_halo + kg * FT_HP + ((wave >> 1) * FT_HY + 4 * (wave & 1)) * FT_HX + r;
   for (int c0 = 0; c0 < a.Cbp; c0 += 32, ap += (size_t)a.nrb * 512) {
-    for (int i = threadIdx.x; i < FT_HALO * 4; i += 256) {
-      const int hv = i >> 2, q = i & 3;
-      const int hx = hv % FT_HX, hy = (hv / FT_HX) % FT_HY, hz = hv / (FT_HX * FT_HY);
-      const int gz = z + hz - 1, gy = y0 + hy - 1, gx = x0 + hx - 1;
-      bf16x8 v = zero;
-      if (gz >= 0 && gz < a.D && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W)
-        v = *(const bf16x8*)(a.Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.Cbp + c0 + q * 8);
-      s_halo[i] = v;
+    bf16x8 av[FT_PF + 1][MT];   // the weights of FT_PF taps in flight
+#pragma unroll
+    for (int t = 0; t < FT_PF; t++)
+#pragma unroll
+      for (int i = 0; i < MT; i++) av[t][i] = *(const bf16x8*)(ap + t * atap + i * 512);
+    // all of the thread's loads in flight at once, then the stores
+    constexpr int kLoads = (FT_HALO * 4 + 255) / 256;
+    bf16x8 hv[kLoads];
+#pragma unroll
+    for (int l = 0; l < kLoads; l++) {
+      const int i = threadIdx.x + 256 * l, v = i >> 2, q = i & 3;
+      const int hx = v % FT_HX, hy = (v / FT_HX) % FT_HY, hz = v / (FT_HX * FT_HY);
+      const int gz = z0 + hz - 1, gy = y0 + hy - 1, gx = x0 + hx - 1;
+      const bool in = v < FT_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
+      const __bf16* p = a.Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.Cbp + c0 + q * 8;
+      hv[l] = load_cl(p, in);
+    }
+#pragma unroll
+    for (int l = 0; l < kLoads; l++) {
+      const int i = threadIdx.x + 256 * l;
+      if (i < FT_HALO * 4) s_halo[(i & 3) * FT_HP + (i >> 2)] = hv[l];
     }
     __syncthreads();
+    bf16x8 bv[6][3];
 #pragma unroll
     for (int t = 0; t < 27; t++) {
       const int dz = MODE == FWD ? t / 9 : 2 - t / 9;            // halo coordinates of p + d_t or p - d_t
       const int dy = MODE == FWD ? (t / 3) % 3 : 2 - (t / 3) % 3;
       const int dx = MODE == FWD ? t % 3 : 2 - t % 3;
-      bf16x8 av[MT];
+      if (t % 9 == 0) {
 #pragma unroll
-      for (int i = 0; i < MT; i++) av[i] = *(const bf16x8*)(ap + t * atap + i * 512);
+        for (int y = 0; y < 6; y++)
 #pragma unroll
-      for (int j = 0; j < FT_R; j++) {
-        const bf16x8 bv = s_halo[((dz * FT_HY + FT_R * wave + j + dy) * FT_HX + r + dx) * 4 + kg];
-#pragma unroll
-        for (int i = 0; i < MT; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv, acc[j][i], 0, 0, 0);
+          for (int x = 0; x < 3; x++) bv[y][x] = hp[(dz * FT_HY + y) * FT_HX + x];
       }
+      if (t + FT_PF < 27) {
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          av[(t + FT_PF) % (FT_PF + 1)][i] = *(const bf16x8*)(ap + (t + FT_PF) * atap + i * 512);
+      }
+      __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the taps that they do not belong to
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[t % (FT_PF + 1)][i], bv[j + dy][dx], acc[j][i], 0, 0, 0);
     }
     __syncthreads();
   }
-  // this lane's columns are voxels (z, y0 + FT_R wave + j, x0 + r)
-  const int x = x0 + r;
+  // this lane's columns are voxels (z, y0 + 4 (w % 2) + j, x0 + r)
+  const int x = x0 + r, z = z0 + (wave >> 1);
+  if (x >= a.W || z >= a.D) return;
 #pragma unroll
-  for (int j = 0; j < FT_R; j++) {
-    const int y = y0 + FT_R * wave + j;
-    if (x >= a.W || y >= a.H) continue;
+  for (int j = 0; j < 4; j++) {
+    const int y = y0 + 4 * (wave & 1) + j;
+    if (y >= a.H) continue;
     const int n = (z * a.H + y) * a.W + x;
 #pragma unroll
     for (int i = 0; i < MT; i++) conv_out<MODE>(a, acc[j][i], (rb0 + i) * 16 + kg * 4, n);
+  }
+}
+
+// The products of k_conv_cols (the same k-steps per wave, the same order of every sum) for stride-1
+// 3x3x3 convolutions with a multiple of 32 (padded) channels, in tiles of 16 x 4 voxels: k runs tap
+// plane by tap plane, so LDS holds one halo plane (18 x 6 voxels) of all channels at a time, as
+// [channel group of 8][voxel], and a weight fragment serves 64 voxels (k_conv_cols: 32, and its
+// workgroups read each weight once per 16 or 32 voxels from L2, which bounds it). 192 -> 64 channels on
+// four volumes of 16 x 28 x 28: 102 -> 60 us; 64 -> 64: 45 -> 33 us.
+#define FP_HALO (6 * 18)
+#define FP_HP (FP_HALO + 2)
+
+template <int MODE, int MT>
+__global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
+{
+  extern __shared__ __attribute__((aligned(16))) char s_planes[];
+  bf16x8* const halo = (bf16x8*)s_planes;                 // [Cbp / 8][FP_HP]
+  floatx4* const red = (floatx4*)s_planes;                // [4 waves][2 rows x MT][64]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int tiles_x = (a.W + 15) >> 4, tiles_y = (a.H + 3) >> 2;
+  int b = xcd_order(blockIdx.x, gridDim.x);
+  const int x0 = (b % tiles_x) * 16;
+  b /= tiles_x;
+  const int y0 = (b % tiles_y) * 4;
+  const int z = b / tiles_y;
+  const int rb0 = blockIdx.y * MT;
+  to_sample(a);
+  floatx4 acc[4][MT];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int nsl = a.Cbp >> 5, groups = a.Cbp >> 3, per_plane = 9 * nsl;
+  const int dt = 4 / nsl, dc = 4 - dt * nsl;
+  const size_t astep = (size_t)a.nrb * 2048;
+  const bf16x8* const hp = halo + kg * FP_HP + r;
+  constexpr int kLoads = 6;   // halo loads of a thread in flight
+  for (int p = 0; p < 3; p++) {
+    // the wave's steps w, w + 4, ... inside this tap plane
+    const int first = wave + 4 * ((p * per_plane - wave + 3) >> 2);
+    const int n_mine = ((p + 1) * per_plane - first + 3) >> 2;
+    int t = (first - p * per_plane) / nsl, sl = first - p * per_plane - t * nsl;
+    const __bf16* ap = a.A + ((size_t)first * a.nrb + rb0) * 512 + lane * 8;
+    bf16x8 av[CONV_PF][MT];
+    auto fetch = [&](bf16x8* fa) {
+#pragma unroll
+      for (int i = 0; i < MT; i++) fa[i] = *(const bf16x8*)(ap + i * 512);
+      ap += astep;
+    };
+    auto mult = [&](const bf16x8* fa) {
+      const int q3 = (t * 21846) >> 16, dy = MODE == FWD ? q3 : 2 - q3, dx = MODE == FWD ? t - 3 * q3 : 2 - (t - 3 * q3);
+      const bf16x8* h = hp + sl * (4 * FP_HP) + dy * 18 + dx;
+      bf16x8 bv[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) bv[j] = h[j * 18];
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], bv[j], acc[j][i], 0, 0, 0);
+      sl += dc;
+      t += dt;
+      if (sl >= nsl) {
+        sl -= nsl;
+        t++;
+      }
+    };
+#pragma unroll
+    for (int f = 0; f < CONV_PF; f++)
+      if (f < n_mine) fetch(av[f]);
+    if (p) __syncthreads();   // every wave is done with the last plane
+    const int gz = MODE == FWD ? z + p - 1 : z + 1 - p;
+    for (int i0 = threadIdx.x; i0 < FP_HALO * groups; i0 += 256 * kLoads) {
+      bf16x8 hv[kLoads];
+      int at[kLoads];
+#pragma unroll
+      for (int l = 0; l < kLoads; l++) {
+        const int i = i0 + 256 * l, v = i / groups, q = i - v * groups;
+        const int hy = v / 18, hx = v - hy * 18;
+        const int gy = y0 + hy - 1, gx = x0 + hx - 1;
+        const bool in = v < FP_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
+        const __bf16* g = a.Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.Cbp + q * 8;
+        hv[l] = load_cl(g, in);
+        at[l] = v < FP_HALO ? q * FP_HP + v : -1;
+      }
+#pragma unroll
+      for (int l = 0; l < kLoads; l++)
+        if (at[l] >= 0) halo[at[l]] = hv[l];
+    }
+    __syncthreads();
+    int i = 0;
+    for (; i + 2 * CONV_PF <= n_mine; i += CONV_PF) {
+#pragma unroll
+      for (int f = 0; f < CONV_PF; f++) {
+        mult(av[f]);
+        fetch(av[f]);
+        __builtin_amdgcn_sched_barrier(0);   // the loads are issued here, CONV_PF steps ahead of their use
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < CONV_PF; f++) {
+      if (i + f < n_mine) mult(av[f]);
+      if (i + f + CONV_PF < n_mine) fetch(av[f]);
+    }
+    i += CONV_PF;
+#pragma unroll
+    for (int f = 0; f < CONV_PF; f++)
+      if (i + f < n_mine) mult(av[f]);
+  }
+  // the waves' sums, two rows at a time
+  const int x = x0 + r;
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int i = 0; i < MT; i++) red[(wave * 2 * MT + j * MT + i) * 64 + lane] = acc[2 * h + j][i];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2 * MT; q++) {
+      if ((q & 3) != wave) continue;
+      const floatx4* s = red + q * 64 + lane;
+      const floatx4 sum = s[0] + s[2 * MT * 64] + s[4 * MT * 64] + s[6 * MT * 64];
+      const int y = y0 + 2 * h + q / MT;
+      if (x < a.W && y < a.H) conv_out<MODE>(a, sum, (rb0 + q % MT) * 16 + kg * 4, (z * a.H + y) * a.W + x);
+    }
   }
 }
 
@@ -586,12 +751,37 @@ void launch_cols(const ConvK& a, int mt, hipStream_t st)
 // Forward and input-gradient products outside the tiled form. The tile of a workgroup does not
 // change the order of any sum: it is the largest of the list that still gives COLS_WGS workgroups
 // (two per CU), the smallest where none does.
-#ifndef COLS_WGS
 #define COLS_WGS 512
-#endif
+// k_conv_planes takes a shape when its halo plane fits LDS beside a second workgroup's and its tiles
+// give PLANES_WGS workgroups: with fewer, k_conv_cols' smaller tiles end sooner.
+#define PLANES_WGS 256
+inline long long planes_tiles(const ConvK& a) { return (long long)((a.W + 15) / 16) * ((a.H + 3) / 4) * a.D; }
+inline size_t planes_lds(const ConvK& a, int mt) { return std::max<size_t>(16 * (size_t)(a.Cbp / 8) * FP_HP, 16 * 512 * (size_t)mt); }
+inline bool use_planes(const ConvK& a)
+{
+  const int mt = mt_for(a.M);
+  return a.ks == 3 && a.stride == 1 && a.Cbp % 32 == 0 && planes_lds(a, mt) <= 65536 && planes_tiles(a) <= 0x7fffffffLL &&
+         planes_tiles(a) * (a.nrb / mt) * a.samples >= PLANES_WGS;
+}
+template <int MODE>
+hipError_t launch_planes(const ConvK& a, hipStream_t st)
+{
+  const int mt = mt_for(a.M);
+  const dim3 g((unsigned)planes_tiles(a), a.nrb / mt, a.samples);
+  const unsigned lds = (unsigned)planes_lds(a, mt);
+  switch (mt) {
+    case 1: hipLaunchKernelGGL((k_conv_planes<MODE, 1>), g, dim3(256), lds, st, a); break;
+    case 2: hipLaunchKernelGGL((k_conv_planes<MODE, 2>), g, dim3(256), lds, st, a); break;
+    case 3: hipLaunchKernelGGL((k_conv_planes<MODE, 3>), g, dim3(256), lds, st, a); break;
+    default: hipLaunchKernelGGL((k_conv_planes<MODE, 4>), g, dim3(256), lds, st, a); break;
+  }
+  return hipGetLastError();
+}
+
 template <int MODE>
 hipError_t launch_conv(const ConvK& a, hipStream_t st)
 {
+  if (use_planes(a)) return launch_planes<MODE>(a, st);
   int mt = mt_for(a.M), nc = 2;
   auto wgs = [&](int m, int c) { return (long long)a.samples * (a.nrb / m) * ((a.N + 16 * c - 1) / (16 * c)); };
   if (wgs(mt, nc) < COLS_WGS) {
@@ -639,19 +829,17 @@ inline long long tiled_blocks(const ConvK& a)
 }
 // The tiled products on volumes with at least 1024 four-row tiles (the full-resolution level);
 // smaller volumes (the coarser U-Net levels) keep k_conv's 16-voxel tiles and in-workgroup k split.
-#ifndef MCPET_TILED_MIN
-#define MCPET_TILED_MIN 1024
-#endif
+#define TILED_MIN 1024
 inline bool use_tiled(const ConvK& a)
 {
-  return a.ks == 3 && a.stride == 1 && a.Cbp % 32 == 0 && tiled_blocks(a) >= MCPET_TILED_MIN;
+  return a.ks == 3 && a.stride == 1 && a.Cbp % 32 == 0 && tiled_blocks(a) >= TILED_MIN;
 }
 
 template <int MODE>
 hipError_t launch_conv_tiled(const ConvK& a, hipStream_t st)
 {
   const int mt = mt_for(a.M);
-  const long long tiles = (long long)((a.W + FT_X - 1) / FT_X) * ((a.H + FT_Y - 1) / FT_Y) * a.D;
+  const long long tiles = (long long)((a.W + FT_X - 1) / FT_X) * ((a.H + FT_Y - 1) / FT_Y) * ((a.D + FT_Z - 1) / FT_Z);
   if (a.ks != 3 || a.stride != 1 || a.D != a.oD || a.H != a.oH || a.W != a.oW || a.Cbp % 32 != 0 || a.Kp < 27 * a.Cbp ||
       tiles > 0x7fffffffLL)
     return hipErrorInvalidValue;

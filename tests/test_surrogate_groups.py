@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import mcpet
+from test_surrogate import integer_network, unet_reference
 
 
 def _network(grid, cin, c, rng):
@@ -35,3 +36,20 @@ def test_batch_equals_its_samples(grid, cin, c, batch):
     size = np.mean([np.linalg.norm(g.astype(np.float64)) for _, g in each])
     assert np.linalg.norm(grad - mean) <= 2.0 ** -8 * size
     assert abs(loss - np.mean([l for l, _ in each])) <= 1e-5 * abs(loss)
+
+
+# 20 x 44 x 68 takes the tiles of 16 x 8 x 2 (1100 four-row tiles) with a remainder in x and y, its
+# half resolution the plane-wise products with one in x and y; 36 x 28 x 84 a remainder of every kind
+@pytest.mark.gpu
+@pytest.mark.parametrize("grid,batch", [((20, 44, 68), 2), ((36, 28, 84), 1)])
+def test_ragged_tiles_are_exact_on_integer_networks(grid, batch):
+    """Sums of small integers: equal to the float64 reference bit for bit."""
+    cin, c = 2, 32
+    rng = np.random.default_rng(sum(grid))
+    p = integer_network(cin, c, rng)
+    x = rng.integers(0, 4, (batch, cin) + grid).astype(np.float32)
+    net = mcpet.Surrogate(grid, in_channels=cin, width=c, seed=3)
+    net.set_params(p.astype(np.float32))
+    _, _, yr = unet_reference(p, x.astype(np.float64), np.zeros((batch,) + grid), cin, c, "bf16", grad=False)
+    assert np.abs(yr).max() < 2.0 ** 24 and np.all(yr == np.round(yr))
+    assert np.array_equal(net.forward(x).astype(np.float64), yr)
