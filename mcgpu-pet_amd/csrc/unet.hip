@@ -114,7 +114,9 @@ hipError_t gemm(AOp A, BOp B, float* C, int M, int N, int K, int ldc, const floa
 // (for the next product) beside the FP32 channel-first tensor (which BWGT, the bias gradients and
 // the ReLU masks read). BWGT splits its (voxel) reduction over workgroups.
 
-enum { FWD = 0, BDATA = 1 };
+// FWDUP: FWD of a concatenation whose first Cu channels are the nearest x2 upsampling of a tensor of
+// half the size, read where it is.
+enum { FWD = 0, BDATA = 1, FWDUP = 2 };
 
 // Where an epilogue writes a channels-last BF16 copy of its output: element (m, n) at
 // p[n * ld + off + m] (p null: no copy).
@@ -127,17 +129,21 @@ struct ConvK {
   const __bf16* A;     // FWD, BDATA: BF16 weights [Kp / 32][nrb][64 lanes][8] (k_derive)
   const float* Ad;     // BWGT: dY [M][K]
   const float* X;      // BWGT: input activations [Cin][D][H][W]
-  const __bf16* Xl;    // FWD: input activations [D][H][W][Cbp]; BDATA: dY [oD][oH][oW][Cbp] (channels-last BF16)
-  ClOut o1, o2;        // FWD, BDATA: channels-last copies of the output
+  const __bf16* Xl;    // FWD: input activations [D][H][W][ldx]; BDATA: dY [oD][oH][oW][ldx] (channels-last BF16)
+  const __bf16* Xu;    // FWDUP: channels 0 .. Cu - 1 at half size, [D/2][H/2][W/2][ldu]; Xl holds the others
+  int ldx, ldu, Cu;
+  ClOut o1;            // FWD, BDATA: channels-last copy of the output
   float* C;            // FWD: Y [M][N]; BDATA: dX [M][N]; BWGT: weight gradient [Cout][Cin][T]
   const float* bias;   // FWD
-  const float* mask;   // BDATA: the layer input (gradient zero where it is <= 0: the ReLU before it); may be null
+  const __bf16* mask;  // BDATA: the layer input's channels from mask0 on, [N][ldm] (gradient zero where it is
+  int ldm, mask0;      // not positive: the ReLU before it); may be null
+  const float* res;    // FWD with M = 1: added to the output; may be null
   int relu, beta;      // FWD: ReLU on the output; BDATA: add to C
   int M, N, K, Kp;     // GEMM sizes; Kp: K padded to whole k-steps
   int nrb;             // 16-row blocks of A
   int Cb, Cbp;         // channels of the B tensor (FWD, BWGT: Cin; BDATA: Cout) and Cb rounded up to 8
   int D, H, W, oD, oH, oW, ks, stride, T;
-  size_t sX, sC;       // from one sample to the next (blockIdx.z): B tensor; C and mask (BWGT: X; Ad)
+  size_t sX, sXu, sC, sR;   // from one sample to the next (blockIdx.z): B tensor(s); C; res (BWGT: X; -; Ad)
   int samples;
   int k_per_split, splits;   // BWGT: voxels per workgroup, workgroups per sample
   int vec;             // BWGT: K % 4 == 0 (dY rows are float4-aligned)
@@ -223,22 +229,62 @@ __global__ __launch_bounds__(256) void k_conv_bwgt(ConvK a)
   }
 }
 
-// the tensors of sample blockIdx.z
-__device__ __forceinline__ void to_sample(ConvK& a)
+// the tensors of sample z
+__device__ __forceinline__ void to_sample(ConvK& a, size_t z)
 {
-  const size_t z = blockIdx.z;
   a.Xl += z * a.sX;
+  if (a.Xu) a.Xu += z * a.sXu;
   if (a.C) a.C += z * a.sC;
-  if (a.mask) a.mask += z * a.sC;
+  if (a.res) a.res += z * a.sR;
+  if (a.mask) a.mask += z * a.N * a.ldm;
   if (a.o1.p) a.o1.p += z * a.N * a.o1.ld;
-  if (a.o2.p) a.o2.p += z * a.N * a.o2.ld;
 }
 
-// One output tile's four rows row0 .. row0 + 3 of column n (FWD: bias, ReLU; BDATA: add, mask) and
-// their channels-last copies.
+// What the epilogue of rows row0 .. row0 + 3 of column n reads: FWD the bias, BDATA the ReLU mask (the
+// sign of the forward's BF16 copy) and what it adds to. Read apart from the stores, so that a wave's
+// reads are in flight together.
+struct ConvIn {
+  float c[4];   // FWD: bias; BDATA: the earlier C, 0 without beta
+  bool on[4];   // BDATA: not masked
+};
 template <int MODE>
-__device__ __forceinline__ void conv_out(const ConvK& a, const floatx4& s, int row0, int n)
+__device__ __forceinline__ ConvIn conv_in(const ConvK& a, int row0, int n)
 {
+  ConvIn q;
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    q.c[v] = 0.0f;
+    q.on[v] = true;
+  }
+  if (row0 >= a.M || (MODE == BDATA && n >= a.N)) return q;
+  if (MODE != BDATA) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) q.c[v] = row0 + v < a.M ? a.bias[row0 + v] : 0.0f;
+    return q;
+  }
+  if (a.beta)
+#pragma unroll
+    for (int v = 0; v < 4; v++) q.c[v] = row0 + v < a.M ? a.C[(size_t)(row0 + v) * a.N + n] : 0.0f;
+  if (a.mask && row0 + 3 >= a.mask0) {
+    const __bf16* m = a.mask + (size_t)n * a.ldm - a.mask0;
+    if ((a.mask0 & 3) == 0) {   // ldm is a multiple of 8: the four exist
+      const bf16x4 m4 = *(const bf16x4*)(m + row0);
+#pragma unroll
+      for (int v = 0; v < 4; v++) q.on[v] = (float)m4[v] > 0.0f;
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        if (row0 + v >= a.mask0 && row0 + v < a.M) q.on[v] = (float)m[row0 + v] > 0.0f;
+    }
+  }
+  return q;
+}
+
+// Those four rows (FWD: bias, ReLU; BDATA: add, mask) and their channels-last copy.
+template <int MODE>
+__device__ __forceinline__ void conv_out(const ConvK& a, const ConvIn& q, const floatx4& s, int row0, int n)
+{
+  if (row0 >= a.M) return;
   float ov[4];
 #pragma unroll
   for (int v = 0; v < 4; v++) {
@@ -246,35 +292,28 @@ __device__ __forceinline__ void conv_out(const ConvK& a, const floatx4& s, int r
     ov[v] = 0.0f;
     if (row >= a.M) continue;
     const size_t idx = (size_t)row * a.N + n;
-    float o;
-    if (MODE == FWD) {
-      o = s[v] + a.bias[row];
+    float o = s[v] + q.c[v];
+    if (MODE != BDATA) {
       if (a.relu) o = fmaxf(o, 0.0f);
-      if (a.C) a.C[idx] = o;   // null: no FP32 copy (inference)
+      if (a.C) a.C[idx] = a.res ? a.res[n] + o : o;   // null: no FP32 copy
     } else {
-      o = s[v] + (a.beta ? a.C[idx] : 0.0f);
-      if (a.mask && !(a.mask[idx] > 0.0f)) o = 0.0f;
+      if (!q.on[v]) o = 0.0f;
       a.C[idx] = o;
     }
     ov[v] = o;
   }
   // the four channels in one 8-byte store when they all exist
-  const ClOut* outs[2] = {&a.o1, &a.o2};
+  if (!a.o1.p) return;
+  __bf16* dst = a.o1.p + (size_t)n * a.o1.ld + a.o1.off + row0;
+  if (row0 + 3 < a.M && ((a.o1.ld | a.o1.off) & 3) == 0) {
+    bf16x4 w;
 #pragma unroll
-  for (int j = 0; j < 2; j++) {
-    const ClOut& o = *outs[j];
-    if (!o.p) continue;
-    __bf16* dst = o.p + (size_t)n * o.ld + o.off + row0;
-    if (row0 + 3 < a.M && ((o.ld | o.off) & 3) == 0) {
-      bf16x4 q;
+    for (int v = 0; v < 4; v++) w[v] = to_bf16(ov[v]);
+    *(bf16x4*)dst = w;
+  } else {
 #pragma unroll
-      for (int v = 0; v < 4; v++) q[v] = to_bf16(ov[v]);
-      *(bf16x4*)dst = q;
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        if (row0 + v < a.M) dst[v] = to_bf16(ov[v]);
-    }
+    for (int v = 0; v < 4; v++)
+      if (row0 + v < a.M) dst[v] = to_bf16(ov[v]);
   }
 }
 
@@ -286,6 +325,18 @@ __device__ __attribute__((aligned(16))) const unsigned k_zeros[4] = {0u, 0u, 0u,
 __device__ __forceinline__ bf16x8 load_cl(const __bf16* p, bool in)
 {
   return *(const __attribute__((address_space(1))) bf16x8*)(in ? (unsigned long long)p : (unsigned long long)k_zeros);
+}
+
+// the 8 channels from c on of input voxel (z, y, x)
+template <int MODE>
+__device__ __forceinline__ const __bf16* voxel_cl(const ConvK& a, int z, int y, int x, int c)
+{
+  if (MODE == FWDUP) {
+    const bool up = c < a.Cu;
+    const size_t v = up ? ((size_t)(z >> 1) * (a.H >> 1) + (y >> 1)) * (a.W >> 1) + (x >> 1) : ((size_t)z * a.H + y) * a.W + x;
+    return (up ? a.Xu : a.Xl) + v * (up ? a.ldu : a.ldx) + (up ? c : c - a.Cu);
+  }
+  return a.Xl + (((size_t)z * a.H + y) * a.W + x) * a.ldx + c;
 }
 
 // bits t of the taps t = 9 (dz + 1) + 3 (dy + 1) + (dx + 1) whose three bits are all set
@@ -309,20 +360,19 @@ __device__ __forceinline__ unsigned tap_mask(unsigned vz, unsigned vy, unsigned 
 template <int MODE, int MT, int NC, bool kSkip>
 __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
 {
-  static_assert(MODE == FWD || MODE == BDATA, "forward and input-gradient products only");
   __shared__ floatx4 red[4][NC * MT][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int r = lane & 15, kg = lane >> 4;
   const int rb0 = blockIdx.y * MT;
-  to_sample(a);
-  int nn[NC], base[NC];
+  to_sample(a, blockIdx.z);
+  int nn[NC], base[NC], cx[NC], cy[NC], cz[NC];   // c?: FWDUP's input voxel
   unsigned mask[NC];
   // the tap's step in the B tensor: rows and planes of that tensor
-  const int bW = MODE == FWD ? a.W : a.oW, bH = MODE == FWD ? a.H : a.oH;
+  const int bW = MODE != BDATA ? a.W : a.oW, bH = MODE != BDATA ? a.H : a.oH;
 #pragma unroll
   for (int j = 0; j < NC; j++) {
     int n = (blockIdx.x * NC + j) * 16 + r;   // this lane's column in tile j
-    const int w = MODE == FWD ? a.oW : a.W, h = MODE == FWD ? a.oH : a.H, d = MODE == FWD ? a.oD : a.D;
+    const int w = MODE != BDATA ? a.oW : a.W, h = MODE != BDATA ? a.oH : a.H, d = MODE != BDATA ? a.oD : a.D;
     int x, y, z;
     if (kSkip) {
       const int per = a.N >> 3, cls = n / per, i = n - cls * per, w2 = w >> 1, h2 = h >> 1;
@@ -338,7 +388,7 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
     }
     nn[j] = n;
     unsigned vx = 7, vy = 7, vz = 7;
-    if (MODE == FWD) {
+    if (MODE != BDATA) {
       x *= a.stride;
       y *= a.stride;
       z *= a.stride;
@@ -369,6 +419,9 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
       if (z + 1 >= d) vz &= ~1u;
       base[j] = (z * h + y) * w + x;
     }
+    cx[j] = x;
+    cy[j] = y;
+    cz[j] = z;
     mask[j] = n < a.N ? (a.ks == 3 ? tap_mask(vz, vy, vx) : 1u) : 0u;
   }
   floatx4 acc[NC][MT];
@@ -399,13 +452,16 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
     }
   };
   auto fetch = [&](bf16x8* fa, bf16x8* fb) {   // step `step`, then on to the wave's next one
-    int off = 0;
+    int off = 0, oz = 0, oy = 0, ox = 0;
     if (a.ks == 3) {   // t / 9 = (7282 t) >> 16 and t / 3 = (21846 t) >> 16, exact for t < 32
       const int q9 = (t * 7282) >> 16, q3 = (t * 21846) >> 16;
       const int uz = q9, uy = q3 - 3 * q9, ux = t - 3 * q3;   // d + 1
       if (kSkip) off = -(((uz >> 1) * bH + (uy >> 1)) * bW + (ux >> 1));
       else {
-        off = ((uz - 1) * bH + (uy - 1)) * bW + (ux - 1);
+        oz = uz - 1;
+        oy = uy - 1;
+        ox = ux - 1;
+        off = (oz * bH + oy) * bW + ox;
         if (MODE == BDATA) off = -off;
       }
     }
@@ -414,7 +470,8 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
 #pragma unroll
     for (int j = 0; j < NC; j++) {
       const bool in = t < 32 && ((mask[j] >> t) & 1u);
-      const __bf16* p = a.Xl + ((size_t)(unsigned)(base[j] + off) * (unsigned)Cbp + (unsigned)c0);
+      const __bf16* p = MODE == FWDUP ? voxel_cl<MODE>(a, cz[j] + oz, cy[j] + oy, cx[j] + ox, c0)
+                                      : a.Xl + ((size_t)(unsigned)(base[j] + off) * (unsigned)a.ldx + (unsigned)c0);
       fb[j] = load_cl(p, in);
     }
     advance();
@@ -470,14 +527,18 @@ __global__ __launch_bounds__(256) void k_conv_cols(ConvK a)
   for (int j = 0; j < NC; j++)
 #pragma unroll
     for (int i = 0; i < MT; i++) red[wave][j * MT + i][lane] = acc[j][i];
-  __syncthreads();
   // wave w finishes the (tile, row block) pairs w, w + 4, ...
+  ConvIn pre[(NC * MT + 3) / 4];
+#pragma unroll
+  for (int q = 0; q < NC * MT; q++)
+    if ((q & 3) == wave) pre[q / 4] = conv_in<MODE>(a, (rb0 + q % MT) * 16 + kg * 4, nn[q / MT]);
+  __syncthreads();
 #pragma unroll
   for (int q = 0; q < NC * MT; q++) {
     if ((q & 3) != wave) continue;
     const floatx4 s = red[0][q][lane] + red[1][q][lane] + red[2][q][lane] + red[3][q][lane];
-    const int j = q / MT, i = q % MT;
-    if (nn[j] < a.N) conv_out<MODE>(a, s, (rb0 + i) * 16 + kg * 4, nn[j]);
+    const int j = q / MT;
+    if (nn[j] < a.N) conv_out<MODE>(a, pre[q / 4], s, (rb0 + q % MT) * 16 + kg * 4, nn[j]);
   }
 }
 
@@ -522,7 +583,7 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
   const int y0 = (b % tiles_y) * FT_Y;
   const int z0 = (b / tiles_y) * FT_Z;
   const int rb0 = blockIdx.y * MT;
-  to_sample(a);
+  to_sample(a, blockIdx.z);
   floatx4 acc[4][MT];
 #pragma unroll
   for (int j = 0; j < 4; j++)
@@ -546,7 +607,7 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
       const int hx = v % FT_HX, hy = (v / FT_HX) % FT_HY, hz = v / (FT_HX * FT_HY);
       const int gz = z0 + hz - 1, gy = y0 + hy - 1, gx = x0 + hx - 1;
       const bool in = v < FT_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
-      const __bf16* p = a.Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.Cbp + c0 + q * 8;
+      const __bf16* p = voxel_cl<MODE>(a, gz, gy, gx, c0 + q * 8);
       hv[l] = load_cl(p, in);
     }
 #pragma unroll
@@ -558,9 +619,9 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
     bf16x8 bv[6][3];
 #pragma unroll
     for (int t = 0; t < 27; t++) {
-      const int dz = MODE == FWD ? t / 9 : 2 - t / 9;            // halo coordinates of p + d_t or p - d_t
-      const int dy = MODE == FWD ? (t / 3) % 3 : 2 - (t / 3) % 3;
-      const int dx = MODE == FWD ? t % 3 : 2 - t % 3;
+      const int dz = MODE != BDATA ? t / 9 : 2 - t / 9;            // halo coordinates of p + d_t or p - d_t
+      const int dy = MODE != BDATA ? (t / 3) % 3 : 2 - (t / 3) % 3;
+      const int dx = MODE != BDATA ? t % 3 : 2 - t % 3;
       if (t % 9 == 0) {
 #pragma unroll
         for (int y = 0; y < 6; y++)
@@ -584,13 +645,20 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
   // this lane's columns are voxels (z, y0 + 4 (w % 2) + j, x0 + r)
   const int x = x0 + r, z = z0 + (wave >> 1);
   if (x >= a.W || z >= a.D) return;
+  constexpr int kIn = MODE == BDATA ? 4 : 1;   // FWD: the rows' bias serves every column
+  ConvIn pre[kIn][MT];
+  const int yw = y0 + 4 * (wave & 1);
+#pragma unroll
+  for (int j = 0; j < kIn; j++)
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+      pre[j][i] = conv_in<MODE>(a, (rb0 + i) * 16 + kg * 4, yw + j < a.H ? (z * a.H + yw + j) * a.W + x : a.N);
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    const int y = y0 + 4 * (wave & 1) + j;
-    if (y >= a.H) continue;
-    const int n = (z * a.H + y) * a.W + x;
+    if (yw + j >= a.H) continue;
+    const int n = (z * a.H + yw + j) * a.W + x;
 #pragma unroll
-    for (int i = 0; i < MT; i++) conv_out<MODE>(a, acc[j][i], (rb0 + i) * 16 + kg * 4, n);
+    for (int i = 0; i < MT; i++) conv_out<MODE>(a, pre[j % kIn][i], acc[j][i], (rb0 + i) * 16 + kg * 4, n);
   }
 }
 
@@ -618,7 +686,7 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
   const int y0 = (b % tiles_y) * 4;
   const int z = b / tiles_y;
   const int rb0 = blockIdx.y * MT;
-  to_sample(a);
+  to_sample(a, blockIdx.z);
   floatx4 acc[4][MT];
 #pragma unroll
   for (int j = 0; j < 4; j++)
@@ -642,7 +710,7 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
       ap += astep;
     };
     auto mult = [&](const bf16x8* fa) {
-      const int q3 = (t * 21846) >> 16, dy = MODE == FWD ? q3 : 2 - q3, dx = MODE == FWD ? t - 3 * q3 : 2 - (t - 3 * q3);
+      const int q3 = (t * 21846) >> 16, dy = MODE != BDATA ? q3 : 2 - q3, dx = MODE != BDATA ? t - 3 * q3 : 2 - (t - 3 * q3);
       const bf16x8* h = hp + sl * (4 * FP_HP) + dy * 18 + dx;
       bf16x8 bv[4];
 #pragma unroll
@@ -662,7 +730,7 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
     for (int f = 0; f < CONV_PF; f++)
       if (f < n_mine) fetch(av[f]);
     if (p) __syncthreads();   // every wave is done with the last plane
-    const int gz = MODE == FWD ? z + p - 1 : z + 1 - p;
+    const int gz = MODE != BDATA ? z + p - 1 : z + 1 - p;
     for (int i0 = threadIdx.x; i0 < FP_HALO * groups; i0 += 256 * kLoads) {
       bf16x8 hv[kLoads];
       int at[kLoads];
@@ -672,7 +740,7 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
         const int hy = v / 18, hx = v - hy * 18;
         const int gy = y0 + hy - 1, gx = x0 + hx - 1;
         const bool in = v < FP_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
-        const __bf16* g = a.Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.Cbp + q * 8;
+        const __bf16* g = voxel_cl<MODE>(a, gz, gy, gx, q * 8);
         hv[l] = load_cl(g, in);
         at[l] = v < FP_HALO ? q * FP_HP + v : -1;
       }
@@ -709,6 +777,13 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
     for (int j = 0; j < 2; j++)
 #pragma unroll
       for (int i = 0; i < MT; i++) red[(wave * 2 * MT + j * MT + i) * 64 + lane] = acc[2 * h + j][i];
+    ConvIn pre[(2 * MT + 3) / 4];
+#pragma unroll
+    for (int q = 0; q < 2 * MT; q++) {
+      const int y = y0 + 2 * h + q / MT;
+      if ((q & 3) == wave)
+        pre[q / 4] = conv_in<MODE>(a, (rb0 + q % MT) * 16 + kg * 4, x < a.W && y < a.H ? (z * a.H + y) * a.W + x : a.N);
+    }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 2 * MT; q++) {
@@ -716,7 +791,89 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
       const floatx4* s = red + q * 64 + lane;
       const floatx4 sum = s[0] + s[2 * MT * 64] + s[4 * MT * 64] + s[6 * MT * 64];
       const int y = y0 + 2 * h + q / MT;
-      if (x < a.W && y < a.H) conv_out<MODE>(a, sum, (rb0 + q % MT) * 16 + kg * 4, (z * a.H + y) * a.W + x);
+      if (x < a.W && y < a.H) conv_out<MODE>(a, pre[q / 4], sum, (rb0 + q % MT) * 16 + kg * 4, (z * a.H + y) * a.W + x);
+    }
+  }
+}
+
+// The products of k_conv_cols with at most SHORT_STEPS k-steps (8 or fewer padded channels, or a
+// 1x1x1 kernel): reading and writing bounds them, so the weights stay in registers and each wave takes
+// 16-voxel tiles by itself, all steps of one (the four sums that k_conv_cols' waves would hold, added
+// in their order), the next tile's voxels in flight. Four volumes of 32 x 56 x 56: 4 -> 32 channels
+// 49 -> 32 us, 32 -> 1 22 -> 8 us, the latter's input gradient 50 -> 22 us.
+#define SHORT_STEPS 8
+template <int MODE, int MT, int NS>
+__global__ __launch_bounds__(256) void k_conv_short(ConvK a)
+{
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int r = lane & 15, kg = lane >> 4;
+  const int rb0 = blockIdx.y * MT;
+  to_sample(a, blockIdx.z);
+  bf16x8 av[NS][MT], bv[NS];
+  int t[NS], c0[NS];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)   // steps that K does not have multiply zeros
+      av[s][i] = load_cl(a.A + ((size_t)s * a.nrb + rb0 + i) * 512 + lane * 8, 32 * s < a.K);
+    const int k = 32 * s + 8 * kg;
+    t[s] = k / a.Cbp;
+    c0[s] = k - t[s] * a.Cbp;
+  }
+  const int tiles = (a.N + 15) >> 4, step = gridDim.x * 4;
+  auto fetch = [&](int tile) {
+    const int n = tile * 16 + r;
+    const int x = n % a.W, y = (n / a.W) % a.H, z = n / (a.W * a.H);
+    unsigned vx = 7, vy = 7, vz = 7;
+    constexpr unsigned lo = MODE == BDATA ? 4u : 1u, hi = 5u - lo;   // the taps that leave at 0 and at the end
+    if (x == 0) vx &= ~lo;
+    if (y == 0) vy &= ~lo;
+    if (z == 0) vz &= ~lo;
+    if (x + 1 >= a.W) vx &= ~hi;
+    if (y + 1 >= a.H) vy &= ~hi;
+    if (z + 1 >= a.D) vz &= ~hi;
+    const unsigned mask = n < a.N ? (a.ks == 3 ? tap_mask(vz, vy, vx) : 1u) : 0u;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      int off = 0;
+      if (a.ks == 3) {
+        const int q9 = (t[s] * 7282) >> 16, q3 = (t[s] * 21846) >> 16;
+        off = ((q9 - 1) * a.H + (q3 - 3 * q9 - 1)) * a.W + (t[s] - 3 * q3 - 1);
+        if (MODE == BDATA) off = -off;
+      }
+      const bool in = t[s] < 32 && ((mask >> t[s]) & 1u);
+      const size_t v = (unsigned)(n + off);
+      bv[s] = load_cl(a.Xl + v * a.ldx + c0[s], in);
+    }
+  };
+  int tile = blockIdx.x * 4 + wave;
+  ConvIn pre[MT];
+#pragma unroll
+  for (int i = 0; i < MT; i++) pre[i] = conv_in<MODE>(a, (rb0 + i) * 16 + kg * 4, tile * 16 + r);
+  if (tile < tiles) fetch(tile);
+  while (tile < tiles) {
+    floatx4 acc[MT][4];   // steps 0, 4, ...; 1, 5, ...; 2, 6, ...; 3, 7, ...
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+      for (int i = 0; i < MT; i++) acc[i][s & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[s][i], bv[s], acc[i][s & 3], 0, 0, 0);
+    const int n = tile * 16 + r;
+    tile += step;
+    if (tile < tiles) fetch(tile);
+    ConvIn now[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      now[i] = pre[i];
+      if (MODE == BDATA && tile < tiles) pre[i] = conv_in<MODE>(a, (rb0 + i) * 16 + kg * 4, tile * 16 + r);
+    }
+    if (n < a.N) {
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+        conv_out<MODE>(a, now[i], acc[i][0] + acc[i][1] + acc[i][2] + acc[i][3], (rb0 + i) * 16 + kg * 4, n);
     }
   }
 }
@@ -778,9 +935,38 @@ hipError_t launch_planes(const ConvK& a, hipStream_t st)
   return hipGetLastError();
 }
 
+inline bool use_short(const ConvK& a) { return a.stride == 1 && a.K <= 32 * SHORT_STEPS; }
+template <int MODE, int MT>
+void launch_short_ns(const ConvK& a, dim3 g, hipStream_t st)
+{
+  const int ns = (a.K + 31) / 32;
+  if (ns == 1) hipLaunchKernelGGL((k_conv_short<MODE, MT, 1>), g, dim3(256), 0, st, a);
+  else if (ns == 2) hipLaunchKernelGGL((k_conv_short<MODE, MT, 2>), g, dim3(256), 0, st, a);
+  else if (ns <= 4) hipLaunchKernelGGL((k_conv_short<MODE, MT, 4>), g, dim3(256), 0, st, a);
+  else if constexpr (MT <= 2) hipLaunchKernelGGL((k_conv_short<MODE, MT, 8>), g, dim3(256), 0, st, a);
+}
+template <int MODE>
+hipError_t launch_short(const ConvK& a, hipStream_t st)
+{
+  int mt = mt_for(a.M);
+  if (a.K > 128) mt = mt == 4 ? 2 : mt == 3 ? 1 : mt;   // eight steps' weights of more blocks take over 256 registers
+  const int tiles = (a.N + 15) / 16;
+  // the workgroups that are resident together, so that a wave's weights serve several tiles
+  const int most = std::max(1, (a.K > 128 ? 512 : 2048) / (a.samples * (a.nrb / mt)));
+  const dim3 g(std::min((tiles + 3) / 4, most), a.nrb / mt, a.samples);
+  switch (mt) {
+    case 1: launch_short_ns<MODE, 1>(a, g, st); break;
+    case 2: launch_short_ns<MODE, 2>(a, g, st); break;
+    case 3: launch_short_ns<MODE, 3>(a, g, st); break;
+    default: launch_short_ns<MODE, 4>(a, g, st); break;
+  }
+  return hipGetLastError();
+}
+
 template <int MODE>
 hipError_t launch_conv(const ConvK& a, hipStream_t st)
 {
+  if (MODE != FWDUP && use_short(a)) return launch_short<MODE == FWDUP ? FWD : MODE>(a, st);
   if (use_planes(a)) return launch_planes<MODE>(a, st);
   int mt = mt_for(a.M), nc = 2;
   auto wgs = [&](int m, int c) { return (long long)a.samples * (a.nrb / m) * ((a.N + 16 * c - 1) / (16 * c)); };
@@ -874,11 +1060,13 @@ hipError_t launch_conv_tiled(const ConvK& a, hipStream_t st)
 
 struct BwK {
   const __bf16* Xl;   // input, channels-last [vox][ldx] (channels >= ldx: zero)
+  const __bf16* Xu;   // its first Cu channels at half size, [vox / 8][ldu] (Cu = 0: none; Xl then holds the others)
+  int ldu, Cu;
   const __bf16* Gl;   // output gradient, channels-last [ovox][ldg]
   float* part;        // [n_slabs][27][32 cob][32 cib]
-  int ldx, ldg, Cin, Cout, D, H, W, oD, oH, oW;
+  int ldx, ldg, gch, Cin, Cout, D, H, W, oD, oH, oW;   // gch: channels from Gl on
   int tiles_x, tiles_y, n_tiles, per_slab, cob, cib;   // n_tiles: of all samples
-  size_t sX, sG;                                       // from one sample to the next
+  size_t sX, sXu, sG;                                  // from one sample to the next
 };
 
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -937,6 +1125,7 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
     b /= a.tiles_y;
     const int z0 = b % a.oD, smp = b / a.oD;
     const __bf16* const Xl = a.Xl + smp * a.sX;
+    const __bf16* const Xu = a.Xu + smp * a.sXu;
     const __bf16* const Gl = a.Gl + smp * a.sG;
     // input region: voxel (S z0 - 1 + hz, S y0 - 1 + hy, S x0 - 1 + hx), 4 groups of 8 channels
     for (int i = threadIdx.x; i < 3 * HY * HX * 4; i += BW_THREADS) {
@@ -945,8 +1134,10 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
       const int gz = S * z0 + hz - 1, gy = S * y0 + hy - 1, gx = S * x0 + hx - 1;
       const int c = ci0 + q * 8;
       bf16x8 v = zero;
-      if (gz >= 0 && gz < a.D && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W && c < a.ldx)
-        v = *(const bf16x8*)(Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.ldx + c);
+      if (gz >= 0 && gz < a.D && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W && c < a.Cu + a.ldx) {
+        if (c < a.Cu) v = *(const bf16x8*)(Xu + (((size_t)(gz >> 1) * (a.H >> 1) + (gy >> 1)) * (a.W >> 1) + (gx >> 1)) * a.ldu + c);
+        else v = *(const bf16x8*)(Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.ldx + (c - a.Cu));
+      }
       if constexpr (S == 1) {
 #pragma unroll
         for (int e = 0; e < 8; e++) L.x[q * 8 + e][hz][hy][hx + 7] = v[e];
@@ -964,7 +1155,7 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
       const int gy = y0 + (qv >> 4), gx = x0 + (qv & 15);
       const int c = co0 + q4 * 8;
       bf16x8 v = zero;
-      if (gy < a.oH && gx < a.oW && c < a.ldg)
+      if (gy < a.oH && gx < a.oW && c < a.gch)
         v = *(const bf16x8*)(Gl + (((size_t)z0 * a.oH + gy) * a.oW + gx) * a.ldg + c);
 #pragma unroll
       for (int e = 0; e < 8; e++) gs[q4 * 8 + e][qv] = v[e];
@@ -1068,47 +1259,29 @@ inline void bwgt_shape(int samples, int oD, int oH, int oW, int Cin, int Cout, B
   b.per_slab = (b.n_tiles + n_slabs - 1) / n_slabs;
   n_slabs = (b.n_tiles + b.per_slab - 1) / b.per_slab;
 }
-constexpr size_t kBwPartFloats = (size_t)BW_WGS * 27 * 1024;
+constexpr size_t kBwPartFloats = (size_t)BW_WGS * 27 * 1024;   // a workgroup writes 27 x 32 x 32
 
-// true when the tiled weight gradient takes this layer (its slab sums fit the buffer)
-inline bool bwgt_fits(int samples, int oD, int oH, int oW, int Cin, int Cout)
+// The input x and its gradient's copy gyl as in conv_bwd_weights; stride 1 (input and output volumes
+// equal) or 2 (output (D/2, H/2, W/2)). Output channels go in passes of as many 32-channel blocks as
+// the partial sums have room for (all of them up to 512 blocks of 32 x 32).
+hipError_t launch_bwgt_tiled(int samples, int stride, BwK b, const __bf16* gyl, float* G, hipStream_t st)
 {
-  BwK b{};
-  int n_slabs = 0;
-  bwgt_shape(samples, oD, oH, oW, Cin, Cout, b, n_slabs);
-  return (size_t)n_slabs * 27 * (32 * b.cob) * (32 * b.cib) <= kBwPartFloats;
-}
-
-// stride 1 (input and output volumes equal) or 2 (output (D/2, H/2, W/2) rounded down or up)
-hipError_t launch_bwgt_tiled(int samples, int stride, const __bf16* xl, int ldx, const __bf16* gyl, int ldg, int Cin, int Cout, int D, int H,
-                             int W, int oD, int oH, int oW, float* part, float* G, hipStream_t st)
-{
-  BwK b{};
-  int n_slabs = 0;
-  bwgt_shape(samples, oD, oH, oW, Cin, Cout, b, n_slabs);
-  if ((size_t)n_slabs * 27 * (32 * b.cob) * (32 * b.cib) > kBwPartFloats || ldx % 8 != 0 || ldg % 8 != 0 ||
-      (stride != 1 && stride != 2))
-    return hipErrorInvalidValue;
-  b.Xl = xl;
-  b.Gl = gyl;
-  b.part = part;
-  b.ldx = ldx;
-  b.sX = (size_t)D * H * W * ldx;
-  b.sG = (size_t)oD * oH * oW * ldg;
-  b.ldg = ldg;
-  b.Cin = Cin;
-  b.Cout = Cout;
-  b.D = D;
-  b.H = H;
-  b.W = W;
-  b.oD = oD;
-  b.oH = oH;
-  b.oW = oW;
-  if (stride == 1) hipLaunchKernelGGL(k_bwgt_tiled<1>, dim3(n_slabs, b.cob, b.cib), dim3(BW_THREADS), 0, st, b);
-  else hipLaunchKernelGGL(k_bwgt_tiled<2>, dim3(n_slabs, b.cob, b.cib), dim3(BW_THREADS), 0, st, b);
-  const long long n = (long long)Cout * Cin * 27;
-  hipLaunchKernelGGL(k_bwgt_reduce, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float*)part, G, Cout, Cin,
-                     32 * b.cob, 32 * b.cib, n_slabs);
+  if (b.ldx % 8 != 0 || b.ldg % 8 != 0 || (stride != 1 && stride != 2)) return hipErrorInvalidValue;
+  const int cout = b.Cout, cib = (b.Cin + 31) / 32, most = BW_WGS / cib * 32;
+  if (most == 0) return hipErrorInvalidValue;
+  for (int co = 0; co < cout; co += most) {
+    b.Cout = std::min(most, cout - co);
+    b.Gl = gyl + co;
+    b.gch = b.ldg - co;
+    int n_slabs = 0;
+    bwgt_shape(samples, b.oD, b.oH, b.oW, b.Cin, b.Cout, b, n_slabs);
+    const dim3 g(n_slabs, b.cob, b.cib);
+    if (stride == 1) hipLaunchKernelGGL(k_bwgt_tiled<1>, g, dim3(BW_THREADS), 0, st, b);
+    else hipLaunchKernelGGL(k_bwgt_tiled<2>, g, dim3(BW_THREADS), 0, st, b);
+    const long long n = (long long)b.Cout * b.Cin * 27;
+    hipLaunchKernelGGL(k_bwgt_reduce, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float*)b.part,
+                       G + (size_t)co * b.Cin * 27, b.Cout, b.Cin, 32 * b.cob, 32 * b.cib, n_slabs);
+  }
   return hipGetLastError();
 }
 
@@ -1134,72 +1307,66 @@ __global__ void k_derive(const float* __restrict__ w, __bf16* __restrict__ out, 
 
 // Elementwise kernels take sample blockIdx.y; a tensor that is part of a larger one comes with its
 // step from sample to sample.
-// nearest x2 upsampling of [C][d][h][w] into [C][2d][2h][2w] (and its channels-last copy o)
-__global__ void k_upsample(const float* __restrict__ x, float* __restrict__ y, size_t sy, int C, int d, int h, int w, ClOut o)
+// Channels-last concatenation of the nearest x2 upsampling of u [D/2][H/2][W/2][ldu] (Cu channels) and of
+// l [D][H][W][ldl] (Cl channels) into o: where Cu is not a multiple of 8 (else the products read u and l
+// themselves).
+__global__ void k_concat(const __bf16* __restrict__ u, int Cu, int ldu, const __bf16* __restrict__ l, int Cl, int ldl, int D, int H,
+                         int W, ClOut o)
 {
-  x += blockIdx.y * ((size_t)C * d * h * w);
-  if (y) y += blockIdx.y * sy;
-  if (o.p) o.p += blockIdx.y * ((size_t)8 * d * h * w) * o.ld;
-  const size_t n = (size_t)C * 8 * d * h * w;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int W2 = 2 * w, H2 = 2 * h, D2 = 2 * d;
-  const size_t vox2 = (size_t)W2 * H2 * D2;
-  const int xx = (int)(i % W2), yy = (int)((i / W2) % H2), zz = (int)((i / ((size_t)W2 * H2)) % D2);
-  const int c = (int)(i / vox2);
-  const float v = x[(((size_t)c * d + zz / 2) * h + yy / 2) * w + xx / 2];
-  if (y) y[i] = v;   // null: no FP32 copy (inference)
-  if (o.p) o.p[(i % vox2) * o.ld + o.off + c] = to_bf16(v);
+  const size_t vox = (size_t)D * H * W, i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= vox * (Cu + Cl)) return;
+  const size_t v = i / (Cu + Cl), vl = blockIdx.y * vox + v;
+  const int c = (int)(i % (Cu + Cl));
+  const int x = (int)(v % W), y = (int)((v / W) % H), z = (int)(v / ((size_t)W * H));
+  const size_t vu = blockIdx.y * (vox / 8) + ((size_t)(z / 2) * (H / 2) + y / 2) * (W / 2) + x / 2;
+  o.p[vl * o.ld + c] = c < Cu ? u[vu * ldu + c] : l[vl * ldl + c - Cu];
 }
-// k_upsample with each thread on 8 channels of one output voxel: the FP32 stores stay
-// coalesced across threads (consecutive voxels), and the channels-last copy of the 8 channels
-// is one 16-byte store (C % 8 == 0, o.ld and o.off multiples of 8).
-__global__ void k_upsample8(const float* __restrict__ x, float* __restrict__ y, size_t sy, int C, int d, int h, int w, ClOut o)
-{
-  x += blockIdx.y * ((size_t)C * d * h * w);
-  if (y) y += blockIdx.y * sy;
-  if (o.p) o.p += blockIdx.y * ((size_t)8 * d * h * w) * o.ld;
-  const int W2 = 2 * w, H2 = 2 * h, D2 = 2 * d;
-  const size_t vox2 = (size_t)W2 * H2 * D2;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vox2 * (size_t)(C / 8)) return;
-  const size_t v = i % vox2;
-  const int c0 = (int)(i / vox2) * 8;
-  const int xx = (int)(v % W2), yy = (int)((v / W2) % H2), zz = (int)(v / ((size_t)W2 * H2));
-  const size_t src = ((size_t)(zz / 2) * h + yy / 2) * w + xx / 2, vin = (size_t)d * h * w;
-  bf16x8 q;
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const float val = x[(size_t)(c0 + e) * vin + src];
-    if (y) y[(size_t)(c0 + e) * vox2 + v] = val;   // null: no FP32 copy (inference)
-    q[e] = to_bf16(val);
-  }
-  if (o.p) *(bf16x8*)(o.p + v * o.ld + o.off + c0) = q;
-}
-// channel-first FP32 [C][vox] -> channels-last BF16 copy
+// channel-first FP32 [C][vox] -> channels-last BF16 copy (zero padded), 8 channels of a voxel per thread
 __global__ void k_to_cl(const float* __restrict__ x, int C, size_t vox, ClOut o)
 {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)C * vox) return;
-  o.p[(blockIdx.y * vox + i % vox) * o.ld + o.off + i / vox] = to_bf16(x[blockIdx.y * (C * vox) + i]);
+  if (i >= vox * (o.ld / 8)) return;
+  const size_t v = i % vox;
+  const int c0 = (int)(i / vox) * 8;
+  bf16x8 q;
+#pragma unroll
+  for (int k = 0; k < 8; k++) q[k] = to_bf16(c0 + k < C ? x[(blockIdx.y * (size_t)C + c0 + k) * vox + v] : 0.0f);
+  *(bf16x8*)(o.p + (blockIdx.y * vox + v) * o.ld + c0) = q;
 }
-__global__ void k_upsample_bwd(const float* __restrict__ gy, size_t sy, float* __restrict__ gx, int C, int d, int h, int w, ClOut o)
+// Gradient of the x2 upsampling: the eight voxels' sum, zero where the upsampled tensor's own copy
+// (mask, [d h w][o.ld]) is not positive, and its channels-last copy. A thread takes 8 channels of a voxel.
+__global__ void k_upsample_bwd(const float* __restrict__ gy, size_t sy, const __bf16* __restrict__ mask, float* __restrict__ gx,
+                               int C, int d, int h, int w, ClOut o)
 {
-  gy += blockIdx.y * sy;
-  gx += blockIdx.y * ((size_t)C * d * h * w);
-  if (o.p) o.p += blockIdx.y * ((size_t)d * h * w) * o.ld;
-  const size_t n = (size_t)C * d * h * w;
+  const size_t vin = (size_t)d * h * w;
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int xx = (int)(i % w), yy = (int)((i / w) % h), zz = (int)((i / ((size_t)w * h)) % d);
-  const int c = (int)(i / ((size_t)w * h * d));
+  if (i >= vin * (size_t)((C + 7) / 8)) return;
+  gy += blockIdx.y * sy;
+  gx += blockIdx.y * (C * vin);
+  const size_t v = i % vin, vl = blockIdx.y * vin + v;
+  const int c0 = (int)(i / vin) * 8;
+  const int xx = (int)(v % w), yy = (int)((v / w) % h), zz = (int)(v / ((size_t)w * h));
   const int W2 = 2 * w, H2 = 2 * h, D2 = 2 * d;
-  float s = 0.0f;
-  for (int a = 0; a < 2; a++)
-    for (int b = 0; b < 2; b++)
-      for (int e = 0; e < 2; e++) s += gy[(((size_t)c * D2 + 2 * zz + a) * H2 + 2 * yy + b) * W2 + 2 * xx + e];
-  gx[i] = s;
-  if (o.p) o.p[(i % ((size_t)w * h * d)) * o.ld + o.off + c] = to_bf16(s);
+  const bf16x8 m = *(const bf16x8*)(mask + vl * o.ld + c0);
+  bf16x8 q;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    q[k] = to_bf16(0.0f);
+    if (c0 + k >= C) continue;
+    float s = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        const float2 p = *(const float2*)(gy + (((size_t)(c0 + k) * D2 + 2 * zz + a) * H2 + 2 * yy + b) * W2 + 2 * xx);
+        s += p.x;
+        s += p.y;
+      }
+    if (!((float)m[k] > 0.0f)) s = 0.0f;
+    gx[(c0 + k) * vin + v] = s;
+    q[k] = to_bf16(s);
+  }
+  *(bf16x8*)(o.p + vl * o.ld + c0) = q;
 }
 // per-channel sum (bias gradient): workgroups (channel, chunk of `per` voxels, sample), added atomically
 __global__ void k_channel_sum(const float* __restrict__ g, size_t sg, float* __restrict__ out, int vox, int per)
@@ -1217,24 +1384,19 @@ __global__ void k_channel_sum(const float* __restrict__ g, size_t sg, float* __r
   }
   if (threadIdx.x == 0) atomicAdd(&out[blockIdx.x], sh[0]);
 }
-// out = x0 + r (residual output) and, with a target, the loss gradient and squared error
-__global__ void k_output(const float* __restrict__ x0, size_t sx, const float* __restrict__ r, float* __restrict__ out,
-                         const float* __restrict__ target, float* __restrict__ g, float scale, float* __restrict__ sse, int n,
-                         ClOut gl)
+// loss gradient (and its channels-last copy) and squared error of the output
+__global__ void k_loss(const float* __restrict__ out, const float* __restrict__ target, float* __restrict__ g, float scale,
+                       float* __restrict__ sse, int n, ClOut gl)
 {
   __shared__ float sh[256];
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   const size_t i = blockIdx.y * (size_t)n + v;
   float e2 = 0.0f;
   if (v < n) {
-    const float o = x0[blockIdx.y * sx + v] + r[i];
-    out[i] = o;
-    if (target) {
-      const float d = o - target[i];
-      g[i] = 2.0f * d * scale;
-      if (gl.p) gl.p[i * gl.ld] = to_bf16(g[i]);
-      e2 = d * d;
-    }
+    const float d = out[i] - target[i];
+    g[i] = 2.0f * d * scale;
+    gl.p[i * gl.ld] = to_bf16(g[i]);
+    e2 = d * d;
   }
   sh[threadIdx.x] = e2;
   __syncthreads();
@@ -1242,7 +1404,36 @@ __global__ void k_output(const float* __restrict__ x0, size_t sx, const float* _
     if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0 && target) atomicAdd(sse, sh[0]);
+  if (threadIdx.x == 0) atomicAdd(sse, sh[0]);
+}
+// Weight gradient of the 1x1x1 output layer (one output channel): the sum over voxels of the output
+// gradient (channel 0 of gl, [vox][8]) times the input copy xl [vox][ld]. A thread adds 8 channels of
+// every (256 / groups)th voxel of its workgroup's chunk; bounded by reading xl once.
+__global__ __launch_bounds__(256) void k_bwgt_point(const __bf16* __restrict__ xl, int ld, const __bf16* __restrict__ gl,
+                                                    float* __restrict__ G, int C, size_t n, int chunk)
+{
+  __shared__ float sh[256][9];
+  const int groups = ld >> 3, per = 256 / groups, q = threadIdx.x % groups, first = threadIdx.x / groups;
+  const size_t b = (size_t)blockIdx.x * chunk, e = min(n, b + chunk);
+  float s[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) s[k] = 0.0f;
+  if (first < per)
+#pragma unroll 4
+    for (size_t v = b + first; v < e; v += per) {
+      const bf16x8 x = *(const bf16x8*)(xl + v * ld + q * 8);
+      const float g = (float)gl[v * 8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) s[k] = __builtin_fmaf(g, (float)x[k], s[k]);   // the product is exact
+    }
+#pragma unroll
+  for (int k = 0; k < 8; k++) sh[threadIdx.x][k] = s[k];
+  __syncthreads();
+  for (int c = threadIdx.x; c < C; c += 256) {
+    float t = 0.0f;
+    for (int i = 0; i < per; i++) t += sh[i * groups + (c >> 3)][c & 7];
+    atomicAdd(&G[c], t);
+  }
 }
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m, float* __restrict__ v, size_t n,
                        float lr, float b1, float b2, float eps, float c1, float c2)
@@ -1341,15 +1532,14 @@ struct mcpet_surrogate {
   size_t n_params = 0, n_bf16 = 0;
   float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;
   __bf16* wbf = nullptr;
-  // activations (post-ReLU) and their gradients; concat buffers hold the skip tensors
+  // the input, the output and the gradients; the concatenations' gradients hold the skip tensors' ones
   Vol vx, va1, vcat1, vd1, vcat2, vd2, vb3, ve2, ve1, vr;
-  float *x0 = nullptr, *a1 = nullptr, *cat1 = nullptr, *d1 = nullptr, *cat2 = nullptr, *d2 = nullptr, *b3 = nullptr,
-        *e2 = nullptr, *e1 = nullptr, *r = nullptr, *out = nullptr, *tgt = nullptr;
+  float *x0 = nullptr, *out = nullptr, *tgt = nullptr;
   float *ga1 = nullptr, *gcat1 = nullptr, *gd1 = nullptr, *gcat2 = nullptr, *gd2 = nullptr, *gb3 = nullptr, *ge2 = nullptr,
         *ge1 = nullptr, *gr = nullptr, *sse = nullptr;
-  // channels-last BF16 copies read as B operands (activations, then gradients)
+  // channels-last BF16 copies: the activations (post-ReLU), then the gradients read as B operands
   __bf16 *x0l = nullptr, *a1l = nullptr, *b1l = nullptr, *cat1l = nullptr, *d1l = nullptr, *b2l = nullptr, *cat2l = nullptr,
-         *d2l = nullptr, *e1l = nullptr;
+         *d2l = nullptr, *b3l = nullptr, *e2l = nullptr, *e1l = nullptr;
   __bf16 *grl = nullptr, *ge1l = nullptr, *ge2l = nullptr, *gb3l = nullptr, *gd2l = nullptr, *gb2l = nullptr, *gd1l = nullptr,
          *gb1l = nullptr;
   float *raw_s = nullptr, *raw_t = nullptr, *est = nullptr;   // the fused estimate's buffers
@@ -1427,16 +1617,32 @@ ConvK conv_args(const Conv& l, const Vol& vin, const Vol& vout)
 
 const ClOut kNoCl{nullptr, 0, 0};
 
-// y = act(conv(x) + b); x read from its channels-last copy xl; o1, o2: copies of y to write
-hipError_t conv_fwd(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, const __bf16* xl, const Vol& vout, float* y,
-                    size_t sy, bool relu, ClOut o1, ClOut o2 = kNoCl)
+// A layer's input as channels-last copies: xl alone, or the concatenation of xu's x2 upsampling (its
+// first Cu channels) and xl.
+struct ClIn {
+  const __bf16* xl;
+  int ld;
+  const __bf16* xu;
+  int Cu;
+};
+
+// act(conv(x) + b) into the channels-last copy o1 and, where y is given, FP32 (with res: res + it)
+hipError_t conv_fwd(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, ClIn x, const Vol& vout, bool relu, ClOut o1,
+                    float* y = nullptr, const float* res = nullptr)
 {
   ConvK a = conv_args(l, vin, vout);
   a.A = s->wbf + l.wf;
-  a.Xl = xl;
+  a.Xl = x.xl;
+  a.ldx = x.ld;
+  a.sX = vin.vox() * x.ld;
+  a.Xu = x.xu;
+  a.Cu = a.ldu = x.Cu;
+  a.sXu = vin.vox() / 8 * x.Cu;
   a.C = y;
+  a.sC = vout.size();
+  a.res = res;
+  a.sR = s->vx.size();
   a.o1 = o1;
-  a.o2 = o2;
   a.bias = s->p + l.b;
   a.relu = relu ? 1 : 0;
   a.M = l.cout;
@@ -1444,158 +1650,178 @@ hipError_t conv_fwd(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, c
   a.Cb = l.cin;
   a.Cbp = rup(l.cin, 8);
   a.samples = ns;
-  a.sX = vin.vox() * a.Cbp;
-  a.sC = sy;
   a.K = a.T * a.Cbp;
   a.Kp = l.kp_f;
   a.nrb = l.rows_f / 16;
   s->flops_fwd += 2.0 * l.cout * (double)l.cin * a.T * a.N;
-  if (use_tiled(a)) return launch_conv_tiled<FWD>(a, s->st);
-  return launch_conv<FWD>(a, s->st);
+  if (x.Cu) return use_tiled(a) ? launch_conv_tiled<FWDUP>(a, s->st) : launch_conv<FWDUP>(a, s->st);
+  return use_tiled(a) ? launch_conv_tiled<FWD>(a, s->st) : launch_conv<FWD>(a, s->st);
 }
-// gx (+)= dL/dx of the layer input, zeroed where mask <= 0; gy read from its channels-last copy
+// gx (+)= dL/dx of the layer input; from channel mask0 on zeroed where the input's copy mask is not
+// positive; gy read from its channels-last copy
 hipError_t conv_bwd_data(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, const Vol& vout, const __bf16* gyl, float* gx,
-                         size_t sx, const float* mask, bool add, ClOut o1)
+                         size_t sx, ClOut mask, int mask0, bool add, ClOut o1)
 {
   ConvK a = conv_args(l, vin, vout);
   a.A = s->wbf + l.wb;
   a.Xl = gyl;
   a.C = gx;
   a.o1 = o1;
-  a.o2 = kNoCl;
-  a.mask = mask;
+  a.mask = mask.p;
+  a.ldm = mask.ld;
+  a.mask0 = mask0;
   a.beta = add ? 1 : 0;
   a.M = l.cin;
   a.N = (int)vin.vox();
   a.Cb = l.cout;
   a.Cbp = rup(l.cout, 8);
+  a.ldx = a.Cbp;
   a.samples = ns;
   a.sX = vout.vox() * a.Cbp;
   a.sC = sx;
   a.K = a.T * a.Cbp;
   a.Kp = l.kp_b;
   a.nrb = l.rows_b / 16;
-  if (use_tiled(a)) return launch_conv_tiled<BDATA>(a, s->st);
-  return launch_conv<BDATA>(a, s->st);
+  return use_tiled(a) ? launch_conv_tiled<BDATA>(a, s->st) : launch_conv<BDATA>(a, s->st);
 }
-// weight and bias gradients accumulated from gy (dL/d pre-activation) and the layer input x;
-// xl, gyl: their channels-last BF16 copies (ClOut ld = row length) or null. 3x3x3 layers with
-// both copies take the LDS-tiled product, the others k_conv's.
-hipError_t conv_bwd_weights(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, const float* x, const Vol& vout,
-                            const float* gy, size_t sg, ClOut xl = ClOut{nullptr, 0, 0}, ClOut gyl = ClOut{nullptr, 0, 0})
+// weight and bias gradients accumulated from gy (dL/d pre-activation, with its channels-last copy
+// gyl) and the layer input x. The output layer and the 3x3x3 layers that the tiled product takes read
+// the copies, the others FP32 x0 and gy.
+hipError_t conv_bwd_weights(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, ClIn x, const Vol& vout, const float* gy,
+                            size_t sg, const __bf16* gyl, const float* x0 = nullptr)
 {
   const int vox = (int)vout.vox(), per = 4096;
-  if (l.ks == 3 && (l.stride == 1 || l.stride == 2) && xl.p && gyl.p && xl.off == 0 && gyl.off == 0 && xl.ld % 8 == 0 &&
-      gyl.ld % 8 == 0 && bwgt_fits(ns, vout.D, vout.H, vout.W, l.cin, l.cout)) {
-    hipError_t e = launch_bwgt_tiled(ns, l.stride, xl.p, xl.ld, gyl.p, gyl.ld, l.cin, l.cout, vin.D, vin.H, vin.W, vout.D, vout.H,
-                                     vout.W, s->bw_part, s->g + l.w, s->st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per, ns), dim3(256), 0, s->st, gy, sg, s->g + l.b, vox, per);
-    return hipGetLastError();
+  hipError_t e = hipSuccess;
+  if (l.ks == 1 && l.cout == 1 && x.ld <= 256) {
+    const size_t n = (size_t)ns * vox;
+    const int chunk = (int)std::max<size_t>(256, (n + 1023) / 1024);
+    hipLaunchKernelGGL(k_bwgt_point, dim3((unsigned)((n + chunk - 1) / chunk)), dim3(256), 0, s->st, x.xl, x.ld, gyl, s->g + l.w,
+                       l.cin, n, chunk);
+    e = hipGetLastError();
+  } else if (!x0) {
+    BwK b{};
+    b.Xl = x.xl;
+    b.Xu = x.xu;
+    b.ldu = b.Cu = x.Cu;
+    b.part = s->bw_part;
+    b.ldx = x.ld;
+    b.ldg = rup(l.cout, 8);
+    b.Cin = l.cin;
+    b.Cout = l.cout;
+    b.D = vin.D, b.H = vin.H, b.W = vin.W;
+    b.oD = vout.D, b.oH = vout.H, b.oW = vout.W;
+    b.sX = vin.vox() * x.ld;
+    b.sXu = vin.vox() / 8 * x.Cu;
+    b.sG = vout.vox() * b.ldg;
+    e = launch_bwgt_tiled(ns, l.stride, b, gyl, s->g + l.w, s->st);
+  } else {
+    ConvK a = conv_args(l, vin, vout);
+    a.Ad = gy;
+    a.X = x0;
+    a.C = s->g + l.w;
+    a.M = l.cout;
+    a.N = a.T * l.cin;
+    a.K = vox;
+    a.Cb = l.cin;
+    a.Cbp = l.cin;
+    a.samples = ns;
+    a.sX = vin.size();
+    a.sC = sg;
+    e = launch_bwgt(a, s->st);
   }
-  ConvK a = conv_args(l, vin, vout);
-  a.Ad = gy;
-  a.X = x;
-  a.C = s->g + l.w;
-  a.M = l.cout;
-  a.N = a.T * l.cin;
-  a.K = (int)vout.vox();
-  a.Cb = l.cin;
-  a.Cbp = l.cin;
-  a.samples = ns;
-  a.sX = vin.size();
-  a.sC = sg;
-  hipError_t e = launch_bwgt(a, s->st);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per, ns), dim3(256), 0, s->st, gy, sg, s->g + l.b, vox, per);
   return hipGetLastError();
 }
-hipError_t upsample(mcpet_surrogate* s, int ns, const Vol& v, const float* x, float* y, size_t sy, ClOut o)
+hipError_t upsample_bwd(mcpet_surrogate* s, int ns, const Vol& v, const float* gy, size_t sy, const __bf16* mask, float* gx, ClOut o)
 {
-  if (v.C % 8 == 0 && (!o.p || (o.ld % 8 == 0 && o.off % 8 == 0)))
-    hipLaunchKernelGGL(k_upsample8, dim3(blocks_for(v.size()), ns), dim3(256), 0, s->st, x, y, sy, v.C, v.D, v.H, v.W, o);
-  else
-    hipLaunchKernelGGL(k_upsample, dim3(blocks_for(v.size() * 8), ns), dim3(256), 0, s->st, x, y, sy, v.C, v.D, v.H, v.W, o);
-  return hipGetLastError();
-}
-hipError_t upsample_bwd(mcpet_surrogate* s, int ns, const Vol& v, const float* gy, size_t sy, float* gx, ClOut o)
-{
-  hipLaunchKernelGGL(k_upsample_bwd, dim3(blocks_for(v.size()), ns), dim3(256), 0, s->st, gy, sy, gx, v.C, v.D, v.H, v.W, o);
+  hipLaunchKernelGGL(k_upsample_bwd, dim3(blocks_for(v.vox() * ((v.C + 7) / 8)), ns), dim3(256), 0, s->st, gy, sy, mask, gx, v.C,
+                     v.D, v.H, v.W, o);
   return hipGetLastError();
 }
 ClOut cl(__bf16* p, int channels, int off = 0) { return ClOut{p, rup(channels, 8), off}; }
 
-// Forward of the ns samples already in s->x0 (r = the residuals). keep: write the FP32 copy of every
-// activation (training reads them); without it only the tensors the forward itself reads in
-// FP32 (the upsampling inputs b3 and e2, the residual r) are written, the layers passing their
-// outputs to the next one through the channels-last BF16 copies alone.
-hipError_t forward(mcpet_surrogate* s, int ns, bool keep)
+ClIn in(const __bf16* p, int channels) { return ClIn{p, rup(channels, 8), nullptr, 0}; }
+
+// The input of a layer after an upsampling: its two tensors where they are, or their concatenation cat
+// (written by concat) where the products cannot read them so.
+ClIn in_up(const __bf16* u, int Cu, const __bf16* l, int Cl, const __bf16* cat)
+{
+  return Cu % 8 == 0 ? ClIn{l, rup(Cl, 8), u, Cu} : in(cat, Cu + Cl);
+}
+hipError_t concat(mcpet_surrogate* s, int ns, const Vol& v, const __bf16* u, int Cu, const __bf16* l, int Cl, __bf16* cat)
+{
+  if (Cu % 8 == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_concat, dim3(blocks_for(v.vox() * (Cu + Cl)), ns), dim3(256), 0, s->st, u, Cu, rup(Cu, 8), l, Cl, rup(Cl, 8),
+                     v.D, v.H, v.W, cl(cat, Cu + Cl));
+  return hipGetLastError();
+}
+
+// Forward of the ns samples already in s->x0, into s->out. The layers pass their outputs on as
+// channels-last BF16 copies, which are also the weight gradients' operands and, by their signs, the
+// ReLU masks.
+hipError_t forward(mcpet_surrogate* s, int ns)
 {
   hipError_t e = hipSuccess;
   const int c = s->c;
   const Vol vb1{c, s->D, s->H, s->W}, vb2{2 * c, s->D / 2, s->H / 2, s->W / 2};
-  const size_t s1 = s->vcat1.size(), s2 = s->vcat2.size();
-  float* b1 = s->cat1 + (size_t)2 * c * vb1.vox();   // enc1 output lives in the concat buffer
-  float* b2 = s->cat2 + (size_t)4 * c * vb2.vox();
   s->flops_fwd = 0.0;
-  hipLaunchKernelGGL(k_to_cl, dim3(blocks_for(s->vx.size()), ns), dim3(256), 0, s->st, s->x0, s->cin, s->vx.vox(),
-                     cl(s->x0l, s->cin));
-  e = hipGetLastError();
 #define STEP(x) \
   if (e == hipSuccess) e = (x)
-  auto k = [keep](float* p) { return keep ? p : nullptr; };
-  STEP(conv_fwd(s, ns, s->L[0], s->vx, s->x0l, s->va1, k(s->a1), s->va1.size(), true, cl(s->a1l, c)));
-  STEP(conv_fwd(s, ns, s->L[1], s->va1, s->a1l, vb1, k(b1), s1, true, cl(s->b1l, c), cl(s->cat1l, 3 * c, 2 * c)));
-  STEP(conv_fwd(s, ns, s->L[2], vb1, s->b1l, s->vd1, k(s->d1), s->vd1.size(), true, cl(s->d1l, 2 * c)));
-  STEP(conv_fwd(s, ns, s->L[3], s->vd1, s->d1l, vb2, k(b2), s2, true, cl(s->b2l, 2 * c), cl(s->cat2l, 6 * c, 4 * c)));
-  STEP(conv_fwd(s, ns, s->L[4], vb2, s->b2l, s->vd2, k(s->d2), s->vd2.size(), true, cl(s->d2l, 4 * c)));
-  STEP(conv_fwd(s, ns, s->L[5], s->vd2, s->d2l, s->vb3, s->b3, s->vb3.size(), true, kNoCl));
-  STEP(upsample(s, ns, s->vb3, s->b3, k(s->cat2), s2, cl(s->cat2l, 6 * c)));    // first 4c channels of cat2
-  STEP(conv_fwd(s, ns, s->L[6], s->vcat2, s->cat2l, s->ve2, s->e2, s->ve2.size(), true, kNoCl));
-  STEP(upsample(s, ns, s->ve2, s->e2, k(s->cat1), s1, cl(s->cat1l, 3 * c)));    // first 2c channels of cat1
-  STEP(conv_fwd(s, ns, s->L[7], s->vcat1, s->cat1l, s->ve1, k(s->e1), s->ve1.size(), true, cl(s->e1l, c)));
-  STEP(conv_fwd(s, ns, s->L[8], s->ve1, s->e1l, s->vr, s->r, s->vr.size(), false, kNoCl));
+  hipLaunchKernelGGL(k_to_cl, dim3(blocks_for(s->vx.vox() * (rup(s->cin, 8) / 8)), ns), dim3(256), 0, s->st, s->x0, s->cin,
+                     s->vx.vox(), cl(s->x0l, s->cin));
+  e = hipGetLastError();
+  STEP(conv_fwd(s, ns, s->L[0], s->vx, in(s->x0l, s->cin), s->va1, true, cl(s->a1l, c)));
+  STEP(conv_fwd(s, ns, s->L[1], s->va1, in(s->a1l, c), vb1, true, cl(s->b1l, c)));
+  STEP(conv_fwd(s, ns, s->L[2], vb1, in(s->b1l, c), s->vd1, true, cl(s->d1l, 2 * c)));
+  STEP(conv_fwd(s, ns, s->L[3], s->vd1, in(s->d1l, 2 * c), vb2, true, cl(s->b2l, 2 * c)));
+  STEP(conv_fwd(s, ns, s->L[4], vb2, in(s->b2l, 2 * c), s->vd2, true, cl(s->d2l, 4 * c)));
+  STEP(conv_fwd(s, ns, s->L[5], s->vd2, in(s->d2l, 4 * c), s->vb3, true, cl(s->b3l, 4 * c)));
+  STEP(concat(s, ns, s->vcat2, s->b3l, 4 * c, s->b2l, 2 * c, s->cat2l));
+  STEP(conv_fwd(s, ns, s->L[6], s->vcat2, in_up(s->b3l, 4 * c, s->b2l, 2 * c, s->cat2l), s->ve2, true, cl(s->e2l, 2 * c)));
+  STEP(concat(s, ns, s->vcat1, s->e2l, 2 * c, s->b1l, c, s->cat1l));
+  STEP(conv_fwd(s, ns, s->L[7], s->vcat1, in_up(s->e2l, 2 * c, s->b1l, c, s->cat1l), s->ve1, true, cl(s->e1l, c)));
+  STEP(conv_fwd(s, ns, s->L[8], s->ve1, in(s->e1l, c), s->vr, false, kNoCl, s->out, s->x0));
 #undef STEP
   return e;
 }
 
 // Backward of ns samples from gr (= dL/dr, with its channels-last copy); accumulates the
-// parameter gradients. The ReLU derivative is applied where each gradient is produced (mask =
-// the post-ReLU activation; the upsampled and concatenated copies carry the same sign as their
-// sources). A gradient's channels-last copy is written by the product that completes it.
+// parameter gradients. The ReLU derivative is applied where each gradient is produced (mask = the
+// sign of the post-ReLU activation), for an upsampled tensor after the sum over its copies. A
+// gradient's channels-last copy is written by the product that completes it.
 hipError_t backward(mcpet_surrogate* s, int ns)
 {
   hipError_t e = hipSuccess;
   const int c = s->c;
   const Vol vb1{c, s->D, s->H, s->W}, vb2{2 * c, s->D / 2, s->H / 2, s->W / 2};
   const size_t s1 = s->vcat1.size(), s2 = s->vcat2.size();
-  const float* b1 = s->cat1 + (size_t)2 * c * vb1.vox();
-  const float* b2 = s->cat2 + (size_t)4 * c * vb2.vox();
   float* gb1 = s->gcat1 + (size_t)2 * c * vb1.vox();
   float* gb2 = s->gcat2 + (size_t)4 * c * vb2.vox();
 #define STEP(x) \
   if (e == hipSuccess) e = (x)
-#define WGT(l, vin, x, vout, gy, sg, ...) STEP(conv_bwd_weights(s, ns, s->L[l], vin, x, vout, gy, sg, ##__VA_ARGS__))
-#define DATA(l, vin, vout, gyl, gx, sx, mask, add, o1) STEP(conv_bwd_data(s, ns, s->L[l], vin, vout, gyl, gx, sx, mask, add, o1))
-  WGT(8, s->ve1, s->e1, s->vr, s->gr, s->vr.size());
-  DATA(8, s->ve1, s->vr, s->grl, s->ge1, s->ve1.size(), s->e1, false, cl(s->ge1l, c));
-  WGT(7, s->vcat1, s->cat1, s->ve1, s->ge1, s->ve1.size(), cl(s->cat1l, 3 * c), cl(s->ge1l, c));
-  DATA(7, s->vcat1, s->ve1, s->ge1l, s->gcat1, s1, s->cat1, false, kNoCl);   // g(up1), g(b1 skip)
-  STEP(upsample_bwd(s, ns, s->ve2, s->gcat1, s1, s->ge2, cl(s->ge2l, 2 * c)));
-  WGT(6, s->vcat2, s->cat2, s->ve2, s->ge2, s->ve2.size(), cl(s->cat2l, 6 * c), cl(s->ge2l, 2 * c));
-  DATA(6, s->vcat2, s->ve2, s->ge2l, s->gcat2, s2, s->cat2, false, kNoCl);   // g(up2), g(b2 skip)
-  STEP(upsample_bwd(s, ns, s->vb3, s->gcat2, s2, s->gb3, cl(s->gb3l, 4 * c)));
-  WGT(5, s->vd2, s->d2, s->vb3, s->gb3, s->vb3.size(), cl(s->d2l, 4 * c), cl(s->gb3l, 4 * c));
-  DATA(5, s->vd2, s->vb3, s->gb3l, s->gd2, s->vd2.size(), s->d2, false, cl(s->gd2l, 4 * c));
-  WGT(4, vb2, b2, s->vd2, s->gd2, s->vd2.size(), cl(s->b2l, 2 * c), cl(s->gd2l, 4 * c));
-  DATA(4, vb2, s->vd2, s->gd2l, gb2, s2, b2, true, cl(s->gb2l, 2 * c));      // + the skip's gradient
-  WGT(3, s->vd1, s->d1, vb2, gb2, s2, cl(s->d1l, 2 * c), cl(s->gb2l, 2 * c));
-  DATA(3, s->vd1, vb2, s->gb2l, s->gd1, s->vd1.size(), s->d1, false, cl(s->gd1l, 2 * c));
-  WGT(2, vb1, b1, s->vd1, s->gd1, s->vd1.size(), cl(s->b1l, c), cl(s->gd1l, 2 * c));
-  DATA(2, vb1, s->vd1, s->gd1l, gb1, s1, b1, true, cl(s->gb1l, c));          // + the skip's gradient
-  WGT(1, s->va1, s->a1, vb1, gb1, s1, cl(s->a1l, c), cl(s->gb1l, c));
-  DATA(1, s->va1, vb1, s->gb1l, s->ga1, s->va1.size(), s->a1, false, kNoCl);
-  WGT(0, s->vx, s->x0, s->va1, s->ga1, s->va1.size());
+#define WGT(l, vin, x, vout, gy, sg, gyl, ...) STEP(conv_bwd_weights(s, ns, s->L[l], vin, x, vout, gy, sg, gyl, ##__VA_ARGS__))
+#define DATA(l, vin, vout, gyl, gx, sx, mask, mask0, add, o1) \
+  STEP(conv_bwd_data(s, ns, s->L[l], vin, vout, gyl, gx, sx, mask, mask0, add, o1))
+  WGT(8, s->ve1, in(s->e1l, c), s->vr, s->gr, s->vr.size(), s->grl);
+  DATA(8, s->ve1, s->vr, s->grl, s->ge1, s->ve1.size(), cl(s->e1l, c), 0, false, cl(s->ge1l, c));
+  WGT(7, s->vcat1, in_up(s->e2l, 2 * c, s->b1l, c, s->cat1l), s->ve1, s->ge1, s->ve1.size(), s->ge1l);
+  DATA(7, s->vcat1, s->ve1, s->ge1l, s->gcat1, s1, cl(s->b1l, c), 2 * c, false, kNoCl);   // g(up1), g(b1 skip)
+  STEP(upsample_bwd(s, ns, s->ve2, s->gcat1, s1, s->e2l, s->ge2, cl(s->ge2l, 2 * c)));
+  WGT(6, s->vcat2, in_up(s->b3l, 4 * c, s->b2l, 2 * c, s->cat2l), s->ve2, s->ge2, s->ve2.size(), s->ge2l);
+  DATA(6, s->vcat2, s->ve2, s->ge2l, s->gcat2, s2, cl(s->b2l, 2 * c), 4 * c, false, kNoCl);   // g(up2), g(b2 skip)
+  STEP(upsample_bwd(s, ns, s->vb3, s->gcat2, s2, s->b3l, s->gb3, cl(s->gb3l, 4 * c)));
+  WGT(5, s->vd2, in(s->d2l, 4 * c), s->vb3, s->gb3, s->vb3.size(), s->gb3l);
+  DATA(5, s->vd2, s->vb3, s->gb3l, s->gd2, s->vd2.size(), cl(s->d2l, 4 * c), 0, false, cl(s->gd2l, 4 * c));
+  WGT(4, vb2, in(s->b2l, 2 * c), s->vd2, s->gd2, s->vd2.size(), s->gd2l);
+  DATA(4, vb2, s->vd2, s->gd2l, gb2, s2, cl(s->b2l, 2 * c), 0, true, cl(s->gb2l, 2 * c));      // + the skip's gradient
+  WGT(3, s->vd1, in(s->d1l, 2 * c), vb2, gb2, s2, s->gb2l);
+  DATA(3, s->vd1, vb2, s->gb2l, s->gd1, s->vd1.size(), cl(s->d1l, 2 * c), 0, false, cl(s->gd1l, 2 * c));
+  WGT(2, vb1, in(s->b1l, c), s->vd1, s->gd1, s->vd1.size(), s->gd1l);
+  DATA(2, vb1, s->vd1, s->gd1l, gb1, s1, cl(s->b1l, c), 0, true, cl(s->gb1l, c));              // + the skip's gradient
+  WGT(1, s->va1, in(s->a1l, c), vb1, gb1, s1, s->gb1l);
+  DATA(1, s->va1, vb1, s->gb1l, s->ga1, s->va1.size(), cl(s->a1l, c), 0, false, kNoCl);
+  WGT(0, s->vx, in(s->x0l, s->cin), s->va1, s->ga1, s->va1.size(), nullptr, s->x0);
 #undef WGT
 #undef DATA
 #undef STEP
@@ -1616,14 +1842,13 @@ std::vector<Slot> sample_tensors(mcpet_surrogate* s)
   std::vector<Slot> t;
   auto f = [&](float** p, const Vol& v) { t.push_back({(void**)p, sizeof(float) * v.size(), false}); };
   auto h = [&](__bf16** p, size_t vox, int ch) { t.push_back({(void**)p, sizeof(__bf16) * vox * rup(ch, 8), true}); };
-  f(&s->x0, s->vx), f(&s->b3, s->vb3), f(&s->e2, s->ve2), f(&s->r, s->vr), f(&s->out, s->vr);
-  f(&s->a1, s->va1), f(&s->cat1, s->vcat1), f(&s->d1, s->vd1), f(&s->cat2, s->vcat2);
-  f(&s->d2, s->vd2), f(&s->e1, s->ve1), f(&s->tgt, s->vr);
+  const bool cat = 2 * c % 8 != 0;   // the concatenations are written (concat)
+  f(&s->x0, s->vx), f(&s->out, s->vr), f(&s->tgt, s->vr);
   f(&s->ga1, s->va1), f(&s->gcat1, s->vcat1), f(&s->gd1, s->vd1), f(&s->gcat2, s->vcat2);
   f(&s->gd2, s->vd2), f(&s->gb3, s->vb3), f(&s->ge2, s->ve2), f(&s->ge1, s->ve1), f(&s->gr, s->vr);
-  h(&s->x0l, v0, ci), h(&s->a1l, v0, c), h(&s->b1l, v0, c), h(&s->cat1l, v0, 3 * c);
-  h(&s->d1l, v1, 2 * c), h(&s->b2l, v1, 2 * c), h(&s->cat2l, v1, 6 * c), h(&s->d2l, v2, 4 * c);
-  h(&s->e1l, v0, c);
+  h(&s->x0l, v0, ci), h(&s->a1l, v0, c), h(&s->b1l, v0, c), h(&s->cat1l, cat ? v0 : 0, 3 * c);
+  h(&s->d1l, v1, 2 * c), h(&s->b2l, v1, 2 * c), h(&s->cat2l, cat ? v1 : 0, 6 * c), h(&s->d2l, v2, 4 * c);
+  h(&s->e1l, v0, c), h(&s->e2l, v1, 2 * c), h(&s->b3l, v2, 4 * c);
   h(&s->grl, v0, 8), h(&s->ge1l, v0, c), h(&s->ge2l, v1, 2 * c), h(&s->gb3l, v2, 4 * c);
   h(&s->gd2l, v2, 4 * c), h(&s->gb2l, v1, 2 * c), h(&s->gd1l, v1, 2 * c), h(&s->gb1l, v0, c);
   return t;
@@ -1808,10 +2033,7 @@ extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float*
     SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx * n, hipMemcpyHostToDevice, s->st));
     const bool last = b + n == batch;
     if (last) SHIP(s, hipEventRecord(s->ev_f0, s->st));
-    SHIP(s, forward(s, n, false));
-    hipLaunchKernelGGL(k_output, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->x0, nx, s->r, s->out, (const float*)nullptr,
-                       (float*)nullptr, 0.0f, (float*)nullptr, (int)nv, kNoCl);
-    SHIP(s, hipGetLastError());
+    SHIP(s, forward(s, n));
     if (last) SHIP(s, hipEventRecord(s->ev_f1, s->st));
     SHIP(s, hipMemcpyAsync(y + b * nv, s->out, sizeof(float) * nv * n, hipMemcpyDeviceToHost, s->st));
   }
@@ -1868,9 +2090,7 @@ extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* 
   hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, s->st, s->sums, 256, s->sums + 256);
   hipLaunchKernelGGL(k_normalize, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->raw_s, s->raw_t, s->x0, nv, s->sums + 256);
   SHIP(s, hipGetLastError());
-  SHIP(s, forward(s, 1, false));
-  hipLaunchKernelGGL(k_output, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->x0, s->vx.size(), s->r, s->out, (const float*)nullptr,
-                     (float*)nullptr, 0.0f, (float*)nullptr, (int)nv, kNoCl);
+  SHIP(s, forward(s, 1));
   hipLaunchKernelGGL(k_estimate, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->out, s->est, nv, s->sums + 256, d_decays);
   SHIP(s, hipGetLastError());
   // through pinned staging (one DMA per output), then host copies into the caller's buffers
@@ -1898,9 +2118,9 @@ static mcpet_status batch_gradients(mcpet_surrogate* s, const float* x, const fl
     const int n = std::min(group, batch - b);
     SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx * n, hipMemcpyHostToDevice, s->st));
     SHIP(s, hipMemcpyAsync(s->tgt, target + b * nv, sizeof(float) * nv * n, hipMemcpyHostToDevice, s->st));
-    SHIP(s, forward(s, n, true));
-    hipLaunchKernelGGL(k_output, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->x0, nx, s->r, s->out, s->tgt, s->gr, scale,
-                       s->sse, (int)nv, ClOut{s->grl, 8, 0});
+    SHIP(s, forward(s, n));
+    hipLaunchKernelGGL(k_loss, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->out, s->tgt, s->gr, scale, s->sse, (int)nv,
+                       ClOut{s->grl, 8, 0});
     SHIP(s, hipGetLastError());
     SHIP(s, backward(s, n));
   }
