@@ -1321,17 +1321,25 @@ __global__ void k_concat(const __bf16* __restrict__ u, int Cu, int ldu, const __
   const size_t vu = blockIdx.y * (vox / 8) + ((size_t)(z / 2) * (H / 2) + y / 2) * (W / 2) + x / 2;
   o.p[vl * o.ld + c] = c < Cu ? u[vu * ldu + c] : l[vl * ldl + c - Cu];
 }
-// channel-first FP32 [C][vox] -> channels-last BF16 copy (zero padded), 8 channels of a voxel per thread
-__global__ void k_to_cl(const float* __restrict__ x, int C, size_t vox, ClOut o)
+// Input voxels v0 .. v0 + range - 1 (x: FP32 [sample][C][range], device or pinned host memory) into their
+// channels-last BF16 copy o (zero padded) and, where x0 is given, the FP32 input [sample][C][vox]; 8
+// channels of a voxel per thread.
+__global__ void k_input(const float* __restrict__ x, int C, size_t vox, size_t v0, size_t range, float* __restrict__ x0, ClOut o)
 {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vox * (o.ld / 8)) return;
-  const size_t v = i % vox;
-  const int c0 = (int)(i / vox) * 8;
+  if (i >= range * (o.ld / 8)) return;
+  const size_t v = i % range;
+  const int c0 = (int)(i / range) * 8;
+  float f[8];
   bf16x8 q;
 #pragma unroll
-  for (int k = 0; k < 8; k++) q[k] = to_bf16(c0 + k < C ? x[(blockIdx.y * (size_t)C + c0 + k) * vox + v] : 0.0f);
-  *(bf16x8*)(o.p + (blockIdx.y * vox + v) * o.ld + c0) = q;
+  for (int k = 0; k < 8; k++) f[k] = c0 + k < C ? x[(blockIdx.y * (size_t)C + c0 + k) * range + v] : 0.0f;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    q[k] = to_bf16(f[k]);
+    if (x0 && c0 + k < C) x0[(blockIdx.y * (size_t)C + c0 + k) * vox + v0 + v] = f[k];
+  }
+  *(bf16x8*)(o.p + (blockIdx.y * vox + v0 + v) * o.ld + c0) = q;
 }
 // Gradient of the x2 upsampling: the eight voxels' sum, zero where the upsampled tensor's own copy
 // (mask, [d h w][o.ld]) is not positive, and its channels-last copy. A thread takes 8 channels of a voxel.
@@ -1534,7 +1542,7 @@ struct mcpet_surrogate {
   __bf16* wbf = nullptr;
   // the input, the output and the gradients; the concatenations' gradients hold the skip tensors' ones
   Vol vx, va1, vcat1, vd1, vcat2, vd2, vb3, ve2, ve1, vr;
-  float *x0 = nullptr, *out = nullptr, *tgt = nullptr;
+  float *x0 = nullptr, *out = nullptr;
   float *ga1 = nullptr, *gcat1 = nullptr, *gd1 = nullptr, *gcat2 = nullptr, *gd2 = nullptr, *gb3 = nullptr, *ge2 = nullptr,
         *ge1 = nullptr, *gr = nullptr, *sse = nullptr;
   // channels-last BF16 copies: the activations (post-ReLU), then the gradients read as B operands
@@ -1550,7 +1558,10 @@ struct mcpet_surrogate {
   int device = 0;
   hipStream_t st = nullptr;
   hipEvent_t ev_f0 = nullptr, ev_f1 = nullptr;   // around the last forward of mcpet_surrogate_forward
-  float* h_stage = nullptr;   // pinned host staging of the fused estimate's two outputs (2 x voxels)
+  float* h_stage = nullptr;   // pinned: a group's outputs or targets; the fused estimate's two outputs
+  float* h_in = nullptr;      // pinned: the two halves of stage_input's buffer, stage_in floats
+  size_t stage_in = 0;
+  hipEvent_t ev_in[2] = {nullptr, nullptr}, ev_out = nullptr;
   unsigned long long* h_decays = nullptr;   // pinned: the estimated run's decays
   int fwd_timed = 0;   // samples between the two events
   std::vector<void*> allocs;
@@ -1757,10 +1768,41 @@ hipError_t concat(mcpet_surrogate* s, int ns, const Vol& v, const __bf16* u, int
   return hipGetLastError();
 }
 
-// Forward of the ns samples already in s->x0, into s->out. The layers pass their outputs on as
-// channels-last BF16 copies, which are also the weight gradients' operands and, by their signs, the
-// ReLU masks.
-hipError_t forward(mcpet_surrogate* s, int ns)
+// n samples of the batch into s->x0 and their copy. A pageable copy of 100 KB takes 48 us, of 6.4 MB
+// 200; so the host fills the two halves of a pinned buffer in turn (whole samples where they fit, else
+// voxel ranges) and k_input reads them where they are.
+hipError_t stage_input(mcpet_surrogate* s, const float* x, int n)
+{
+  const size_t C = s->cin, vox = s->vx.vox(), half = s->stage_in / 2;
+  const size_t range = std::min(vox, half / C);
+  const int per = range == vox ? (int)std::min<size_t>(n, half / (C * vox)) : 1;
+  int turn = 0;
+  bool used[2] = {false, false};
+  for (int b = 0; b < n; b += per)
+    for (size_t v0 = 0; v0 < vox; v0 += range, turn ^= 1) {
+      const int m = std::min(per, n - b);
+      const size_t r = std::min(range, vox - v0);
+      float* h = s->h_in + turn * half;
+      hipError_t e = used[turn] ? hipEventSynchronize(s->ev_in[turn]) : hipSuccess;
+      if (e != hipSuccess) return e;
+      if (r == vox) std::memcpy(h, x + b * C * vox, sizeof(float) * m * C * vox);
+      else
+        for (size_t c = 0; c < C; c++) std::memcpy(h + c * r, x + (b * C + c) * vox + v0, sizeof(float) * r);
+      const ClOut o{s->x0l + (size_t)b * vox * rup(s->cin, 8), rup(s->cin, 8), 0};
+      hipLaunchKernelGGL(k_input, dim3(blocks_for(r * (o.ld / 8)), m), dim3(256), 0, s->st, (const float*)h, (int)C, vox, v0, r,
+                         s->x0 + (size_t)b * C * vox, o);
+      e = hipGetLastError();
+      if (e == hipSuccess) e = hipEventRecord(s->ev_in[turn], s->st);
+      if (e != hipSuccess) return e;
+      used[turn] = true;
+    }
+  return hipSuccess;
+}
+
+// Forward of the ns samples already in s->x0 and their copy, into out (device, or pinned host memory).
+// The layers pass their outputs on as channels-last BF16 copies, which are also the weight gradients'
+// operands and, by their signs, the ReLU masks.
+hipError_t forward(mcpet_surrogate* s, int ns, float* out)
 {
   hipError_t e = hipSuccess;
   const int c = s->c;
@@ -1768,9 +1810,6 @@ hipError_t forward(mcpet_surrogate* s, int ns)
   s->flops_fwd = 0.0;
 #define STEP(x) \
   if (e == hipSuccess) e = (x)
-  hipLaunchKernelGGL(k_to_cl, dim3(blocks_for(s->vx.vox() * (rup(s->cin, 8) / 8)), ns), dim3(256), 0, s->st, s->x0, s->cin,
-                     s->vx.vox(), cl(s->x0l, s->cin));
-  e = hipGetLastError();
   STEP(conv_fwd(s, ns, s->L[0], s->vx, in(s->x0l, s->cin), s->va1, true, cl(s->a1l, c)));
   STEP(conv_fwd(s, ns, s->L[1], s->va1, in(s->a1l, c), vb1, true, cl(s->b1l, c)));
   STEP(conv_fwd(s, ns, s->L[2], vb1, in(s->b1l, c), s->vd1, true, cl(s->d1l, 2 * c)));
@@ -1781,7 +1820,7 @@ hipError_t forward(mcpet_surrogate* s, int ns)
   STEP(conv_fwd(s, ns, s->L[6], s->vcat2, in_up(s->b3l, 4 * c, s->b2l, 2 * c, s->cat2l), s->ve2, true, cl(s->e2l, 2 * c)));
   STEP(concat(s, ns, s->vcat1, s->e2l, 2 * c, s->b1l, c, s->cat1l));
   STEP(conv_fwd(s, ns, s->L[7], s->vcat1, in_up(s->e2l, 2 * c, s->b1l, c, s->cat1l), s->ve1, true, cl(s->e1l, c)));
-  STEP(conv_fwd(s, ns, s->L[8], s->ve1, in(s->e1l, c), s->vr, false, kNoCl, s->out, s->x0));
+  STEP(conv_fwd(s, ns, s->L[8], s->ve1, in(s->e1l, c), s->vr, false, kNoCl, out, s->x0));
 #undef STEP
   return e;
 }
@@ -1843,7 +1882,7 @@ std::vector<Slot> sample_tensors(mcpet_surrogate* s)
   auto f = [&](float** p, const Vol& v) { t.push_back({(void**)p, sizeof(float) * v.size(), false}); };
   auto h = [&](__bf16** p, size_t vox, int ch) { t.push_back({(void**)p, sizeof(__bf16) * vox * rup(ch, 8), true}); };
   const bool cat = 2 * c % 8 != 0;   // the concatenations are written (concat)
-  f(&s->x0, s->vx), f(&s->out, s->vr), f(&s->tgt, s->vr);
+  f(&s->x0, s->vx), f(&s->out, s->vr);
   f(&s->ga1, s->va1), f(&s->gcat1, s->vcat1), f(&s->gd1, s->vd1), f(&s->gcat2, s->vcat2);
   f(&s->gd2, s->vd2), f(&s->gb3, s->vb3), f(&s->ge2, s->ve2), f(&s->ge1, s->ve1), f(&s->gr, s->vr);
   h(&s->x0l, v0, ci), h(&s->a1l, v0, c), h(&s->b1l, v0, c), h(&s->cat1l, cat ? v0 : 0, 3 * c);
@@ -1955,7 +1994,8 @@ extern "C" mcpet_status mcpet_surrogate_create(int32_t D, int32_t H, int32_t W, 
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&s->st, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&s->ev_f0);
   if (e == hipSuccess) e = hipEventCreate(&s->ev_f1);
-  if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_stage, 2 * sizeof(float) * (size_t)D * H * W, hipHostMallocDefault);
+  for (hipEvent_t* ev : {&s->ev_in[0], &s->ev_in[1], &s->ev_out})
+    if (e == hipSuccess) e = hipEventCreateWithFlags(ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_decays, sizeof(unsigned long long), hipHostMallocDefault);
   struct A {
     float** p;
@@ -1968,6 +2008,12 @@ extern "C" mcpet_status mcpet_surrogate_create(int32_t D, int32_t H, int32_t W, 
   if (e == hipSuccess) e = dalloc_t(s, &s->sums, 257);
   if (e == hipSuccess) e = dalloc_t(s, &s->bw_part, kBwPartFloats);
   if (e == hipSuccess) e = hold_samples(s);
+  const size_t vox = (size_t)D * H * W;
+  if (e == hipSuccess)
+    e = hipHostMalloc((void**)&s->h_stage, sizeof(float) * vox * std::max(2, s->slots), hipHostMallocDefault);
+  // at most 2 MB a half
+  s->stage_in = 2 * std::min<size_t>((size_t)1 << 19, vox * in_channels * s->slots);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&s->h_in, sizeof(float) * s->stage_in, hipHostMallocDefault);
   if (e != hipSuccess) {
     std::string m = std::string("mcpet_surrogate_create: ") + hipGetErrorString(e);
     mcpet_surrogate_destroy(s);
@@ -2022,22 +2068,30 @@ extern "C" mcpet_status mcpet_surrogate_set_params(mcpet_surrogate* s, const flo
   return MCPET_OK;
 }
 
+// The host's halves of the staging buffers are free whenever a call begins: every call that uses them
+// waits for its stream before it returns.
 // x: batch x cin x D x H x W, y (out): batch x D x H x W; returns the forward GFLOP per sample.
 extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float* x, int32_t batch, float* y, double* gflop)
 {
   if (!s || !x || !y || batch < 1) return serr(s, MCPET_E_ARG, "mcpet_surrogate_forward: bad arguments");
   const size_t nx = s->vx.size(), nv = s->vr.size();
   const int group = sample_group(s, batch);
+  SHIP(s, stage_input(s, x, std::min(group, batch)));
   for (int b = 0; b < batch; b += group) {
-    const int n = std::min(group, batch - b);
-    SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx * n, hipMemcpyHostToDevice, s->st));
-    const bool last = b + n == batch;
+    const int n = std::min(group, batch - b), next = std::min(group, batch - b - n);
+    const bool last = next == 0;
     if (last) SHIP(s, hipEventRecord(s->ev_f0, s->st));
-    SHIP(s, forward(s, n));
+    SHIP(s, forward(s, n, s->h_stage));   // the last layer writes to the host
     if (last) SHIP(s, hipEventRecord(s->ev_f1, s->st));
-    SHIP(s, hipMemcpyAsync(y + b * nv, s->out, sizeof(float) * nv * n, hipMemcpyDeviceToHost, s->st));
+    if (last) {
+      SHIP(s, hipStreamSynchronize(s->st));
+    } else {
+      SHIP(s, hipEventRecord(s->ev_out, s->st));
+      SHIP(s, stage_input(s, x + (b + n) * nx, next));   // the next group's input, behind this one's layers
+      SHIP(s, hipEventSynchronize(s->ev_out));
+    }
+    std::memcpy(y + b * nv, s->h_stage, sizeof(float) * nv * n);
   }
-  SHIP(s, hipStreamSynchronize(s->st));
   s->fwd_timed = batch - (batch - 1) / group * group;
   if (gflop) *gflop = s->flops_fwd * 1e-9;
   return MCPET_OK;
@@ -2090,7 +2144,10 @@ extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* 
   hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(256), 0, s->st, s->sums, 256, s->sums + 256);
   hipLaunchKernelGGL(k_normalize, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->raw_s, s->raw_t, s->x0, nv, s->sums + 256);
   SHIP(s, hipGetLastError());
-  SHIP(s, forward(s, 1));
+  hipLaunchKernelGGL(k_input, dim3(blocks_for(nv * (rup(s->cin, 8) / 8))), dim3(256), 0, s->st, (const float*)s->x0, s->cin, nv,
+                     (size_t)0, nv, (float*)nullptr, cl(s->x0l, s->cin));
+  SHIP(s, hipGetLastError());
+  SHIP(s, forward(s, 1, s->out));
   hipLaunchKernelGGL(k_estimate, dim3(blocks_for(nv)), dim3(256), 0, s->st, s->out, s->est, nv, s->sums + 256, d_decays);
   SHIP(s, hipGetLastError());
   // through pinned staging (one DMA per output), then host copies into the caller's buffers
@@ -2116,11 +2173,13 @@ static mcpet_status batch_gradients(mcpet_surrogate* s, const float* x, const fl
   const int group = sample_group(s, batch);
   for (int b = 0; b < batch; b += group) {
     const int n = std::min(group, batch - b);
-    SHIP(s, hipMemcpyAsync(s->x0, x + b * nx, sizeof(float) * nx * n, hipMemcpyHostToDevice, s->st));
-    SHIP(s, hipMemcpyAsync(s->tgt, target + b * nv, sizeof(float) * nv * n, hipMemcpyHostToDevice, s->st));
-    SHIP(s, forward(s, n));
-    hipLaunchKernelGGL(k_loss, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->out, s->tgt, s->gr, scale, s->sse, (int)nv,
-                       ClOut{s->grl, 8, 0});
+    if (b) SHIP(s, hipEventSynchronize(s->ev_out));   // the last group's targets have been read
+    std::memcpy(s->h_stage, target + b * nv, sizeof(float) * nv * n);
+    SHIP(s, stage_input(s, x + b * nx, n));
+    SHIP(s, forward(s, n, s->out));
+    hipLaunchKernelGGL(k_loss, dim3(blocks_for(nv), n), dim3(256), 0, s->st, s->out, (const float*)s->h_stage, s->gr, scale, s->sse,
+                       (int)nv, ClOut{s->grl, 8, 0});
+    SHIP(s, hipEventRecord(s->ev_out, s->st));
     SHIP(s, hipGetLastError());
     SHIP(s, backward(s, n));
   }
@@ -2164,6 +2223,9 @@ extern "C" void mcpet_surrogate_destroy(mcpet_surrogate* s)
   if (s->st) (void)hipStreamSynchronize(s->st);
   for (void* p : s->allocs) (void)hipFree(p);
   if (s->h_stage) (void)hipHostFree(s->h_stage);
+  if (s->h_in) (void)hipHostFree(s->h_in);
+  for (hipEvent_t ev : {s->ev_in[0], s->ev_in[1], s->ev_out})
+    if (ev) (void)hipEventDestroy(ev);
   if (s->h_decays) (void)hipHostFree(s->h_decays);
   if (s->ev_f0) (void)hipEventDestroy(s->ev_f0);
   if (s->ev_f1) (void)hipEventDestroy(s->ev_f1);

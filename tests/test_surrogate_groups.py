@@ -16,10 +16,11 @@ def _network(grid, cin, c, rng):
 
 
 # one group, a full one, two unequal ones of 64 at most (35 + 34); widths with and without whole
-# 32-channel slices; volumes below and above one tile; one whose group is bounded by its voxels
+# 32-channel slices; volumes below and above one tile; one whose group is bounded by its voxels; one whose
+# sample does not fit half of the input staging (2 MB)
 @pytest.mark.gpu
 @pytest.mark.parametrize("grid,cin,c,batch", [((4, 4, 4), 1, 3, 69), ((4, 8, 20), 2, 16, 5), ((8, 12, 16), 4, 32, 3),
-                                              ((12, 36, 36), 2, 32, 7), ((32, 68, 64), 2, 8, 5)])
+                                              ((12, 36, 36), 2, 32, 7), ((32, 68, 64), 2, 8, 5), ((16, 48, 48), 16, 4, 3)])
 def test_batch_equals_its_samples(grid, cin, c, batch):
     rng = np.random.default_rng(5)
     net = _network(grid, cin, c, rng)
