@@ -127,8 +127,6 @@ struct ClOut {
 
 struct ConvK {
   const __bf16* A;     // FWD, BDATA: BF16 weights [Kp / 32][nrb][64 lanes][8] (k_derive)
-  const float* Ad;     // BWGT: dY [M][K]
-  const float* X;      // BWGT: input activations [Cin][D][H][W]
   const __bf16* Xl;    // FWD: input activations [D][H][W][ldx]; BDATA: dY [oD][oH][oW][ldx] (channels-last BF16)
   const __bf16* Xu;    // FWDUP: channels 0 .. Cu - 1 at half size, [D/2][H/2][W/2][ldu]; Xl holds the others
   int ldx, ldu, Cu;
@@ -143,91 +141,9 @@ struct ConvK {
   int nrb;             // 16-row blocks of A
   int Cb, Cbp;         // channels of the B tensor (FWD, BWGT: Cin; BDATA: Cout) and Cb rounded up to 8
   int D, H, W, oD, oH, oW, ks, stride, T;
-  size_t sX, sXu, sC, sR;   // from one sample to the next (blockIdx.z): B tensor(s); C; res (BWGT: X; -; Ad)
+  size_t sX, sXu, sC, sR;   // from one sample to the next (blockIdx.z): B tensor(s); C; res
   int samples;
-  int k_per_split, splits;   // BWGT: voxels per workgroup, workgroups per sample
-  int vec;             // BWGT: K % 4 == 0 (dY rows are float4-aligned)
 };
-
-__device__ __forceinline__ void tap3(int t, int ks, int& dz, int& dy, int& dx)
-{
-  if (ks == 1) {
-    dz = dy = dx = 0;
-  } else {
-    dz = t / 9 - 1;
-    dy = (t / 3) % 3 - 1;
-    dx = t % 3 - 1;
-  }
-}
-
-// Weight-gradient product of the layers without the tiled form: four waves split a slab of voxels
-// (the K range of the workgroup) and reduce through LDS, workgroups add with atomics.
-template <int MT>
-__global__ __launch_bounds__(256) void k_conv_bwgt(ConvK a)
-{
-  __shared__ floatx4 red[4][MT][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r = lane & 15, kg = lane >> 4;
-  const int m0 = blockIdx.y * (16 * MT);
-  const int n = blockIdx.x * 16 + r;                 // this lane's B column
-  const bool nvalid = n < a.N;
-  const size_t vin = (size_t)a.D * a.H * a.W;
-  floatx4 acc[MT];
-#pragma unroll
-  for (int i = 0; i < MT; i++) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const int bt = n / a.Cb, bci = n - bt * a.Cb;
-  const int smp = blockIdx.z / a.splits, kb = (blockIdx.z - smp * a.splits) * a.k_per_split, ke = min(a.K, kb + a.k_per_split);
-  a.X += smp * a.sX;
-  a.Ad += smp * a.sC;
-  for (int k0 = kb + wave * 32; k0 < ke; k0 += 128) {
-    const int k = k0 + kg * 8;
-    bf16x8 b;
-    // B: X[ci][s q + d_t] for q = k .. k + 7
-    int dz, dy, dx;
-    tap3(bt, a.ks, dz, dy, dx);
-    int ox = k % a.oW, oy = (k / a.oW) % a.oH, oz = k / (a.oW * a.oH);
-    const float* xc = a.X + (size_t)bci * vin;
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const int z = oz * a.stride + dz, y = oy * a.stride + dy, x = ox * a.stride + dx;
-      const bool in = nvalid && k + e < ke && z >= 0 && y >= 0 && x >= 0 && z < a.D && y < a.H && x < a.W;
-      b[e] = to_bf16(in ? xc[((size_t)z * a.H + y) * a.W + x] : 0.0f);
-      if (++ox == a.oW) {
-        ox = 0;
-        if (++oy == a.oH) {
-          oy = 0;
-          ++oz;
-        }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < MT; i++) {
-      const int m = m0 + 16 * i + r;
-      bf16x8 av;
-      if (m < a.M && a.vec && k + 8 <= ke) {
-        const float4* p4 = (const float4*)(a.Ad + (size_t)m * a.K + k);
-        const float4 u = p4[0], w = p4[1];
-        av[0] = to_bf16(u.x); av[1] = to_bf16(u.y); av[2] = to_bf16(u.z); av[3] = to_bf16(u.w);
-        av[4] = to_bf16(w.x); av[5] = to_bf16(w.y); av[6] = to_bf16(w.z); av[7] = to_bf16(w.w);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) av[e] = to_bf16((m < a.M && k + e < ke) ? a.Ad[(size_t)m * a.K + k + e] : 0.0f);
-      }
-      acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, b, acc[i], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < MT; i++) red[wave][i][lane] = acc[i];
-  __syncthreads();
-  for (int i = wave; i < MT; i += 4) {   // wave w finishes the row blocks w, w + 4, ...
-    const floatx4 s = red[0][i][lane] + red[1][i][lane] + red[2][i][lane] + red[3][i][lane];
-    const int row0 = m0 + 16 * i + kg * 4;   // this lane's four rows row0 .. row0 + 3
-    if (!nvalid) continue;
-#pragma unroll
-    for (int v = 0; v < 4; v++)
-      if (row0 + v < a.M) atomicAdd(&a.C[((size_t)(row0 + v) * a.Cb + bci) * a.T + bt], s[v]);
-  }
-}
 
 // the tensors of sample z
 __device__ __forceinline__ void to_sample(ConvK& a, size_t z)
@@ -337,6 +253,36 @@ __device__ __forceinline__ const __bf16* voxel_cl(const ConvK& a, int z, int y, 
     return (up ? a.Xu : a.Xl) + v * (up ? a.ldu : a.ldx) + (up ? c : c - a.Cu);
   }
   return a.Xl + (((size_t)z * a.H + y) * a.W + x) * a.ldx + c;
+}
+
+// A thread's place in a halo tile that begins one voxel before (z0, y0, x0): halo coordinates packed
+// once, so that a load is a few integer operations (divisions by the halo's sides and 64-bit index
+// products took longer than the products that they feed).
+__device__ __forceinline__ unsigned halo_pack(int hx, int hy, int hz) { return (unsigned)(hx | hy << 8 | hz << 16); }
+
+// Where a thread's 8 channels come from: Xl, or (up) the tensor of half the size. The tile's first voxel
+// is even, so the half-size offset of a halo voxel does not depend on the tile. Offsets in units of 8
+// channels fit 32 bits: two planes of a tensor that the device can hold have fewer than 2^34 elements.
+struct HaloFrom {
+  const __bf16* base;   // the tile's first voxel (not the halo's), the thread's channels
+  int row, plane, ld8, up;
+};
+__device__ __forceinline__ HaloFrom halo_from(const __bf16* Xl, int ldx, const __bf16* Xu, int ldu, int Cu, int H, int W, int z, int y,
+                                              int x, int c)
+{
+  HaloFrom f;
+  f.up = c < Cu;
+  f.row = f.up ? W >> 1 : W;
+  f.plane = f.up ? (H >> 1) * (W >> 1) : H * W;
+  f.ld8 = (f.up ? ldu : ldx) >> 3;
+  const size_t v = f.up ? ((size_t)(z >> 1) * (H >> 1) + (y >> 1)) * (W >> 1) + (x >> 1) : ((size_t)z * H + y) * W + x;
+  f.base = (f.up ? Xu : Xl) + v * (f.up ? ldu : ldx) + (f.up ? c : c - Cu);
+  return f;
+}
+__device__ __forceinline__ bf16x8 halo_load(const HaloFrom& f, unsigned h, bool in)
+{
+  const int dx = ((int)(h & 255u) - 1) >> f.up, dy = ((int)(h >> 8 & 255u) - 1) >> f.up, dz = ((int)(h >> 16) - 1) >> f.up;
+  return load_cl(f.base + (ptrdiff_t)((dz * f.plane + dy * f.row + dx) * f.ld8) * 8, in);
 }
 
 // bits t of the taps t = 9 (dz + 1) + 3 (dy + 1) + (dx + 1) whose three bits are all set
@@ -591,6 +537,15 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
     for (int i = 0; i < MT; i++) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
   const __bf16* ap = a.A + (size_t)rb0 * 512 + lane * 8;
   const size_t atap = (size_t)(a.Cbp >> 5) * a.nrb * 512;   // weights of the next tap
+  constexpr int kLoads = (FT_HALO * 4 + 255) / 256;
+  unsigned at[kLoads], ok = 0;
+#pragma unroll
+  for (int l = 0; l < kLoads; l++) {
+    const int v = (threadIdx.x + 256 * l) >> 2, hx = v % FT_HX, hy = (v / FT_HX) % FT_HY, hz = v / (FT_HX * FT_HY);
+    const int gz = z0 + hz - 1, gy = y0 + hy - 1, gx = x0 + hx - 1;
+    at[l] = halo_pack(hx, hy, hz);
+    if (v < FT_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W) ok |= 1u << l;
+  }
   const bf16x8* const hp = s_halo + kg * FT_HP + ((wave >> 1) * FT_HY + 4 * (wave & 1)) * FT_HX + r;
   for (int c0 = 0; c0 < a.Cbp; c0 += 32, ap += (size_t)a.nrb * 512) {
     bf16x8 av[FT_PF + 1][MT];   // the weights of FT_PF taps in flight
@@ -599,17 +554,10 @@ __global__ __launch_bounds__(256) void k_conv_tiled(ConvK a)
 #pragma unroll
       for (int i = 0; i < MT; i++) av[t][i] = *(const bf16x8*)(ap + t * atap + i * 512);
     // all of the thread's loads in flight at once, then the stores
-    constexpr int kLoads = (FT_HALO * 4 + 255) / 256;
+    const HaloFrom from = halo_from(a.Xl, a.ldx, a.Xu, a.ldu, MODE == FWDUP ? a.Cu : 0, a.H, a.W, z0, y0, x0, c0 + (threadIdx.x & 3) * 8);
     bf16x8 hv[kLoads];
 #pragma unroll
-    for (int l = 0; l < kLoads; l++) {
-      const int i = threadIdx.x + 256 * l, v = i >> 2, q = i & 3;
-      const int hx = v % FT_HX, hy = (v / FT_HX) % FT_HY, hz = v / (FT_HX * FT_HY);
-      const int gz = z0 + hz - 1, gy = y0 + hy - 1, gx = x0 + hx - 1;
-      const bool in = v < FT_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
-      const __bf16* p = voxel_cl<MODE>(a, gz, gy, gx, c0 + q * 8);
-      hv[l] = load_cl(p, in);
-    }
+    for (int l = 0; l < kLoads; l++) hv[l] = halo_load(from, at[l], ok >> l & 1u);
 #pragma unroll
     for (int l = 0; l < kLoads; l++) {
       const int i = threadIdx.x + 256 * l;
@@ -697,6 +645,7 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
   const size_t astep = (size_t)a.nrb * 2048;
   const bf16x8* const hp = halo + kg * FP_HP + r;
   constexpr int kLoads = 6;   // halo loads of a thread in flight
+  const int v_first = threadIdx.x / groups, q_first = threadIdx.x - v_first * groups, dv = 256 / groups, dq = 256 - dv * groups;
   for (int p = 0; p < 3; p++) {
     // the wave's steps w, w + 4, ... inside this tap plane
     const int first = wave + 4 * ((p * per_plane - wave + 3) >> 2);
@@ -731,18 +680,22 @@ __global__ __launch_bounds__(256) void k_conv_planes(ConvK a)
       if (f < n_mine) fetch(av[f]);
     if (p) __syncthreads();   // every wave is done with the last plane
     const int gz = MODE != BDATA ? z + p - 1 : z + 1 - p;
-    for (int i0 = threadIdx.x; i0 < FP_HALO * groups; i0 += 256 * kLoads) {
+    for (int v = v_first, q = q_first; v < FP_HALO;) {
       bf16x8 hv[kLoads];
       int at[kLoads];
 #pragma unroll
       for (int l = 0; l < kLoads; l++) {
-        const int i = i0 + 256 * l, v = i / groups, q = i - v * groups;
-        const int hy = v / 18, hx = v - hy * 18;
+        const int hy = (v * 3641) >> 16, hx = v - 18 * hy;   // v / 18, exact for v < 2^11
         const int gy = y0 + hy - 1, gx = x0 + hx - 1;
         const bool in = v < FP_HALO && (unsigned)gz < (unsigned)a.D && (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
-        const __bf16* g = voxel_cl<MODE>(a, gz, gy, gx, q * 8);
-        hv[l] = load_cl(g, in);
+        hv[l] = load_cl(voxel_cl<MODE>(a, gz, gy, gx, q * 8), in);
         at[l] = v < FP_HALO ? q * FP_HP + v : -1;
+        v += dv;
+        q += dq;
+        if (q >= groups) {
+          q -= groups;
+          v++;
+        }
       }
 #pragma unroll
       for (int l = 0; l < kLoads; l++)
@@ -985,28 +938,6 @@ hipError_t launch_conv(const ConvK& a, hipStream_t st)
   return hipGetLastError();
 }
 
-// Weight gradients outside the tiled form: about 2048 workgroups, of at least 256 voxels.
-hipError_t launch_bwgt(const ConvK& a, hipStream_t st)
-{
-  const int mt = mt_for(a.M);
-  dim3 grid((a.N + 15) / 16, (a.M + 16 * mt - 1) / (16 * mt), 1);
-  ConvK b = a;
-  const long long xy = (long long)grid.x * grid.y * a.samples;
-  int split = (int)std::max<long long>(1, std::min<long long>(2048 / std::max<long long>(1, xy), (a.K + 255) / 256));
-  const int kps = rup((a.K + split - 1) / split, 128);
-  b.splits = (a.K + kps - 1) / kps;
-  grid.z = b.splits * a.samples;
-  b.k_per_split = kps;
-  b.vec = (a.K % 4 == 0) ? 1 : 0;
-  switch (mt) {
-    case 1: hipLaunchKernelGGL(k_conv_bwgt<1>, grid, dim3(256), 0, st, b); break;
-    case 2: hipLaunchKernelGGL(k_conv_bwgt<2>, grid, dim3(256), 0, st, b); break;
-    case 3: hipLaunchKernelGGL(k_conv_bwgt<3>, grid, dim3(256), 0, st, b); break;
-    default: hipLaunchKernelGGL(k_conv_bwgt<4>, grid, dim3(256), 0, st, b); break;
-  }
-  return hipGetLastError();
-}
-
 // Stride-1 3x3x3 FWD / BDATA products with Cbp % 32 == 0 (k_conv_tiled); the row blocks as
 // k_conv's, so the A rows read stay inside the padded weight copy. Counted in 4-row tiles.
 inline long long tiled_blocks(const ConvK& a)
@@ -1043,20 +974,24 @@ hipError_t launch_conv_tiled(const ConvK& a, hipStream_t st)
 // its input X and of its output gradient dY:
 //   G[co][ci][t] = sum_q dY[co][q] X[ci][S q + d_t]      (MFMA m = co, n = ci, k = q)
 // A workgroup owns one block of 32 output and 32 input channels and a slab of output-voxel tiles
-// (4 rows x 16 voxels of one z-plane, 64 voxels = two 32-voxel k-steps); six waves split the
-// accumulators by tap plane dz (3) and input-channel half (2), each holding the 3 x 3 (dy, dx)
-// taps x 2 output-channel halves = 18 MFMA tiles. Per tile the workgroup stages in LDS, both
-// transposed to voxel-contiguous rows: dY of the tile's 64 voxels (32 x 64) and X of the input
-// region the tile's taps read (32 channels x 3 planes x 6 rows x 18 voxels for S = 1; 3 planes x
-// 9 rows x 33 voxels for S = 2, each row split into its even and odd voxels), so that each 8-voxel
-// k-group of a fragment is one aligned 16-byte LDS read: S = 1 voxel x at index x - x0 + 8, the
-// dx = -1 / +1 taps that read shifted by one voxel with v_alignbit across the neighbouring words;
-// S = 2 the even voxels 2 (x0 + j) at E[j] (dx = 0), the odd voxels 2 (x0 + j) - 1 at O[j] (dx = -1,
-// and shifted by one, dx = +1). Each workgroup writes its slab's sums to part[slab][t][co][ci];
+// (16 x 8 x 2 voxels for S = 1, 16 x 4 x 1 for S = 2); each half of a tile's voxels has six waves, which
+// split the accumulators by tap plane dz (3) and input-channel half (2), each holding the 3 x 3 (dy, dx)
+// taps x 2 output-channel halves = 18 MFMA tiles. dY of the tile and X of the region its taps read (18 x 10 x 4 voxels, 33 x 9 x 3 for
+// S = 2) are staged in LDS as they are, [voxel][32 channels], and the fragments, which want 8 voxels of
+// a channel per lane, are transposing reads (16 lanes give the addresses of 4 voxels x 4 channel quads
+// and get 4 voxels of one channel each), so a tap is an address offset. The next tile is on its way to
+// registers while one is multiplied. Each half writes its slab's sums to part[2 slab + half][t][co][ci];
 // k_bwgt_reduce adds the slabs in a fixed order into the gradient (deterministic, no atomics).
-#define BW_Y 4
+// 96 -> 32 channels on four volumes of 32 x 56 x 56: 234 us with element-wise transposed
+// stores, 140 with these reads and six waves per CU, 101 with twelve, 89 with the loads' places packed once
 #define BW_X 16
-#define BW_THREADS 384
+#define BW_THREADS 768
+template <int S>
+struct BwTile {
+  static constexpr int Y = S == 1 ? 8 : 4, Z = S == 1 ? 2 : 1;
+  static constexpr int HX = S * (BW_X - 1) + 3, HY = S * (Y - 1) + 3, HZ = S * (Z - 1) + 3;
+  static constexpr int NX = (HX * HY * HZ * 4 + BW_THREADS - 1) / BW_THREADS, NG = (BW_X * Y * Z * 4 + BW_THREADS - 1) / BW_THREADS;
+};
 
 struct BwK {
   const __bf16* Xl;   // input, channels-last [vox][ldx] (channels >= ldx: zero)
@@ -1065,46 +1000,31 @@ struct BwK {
   const __bf16* Gl;   // output gradient, channels-last [ovox][ldg]
   float* part;        // [n_slabs][27][32 cob][32 cib]
   int ldx, ldg, gch, Cin, Cout, D, H, W, oD, oH, oW;   // gch: channels from Gl on
-  int tiles_x, tiles_y, n_tiles, per_slab, cob, cib;   // n_tiles: of all samples
+  int tiles_x, tiles_y, tiles_z, n_tiles, per_slab, cob, cib;   // n_tiles: of all samples
   size_t sX, sXu, sG;                                  // from one sample to the next
 };
 
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef short short4v __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
-
-// words of v shifted by one BF16 element towards lower indices, the last one from `next`
-__device__ __forceinline__ u32x4 shift_down1(u32x4 v, unsigned next)
+// the lane's 8 voxels of its channel: two transposing reads, the second `next` bytes on
+__device__ __forceinline__ bf16x8 read_tr(const char* lds, int next)
 {
-  u32x4 o;
-  o[0] = __builtin_amdgcn_alignbit(v[1], v[0], 16);
-  o[1] = __builtin_amdgcn_alignbit(v[2], v[1], 16);
-  o[2] = __builtin_amdgcn_alignbit(v[3], v[2], 16);
-  o[3] = __builtin_amdgcn_alignbit(next, v[3], 16);
-  return o;
+  typedef __attribute__((address_space(3))) short4v lds4;
+  const short4v a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)lds);
+  const short4v b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(lds + next));
+  typedef short short8v __attribute__((ext_vector_type(8)));
+  return __builtin_bit_cast(bf16x8, (short8v)__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
 template <int S>
-struct BwLds;
-template <>
-struct BwLds<1> {
-  __bf16 x[32][3][6][32];   // 36 KB: [channel][plane][row][x - x0 + 8]
-};
-template <>
-struct BwLds<2> {
-  __bf16 e[32][3][9][16];   // even input voxels 2 (x0 + j), j = 0..15
-  __bf16 o[32][3][9][24];   // odd input voxels 2 (x0 + j) - 1, j = 0..16
-};
-
-template <int S>
-__global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
+__global__ __launch_bounds__(BW_THREADS, 3) void k_bwgt_tiled(BwK a)
 {
-  constexpr int HY = S == 1 ? 6 : 9, HX = S == 1 ? 18 : 33;   // input region: 3 x HY x HX voxels
-  __shared__ __attribute__((aligned(16))) BwLds<S> L;
-  __shared__ __attribute__((aligned(16))) __bf16 gs[32][64];   // 4 KB
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  typedef BwTile<S> T;
+  __shared__ __attribute__((aligned(16))) char s_x[T::HX * T::HY * T::HZ * 64];   // [voxel][32 channels]
+  __shared__ __attribute__((aligned(16))) char s_g[BW_X * T::Y * T::Z * 64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int lr = lane & 15, g = lane >> 4;
-  const int dz = wave % 3, nj = wave / 3;   // tap plane and input-channel half of this wave
+  const int dz = wave % 3, nj = wave / 3 & 1, half = wave / 6;   // tap plane, input-channel half, half of the k-steps
   const int slab = blockIdx.x, co0 = blockIdx.y * 32, ci0 = blockIdx.z * 32;
   floatx4 acc[3][3][2];
 #pragma unroll
@@ -1113,91 +1033,83 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
     for (int j = 0; j < 3; j++)
 #pragma unroll
       for (int m = 0; m < 2; m++) acc[i][j][m] = floatx4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 zero;
+  // the thread's channels and places are the same in every tile (BW_THREADS is a multiple of 4)
+  const int cx = ci0 + (threadIdx.x & 3) * 8, cg = co0 + (threadIdx.x & 3) * 8;
+  const bool x_in = cx < a.Cu + a.ldx;
+  unsigned at[T::NX];
 #pragma unroll
-  for (int e = 0; e < 8; e++) zero[e] = to_bf16(0.0f);
-  const int t_end = min(a.n_tiles, (slab + 1) * a.per_slab);
-  for (int tile = slab * a.per_slab; tile < t_end; tile++) {
+  for (int l = 0; l < T::NX; l++) {
+    const int v = (threadIdx.x + l * BW_THREADS) >> 2, hz = v / (T::HX * T::HY);
+    // 0xffff: past the region (the last one only)
+    at[l] = halo_pack(v % T::HX, (v / T::HX) % T::HY, hz < T::HZ ? hz : 0xffff);
+  }
+  bf16x8 xv[T::NX], gv[T::NG];
+  auto load = [&](int tile) {
     int b = tile;
     const int x0 = (b % a.tiles_x) * BW_X;
     b /= a.tiles_x;
-    const int y0 = (b % a.tiles_y) * BW_Y;
+    const int y0 = (b % a.tiles_y) * T::Y;
     b /= a.tiles_y;
-    const int z0 = b % a.oD, smp = b / a.oD;
+    const int z0 = (b % a.tiles_z) * T::Z, smp = b / a.tiles_z;
     const __bf16* const Xl = a.Xl + smp * a.sX;
     const __bf16* const Xu = a.Xu + smp * a.sXu;
     const __bf16* const Gl = a.Gl + smp * a.sG;
     // input region: voxel (S z0 - 1 + hz, S y0 - 1 + hy, S x0 - 1 + hx), 4 groups of 8 channels
-    for (int i = threadIdx.x; i < 3 * HY * HX * 4; i += BW_THREADS) {
-      const int q = i & 3, hv = i >> 2;
-      const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-      const int gz = S * z0 + hz - 1, gy = S * y0 + hy - 1, gx = S * x0 + hx - 1;
-      const int c = ci0 + q * 8;
-      bf16x8 v = zero;
-      if (gz >= 0 && gz < a.D && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W && c < a.Cu + a.ldx) {
-        if (c < a.Cu) v = *(const bf16x8*)(Xu + (((size_t)(gz >> 1) * (a.H >> 1) + (gy >> 1)) * (a.W >> 1) + (gx >> 1)) * a.ldu + c);
-        else v = *(const bf16x8*)(Xl + (((size_t)gz * a.H + gy) * a.W + gx) * a.ldx + (c - a.Cu));
-      }
-      if constexpr (S == 1) {
+    const int xz = S * z0, xy = S * y0, xx = S * x0;
+    const HaloFrom from = halo_from(Xl, a.ldx, Xu, a.ldu, a.Cu, a.H, a.W, xz, xy, xx, cx);
 #pragma unroll
-        for (int e = 0; e < 8; e++) L.x[q * 8 + e][hz][hy][hx + 7] = v[e];
-      } else if (hx & 1) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) L.e[q * 8 + e][hz][hy][hx >> 1] = v[e];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; e++) L.o[q * 8 + e][hz][hy][hx >> 1] = v[e];
-      }
+    for (int l = 0; l < T::NX; l++) {
+      const int gz = xz + (int)(at[l] >> 16) - 1, gy = xy + (int)(at[l] >> 8 & 255u) - 1, gx = xx + (int)(at[l] & 255u) - 1;
+      const bool in = x_in && (l + 1 < T::NX || at[l] >> 16 != 0xffff) && (unsigned)gz < (unsigned)a.D &&
+                      (unsigned)gy < (unsigned)a.H && (unsigned)gx < (unsigned)a.W;
+      xv[l] = halo_load(from, at[l], in);
     }
-    // dY of the tile's 64 output voxels, transposed into gs[c][q] (q = row * 16 + x)
-    for (int i = threadIdx.x; i < 64 * 4; i += BW_THREADS) {
-      const int q4 = i & 3, qv = i >> 2;
-      const int gy = y0 + (qv >> 4), gx = x0 + (qv & 15);
-      const int c = co0 + q4 * 8;
-      bf16x8 v = zero;
-      if (gy < a.oH && gx < a.oW && c < a.gch)
-        v = *(const bf16x8*)(Gl + (((size_t)z0 * a.oH + gy) * a.oW + gx) * a.ldg + c);
+    const __bf16* const gb = Gl + (((size_t)z0 * a.oH + y0) * a.oW + x0) * a.ldg + cg;
 #pragma unroll
-      for (int e = 0; e < 8; e++) gs[q4 * 8 + e][qv] = v[e];
+    for (int l = 0; l < T::NG; l++) {
+      const int v = (threadIdx.x + l * BW_THREADS) >> 2, dx = v % BW_X, dy = (v / BW_X) % T::Y, dz = v / (BW_X * T::Y);
+      const bool in = dz < T::Z && z0 + dz < a.oD && y0 + dy < a.oH && x0 + dx < a.oW && cg < a.gch;
+      gv[l] = load_cl(gb + (ptrdiff_t)((dz * a.oH + dy) * a.oW + dx) * a.ldg, in);
+    }
+  };
+  // what this lane reads of each fragment: voxel (lr / 4) of four, channels 4 (lr % 4) .. + 3 of 16
+  const int vj = lr >> 2, qb = (lr & 3) * 8;
+  const int hz = S == 1 ? half : 0, hy = S == 1 ? 0 : 2 * half;   // where the half begins: a plane, or two rows
+  const char* const ga = s_g + ((hz * T::Y + hy + (g >> 1)) * BW_X + (g & 1) * 8 + vj) * 64 + qb;
+  const char* const xa = s_x + (((S * hz + dz) * T::HY + S * (hy + (g >> 1))) * T::HX + S * ((g & 1) * 8 + vj)) * 64 + 32 * nj + qb;
+  const int t_end = min(a.n_tiles, (slab + 1) * a.per_slab);
+  int tile = slab * a.per_slab;
+  if (tile < t_end) load(tile);
+  for (; tile < t_end; tile++) {
+#pragma unroll
+    for (int l = 0; l < T::NX; l++) {
+      const int i = threadIdx.x + l * BW_THREADS;
+      if (i < T::HX * T::HY * T::HZ * 4) *(bf16x8*)(s_x + i * 16) = xv[l];
+    }
+#pragma unroll
+    for (int l = 0; l < T::NG; l++) {
+      const int i = threadIdx.x + l * BW_THREADS;
+      if (i < BW_X * T::Y * T::Z * 4) *(bf16x8*)(s_g + i * 16) = gv[l];
     }
     __syncthreads();
+    if (tile + 1 < t_end) load(tile + 1);
+    __builtin_amdgcn_sched_barrier(0);   // the loads are issued before the products
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      const int r = 2 * ks + (g >> 1), xh = (g & 1) * 8;   // this lane's 8 voxels: row r, x = xh .. xh + 7
+    for (int ks = 0; ks < T::Y * T::Z / 4; ks++) {   // 32 voxels: two rows of the wave's half of the tile
+      constexpr int rows = T::Y / (S == 1 ? 2 : 4);   // pairs of rows in a plane of the half
+      const int oz = ks / rows, oy = 2 * (ks % rows);
       bf16x8 av[2];
 #pragma unroll
-      for (int m = 0; m < 2; m++) av[m] = *(const bf16x8*)&gs[16 * m + lr][r * 16 + xh];
+      for (int m = 0; m < 2; m++) av[m] = read_tr(ga + (oz * T::Y + oy) * (BW_X * 64) + 32 * m, 256);
 #pragma unroll
-      for (int dy = 0; dy < 3; dy++) {
-        bf16x8 bx[3];   // the dx = -1, 0, +1 fragments
-        if constexpr (S == 1) {
-          const __bf16* row = &L.x[16 * nj + lr][dz][r + dy][0];
-          const u32x4 bm = *(const u32x4*)(row + xh + 8);          // x = xh .. xh + 7
-          const unsigned lo = *(const unsigned*)(row + xh + 6);    // x = xh - 2, xh - 1
-          const unsigned hi = *(const unsigned*)(row + xh + 16);   // x = xh + 8, xh + 9
-          u32x4 bl;
-          bl[0] = __builtin_amdgcn_alignbit(bm[0], lo, 16);
-          bl[1] = __builtin_amdgcn_alignbit(bm[1], bm[0], 16);
-          bl[2] = __builtin_amdgcn_alignbit(bm[2], bm[1], 16);
-          bl[3] = __builtin_amdgcn_alignbit(bm[3], bm[2], 16);
-          bx[0] = as_bf16x8(bl);
-          bx[1] = as_bf16x8(bm);
-          bx[2] = as_bf16x8(shift_down1(bm, hi));
-        } else {
-          const int yy = 2 * r + dy;
-          const __bf16* orow = &L.o[16 * nj + lr][dz][yy][0];
-          const u32x4 ov = *(const u32x4*)(orow + xh);             // O[xh .. xh + 7]: x = 2 j - 1
-          const unsigned hi = *(const unsigned*)(orow + xh + 8);   // O[xh + 8], O[xh + 9]
-          bx[0] = as_bf16x8(ov);
-          bx[1] = *(const bf16x8*)&L.e[16 * nj + lr][dz][yy][xh];  // x = 2 j
-          bx[2] = as_bf16x8(shift_down1(ov, hi));                  // x = 2 j + 1
-        }
+      for (int dy = 0; dy < 3; dy++)
 #pragma unroll
-        for (int dx = 0; dx < 3; dx++)
+        for (int dx = 0; dx < 3; dx++) {
+          const bf16x8 bx = read_tr(xa + ((S * oz * T::HY + S * oy + dy) * T::HX + dx) * 64, S * 256);
 #pragma unroll
           for (int m = 0; m < 2; m++)
-            acc[dy][dx][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bx[dx], acc[dy][dx][m], 0, 0, 0);
-      }
+            acc[dy][dx][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bx, acc[dy][dx][m], 0, 0, 0);
+        }
     }
     __syncthreads();
   }
@@ -1208,7 +1120,7 @@ __global__ __launch_bounds__(BW_THREADS) void k_bwgt_tiled(BwK a)
 #pragma unroll
     for (int dx = 0; dx < 3; dx++) {
       const int t = dz * 9 + dy * 3 + dx;
-      float* p = a.part + ((size_t)slab * 27 + t) * CoutR * CinR + (ci0 + 16 * nj + lr);
+      float* p = a.part + ((size_t)(2 * slab + half) * 27 + t) * CoutR * CinR + (ci0 + 16 * nj + lr);
 #pragma unroll
       for (int m = 0; m < 2; m++)
 #pragma unroll
@@ -1243,23 +1155,23 @@ __global__ __launch_bounds__(256) void k_bwgt_reduce(const float* __restrict__ p
   if (ph == 0 && i < n) G[((size_t)co * Cin + ci) * 27 + t] += ((ps[0][j] + ps[1][j]) + ps[2][j]) + ps[3][j];
 }
 
-// Workgroups of the tiled weight gradient: about BW_WGS in total, the output-voxel tiles dealt
-// to slabs of equal length; the partial sums then fit in BW_WGS x 27 x 1024 floats.
-#ifndef BW_WGS
-#define BW_WGS 512
-#endif
-inline void bwgt_shape(int samples, int oD, int oH, int oW, int Cin, int Cout, BwK& b, int& n_slabs)
+// Workgroups of the tiled weight gradient: about BW_WGS in total (one per CU), the output-voxel tiles
+// dealt to slabs of equal length; each workgroup's two halves write their own partial sums.
+#define BW_WGS 256
+inline void bwgt_shape(int samples, int stride, BwK& b, int& n_slabs)
 {
-  b.tiles_x = (oW + BW_X - 1) / BW_X;
-  b.tiles_y = (oH + BW_Y - 1) / BW_Y;
-  b.n_tiles = b.tiles_x * b.tiles_y * oD * samples;
-  b.cob = (Cout + 31) / 32;
-  b.cib = (Cin + 31) / 32;
+  const int ty = stride == 1 ? BwTile<1>::Y : BwTile<2>::Y, tz = stride == 1 ? BwTile<1>::Z : BwTile<2>::Z;
+  b.tiles_x = (b.oW + BW_X - 1) / BW_X;
+  b.tiles_y = (b.oH + ty - 1) / ty;
+  b.tiles_z = (b.oD + tz - 1) / tz;
+  b.n_tiles = b.tiles_x * b.tiles_y * b.tiles_z * samples;
+  b.cob = (b.Cout + 31) / 32;
+  b.cib = (b.Cin + 31) / 32;
   n_slabs = std::max(1, std::min(b.n_tiles, BW_WGS / (b.cob * b.cib)));
   b.per_slab = (b.n_tiles + n_slabs - 1) / n_slabs;
   n_slabs = (b.n_tiles + b.per_slab - 1) / b.per_slab;
 }
-constexpr size_t kBwPartFloats = (size_t)BW_WGS * 27 * 1024;   // a workgroup writes 27 x 32 x 32
+constexpr size_t kBwPartFloats = (size_t)BW_WGS * 2 * 27 * 1024;   // half a workgroup writes 27 x 32 x 32
 
 // The input x and its gradient's copy gyl as in conv_bwd_weights; stride 1 (input and output volumes
 // equal) or 2 (output (D/2, H/2, W/2)). Output channels go in passes of as many 32-channel blocks as
@@ -1274,13 +1186,13 @@ hipError_t launch_bwgt_tiled(int samples, int stride, BwK b, const __bf16* gyl, 
     b.Gl = gyl + co;
     b.gch = b.ldg - co;
     int n_slabs = 0;
-    bwgt_shape(samples, b.oD, b.oH, b.oW, b.Cin, b.Cout, b, n_slabs);
+    bwgt_shape(samples, stride, b, n_slabs);
     const dim3 g(n_slabs, b.cob, b.cib);
     if (stride == 1) hipLaunchKernelGGL(k_bwgt_tiled<1>, g, dim3(BW_THREADS), 0, st, b);
     else hipLaunchKernelGGL(k_bwgt_tiled<2>, g, dim3(BW_THREADS), 0, st, b);
     const long long n = (long long)b.Cout * b.Cin * 27;
     hipLaunchKernelGGL(k_bwgt_reduce, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, (const float*)b.part,
-                       G + (size_t)co * b.Cin * 27, b.Cout, b.Cin, 32 * b.cob, 32 * b.cib, n_slabs);
+                       G + (size_t)co * b.Cin * 27, b.Cout, b.Cin, 32 * b.cob, 32 * b.cib, 2 * n_slabs);
   }
   return hipGetLastError();
 }
@@ -1376,21 +1288,34 @@ __global__ void k_upsample_bwd(const float* __restrict__ gy, size_t sy, const __
   }
   *(bf16x8*)(o.p + vl * o.ld + c0) = q;
 }
-// per-channel sum (bias gradient): workgroups (channel, chunk of `per` voxels, sample), added atomically
-__global__ void k_channel_sum(const float* __restrict__ g, size_t sg, float* __restrict__ out, int vox, int per)
+// per-channel sum (bias gradient): workgroups (channel, chunk of `per` voxels, sample), added
+// atomically; four voxels a read where the channels' beginnings allow it
+__global__ __launch_bounds__(256) void k_channel_sum(const float* __restrict__ g, size_t sg, float* __restrict__ out, int vox, int per)
 {
-  __shared__ float sh[256];
+  __shared__ float sh[4];
   const float* p = g + blockIdx.z * sg + (size_t)blockIdx.x * vox;
   const int b = blockIdx.y * per, e = min(vox, b + per);
   float s = 0.0f;
-  for (int i = b + threadIdx.x; i < e; i += blockDim.x) s += p[i];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
+  if ((vox & 3) == 0 && ((uintptr_t)p & 15) == 0) {   // per is a multiple of 4
+    const float4* p4 = (const float4*)p;
+    float4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int i = b / 4 + threadIdx.x; i < e / 4; i += 256) {
+      const float4 v = p4[i];
+      t.x += v.x;
+      t.y += v.y;
+      t.z += v.z;
+      t.w += v.w;
+    }
+    s = (t.x + t.y) + (t.z + t.w);
+  } else {
+    for (int i = b + threadIdx.x; i < e; i += 256) s += p[i];
   }
-  if (threadIdx.x == 0) atomicAdd(&out[blockIdx.x], sh[0]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(&out[blockIdx.x], (sh[0] + sh[1]) + (sh[2] + sh[3]));
 }
 // loss gradient (and its channels-last copy) and squared error of the output
 __global__ void k_loss(const float* __restrict__ out, const float* __restrict__ target, float* __restrict__ g, float scale,
@@ -1549,7 +1474,7 @@ struct mcpet_surrogate {
   __bf16 *x0l = nullptr, *a1l = nullptr, *b1l = nullptr, *cat1l = nullptr, *d1l = nullptr, *b2l = nullptr, *cat2l = nullptr,
          *d2l = nullptr, *b3l = nullptr, *e2l = nullptr, *e1l = nullptr;
   __bf16 *grl = nullptr, *ge1l = nullptr, *ge2l = nullptr, *gb3l = nullptr, *gd2l = nullptr, *gb2l = nullptr, *gd1l = nullptr,
-         *gb1l = nullptr;
+         *gb1l = nullptr, *ga1l = nullptr;
   float *raw_s = nullptr, *raw_t = nullptr, *est = nullptr;   // the fused estimate's buffers
   int slots = 0;                                                // samples that the tensors above have room for
   double* sums = nullptr;                                       // 256 partial totals + the total
@@ -1696,20 +1621,19 @@ hipError_t conv_bwd_data(mcpet_surrogate* s, int ns, const Conv& l, const Vol& v
   return use_tiled(a) ? launch_conv_tiled<BDATA>(a, s->st) : launch_conv<BDATA>(a, s->st);
 }
 // weight and bias gradients accumulated from gy (dL/d pre-activation, with its channels-last copy
-// gyl) and the layer input x. The output layer and the 3x3x3 layers that the tiled product takes read
-// the copies, the others FP32 x0 and gy.
+// gyl) and the layer input x
 hipError_t conv_bwd_weights(mcpet_surrogate* s, int ns, const Conv& l, const Vol& vin, ClIn x, const Vol& vout, const float* gy,
-                            size_t sg, const __bf16* gyl, const float* x0 = nullptr)
+                            size_t sg, const __bf16* gyl)
 {
   const int vox = (int)vout.vox(), per = 4096;
   hipError_t e = hipSuccess;
-  if (l.ks == 1 && l.cout == 1 && x.ld <= 256) {
+  if (l.ks == 1) {   // the output layer: one channel from at most 256
     const size_t n = (size_t)ns * vox;
     const int chunk = (int)std::max<size_t>(256, (n + 1023) / 1024);
     hipLaunchKernelGGL(k_bwgt_point, dim3((unsigned)((n + chunk - 1) / chunk)), dim3(256), 0, s->st, x.xl, x.ld, gyl, s->g + l.w,
                        l.cin, n, chunk);
     e = hipGetLastError();
-  } else if (!x0) {
+  } else {
     BwK b{};
     b.Xl = x.xl;
     b.Xu = x.xu;
@@ -1725,20 +1649,6 @@ hipError_t conv_bwd_weights(mcpet_surrogate* s, int ns, const Conv& l, const Vol
     b.sXu = vin.vox() / 8 * x.Cu;
     b.sG = vout.vox() * b.ldg;
     e = launch_bwgt_tiled(ns, l.stride, b, gyl, s->g + l.w, s->st);
-  } else {
-    ConvK a = conv_args(l, vin, vout);
-    a.Ad = gy;
-    a.X = x0;
-    a.C = s->g + l.w;
-    a.M = l.cout;
-    a.N = a.T * l.cin;
-    a.K = vox;
-    a.Cb = l.cin;
-    a.Cbp = l.cin;
-    a.samples = ns;
-    a.sX = vin.size();
-    a.sC = sg;
-    e = launch_bwgt(a, s->st);
   }
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_channel_sum, dim3(l.cout, (vox + per - 1) / per, ns), dim3(256), 0, s->st, gy, sg, s->g + l.b, vox, per);
@@ -1839,7 +1749,7 @@ hipError_t backward(mcpet_surrogate* s, int ns)
   float* gb2 = s->gcat2 + (size_t)4 * c * vb2.vox();
 #define STEP(x) \
   if (e == hipSuccess) e = (x)
-#define WGT(l, vin, x, vout, gy, sg, gyl, ...) STEP(conv_bwd_weights(s, ns, s->L[l], vin, x, vout, gy, sg, gyl, ##__VA_ARGS__))
+#define WGT(l, vin, x, vout, gy, sg, gyl) STEP(conv_bwd_weights(s, ns, s->L[l], vin, x, vout, gy, sg, gyl))
 #define DATA(l, vin, vout, gyl, gx, sx, mask, mask0, add, o1) \
   STEP(conv_bwd_data(s, ns, s->L[l], vin, vout, gyl, gx, sx, mask, mask0, add, o1))
   WGT(8, s->ve1, in(s->e1l, c), s->vr, s->gr, s->vr.size(), s->grl);
@@ -1859,8 +1769,8 @@ hipError_t backward(mcpet_surrogate* s, int ns)
   WGT(2, vb1, in(s->b1l, c), s->vd1, s->gd1, s->vd1.size(), s->gd1l);
   DATA(2, vb1, s->vd1, s->gd1l, gb1, s1, cl(s->b1l, c), 0, true, cl(s->gb1l, c));              // + the skip's gradient
   WGT(1, s->va1, in(s->a1l, c), vb1, gb1, s1, s->gb1l);
-  DATA(1, s->va1, vb1, s->gb1l, s->ga1, s->va1.size(), cl(s->a1l, c), 0, false, kNoCl);
-  WGT(0, s->vx, in(s->x0l, s->cin), s->va1, s->ga1, s->va1.size(), nullptr, s->x0);
+  DATA(1, s->va1, vb1, s->gb1l, s->ga1, s->va1.size(), cl(s->a1l, c), 0, false, cl(s->ga1l, c));
+  WGT(0, s->vx, in(s->x0l, s->cin), s->va1, s->ga1, s->va1.size(), s->ga1l);
 #undef WGT
 #undef DATA
 #undef STEP
@@ -1889,7 +1799,7 @@ std::vector<Slot> sample_tensors(mcpet_surrogate* s)
   h(&s->d1l, v1, 2 * c), h(&s->b2l, v1, 2 * c), h(&s->cat2l, cat ? v1 : 0, 6 * c), h(&s->d2l, v2, 4 * c);
   h(&s->e1l, v0, c), h(&s->e2l, v1, 2 * c), h(&s->b3l, v2, 4 * c);
   h(&s->grl, v0, 8), h(&s->ge1l, v0, c), h(&s->ge2l, v1, 2 * c), h(&s->gb3l, v2, 4 * c);
-  h(&s->gd2l, v2, 4 * c), h(&s->gb2l, v1, 2 * c), h(&s->gd1l, v1, 2 * c), h(&s->gb1l, v0, c);
+  h(&s->gd2l, v2, 4 * c), h(&s->gb2l, v1, 2 * c), h(&s->gd1l, v1, 2 * c), h(&s->gb1l, v0, c), h(&s->ga1l, v0, c);
   return t;
 }
 

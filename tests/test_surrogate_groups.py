@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import mcpet
-from test_surrogate import integer_network, unet_reference
+from test_surrogate import _layer_rel, integer_network, unet_reference
 
 
 def _network(grid, cin, c, rng):
@@ -54,3 +54,22 @@ def test_ragged_tiles_are_exact_on_integer_networks(grid, batch):
     _, _, yr = unet_reference(p, x.astype(np.float64), np.zeros((batch,) + grid), cin, c, "bf16", grad=False)
     assert np.abs(yr).max() < 2.0 ** 24 and np.all(yr == np.round(yr))
     assert np.array_equal(net.forward(x).astype(np.float64), yr)
+
+
+# width 160: the weight gradient of 960 -> 320 channels goes in two passes of output channels, the
+# others in one; remainders of the tiles of both strides in x, y and z
+@pytest.mark.gpu
+@pytest.mark.parametrize("grid,c,batch", [((4, 4, 4), 160, 1), ((12, 20, 36), 8, 2)])
+def test_weight_gradients_match_the_reference(grid, c, batch):
+    """The bounds of test_surrogate's comparison: 2e-3 a layer, or four times what float32 sums in
+    another order change."""
+    cin = 2
+    rng = np.random.default_rng(c)
+    net = _network(grid, cin, c, rng)
+    p = net.params().astype(np.float64)
+    x, t = rng.random((batch, cin) + grid), rng.random((batch,) + grid)
+    x, t = x.astype(np.float32), t.astype(np.float32)
+    _, g = net.gradients(x, t)
+    gr, g32 = (unet_reference(p, x.astype(np.float64), t.astype(np.float64), cin, c, m)[1] for m in ("bf16", "bf16f32"))
+    rel, rel32 = _layer_rel(g.astype(np.float64), gr, cin, c), _layer_rel(g32, gr, cin, c)
+    assert all(r <= max(2e-3, 4 * r32) for r, r32 in zip(rel, rel32)), (rel, rel32)
