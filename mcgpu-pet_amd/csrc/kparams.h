@@ -165,7 +165,7 @@ hipError_t mcpet_launch_transport(const KParams& P, const KParams* d_P, int kind
 int mcpet_transport_resident(const KParams& P, int count_events, int block_size);
 // dynamic LDS of a single-phantom launch (bytes)
 size_t mcpet_transport_dyn_lds(const KParams& P);
-hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, int n_shells, bool ext, int count_events, int blocks,
+hipError_t mcpet_launch_transport_batch(const KParams* d_params, int n, int n_shells, int n_spec, bool ext, int count_events, int blocks,
                                         int block_size, hipStream_t stream);
 hipError_t mcpet_launch_fill_u32(void* p, size_t n_words, hipStream_t stream);
 // zero n regions of n_words[i] 4-byte words at p[i], K_FILL_MAX regions per launch

@@ -1687,6 +1687,7 @@ mcpet_status mcpet_run_contexts(const CtxRun* runs, int n, hipStream_t stream, K
     return set_err(nullptr, st, m);
   };
   bool ext = false;
+  int n_spec = 0;
   for (int k = 0; k < n; k++) {
     mcpet_ctx* c = runs[k].c;
     KParams P = c->P;
@@ -1695,7 +1696,7 @@ mcpet_status mcpet_run_contexts(const CtxRun* runs, int n, hipStream_t stream, K
     P.stream_base = runs[k].begin;
     P.n_streams = runs[k].end;
     P.sm_policy = 0;
-    P.lds_spectrum = 0;
+    if (P.lds_spectrum) n_spec = std::max(n_spec, P.ne);
     P.lds_palette = 0;
     set_claims(P, c->expected_rate * effective_seconds(c->cfg.mean_life, P.acq_ps) * (double)(P.n_streams - P.stream_base) /
                       (double)std::max(1LL, c->P.n_streams), (long long)blocks * (block_size / 64), false);
@@ -1709,7 +1710,7 @@ mcpet_status mcpet_run_contexts(const CtxRun* runs, int n, hipStream_t stream, K
     c->ran = true;
   }
   hipError_t e = hipMemcpyAsync(d_params, h_params, sizeof(KParams) * (size_t)n, hipMemcpyHostToDevice, stream);
-  if (e == hipSuccess) e = mcpet_launch_transport_batch(d_params, n, h_params[0].n_shells, ext, 0, blocks, block_size, stream);
+  if (e == hipSuccess) e = mcpet_launch_transport_batch(d_params, n, h_params[0].n_shells, n_spec, ext, 0, blocks, block_size, stream);
   for (int k = 0; k < n && e == hipSuccess; k++) e = hipEventRecord(runs[k].c->ev_done, stream);
   if (e != hipSuccess) return fail(MCPET_E_HIP, std::string("batched launch: ") + hipGetErrorString(e));
   return MCPET_OK;
@@ -1816,6 +1817,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
   BHIP(b, hipStreamSynchronize(b->stream));   // the staging copy of the parameters is reused
   const int n = (int)b->ctx.size();
   bool ext = false;
+  int n_spec = 0;
   for (int k = 0; k < n; k++) {
     KParams P = b->ctx[k]->P;
     if (p.seed != 0) P.seed = p.seed;
@@ -1826,7 +1828,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
     P.sm_policy = (policy == 2) ? 1 : 0;
     static const int default_cost[MCPET_NPHASES] = {4, 6, 1, 3, 6, 3, 2, 4, 4, 1};
     for (int i = 0; i < MCPET_NPHASES; i++) P.sm_cost[i] = p.phase_cost[i] > 0 ? p.phase_cost[i] : default_cost[i];
-    P.lds_spectrum = 0;   // per phantom: global atomics
+    if (P.lds_spectrum) n_spec = std::max(n_spec, P.ne);
     P.lds_palette = 0;
     ext = ext || P.prompt_frac > 0.0f || P.mode != 2;
     b->h_params[k] = P;
@@ -1852,7 +1854,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
       mcpet_status st = MCPET_OK;
       for (int k = 0; k < n && st == MCPET_OK; k++) st = clear_buffers(b->ctx[k], b->stream, p.zero_tallies != 0, true);
       hipError_t e = hipSuccess;
-      if (st == MCPET_OK) e = mcpet_launch_transport_batch(b->d_params, n, b->h_params[0].n_shells, ext, p.count_events, blocks, bs, b->stream);
+      if (st == MCPET_OK) e = mcpet_launch_transport_batch(b->d_params, n, b->h_params[0].n_shells, n_spec, ext, p.count_events, blocks, bs, b->stream);
       hipGraph_t g = nullptr;
       hipError_t e2 = hipStreamEndCapture(b->stream, &g);
       if ((st != MCPET_OK || e != hipSuccess || e2 != hipSuccess) && g) (void)hipGraphDestroy(g);
@@ -1872,7 +1874,7 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
       if (st != MCPET_OK) return st;
     }
     BHIP(b, hipEventRecord(b->ev0, b->stream));
-    hipError_t e = mcpet_launch_transport_batch(b->d_params, n, b->h_params[0].n_shells, ext, p.count_events, blocks, bs, b->stream);
+    hipError_t e = mcpet_launch_transport_batch(b->d_params, n, b->h_params[0].n_shells, n_spec, ext, p.count_events, blocks, bs, b->stream);
     if (e != hipSuccess) return bset_err(b, MCPET_E_HIP, std::string("batch launch failed: ") + hipGetErrorString(e));
     BHIP(b, hipEventRecord(b->ev1, b->stream));
   }
