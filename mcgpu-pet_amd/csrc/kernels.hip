@@ -69,13 +69,12 @@
 #ifndef MCPET_CHAIN
 #define MCPET_CHAIN 31
 #endif
+// Five waves per SIMD (96 registers, 32 KB of LDS a workgroup): head, 1e8 decays, 31.9 ms with four, 29.0
+// with five, 29.1 with six, whose 80 registers spill.
 #ifndef MCPET_WAVES_PER_EU
-#define MCPET_WAVES_PER_EU 6
+#define MCPET_WAVES_PER_EU 5
 #endif
-#ifndef MCPET_WAVES_PER_EU_EXT
-#define MCPET_WAVES_PER_EU_EXT 5
-#endif
-#define K_OCCUPANCY(ext) __attribute__((amdgpu_waves_per_eu((ext) ? MCPET_WAVES_PER_EU_EXT : MCPET_WAVES_PER_EU, 8)))
+#define K_OCCUPANCY __attribute__((amdgpu_waves_per_eu(MCPET_WAVES_PER_EU, 8)))
 // Per-phase execution statistics of the persistent kernel (diagnostic builds only).
 #ifndef MCPET_SM_STATS
 #define MCPET_SM_STATS 0
@@ -582,10 +581,69 @@ __device__ __forceinline__ void spectrum_add(const KParams& P, int* s_spec, int 
   else gatomic_add(&P.spectrum[iE], 1);
 }
 
+// Pairs whose bin is known wait in LDS for the rest of their tally, HIT_LEN a wave: about one decay in
+// ten gets that far, three lanes of a wave at a time, and the energy blur of 64 lanes costs as much.
+// An entry holds what is left to compute with, the four random numbers (drawn in their turn) among it;
+// the tallies are integer sums, whose order does not matter. The number of entries is wq[3]. Not with
+// lists (kExt), whose registers it would cost more than it gives (torso 34.0 -> 34.2 ms). Head, 1e8
+// decays, 29.3 -> 28.5 ms; 5e6 decays on the estimate's phantom 1.67 -> 1.61.
+#define HIT_LEN 24
+#define HIT_FULL 16   // enough to take them all
+enum HitWord { HIT_E1 = 0, HIT_E2, HIT_R1, HIT_R2, HIT_R3, HIT_R4, HIT_BIN, HIT_VOX, HIT_WORDS };   // HIT_VOX: voxel, sign: scattered
+typedef K_LDS float* HitQueue;   // [HIT_WORDS][HIT_LEN]
+
+template <class CN>
+__device__ __forceinline__ void tally_hit(const KParams& P, float energy, float energyFirst, float randno1, float randno2,
+                                          float randno3, float randno4, int ibin, int absvox, bool scattered, CN& C, int* s_spec)
+{
+  // -2 log(u) is zero or above 1e-7; the doubling is exact
+  float g1 = sqrt_nz(-2.0f * log_n(randno1 + 1e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno2));
+  float g2 = sqrt_nz(-2.0f * log_n(randno3 + 1.0e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno4));
+  float Energia1 = energy + ((P.e_resol) / 2.35f) * energy * g1;
+  float Energia2 = energyFirst + ((P.e_resol) / 2.35f) * energyFirst * g2;
+  int iE1 = floor_i32(div_r(Energia1, 1000.0f, 1.0f / 1000.0f));
+  int iE2 = floor_i32(div_r(Energia2, 1000.0f, 1.0f / 1000.0f));
+  if ((iE1 < P.ne) && (iE1 >= 0)) spectrum_add(P, s_spec, iE1);
+  if ((iE2 < P.ne) && (iE2 >= 0)) spectrum_add(P, s_spec, iE2);
+  C.inc(KC_PAIRS);
+  if ((Energia1) > (P.e_low) && (Energia1) < (P.e_high) && (Energia2) > (P.e_low) && (Energia2) < (P.e_high)) {
+    C.inc(KC_COINC);
+    gatomic_add(scattered ? &P.scatter[ibin] : &P.trues[ibin], 1);
+    gatomic_add(scattered ? &P.img_sc[absvox] : &P.img_t[absvox], 1);
+    if (P.rb_trues) {   // the same event on the rebinning grid (sinogram, angle, radial bin of ibin)
+      const int per = P.nangles * P.nrad;
+      const int izm = ibin / per, rem = ibin - izm * per;
+      const int ith = rem / P.nrad, ir = rem - ith * P.nrad;
+      const int cb = (P.rb_plane[izm] * P.rb_H + ith / P.rb_gh) * P.rb_W + ir / P.rb_gw;
+      gatomic_add(scattered ? &P.rb_scatter[cb] : &P.rb_trues[cb], 1);
+    }
+  }
+}
+
+// every waiting entry; by the whole wave
+template <class CN>
+__device__ __forceinline__ void hits_take(const KParams& P, HitQueue hq, volatile K_LDS long long* wq, CN& C, int* s_spec)
+{
+  const int lane = (int)(threadIdx.x & 63);
+  const int c = __builtin_amdgcn_readfirstlane((int)wq[3]);
+  __builtin_amdgcn_wave_barrier();
+  if (lane < c) {
+    float e[HIT_WORDS];
+#pragma unroll
+    for (int k = 0; k < HIT_WORDS; k++) e[k] = ((volatile K_LDS float*)hq)[k * HIT_LEN + lane];
+    const int v = __float_as_int(e[HIT_VOX]);
+    tally_hit(P, e[HIT_E1], e[HIT_E2], e[HIT_R1], e[HIT_R2], e[HIT_R3], e[HIT_R4], __float_as_int(e[HIT_BIN]), v & 0x7fffffff,
+              v < 0, C, s_spec);
+  }
+  __builtin_amdgcn_wave_barrier();
+  if (lane == 0) wq[3] = 0;
+}
+
 // tally_Sinogram (K:1623-1836).
 template <class CN>
 K_RARE void tally_sinogram(const KParams& P, float energy, float energyFirst, const float* pos, const float* posf,
-                               const float* dir, const float* dirf, int ss, int ssf, Stream& st, CN& C, int* s_spec)
+                               const float* dir, const float* dirf, int ss, int ssf, Stream& st, CN& C, int* s_spec,
+                               HitQueue hq, volatile K_LDS long long* wq)
 {
   float x0 = pos[0] - P.cx, y0 = pos[1] - P.cy;
   float dist = cyl_dist(P, x0, y0, dir);
@@ -605,39 +663,26 @@ K_RARE void tally_sinogram(const KParams& P, float energy, float energyFirst, co
   const float phi1 = mcf_atan2f(pfyn, pfxn);
   int ibin = sino_bin(P, phi, pzn, phi1, pfzn);
   if (ibin < 0) return;
-  float randno1 = rn(st.r, C);
-  float randno2 = rn(st.r, C);
-  // -2 log(u) is zero or above 1e-7; the doubling is exact
-  float g1 = sqrt_nz(-2.0f * log_n(randno1 + 1e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno2));
-  float randno3 = rn(st.r, C);
-  float randno4 = rn(st.r, C);
-  float g2 = sqrt_nz(-2.0f * log_n(randno3 + 1.0e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno4));
-  float Energia1 = energy + ((P.e_resol) / 2.35f) * energy * g1;
-  float Energia2 = energyFirst + ((P.e_resol) / 2.35f) * energyFirst * g2;
-  int iE1 = floor_i32(div_r(Energia1, 1000.0f, 1.0f / 1000.0f));
-  int iE2 = floor_i32(div_r(Energia2, 1000.0f, 1.0f / 1000.0f));
-  if ((iE1 < P.ne) && (iE1 >= 0)) spectrum_add(P, s_spec, iE1);
-  if ((iE2 < P.ne) && (iE2 >= 0)) spectrum_add(P, s_spec, iE2);
-  C.inc(KC_PAIRS);
-  if ((Energia1) > (P.e_low) && (Energia1) < (P.e_high) && (Energia2) > (P.e_low) && (Energia2) < (P.e_high)) {
-    if (ss == 0 && ssf == 0) {
-      gatomic_add(&P.trues[ibin], 1);
-      gatomic_add(&P.img_t[st.absvox], 1);
-      C.inc(KC_COINC);
-    }
-    if (ss > 0 || ssf > 0) {
-      gatomic_add(&P.scatter[ibin], 1);
-      gatomic_add(&P.img_sc[st.absvox], 1);
-      C.inc(KC_COINC);
-    }
-    if (P.rb_trues) {   // the same event on the rebinning grid (sinogram, angle, radial bin of ibin)
-      const int per = P.nangles * P.nrad;
-      const int izm = ibin / per, rem = ibin - izm * per;
-      const int ith = rem / P.nrad, ir = rem - ith * P.nrad;
-      const int cb = (P.rb_plane[izm] * P.rb_H + ith / P.rb_gh) * P.rb_W + ir / P.rb_gw;
-      gatomic_add((ss == 0 && ssf == 0) ? &P.rb_trues[cb] : &P.rb_scatter[cb], 1);
+  const float randno1 = rn(st.r, C);
+  const float randno2 = rn(st.r, C);
+  const float randno3 = rn(st.r, C);
+  const float randno4 = rn(st.r, C);
+  const bool scattered = ss > 0 || ssf > 0;
+  if (hq) {
+    const unsigned long long here = __ballot(1);
+    const int n = __popcll(here), rank = __popcll(here & ((1ull << __lane_id()) - 1ull));
+    const int at = __builtin_amdgcn_readfirstlane((int)wq[3]);
+    __builtin_amdgcn_wave_barrier();
+    if (at + n <= HIT_LEN) {
+      const float e[HIT_WORDS] = {energy, energyFirst, randno1, randno2, randno3, randno4, __int_as_float(ibin),
+                                  __int_as_float(st.absvox | (scattered ? (int)0x80000000 : 0))};
+#pragma unroll
+      for (int k = 0; k < HIT_WORDS; k++) ((volatile K_LDS float*)hq)[k * HIT_LEN + at + rank] = e[k];
+      if (rank == 0) wq[3] = at + n;
+      return;
     }
   }
+  tally_hit(P, energy, energyFirst, randno1, randno2, randno3, randno4, ibin, st.absvox, scattered, C, s_spec);
 }
 
 __device__ __forceinline__ void write_psf(DU_GLOBAL mcpet_psf_record* rec, unsigned long long t_ps, float travel_ps, int vox, float e,
@@ -1055,9 +1100,10 @@ __device__ __forceinline__ bool pair_selected(const KParams& P, int ss, int ssF)
 
 template <class CN, bool kLists = true>
 __device__ __forceinline__ void tally_pair(const KParams& P, const Photon& ph, const Pair& pr, Stream& st, CN& C, int* s_spec, char* stage = nullptr,
-                                           volatile K_LDS long long* wq = nullptr)
+                                           volatile K_LDS long long* wq = nullptr, HitQueue hq = nullptr)
 {
-  if (!kLists || P.mode == 0 || P.mode == 2) tally_sinogram(P, ph.E, pr.EF, ph.pos, pr.posF, ph.dir, pr.dirF, ph.ss, pr.ssF, st, C, s_spec);
+  if (!kLists || P.mode == 0 || P.mode == 2)
+    tally_sinogram(P, ph.E, pr.EF, ph.pos, pr.posF, ph.dir, pr.dirF, ph.ss, pr.ssF, st, C, s_spec, hq, wq);
   if (kLists && (P.mode == 0 || P.mode == 1))
     tally_psf(P, ph.E, pr.EF, ph.pos, pr.posF, ph.dir, pr.dirF, ph.ss, pr.ssF, ph.travel, pr.travelF, st, C, stage, wq);
 }
@@ -1390,8 +1436,8 @@ __device__ __attribute__((noinline)) long long claim_stream(unsigned long long* 
 
 template <class CN, bool kExt>
 __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& s_cmp, int* s_spec,
-                                         unsigned long long* s_mat, const LaneSlots& L, volatile K_LDS long long* wq, int wave = 0,
-                                         int first = 0)
+                                         unsigned long long* s_mat, const LaneSlots& L, volatile K_LDS long long* wq, HitQueue hq,
+                                         int wave = 0, int first = 0)
 {
   constexpr int kPhases = kExt ? LS_N : LS_CPZ + 1;
   if (__lane_id() == 0) {
@@ -1407,6 +1453,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
       wq[1] = first ? P.chunk0 : 0;
     }
     wq[2] = 0;
+    wq[3] = 0;
   }
   __builtin_amdgcn_wave_barrier();
   char* const stage = kExt ? stage_of(P) : nullptr;
@@ -1523,9 +1570,10 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
     if (run_tally && state == LS_TALLY) {
       Pair pr;
       pair_load<kExt>(L, pr);
-      tally_pair<CN, kExt>(P, ph, pr, st, C, s_spec, stage, wq);
+      tally_pair<CN, kExt>(P, ph, pr, st, C, s_spec, stage, wq, kExt ? nullptr : hq);
       state = prompt ? LS_SOURCE3 : LS_DECAY;
     }
+    if (!kExt && run_tally && __builtin_amdgcn_readfirstlane((int)wq[3]) >= HIT_FULL) hits_take(P, hq, wq, C, s_spec);
     const bool run_decay = best == LS_DECAY || ((MCPET_CHAIN & 16) && run_tally);
     if (run_decay && state == LS_DECAY) {
       for (;;) {
@@ -1619,6 +1667,7 @@ __device__ __forceinline__ void sm_waves(const KParams& P, CN& C, const Shells& 
     if (__lane_id() == 0) C.add(KC_PHASE_CYCLES + best, (unsigned)(clock64() - t_phase));
 #endif
   }
+  if (!kExt) hits_take(P, hq, wq, C, s_spec);   // the last ones
 }
 
 // Persistent kernel over one phantom.
@@ -1626,15 +1675,16 @@ template <class CN, bool kExt>
 // Parameters are read through a pointer to device memory: only the fields a phase uses are
 // loaded (as scalars), instead of a by-value block that would be kept in scalar registers
 // (and spilled) or copied to private memory.
-__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_sm(const KParams* __restrict__ Pd)
+__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_sm(const KParams* __restrict__ Pd)
 {
   const KParams& P = *Pd;
   K_PROLOGUE(CN)
   __shared__ float s_slots[kExt ? LANE_SLOTS_EXT : LANE_SLOTS][K_BLOCK];
-  __shared__ long long s_wq[K_BLOCK / 64][3];
+  __shared__ long long s_wq[K_BLOCK / 64][4];
+  __shared__ float s_hits[K_BLOCK / 64][kExt ? 1 : HIT_WORDS * HIT_LEN];
   const LaneSlots L{&s_slots[0][threadIdx.x]};
   const int waves = (int)(blockDim.x >> 6), wave = (int)(threadIdx.x >> 6);
-  sm_waves<CN, kExt>(P, C, s_cmp, s_spec, s_mat, L, (volatile K_LDS long long*)s_wq[wave], (int)blockIdx.x * waves + wave,
+  sm_waves<CN, kExt>(P, C, s_cmp, s_spec, s_mat, L, (volatile K_LDS long long*)s_wq[wave], (HitQueue)s_hits[wave], (int)blockIdx.x * waves + wave,
                      P.chunk0 ? (int)gridDim.x * waves : 0);
   K_EPILOGUE
 }
@@ -1651,7 +1701,7 @@ __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_sm(cons
 // memory. Per phantom, streams and random numbers are those of a single-phantom run, so each
 // phantom's tallies equal its own run's bit for bit.
 template <class CN, bool kExt>
-__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_batch(const KParams* __restrict__ Ps, int n, int n_spec)
+__global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY void k_transport_batch(const KParams* __restrict__ Ps, int n, int n_spec)
 {
   __shared__ unsigned s_shell_of[K_MAXMAT];
   extern __shared__ v4f s_dyn[];                          // the shells, n_spec spectrum bins
@@ -1659,7 +1709,8 @@ __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_batch(c
   __shared__ unsigned long long s_matw[K_BLOCK / 64][2 * K_MAXMAT];
   __shared__ unsigned s_cntw[K_BLOCK / 64][KC_N];
   __shared__ float s_slots[kExt ? LANE_SLOTS_EXT : LANE_SLOTS][K_BLOCK];
-  __shared__ long long s_wq[K_BLOCK / 64][3];
+  __shared__ long long s_wq[K_BLOCK / 64][4];
+  __shared__ float s_hits[K_BLOCK / 64][kExt ? 1 : HIT_WORDS * HIT_LEN];
   {
     for (int i = threadIdx.x; i < Ps[0].n_shells; i += blockDim.x) {
       const float4 v = gld(Ps[0].shells, i);
@@ -1681,7 +1732,7 @@ __global__ __launch_bounds__(K_BLOCK) K_OCCUPANCY(kExt) void k_transport_batch(c
     const KParams& P = Ps[k];
     CN C;
     C.init(s_cntw[wave]);
-    sm_waves<CN, kExt>(P, C, s_cmp, s_spec, s_matw[wave], L, (volatile K_LDS long long*)s_wq[wave]);
+    sm_waves<CN, kExt>(P, C, s_cmp, s_spec, s_matw[wave], L, (volatile K_LDS long long*)s_wq[wave], (HitQueue)s_hits[wave]);
     C.flush(P, s_cntw[wave]);
     __builtin_amdgcn_wave_barrier();
     if (lane < KC_N && s_cntw[wave][lane]) {

@@ -921,8 +921,8 @@ extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
   if (kind == MCPET_KERNEL_PERSISTENT) {
     const int resident = mcpet_transport_resident(P, p.count_events, bs);
     // Short runs end with lanes waiting for the last streams, the longer the more lanes share the
-    // device: about 16 decays a lane, from four workgroups per CU up (4e6 decays: 6 / 5 / 4
-    // workgroups 1.10 / 1.04 / 1.00 ms, 5e6: 1.67 / 1.62 / 1.66 ms; 2e7: 6 are best).
+    // device: about 16 decays a lane, from four workgroups per CU up (4e6 decays: 5 / 4 workgroups
+    // 1.04 / 1.00 ms, 5e6: 1.61 / 1.59 ms; from 2e7 on as many as fit are best).
     const double decays = c->expected_rate * effective_seconds(c->cfg.mean_life, P.acq_ps);
     const int wanted = (int)std::min((double)resident, std::ceil(decays / (16.0 * c->num_cus * bs)));
     const int per_cu = p.blocks_per_cu > 0 ? p.blocks_per_cu : std::min(resident, std::max(4, wanted));
