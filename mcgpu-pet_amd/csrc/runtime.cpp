@@ -855,10 +855,10 @@ static mcpet_status clear_buffers(mcpet_ctx* c, hipStream_t stream, bool tallies
 // How the waves of a launch claim streams from the queue: an eighth of their part of the rest at
 // a time (a wave knows the queue's position from its last claim, so half of it, 512 streams at
 // once, left the last waves too much: head, 1e8 decays, 27.7 -> 33.2 ms), down to chunks worth
-// about 64 decays, since a claim costs the device about 6 ns and one address serves them all:
-// 16-64 streams. own: the first claim is the wave's by its number, without an atomic (only if
-// every wave is resident from the start). 5e6 decays at 4 a stream: fixed chunks of 64, 1.79 ms,
-// now 1.62; 4e7 torso decays 36.4 -> 33.8 ms.
+// about 64 decays, since a claim costs the device about 6 ns and one address serves them all, and to
+// what a wave makes ready together: 16-128 streams. own: the first claim is the wave's by its number,
+// without an atomic (only if every wave is resident from the start). 5e6 decays at 4 a stream: 1.44 ms;
+// with chunks of half the size 1.67-2.1, eight phantoms 6.7 -> 7.9.
 static void set_claims(KParams& P, double expected_decays, long long n_waves, bool own)
 {
   P.n_claims = std::max(0LL, (P.n_streams - P.stream_base + P.stream_stride - 1) / std::max(1LL, P.stream_stride));
@@ -866,8 +866,9 @@ static void set_claims(KParams& P, double expected_decays, long long n_waves, bo
   while (shift < 40 && (1LL << shift) < 8 * n_waves) shift++;
   P.chunk_shift = shift;
   const double per_stream = expected_decays / (double)std::max(1LL, P.n_streams);
-  P.chunk_min = per_stream >= 4.0 ? 16 : per_stream >= 2.0 ? 32 : 64;
-  P.chunk0 = own ? (int)std::min(512LL, std::max(1LL, P.n_claims >> shift)) : 0;
+  P.chunk_min = per_stream >= 4.0 ? 16 : per_stream >= 2.0 ? 64 : 128;
+  // at least 96, so that a wave fills its lanes at the start from what is its own (4e6 decays 1.15 -> 1.08 ms)
+  P.chunk0 = own ? (int)std::min(512LL, std::max<long long>(P.n_claims >= 192 * n_waves ? 96 : 1, P.n_claims >> shift)) : 0;
 }
 
 extern "C" mcpet_status mcpet_run(mcpet_ctx* c, const mcpet_run_params* rp)
