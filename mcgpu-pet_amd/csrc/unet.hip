@@ -863,8 +863,9 @@ void launch_cols(const ConvK& a, int mt, hipStream_t st)
 // (two per CU), the smallest where none does.
 #define COLS_WGS 512
 // k_conv_planes takes a shape when its halo plane fits LDS beside a second workgroup's and its tiles
-// give PLANES_WGS workgroups: with fewer, k_conv_cols' smaller tiles end sooner.
-#define PLANES_WGS 256
+// give PLANES_WGS workgroups: with fewer, k_conv_cols' smaller tiles end as soon (one sample of 32 x 56 x 56,
+// whose half resolution has 224: 0.157 -> 0.144 ms; thresholds of 100 and 48 no better on smaller volumes).
+#define PLANES_WGS 200
 inline long long planes_tiles(const ConvK& a) { return (long long)((a.W + 15) / 16) * ((a.H + 3) / 4) * a.D; }
 inline size_t planes_lds(const ConvK& a, int mt) { return std::max<size_t>(16 * (size_t)(a.Cbp / 8) * FP_HP, 16 * 512 * (size_t)mt); }
 inline bool use_planes(const ConvK& a)
