@@ -18,7 +18,7 @@
 //     compacted, activity-sorted list of emitting voxels;
 //   - cross sections: total (a,b) pairs in an 8-byte table read in the Woodcock loop,
 //     Compton/Rayleigh (a,b) in a separate 16-byte table read only at real events;
-//   - Compton shell table (5460 B), the energy spectrum and the per-material dose
+//   - the Compton shells of the phantom's materials, the energy spectrum and the per-material dose
 //     are kept in LDS and flushed once per workgroup;
 //   - per-lane state touched by only some phases of the persistent kernel (the pair kept
 //     between the two photons, the Compton sampler between rejection trials) lives in
@@ -42,15 +42,9 @@
 #define K_LDS __attribute__((address_space(3)))
 // Upper bound on the iterations of each rejection loop (GRAa, GCOa). Valid tables accept
 // within a few trials; the bound only guarantees that no lane can loop forever on
-// corrupt input. The CPU checker applies the same bound.
+// corrupt input. The oracle applies the same bound.
 #define K_MAX_TRIALS (1 << 20)
 
-// Occupancy targets of the persistent transport kernels (waves per SIMD). They wait on dependent
-// gathers and on chains of dependent operations, so waves pay up to the last one that fits: 6 (80
-// VGPRs, one spilled; 26.4 KB of LDS per workgroup with the shells and the palette at the phantom's
-// own sizes) where only sinograms are tallied (head, 1e8 decays, at 4 / 5 / 6 waves: 31.6 / 29.0 /
-// 27.8 ms; eight phantoms in one launch 10.75 / 10.2 / 10.1 ms), 5 (96 VGPRs) with lists or
-// prompt gammas (4e7 torso decays with singles, 4 / 5 / 6 waves: 38.1 / 36.3 / 36.8 ms).
 // Woodcock steps a lane may take in one STEP phase while its steps stay virtual, and GCOa
 // rejection trials (tau loop, p_z loop) in one CTAU / CPZ phase: the phase selection's ballots
 // are paid once for several. 3 and 2 measured best on the head workload (1-4 steps, 1-3
@@ -69,8 +63,10 @@
 #ifndef MCPET_CHAIN
 #define MCPET_CHAIN 31
 #endif
-// Five waves per SIMD (96 registers, 32 KB of LDS a workgroup): head, 1e8 decays, 31.9 ms with four, 29.0
-// with five, 29.1 with six, whose 80 registers spill.
+// Occupancy target of the persistent transport kernels: five waves per SIMD (96 registers, none spilled, up to
+// 32 KB of LDS a workgroup). Waves hide the dependent gathers until the vector ALUs' issue bounds the
+// kernel: head, 1e8 decays, 31.9 ms with four, 29.0 with five, 29.1 with six, whose 80 registers spill; 4e7
+// torso decays with singles, 4 / 5 / 6 waves: 38.1 / 36.3 / 36.8 ms.
 #ifndef MCPET_WAVES_PER_EU
 #define MCPET_WAVES_PER_EU 5
 #endif
@@ -1274,9 +1270,9 @@ enum LaneState {
 
 // Per-lane state that only some phases touch lives in LDS slots instead of registers
 // (structure of arrays, slot k of lane i at [k][i]: consecutive lanes, consecutive banks):
-// the pair kept between the two photons (15 words) and the Compton sampler's state
-// between its rejection trials (14 words). Only the stream and the current photon stay
-// in registers across iterations.
+// the pair kept between the two photons and the Compton sampler's state between its rejection
+// trials (22 words in all). Only the stream, the current photon and a ready next stream stay in
+// registers across iterations.
 #define K_BLOCK 256
 // Slots whose contents are never needed together share a place: photon 1's direction waits for
 // photon 2's emission where the pair's first hit goes later, and moves to the Compton sampler's
