@@ -35,7 +35,7 @@ HIP_FLAGS = [
     "-I" + INC, "-I" + CSRC,
 ]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-I" + INC, "-I" + CSRC]
-# Oracle: portable x86-64-v3 (AVX2 + FMA) so it runs on the host of any GPU box.
+# Oracle: portable x86-64-v3 (AVX2 + FMA) so it runs on x86-64 hosts other than the build machine.
 ORACLE_FLAGS = ["-O3", "-std=gnu11", "-fPIC", "-shared", "-march=x86-64-v3", "-ffp-contract=off"]
 
 
