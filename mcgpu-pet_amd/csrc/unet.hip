@@ -1487,6 +1487,8 @@ struct mcpet_surrogate {
   float* h_stage = nullptr;   // pinned: a group's outputs or targets; the fused estimate's two outputs
   float* h_in = nullptr;      // pinned: the two halves of stage_input's buffer, stage_in floats
   size_t stage_in = 0;
+  int in_turn = 0;                      // the half that stage_input fills next
+  bool in_used[2] = {false, false};     // halves that kernels of the current call may still read (until ev_in)
   hipEvent_t ev_in[2] = {nullptr, nullptr}, ev_out = nullptr;
   unsigned long long* h_decays = nullptr;   // pinned: the estimated run's decays
   int fwd_timed = 0;   // samples between the two events
@@ -1681,20 +1683,19 @@ hipError_t concat(mcpet_surrogate* s, int ns, const Vol& v, const __bf16* u, int
 
 // n samples of the batch into s->x0 and their copy. A pageable copy of 100 KB takes 48 us, of 6.4 MB
 // 200; so the host fills the two halves of a pinned buffer in turn (whole samples where they fit, else
-// voxel ranges) and k_input reads them where they are.
+// voxel ranges) and k_input reads them where they are. A half that was filled before in this call, for
+// this group of samples or an earlier one, is filled again only after its k_input has ended.
 hipError_t stage_input(mcpet_surrogate* s, const float* x, int n)
 {
   const size_t C = s->cin, vox = s->vx.vox(), half = s->stage_in / 2;
   const size_t range = std::min(vox, half / C);
   const int per = range == vox ? (int)std::min<size_t>(n, half / (C * vox)) : 1;
-  int turn = 0;
-  bool used[2] = {false, false};
   for (int b = 0; b < n; b += per)
-    for (size_t v0 = 0; v0 < vox; v0 += range, turn ^= 1) {
-      const int m = std::min(per, n - b);
+    for (size_t v0 = 0; v0 < vox; v0 += range, s->in_turn ^= 1) {
+      const int m = std::min(per, n - b), turn = s->in_turn;
       const size_t r = std::min(range, vox - v0);
       float* h = s->h_in + turn * half;
-      hipError_t e = used[turn] ? hipEventSynchronize(s->ev_in[turn]) : hipSuccess;
+      hipError_t e = s->in_used[turn] ? hipEventSynchronize(s->ev_in[turn]) : hipSuccess;
       if (e != hipSuccess) return e;
       if (r == vox) std::memcpy(h, x + b * C * vox, sizeof(float) * m * C * vox);
       else
@@ -1705,7 +1706,7 @@ hipError_t stage_input(mcpet_surrogate* s, const float* x, int n)
       e = hipGetLastError();
       if (e == hipSuccess) e = hipEventRecord(s->ev_in[turn], s->st);
       if (e != hipSuccess) return e;
-      used[turn] = true;
+      s->in_used[turn] = true;
     }
   return hipSuccess;
 }
@@ -1979,12 +1980,18 @@ extern "C" mcpet_status mcpet_surrogate_set_params(mcpet_surrogate* s, const flo
   return MCPET_OK;
 }
 
-// The host's halves of the staging buffers are free whenever a call begins: every call that uses them
-// waits for its stream before it returns.
-// x: batch x cin x D x H x W, y (out): batch x D x H x W; returns the forward GFLOP per sample.
-extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float* x, int32_t batch, float* y, double* gflop)
+// The pinned buffers (h_in, h_stage) are free whenever a call begins: every call that uses them waits for
+// its stream before it returns, also where it returns an error (staged_end).
+static mcpet_status staged_end(mcpet_surrogate* s, mcpet_status st)
 {
-  if (!s || !x || !y || batch < 1) return serr(s, MCPET_E_ARG, "mcpet_surrogate_forward: bad arguments");
+  if (st != MCPET_OK) (void)hipStreamSynchronize(s->st);
+  s->in_turn = 0;
+  s->in_used[0] = s->in_used[1] = false;
+  return st;
+}
+
+static mcpet_status batch_forward(mcpet_surrogate* s, const float* x, int32_t batch, float* y, double* gflop)
+{
   const size_t nx = s->vx.size(), nv = s->vr.size();
   const int group = sample_group(s, batch);
   SHIP(s, stage_input(s, x, std::min(group, batch)));
@@ -2006,6 +2013,13 @@ extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float*
   s->fwd_timed = batch - (batch - 1) / group * group;
   if (gflop) *gflop = s->flops_fwd * 1e-9;
   return MCPET_OK;
+}
+
+// x: batch x cin x D x H x W, y (out): batch x D x H x W; returns the forward GFLOP per sample.
+extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float* x, int32_t batch, float* y, double* gflop)
+{
+  if (!s || !x || !y || batch < 1) return serr(s, MCPET_E_ARG, "mcpet_surrogate_forward: bad arguments");
+  return staged_end(s, batch_forward(s, x, batch, y, gflop));
 }
 
 // Device time per sample of the network in the last mcpet_surrogate_forward (its last samples that
@@ -2033,10 +2047,8 @@ void mcpet_surrogate_dims(const mcpet_surrogate* s, int* D, int* H, int* W, int*
   *cin = s->cin;
 }
 
-extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* ctx, float* estimate, float* scatter_counts,
-                                                 int64_t* decays)
+static mcpet_status run_estimate(mcpet_surrogate* s, mcpet_ctx* ctx, float* estimate, float* scatter_counts, int64_t* decays)
 {
-  if (!s || !ctx || !estimate) return serr(s, MCPET_E_ARG, "mcpet_surrogate_estimate: null argument");
   if (s->cin != 2 && s->cin != 4)
     return serr(s, MCPET_E_ARG, "mcpet_surrogate_estimate: the network must take 2 or 4 input channels");
   if (mcpet_ctx_device(ctx) != s->device) return serr(s, MCPET_E_ARG, "mcpet_surrogate_estimate: context on another device");
@@ -2072,6 +2084,13 @@ extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* 
   return MCPET_OK;
 }
 
+extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* ctx, float* estimate, float* scatter_counts,
+                                                 int64_t* decays)
+{
+  if (!s || !ctx || !estimate) return serr(s, MCPET_E_ARG, "mcpet_surrogate_estimate: null argument");
+  return staged_end(s, run_estimate(s, ctx, estimate, scatter_counts, decays));
+}
+
 // Mean-squared-error gradients of the batch (loss = mean over batch and voxels); leaves them
 // in the device buffer for an optimiser step.
 static mcpet_status batch_gradients(mcpet_surrogate* s, const float* x, const float* target, int32_t batch, float* loss)
@@ -2105,7 +2124,7 @@ extern "C" mcpet_status mcpet_surrogate_gradients(mcpet_surrogate* s, const floa
                                                   float* loss, float* grad)
 {
   if (!s || !x || !target || batch < 1) return serr(s, MCPET_E_ARG, "mcpet_surrogate_gradients: bad arguments");
-  mcpet_status st = batch_gradients(s, x, target, batch, loss);
+  mcpet_status st = staged_end(s, batch_gradients(s, x, target, batch, loss));
   if (st != MCPET_OK || !grad) return st;
   SHIP(s, hipMemcpy(grad, s->g, sizeof(float) * s->n_params, hipMemcpyDeviceToHost));
   return MCPET_OK;
@@ -2116,7 +2135,7 @@ extern "C" mcpet_status mcpet_surrogate_train_step(mcpet_surrogate* s, const flo
                                                    float lr, float* loss)
 {
   if (!s || !x || !target || batch < 1 || !(lr > 0.0f)) return serr(s, MCPET_E_ARG, "mcpet_surrogate_train_step: bad arguments");
-  mcpet_status st = batch_gradients(s, x, target, batch, loss);
+  mcpet_status st = staged_end(s, batch_gradients(s, x, target, batch, loss));
   if (st != MCPET_OK) return st;
   s->t_adam++;
   const float c1 = 1.0f - std::pow(0.9f, (float)s->t_adam), c2 = 1.0f - std::pow(0.999f, (float)s->t_adam);

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import mcpet
+from harness import head_scenario
 from test_surrogate import _layer_rel, integer_network, unet_reference
 
 
@@ -37,6 +38,26 @@ def test_batch_equals_its_samples(grid, cin, c, batch):
     size = np.mean([np.linalg.norm(g.astype(np.float64)) for _, g in each])
     assert np.linalg.norm(grad - mean) <= 2.0 ** -8 * size
     assert abs(loss - np.mean([l for l, _ in each])) <= 1e-5 * abs(loss)
+
+
+# three groups, staged in one piece each; in five, five and four pieces of one sample each; in three pieces of
+# a sample's voxels each
+@pytest.mark.gpu
+@pytest.mark.parametrize("grid,cin,c,batch", [((4, 4, 4), 1, 3, 150), ((32, 56, 56), 4, 8, 14), ((32, 68, 132), 4, 4, 5)])
+def test_groups_behind_a_transport_run_keep_their_samples(grid, cin, c, batch):
+    """While a run (some 50 ms) holds the device, the kernels that read a group's input wait behind it, and the
+    host must not fill the staging with the next group's until they have."""
+    rng = np.random.default_rng(batch)
+    net = _network(grid, cin, c, rng)
+    x = rng.random((batch, cin) + grid).astype(np.float32)
+    alone = np.concatenate([net.forward(x[i:i + 1]) for i in range(batch)])
+    sc = head_scenario(n_decays=1e8)
+    with mcpet.Simulation(sc.cfg, sc.phantom, sc.tables) as sim:
+        for _ in range(2):
+            sim.run()
+            together = net.forward(x)
+            sim.sync()
+            assert np.array_equal(together, alone)
 
 
 # 20 x 44 x 68 takes the tiles of 16 x 8 x 2 (1100 four-row tiles) with a remainder in x and y, its
