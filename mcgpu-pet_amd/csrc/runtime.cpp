@@ -1808,7 +1808,7 @@ struct mcpet_batch {
   int tuned_bs = 0, tuned_per_cu = 0, tuned_policy = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
-  int graph_key[3] = {-1, -1, -1};  // block size, blocks, count_events of the captured launch
+  int graph_key[4] = {-1, -1, -1, -1};  // block size, blocks, count_events of the captured launch; whether it clears the tallies
   bool ran = false;
   std::string err;
 };
@@ -1923,8 +1923,8 @@ static mcpet_status batch_run(mcpet_batch* b, const mcpet_run_params* rp, double
   }
   BHIP(b, hipMemcpyAsync(b->d_params, b->h_params, sizeof(KParams) * (size_t)n, hipMemcpyHostToDevice, b->stream));
   if (p.use_graph) {
-    const int key[3] = {bs, blocks, p.count_events ? 1 : 0};
-    if (!b->gexec || std::memcmp(key, b->graph_key, sizeof key) != 0 || !p.zero_tallies) {
+    const int key[4] = {bs, blocks, p.count_events ? 1 : 0, p.zero_tallies ? 1 : 0};
+    if (!b->gexec || std::memcmp(key, b->graph_key, sizeof key) != 0) {
       if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
       if (b->graph) (void)hipGraphDestroy(b->graph);
       b->gexec = nullptr;

@@ -73,6 +73,24 @@ def test_batch_graph_replays_match_eager_runs():
 
 
 @pytest.mark.gpu
+def test_batch_graph_replays_clear_the_tallies_only_where_asked():
+    """Graph runs that keep and that clear the tallies, in every order: each equal to the eager run."""
+    cfg, phs, tab = _batch_inputs(count=2, seed=8)
+    clears = (True, False, False, True, True, False, True)   # zero_tallies of the runs in turn
+    with mcpet.Batch(cfg, phs, tab) as b:
+        got = []
+        for graph in (False, True):
+            got.append([])
+            for i, zero in enumerate(clears):
+                b.run(seed=900 + i, zero_tallies=zero, use_graph=graph)
+                b.sync()
+                got[-1].append([b.fetch(k, psf=False) for k in range(len(phs))])
+    for eager, replay in zip(*got):
+        for k in range(len(phs)):
+            _same(replay[k], eager[k])
+
+
+@pytest.mark.gpu
 def test_batch_autotune_keeps_results():
     cfg, phs, tab = _batch_inputs(count=4, seed=7)
     with mcpet.Batch(cfg, phs, tab) as b:
