@@ -176,10 +176,13 @@ mcpet_status dalloc_planned(mcpet_ctx* c)
   c->plan.shrink_to_fit();
   return MCPET_OK;
 }
-// frees what dalloc gave on its own; what is part of the context's block goes with the block
-void dfree(mcpet_ctx* c, void* p)
+// frees what dalloc gave on its own (true); what is part of the context's block stays held until the
+// block goes
+bool dfree(mcpet_ctx* c, void* p)
 {
-  if (p && !(c->slab && (char*)p >= c->slab && (char*)p < c->slab + c->slab_bytes)) (void)hipFree(p);
+  if (!p || (c->slab && (char*)p >= c->slab && (char*)p < c->slab + c->slab_bytes)) return false;
+  (void)hipFree(p);
+  return true;
 }
 
 // Idle streams with the pinned staging of a run's parameters, per device: creating and destroying
@@ -1034,8 +1037,7 @@ static mcpet_status apply_stream_layout(mcpet_ctx* c, long long stream_decays)
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (hint.size() > c->hint_cap) {   // at most n + 2 entries: allocated once at that size
     if (c->d_stream_hint) {
-      dfree(c, c->d_stream_hint);
-      c->dev_bytes -= c->hint_cap * sizeof(int);
+      if (dfree(c, c->d_stream_hint)) c->dev_bytes -= c->hint_cap * sizeof(int);
       c->d_stream_hint = nullptr;
       c->hint_cap = 0;
     }

@@ -79,3 +79,24 @@ def test_tuned_decays_per_stream_reproduce_a_context_created_with_them():
         other = sim.fetch(psf=False)
     a, b = int(tuned["trues"].sum()), int(other["trues"].sum())
     assert abs(a - b) < 6 * np.sqrt(a + b) + 10
+
+
+@pytest.mark.gpu
+def test_a_larger_lookup_of_the_tuned_layout_adds_to_the_device_bytes():
+    """Three streams a voxel at creation (look-up of 0.75 n + 2 entries, part of the context's one block), one
+    a voxel while tuning (n + 1 entries, a buffer of n + 2 of its own): the block's part stays held."""
+    n = 8 * 8 * 8
+    shape = (8, 8, 8)
+    sc = water_cube_scenario(n_decays=1e4)
+    cfg = sc.cfg
+    activity, per_voxel = 100.0, 100.0 * cfg.mean_life * (1.0 - np.exp(-cfg.acquisition_time_ps * 1e-12 / cfg.mean_life))
+    cfg.stream_decays = int(per_voxel / 2.5)
+    assert np.ceil(per_voxel / cfg.stream_decays) == 3
+    ph = mcpet.phantom_from_arrays(np.full(shape, 2, np.int32), np.ones(shape, np.float32),
+                                   np.full(shape, activity, np.float32), (0.5, 0.5, 0.5))
+    held = getattr(mcpet.lib(), "_Z22mcpet_ctx_device_bytesPK9mcpet_ctx")
+    held.argtypes, held.restype = [C.c_void_p], C.c_size_t
+    with mcpet.Simulation(cfg, ph, sc.tables) as sim:
+        before = held(sim.ctx)
+        sim.autotune(fraction=0.5, layout=False, stream_decays=[int(2 * per_voxel)])
+        assert held(sim.ctx) == before + 4 * (n + 2)
