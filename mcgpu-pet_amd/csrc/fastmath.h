@@ -22,13 +22,16 @@ static __device__ __forceinline__ double sconst(double c)
   return c;
 }
 
-// floor(x) as an integer, |x| < 2^31 (one instruction; saturating, NaN gives 0).
+// floor(x) as an integer (one instruction; saturating). x is not NaN: that gives 0.
 static __device__ __forceinline__ int floor_i32(float x)
 {
   int r;
   asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
   return r;
 }
+
+// The same with INT_MIN for NaN (f2i_rd's results), so that an undefined value stays out of a table.
+static __device__ __forceinline__ int floor_i32_nan(float x) { return x == x ? floor_i32(x) : INT32_MIN; }
 
 // sqrt(x), x normal and above 2^-100, or zero of either sign: one Newton step on the reciprocal
 // root and two on the root with exact residuals (the sequence of the compiler's own expansion of

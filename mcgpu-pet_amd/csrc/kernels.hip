@@ -597,8 +597,8 @@ __device__ __forceinline__ void tally_hit(const KParams& P, float energy, float 
   float g2 = sqrt_nz(-2.0f * log_n(randno3 + 1.0e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno4));
   float Energia1 = energy + ((P.e_resol) / 2.35f) * energy * g1;
   float Energia2 = energyFirst + ((P.e_resol) / 2.35f) * energyFirst * g2;
-  int iE1 = floor_i32(div_r(Energia1, 1000.0f, 1.0f / 1000.0f));
-  int iE2 = floor_i32(div_r(Energia2, 1000.0f, 1.0f / 1000.0f));
+  int iE1 = floor_i32_nan(div_r(Energia1, 1000.0f, 1.0f / 1000.0f));   // (no bin for an undefined energy)
+  int iE2 = floor_i32_nan(div_r(Energia2, 1000.0f, 1.0f / 1000.0f));
   if ((iE1 < P.ne) && (iE1 >= 0)) spectrum_add(P, s_spec, iE1);
   if ((iE2 < P.ne) && (iE2 >= 0)) spectrum_add(P, s_spec, iE2);
   C.inc(KC_PAIRS);
@@ -779,7 +779,7 @@ __device__ __forceinline__ void record_single(const KParams& P, const float* pos
   const float randno2 = rn(st.r, C);
   const float g = sqrt_nz(-2.0f * log_n(randno1 + 1e-8f)) * cos_n((float)(2.0f * K_PI * (double)randno2));
   const float e = energy + ((P.e_resol) * (1.0f / 2.35f)) * energy * g;
-  const int iE = floor_i32(div_r(e, 1000.0f, 1.0f / 1000.0f));
+  const int iE = floor_i32_nan(div_r(e, 1000.0f, 1.0f / 1000.0f));
   if ((iE < P.ne) && (iE >= 0)) spectrum_add(P, s_spec, iE);
   if (!(e > P.e_low && e < P.e_high)) return;
   const float phi = mcf_atan2f(y0 + dist * dir[1], x0 + dist * dir[0]);
@@ -940,7 +940,7 @@ __device__ __forceinline__ bool compton_end(const KParams& P, Photon& ph, Rng& r
   const double costh_Compton = gcoa_finish(&ph.E, cs);
   rotate_double(ph.dir, costh_Compton, 6.28318530717958647693 * rnd(r, C));
   const float randno = ph.E - e_before;
-  ph.index = floor_i32((ph.E - P.e0) * P.ide);
+  ph.index = floor_i32_nan((ph.E - P.e0) * P.ide);   // an undefined energy lies below the tables: absorbed
   if (ph.index > -1) {
     const float2 w = gld32(P.woodcock, ph.index);
     ph.mfpW = w.x + ph.E * w.y;
