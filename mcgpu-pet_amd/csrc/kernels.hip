@@ -464,13 +464,15 @@ __device__ __forceinline__ bool gcoa_pz_trial(float E, int mat, Rng& r, CN& C, c
   temp = rn(r, C) * gcoa_rnv(E, table, cs, ishell);
   const float fj = table[ishell].z;
   // both halves of the profile through one logarithm and root; its argument is below 1, and zero
-  // (pzomc = -infinity) or subnormal only where the profile term underflows (lower half)
+  // (an infinite root) or subnormal only where the profile term underflows (lower half)
   const bool low = temp < 0.5f;
   const float y = low ? temp + temp : 2.0f - 2.0f * temp;
-  const float root = sqrt_nz(0.5f - (y < 0x1p-126f ? mcf_logf(y) : log_n(y)));
+  float root = sqrt_nz(0.5f - (y >= 0x1p-126f ? log_n(y) : mcf_logf(y)));
+  if (y == 0.0f) root = MCF_INFF;
   const float dev = root - 0.70710678118654502f;
-  float pzomc = div_n(low ? -dev : dev, fj * 1.4142135623731f);
-  if (y == 0.0f) pzomc = -MCF_INFF;
+  const float num = low ? -dev : dev, den = fj * 1.4142135623731f;
+  // a profile of zero width (the quotient is infinite) or nearly so takes the general division
+  const float pzomc = fabsf(den) >= 0x1p-80f && y != 0.0f ? div_n(num, den) : num / den;
   cs.pzomc = pzomc;
   if (!(pzomc < -1.0f)) {
     float af;

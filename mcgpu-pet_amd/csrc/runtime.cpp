@@ -591,7 +591,10 @@ extern "C" mcpet_status mcpet_create(const mcpet_config* cfg, const mcpet_phanto
     std::vector<float4> sh((size_t)n);
     for (int i = 0; i < n; i++) {
       const int k = m + i * MCPET_MAX_MATERIALS;
-      sh[(size_t)i] = make_float4(ct.uico[k], ct.fco[k], ct.fj0[k], ct.uico[k] * 510998.918f);
+      // J0 (in atomic units of 1 to 100) within 2^80: beyond, every profile is a step and the products of J0
+      // would overflow; the limit gives the same samples
+      const float j0 = std::min(std::max(ct.fj0[k], -0x1p80f), 0x1p80f);
+      sh[(size_t)i] = make_float4(ct.uico[k], ct.fco[k], j0, ct.uico[k] * 510998.918f);
     }
     size_t first = hsh.size();
     for (int m2 = 0; m2 < m && n > 0; m2++)

@@ -47,3 +47,14 @@ def test_undefined_energies_follow_the_oracle(tmp_path, kernel, j0, e_resol):
     o = sc.run_oracle()
     assert o["counters"]["compton"] > 1000 and o["spectrum"].sum() == (0 if np.isnan(e_resol) else 2 * o["counters"]["pairs_tallied"])
     assert_tallies_equal(sc.run_gpu(kernel=kernel), o)
+
+
+# a profile of no, hardly any, negative and (beyond what a product in binary32 holds) unbounded width
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("shell,j0", [(0, "0"), (2, "0"), (1, "-0.0"), (0, "1e-40"), (0, "3e-25"), (1, "-20.0"), (0, "1e30"), (1, "inf")])
+def test_momentum_profiles_of_any_width_follow_the_oracle(tmp_path, kernel, shell, j0):
+    sc = _scenario(_water_file(tmp_path, "[NUMBER OF SHELLS", _profile(shell, j0)))
+    o = sc.run_oracle()
+    assert o["counters"]["compton"] > 1000
+    assert_tallies_equal(sc.run_gpu(kernel=kernel), o)
