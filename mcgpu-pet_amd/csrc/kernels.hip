@@ -235,8 +235,10 @@ __device__ __forceinline__ void rotate_double(float* d, double costh, double phi
     DXY = (double)(d[0] * d[0] + d[1] * d[1]);
   }
   if (DXY > 1.0e-28) {
-    const double sin2 = 1.0 - costh * costh;   // zero or above 2^-53; DXY lies in (1e-28, 1]
-    SDT = sin2 > 0.0 ? sqrt_n(div_n(sin2, DXY)) : 0.0;
+    // zero or above 2^-53 (negative, and the direction undefined, only where a table gives |costh| > 1);
+    // DXY lies in (1e-28, 1]
+    const double sin2 = 1.0 - costh * costh;
+    SDT = sin2 != 0.0 ? sqrt_n(div_n(sin2, DXY)) : 0.0;
     float xin = d[0];
     float yz = d[1] * d[2];
     float xz = xin * d[2];

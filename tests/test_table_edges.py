@@ -58,3 +58,14 @@ def test_momentum_profiles_of_any_width_follow_the_oracle(tmp_path, kernel, shel
     o = sc.run_oracle()
     assert o["counters"]["compton"] > 1000
     assert_tallies_equal(sc.run_gpu(kernel=kernel), o)
+
+
+# negative squared momentum transfers: Rayleigh cosines above 1, whose direction is undefined (the photon leaves)
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_rayleigh_cosines_above_one_follow_the_oracle(tmp_path, kernel):
+    sc = _scenario(_water_file(tmp_path, "[DATA VALUES TO SAMPLE SQUARED",
+                               lambda i, f: [f"{-1.0 + 0.01 * i:.3f}"] + f[1:] if i < 64 else f))
+    o = sc.run_oracle()
+    assert o["counters"]["rayleigh"] > 100
+    assert_tallies_equal(sc.run_gpu(kernel=kernel), o)
