@@ -524,7 +524,8 @@ mcpet_status mcpet_batch_project_maps(mcpet_batch* b, int32_t k, int32_t D, int3
  * accumulation; parameters, activations and optimiser state are FP32. Parameter layout: per
  * layer W[Cout][Cin][k^3] then b[Cout], layers in the order above. Created with He-normal
  * weights from `seed`, zero biases and a zero output layer (the identity on channel 0). Holds the
- * tensors of a group of samples (about 2^19 voxels, at most 1 GiB or one sample) and pinned staging. */
+ * tensors of a group of samples (about 2^19 voxels, at most 1 GiB or one sample; what only the gradients
+ * need, four fifths of it, for one sample until the first gradients of more) and pinned staging. */
 mcpet_status mcpet_surrogate_create(int32_t D, int32_t H, int32_t W, int32_t in_channels, int32_t width, uint64_t seed,
                                     mcpet_surrogate** out);
 int64_t mcpet_surrogate_param_count(const mcpet_surrogate* s);

@@ -1477,7 +1477,9 @@ struct mcpet_surrogate {
   __bf16 *grl = nullptr, *ge1l = nullptr, *ge2l = nullptr, *gb3l = nullptr, *gd2l = nullptr, *gb2l = nullptr, *gd1l = nullptr,
          *gb1l = nullptr, *ga1l = nullptr;
   float *raw_s = nullptr, *raw_t = nullptr, *est = nullptr;   // the fused estimate's buffers
-  int slots = 0;                                                // samples that the tensors above have room for
+  int slots = 0, grad_slots = 0;   // samples that the tensors above have room for: the forward's, the gradients'
+  bool grad_full = false;          // more gradients did not fit
+  void *held = nullptr, *grad_held = nullptr;
   double* sums = nullptr;                                       // 256 partial totals + the total
   float* bw_part = nullptr;                                     // slab sums of the tiled weight gradient
   long long t_adam = 0;
@@ -1779,60 +1781,47 @@ hipError_t backward(mcpet_surrogate* s, int ns)
   return e;
 }
 
-// The tensors held per sample.
+// The tensors held per sample: the forward's (the weight gradients' operands and the ReLU masks too), and
+// what only the gradients need.
 struct Slot {
   void** p;
   size_t bytes;   // of one sample
   bool zero;
 };
 
-std::vector<Slot> sample_tensors(mcpet_surrogate* s)
+std::vector<Slot> sample_tensors(mcpet_surrogate* s, bool gradients)
 {
   const int c = s->c, ci = s->cin;
   const size_t v0 = s->vx.vox(), v1 = s->vd1.vox(), v2 = s->vd2.vox();
   std::vector<Slot> t;
   auto f = [&](float** p, const Vol& v) { t.push_back({(void**)p, sizeof(float) * v.size(), false}); };
   auto h = [&](__bf16** p, size_t vox, int ch) { t.push_back({(void**)p, sizeof(__bf16) * vox * rup(ch, 8), true}); };
-  const bool cat = 2 * c % 8 != 0;   // the concatenations are written (concat)
-  f(&s->x0, s->vx), f(&s->out, s->vr);
-  f(&s->ga1, s->va1), f(&s->gcat1, s->vcat1), f(&s->gd1, s->vd1), f(&s->gcat2, s->vcat2);
-  f(&s->gd2, s->vd2), f(&s->gb3, s->vb3), f(&s->ge2, s->ve2), f(&s->ge1, s->ve1), f(&s->gr, s->vr);
-  h(&s->x0l, v0, ci), h(&s->a1l, v0, c), h(&s->b1l, v0, c), h(&s->cat1l, cat ? v0 : 0, 3 * c);
-  h(&s->d1l, v1, 2 * c), h(&s->b2l, v1, 2 * c), h(&s->cat2l, cat ? v1 : 0, 6 * c), h(&s->d2l, v2, 4 * c);
-  h(&s->e1l, v0, c), h(&s->e2l, v1, 2 * c), h(&s->b3l, v2, 4 * c);
-  h(&s->grl, v0, 8), h(&s->ge1l, v0, c), h(&s->ge2l, v1, 2 * c), h(&s->gb3l, v2, 4 * c);
-  h(&s->gd2l, v2, 4 * c), h(&s->gb2l, v1, 2 * c), h(&s->gd1l, v1, 2 * c), h(&s->gb1l, v0, c), h(&s->ga1l, v0, c);
+  if (!gradients) {
+    const bool cat = 2 * c % 8 != 0;   // the concatenations are written (concat)
+    f(&s->x0, s->vx), f(&s->out, s->vr);
+    h(&s->x0l, v0, ci), h(&s->a1l, v0, c), h(&s->b1l, v0, c), h(&s->cat1l, cat ? v0 : 0, 3 * c);
+    h(&s->d1l, v1, 2 * c), h(&s->b2l, v1, 2 * c), h(&s->cat2l, cat ? v1 : 0, 6 * c), h(&s->d2l, v2, 4 * c);
+    h(&s->e1l, v0, c), h(&s->e2l, v1, 2 * c), h(&s->b3l, v2, 4 * c);
+  } else {
+    f(&s->ga1, s->va1), f(&s->gcat1, s->vcat1), f(&s->gd1, s->vd1), f(&s->gcat2, s->vcat2);
+    f(&s->gd2, s->vd2), f(&s->gb3, s->vb3), f(&s->ge2, s->ve2), f(&s->ge1, s->ve1), f(&s->gr, s->vr);
+    h(&s->grl, v0, 8), h(&s->ge1l, v0, c), h(&s->ge2l, v1, 2 * c), h(&s->gb3l, v2, 4 * c);
+    h(&s->gd2l, v2, 4 * c), h(&s->gb2l, v1, 2 * c), h(&s->gd1l, v1, 2 * c), h(&s->gb1l, v0, c), h(&s->ga1l, v0, c);
+  }
   return t;
 }
 
-// Samples that go through the network together: one launch per layer serves them all, so the
-// coarse levels and the short launches fill the device. About 2^19 voxels are enough, and at most
-// 1 GiB is held for them. Four samples of 32 x 56 x 56 on width 32: 1.09 ms of device time one by
-// one, 0.56 together; eight of 16 x 28 x 28 on width 16: 0.77 and 0.11.
-hipError_t hold_samples(mcpet_surrogate* s)
+// Room for n samples of the tensors t in one allocation, the BF16 copies first: zeroed, their padding
+// channels stay zero. The tensors' pointers change only where it succeeds.
+hipError_t hold(mcpet_surrogate* s, const std::vector<Slot>& t, int n, void** block)
 {
-  const std::vector<Slot> t = sample_tensors(s);
-  size_t per = 0;
-  for (const Slot& b : t) per += b.bytes;
-  const size_t by_vox = (((size_t)1 << 19) + s->vr.vox() - 1) / s->vr.vox(), by_mem = ((size_t)1 << 30) / per;
-  s->slots = (int)std::max<size_t>(1, std::min(std::min<size_t>(by_vox, 64), by_mem));
-  // one allocation, the BF16 copies first: zeroed, their padding channels stay zero
-  auto room = [s](const Slot& b) { return (b.bytes * s->slots + 255) / 256 * 256; };
+  auto room = [n](const Slot& b) { return (b.bytes * n + 255) / 256 * 256; };
   size_t zeroed = 0, plain = 0;
-  auto total = [&]() {
-    zeroed = plain = 0;
-    for (const Slot& b : t) (b.zero ? zeroed : plain) += room(b);
-    return zeroed + plain;
-  };
+  for (const Slot& b : t) (b.zero ? zeroed : plain) += room(b);
   char* q = nullptr;
-  hipError_t e = hipMalloc((void**)&q, total());
-  if (e != hipSuccess && s->slots > 1) {
-    (void)hipGetLastError();
-    s->slots = 1;
-    e = hipMalloc((void**)&q, total());
-  }
+  const hipError_t e = hipMalloc((void**)&q, zeroed + plain);
   if (e != hipSuccess) return e;
-  s->allocs.push_back(q);
+  *block = q;
   char *z = q, *p = q + zeroed;
   for (const Slot& b : t) {
     char*& at = b.zero ? z : p;
@@ -1842,10 +1831,50 @@ hipError_t hold_samples(mcpet_surrogate* s)
   return hipMemsetAsync(q, 0, zeroed, s->st);
 }
 
-// samples per pass of a batch: equal groups of at most s->slots
-int sample_group(const mcpet_surrogate* s, int batch)
+// Samples that go through the network together: one launch per layer serves them all, so the
+// coarse levels and the short launches fill the device. About 2^19 voxels are enough, and at most
+// 1 GiB is held for them, the gradients' part of it (four fifths; one sample's until then) from the first
+// gradients of more than one sample. Four samples of 32 x 56 x 56 on width 32: 1.09 ms of device time one by
+// one, 0.56 together; eight of 16 x 28 x 28 on width 16: 0.77 and 0.11.
+hipError_t hold_samples(mcpet_surrogate* s)
 {
-  const int groups = (batch + s->slots - 1) / s->slots;
+  const std::vector<Slot> t = sample_tensors(s, false), g = sample_tensors(s, true);
+  size_t per = 0;
+  for (const auto* v : {&t, &g})
+    for (const Slot& b : *v) per += b.bytes;
+  const size_t by_vox = (((size_t)1 << 19) + s->vr.vox() - 1) / s->vr.vox(), by_mem = ((size_t)1 << 30) / per;
+  s->slots = (int)std::max<size_t>(1, std::min(std::min<size_t>(by_vox, 64), by_mem));
+  hipError_t e = hold(s, t, s->slots, &s->held);
+  if (e != hipSuccess && s->slots > 1) {
+    (void)hipGetLastError();
+    s->slots = 1;
+    e = hold(s, t, 1, &s->held);
+  }
+  s->grad_slots = 1;
+  return e == hipSuccess ? hold(s, g, 1, &s->grad_held) : e;
+}
+
+// The gradients' tensors for as many samples as the forward's, at the first batch that has more than one;
+// one sample at a time stays possible where the device has no room. No kernel of the network is running.
+hipError_t hold_gradients(mcpet_surrogate* s, int batch)
+{
+  if (batch <= s->grad_slots || s->grad_slots == s->slots || s->grad_full) return hipSuccess;
+  void* const one = s->grad_held;
+  const hipError_t e = hold(s, sample_tensors(s, true), s->slots, &s->grad_held);
+  if (s->grad_held == one) {   // no room
+    (void)hipGetLastError();
+    s->grad_full = true;
+    return hipSuccess;
+  }
+  s->grad_slots = s->slots;
+  const hipError_t f = hipFree(one);
+  return e == hipSuccess ? f : e;
+}
+
+// samples per pass of a batch: equal groups of at most `slots`
+int sample_group(int slots, int batch)
+{
+  const int groups = (batch + slots - 1) / slots;
   return (batch + groups - 1) / groups;
 }
 
@@ -1993,7 +2022,7 @@ static mcpet_status staged_end(mcpet_surrogate* s, mcpet_status st)
 static mcpet_status batch_forward(mcpet_surrogate* s, const float* x, int32_t batch, float* y, double* gflop)
 {
   const size_t nx = s->vx.size(), nv = s->vr.size();
-  const int group = sample_group(s, batch);
+  const int group = sample_group(s->slots, batch);
   SHIP(s, stage_input(s, x, std::min(group, batch)));
   for (int b = 0; b < batch; b += group) {
     const int n = std::min(group, batch - b), next = std::min(group, batch - b - n);
@@ -2096,11 +2125,12 @@ extern "C" mcpet_status mcpet_surrogate_estimate(mcpet_surrogate* s, mcpet_ctx* 
 static mcpet_status batch_gradients(mcpet_surrogate* s, const float* x, const float* target, int32_t batch, float* loss)
 {
   const size_t nx = s->vx.size(), nv = s->vr.size();
+  SHIP(s, hold_gradients(s, batch));
   hipLaunchKernelGGL(k_zero, dim3(blocks_for(s->n_params)), dim3(256), 0, s->st, s->g, s->n_params);
   hipLaunchKernelGGL(k_zero, dim3(1), dim3(256), 0, s->st, s->sse, (size_t)1);
   SHIP(s, hipGetLastError());
   const float scale = 1.0f / ((float)nv * (float)batch);
-  const int group = sample_group(s, batch);
+  const int group = sample_group(s->grad_slots, batch);
   for (int b = 0; b < batch; b += group) {
     const int n = std::min(group, batch - b);
     if (b) SHIP(s, hipEventSynchronize(s->ev_out));   // the last group's targets have been read
@@ -2152,6 +2182,8 @@ extern "C" void mcpet_surrogate_destroy(mcpet_surrogate* s)
   if (!s) return;
   if (s->st) (void)hipStreamSynchronize(s->st);
   for (void* p : s->allocs) (void)hipFree(p);
+  for (void* p : {s->held, s->grad_held})
+    if (p) (void)hipFree(p);
   if (s->h_stage) (void)hipHostFree(s->h_stage);
   if (s->h_in) (void)hipHostFree(s->h_in);
   for (hipEvent_t ev : {s->ev_in[0], s->ev_in[1], s->ev_out})

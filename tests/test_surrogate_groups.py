@@ -1,5 +1,7 @@
 """Samples of a batch go through the network together, in equal groups: every sample's output has
 the same bits as alone, and the gradients are the mean of the samples' own ones."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -58,6 +60,30 @@ def test_groups_behind_a_transport_run_keep_their_samples(grid, cin, c, batch):
             together = net.forward(x)
             sim.sync()
             assert np.array_equal(together, alone)
+
+
+@pytest.mark.gpu
+def test_gradient_tensors_of_a_group_wait_for_its_first_gradients():
+    """Width 32 on 32 x 56 x 56 in groups of six: the forward's tensors are 285 bytes a voxel and sample, the
+    gradients' 1084; beside them the weight gradients' partial sums (57 MB), parameters and optimiser state (27 MB)."""
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert mcpet.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    grid, vox = (32, 56, 56), 32 * 56 * 56
+    x = np.random.default_rng(2).random((6, 4) + grid).astype(np.float32)
+    warm = mcpet.Surrogate(grid, in_channels=4, width=32, seed=1)   # the kernels' code and scratch
+    warm.gradients(x, x[:, 0])
+    free = [free_bytes()]
+    net = mcpet.Surrogate(grid, in_channels=4, width=32, seed=1)
+    for call in (lambda: net.forward(x), lambda: net.gradients(x, x[:, 0])):
+        call()
+        free.append(free_bytes())
+    held = free[0] - np.array(free[1:], float)
+    slack = 40e6                                                    # the allocations' granularity
+    assert held[0] < (6 * 285 + 1084) * vox + 84e6 + slack
+    assert abs(held[1] - held[0] - 5 * 1084 * vox) < slack
 
 
 # 20 x 44 x 68 takes the tiles of 16 x 8 x 2 (1100 four-row tiles) with a remainder in x and y, its
