@@ -605,6 +605,14 @@ mcpet_status mcpet_selftest_ranecu(int32_t seed, const int64_t* stream_ids, int3
 mcpet_status mcpet_selftest_fmath(const double* x, const double* y, int32_t n, double* out_d /* 7*n */,
                                   float* out_f /* 8*n */);
 
+/* The transport's in-range functions against the general ones on n arguments, bit for bit. fn: 0 floor, 1 floor with
+ * NaN, 2 sqrtf, 3 logf, 4 expf, 5 sincosf, 6 x / 1000 and its floor (argument: the float of bit pattern
+ * first + i, compared where it lies in the function's range); 7 RANECU's step (both states first + i);
+ * 8 float division, 9 with a given reciprocal, 10 double division, 11 sqrt, 12 log, 13 exp, 14 sincos
+ * (arguments drawn from first + i). res[0]: how many differ, res[1]: the smallest i that does, res[2]: how
+ * many arguments lie in the range. */
+mcpet_status mcpet_selftest_fastmath(int32_t fn, uint64_t first, uint64_t n, uint64_t* res /* 3 */);
+
 /* Stable device radix sort of n 64-bit keys by their low 8*passes bits (passes 1..8), the
  * sort of the singles pipeline; perm receives the sorted order of the input indices. */
 mcpet_status mcpet_selftest_sort(const uint64_t* keys, int64_t n, int32_t passes, uint32_t* perm);

@@ -1902,6 +1902,155 @@ __global__ void k_selftest_fmath(const double* x, const double* y, int n, double
   of[7 * (size_t)n + i] = mcf_acosf(fminf(fmaxf(bf, -1.0f), 1.0f));
 }
 
+// Differences between the functions of fastmath.h (and mcr_step) and the general ones (fmath.h, f2i_rd, IEEE
+// division and root, 64-bit remainders) over n arguments of the stated ranges: every float from bit
+// pattern `first` on where a range is a set of floats (every state of both generators for mcr_step), else drawn from the
+// argument's number, in part next to the values where a rounding, an exponent or a quadrant changes.
+// res[0]: the differences, res[1]: the smallest argument number with one, res[2]: the arguments in range.
+enum FastFn {
+  FF_FLOOR, FF_FLOOR_NAN, FF_SQRT, FF_LOG, FF_EXP, FF_SINCOS, FF_DIV_1000, FF_RANECU,   // argument: first + i
+  FF_DIV, FF_DIV_R, FF_DDIV, FF_DSQRT, FF_DLOG, FF_DEXP, FF_DSINCOS,                             // drawn
+  FF_N
+};
+__device__ __forceinline__ unsigned long long ff_draw(unsigned long long& z)   // splitmix64
+{
+  z += 0x9E3779B97F4A7C15ull;
+  unsigned long long x = z;
+  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
+  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
+  return x ^ (x >> 31);
+}
+// a float with exponent in [-e, e]; of its mantissas one in four has only its first or last bits set or cleared
+__device__ __forceinline__ float ff_float(unsigned long long& z, int e)
+{
+  const unsigned long long h = ff_draw(z);
+  unsigned m = (unsigned)h & 0x7fffffu;
+  if ((h >> 60) == 0) m &= 7u;
+  if ((h >> 60) == 1) m |= 0x7ffff8u;
+  if ((h >> 60) == 2) m &= 0x700000u;
+  if ((h >> 60) == 3) m |= 0x0fffffu;
+  return mcf_ffrom((unsigned)(127 + (int)((h >> 32) % (2 * e + 1)) - e) << 23 | m | ((unsigned)(h >> 59) & 1u) << 31);
+}
+__device__ __forceinline__ double ff_double(unsigned long long& z, int e)
+{
+  const unsigned long long h = ff_draw(z), k = ff_draw(z);
+  unsigned long long m = h & 0xfffffffffffffull;
+  if ((k >> 60) == 0) m &= 7ull;
+  if ((k >> 60) == 1) m |= 0xffffffffffff8ull;
+  if ((k >> 60) == 2) m &= 0xe000000000000ull;
+  if ((k >> 60) == 3) m |= 0x1ffffffffffffull;
+  return mcf_from_bits((unsigned long long)(1023 + (int)((unsigned)(k >> 32) % (unsigned)(2 * e + 1)) - e) << 52 | m | (k & 1ull) << 63);
+}
+// x moved by -2 .. 2 of its last places
+__device__ __forceinline__ float ff_near(float x, unsigned long long& z) { return mcf_ffrom(mcf_fbits(x) + (unsigned)(ff_draw(z) % 5) - 2u); }
+__device__ __forceinline__ double ff_near(double x, unsigned long long& z) { return mcf_from_bits(mcf_bits(x) + ff_draw(z) % 5 - 2ull); }
+// equal bits; a NaN equals any
+__device__ __forceinline__ bool ff_same(float a, float b) { return mcf_fbits(a) == mcf_fbits(b) || (a != a && b != b); }
+__device__ __forceinline__ bool ff_same(double a, double b) { return mcf_bits(a) == mcf_bits(b) || (a != a && b != b); }
+
+// 1: they differ on argument i, 0: they do not, -1: it is outside the function's range
+template <int FN>
+__device__ __forceinline__ int ff_compare(unsigned long long first, unsigned long long i)
+{
+  const float x = mcf_ffrom((unsigned)(first + i));
+  const int state = (int)(first + i);
+  unsigned long long z = (first + i) * 0xD1342543DE82EF95ull;
+  if (FN == FF_FLOOR) return x != x ? -1 : floor_i32(x) != f2i_rd(x);
+  if (FN == FF_FLOOR_NAN) return floor_i32_nan(x) != f2i_rd(x);
+  if (FN == FF_SQRT) return !(x == 0.0f || (x > 0x1p-100f && x < MCF_INFF)) ? -1 : !ff_same(sqrt_nz(x), sqrtf(x));
+  if (FN == FF_LOG) return !(x >= 0x1p-126f && x < MCF_INFF) ? -1 : !ff_same(log_n(x), mcf_logf(x));
+  if (FN == FF_EXP) return x > 88.0f ? -1 : !ff_same(exp_n(x), mcf_expf(x));   // NaN stays NaN
+  if (FN == FF_SINCOS) {
+    if (!(fabsf(x) < 8192.0f)) return -1;
+    float s, c, ms, mc;
+    sincos_n(x, &s, &c);
+    mcf_sincosf(x, &ms, &mc);
+    return !ff_same(s, ms) || !ff_same(c, mc) || !ff_same(cos_n(x), mc);
+  }
+  if (FN == FF_DIV_1000) {   // (tallied energies over 1000: quotients from 2^-80 up, and floors of positive ones anywhere)
+    const bool normal = fabsf(x) >= 0x1p-80f;
+    if (!(fabsf(x) < MCF_INFF) || !(normal || x >= 0.0f)) return -1;
+    const float q = div_r(x, 1000.0f, 1.0f / 1000.0f);
+    return (normal && !ff_same(q, x / 1000.0f)) || floor_i32_nan(q) != f2i_rd(x / 1000.0f);
+  }
+  if (FN == FF_RANECU) {
+    if (state < 1 || state >= MCR_M1) return -1;
+    const int y0 = state < MCR_M2 ? state : 1;
+    int sx = state, sy = y0;
+    const int out = mcr_step(&sx, &sy);
+    const int x1 = (int)(40014ull * (unsigned)state % (unsigned)MCR_M1), y1 = (int)(40692ull * (unsigned)y0 % (unsigned)MCR_M2);
+    return sx != x1 || sy != y1 || out != (x1 - y1 < 1 ? x1 - y1 + (MCR_M1 - 1) : x1 - y1);
+  }
+  if (FN == FF_DIV || FN == FF_DIV_R) {   // half of the quotients next to a float, some of these next to an integer
+    const float b = ff_float(z, 30);
+    float a = ff_float(z, 30);
+    const unsigned long long how = ff_draw(z) & 3;
+    if (how < 2) a = ff_near((how ? rintf(ff_float(z, 12)) : ff_float(z, 30)) * b, z);
+    if (!(fabsf(a) >= 0x1p-62f && fabsf(a) < 0x1p62f)) return -1;
+    return !ff_same(FN == FF_DIV ? div_n(a, b) : div_r(a, b, 1.0f / b), a / b);
+  }
+  if (FN == FF_DDIV) {
+    const double b = ff_double(z, 200);
+    double a = ff_double(z, 200);
+    const unsigned long long how = ff_draw(z) & 3;
+    if (how < 2) a = ff_near((how ? rint(ff_double(z, 20)) : ff_double(z, 200)) * b, z);
+    if (!(fabs(a) >= 0x1p-402 && fabs(a) < 0x1p402)) return -1;
+    return !ff_same(div_n(a, b), a / b);
+  }
+  if (FN == FF_DSQRT) {   // half of them next to a square
+    double a = fabs(ff_double(z, 200));
+    if (ff_draw(z) & 1) {
+      const double r = ff_double(z, 100);
+      a = ff_near(r * r, z);
+    }
+    return !ff_same(sqrt_n(a), sqrt(a));
+  }
+  if (FN == FF_DLOG) {   // all exponents, the generator's outputs, and next to 1 and sqrt(2)
+    const unsigned long long how = ff_draw(z) & 3;
+    double a = fabs(ff_double(z, 1021));
+    if (how == 1) a = (double)(1 + ff_draw(z) % 2147483561ull) * (1.0 / 2147483562.0);
+    if (how == 2) a = 1.0 + ff_double(z, 52) * 0x1p-53;
+    if (how == 3) a = ff_near((ff_draw(z) & 1 ? 1.0 : 0x1.6a09e667f3bcdp+0) * mcf_pow2i((int)(ff_draw(z) % 101) - 50), z);
+    return !(a >= 0x1p-1022) ? -1 : !ff_same(log_n(a), mcf_log(a));
+  }
+  if (FN == FF_DEXP) {   // every exponent below 2^10, next to where the power of two changes, and the ends
+    const unsigned long long how = ff_draw(z) & 3;
+    double a = (double)(ff_draw(z) >> 11) * 0x1p-53 * 712.0;
+    if (how == 1) a = fabs(ff_double(z, 1000)) * 0x1p-991;
+    if (how == 2) a = ff_near(((double)(ff_draw(z) % 1026) + 0.5) * 0x1.62e42fefa39efp-1, z);
+    if (how == 3) a = (ff_draw(z) & 7) ? ff_near(0x1.62e42fefa39efp+9, z) : (ff_draw(z) & 1) ? 0.0 : MCF_INF;
+    return !ff_same(exp_nonneg(a), mcf_exp(a));
+  }
+  // angles of up to 2^30 either way, and next to where the quadrant changes
+  const unsigned long long how = ff_draw(z) & 3;
+  double a = ((double)(ff_draw(z) >> 11) * 0x1p-52 - 1.0) * (how == 0 ? 0x1p30 : 7.0);
+  if (how == 2) a = ff_near(((double)(int)(ff_draw(z) % 2000001) - 1000000.0) * 0x1.921fb54442d18p-1, z);
+  if (how == 3) a = ff_double(z, 29);
+  if (!(fabs(a) < 0x1p30)) return -1;
+  double s, c, ms, mc;
+  sincos_n(a, &s, &c);
+  mcf_sincos(a, &ms, &mc);
+  return !ff_same(s, ms) || !ff_same(c, mc);
+}
+template <int FN>
+__global__ __launch_bounds__(256) void k_selftest_fastmath(unsigned long long first, unsigned long long n, unsigned long long* res)
+{
+  unsigned long long count = 0, least = ~0ull, compared = 0;
+  for (unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (unsigned long long)gridDim.x * 256) {
+    const int d = ff_compare<FN>(first, i);
+    if (d >= 0) compared++;
+    if (d > 0) {
+      count++;
+      least = min(least, i);
+    }
+  }
+  atomicAdd(&res[2], compared);
+  if (count) {
+    atomicAdd(&res[0], count);
+    atomicMin(&res[1], least);
+  }
+}
+
 // Clear n words (a memset that a captured graph may hold).
 __global__ void k_fill_u32(unsigned* __restrict__ p, size_t n)
 {
@@ -2190,6 +2339,22 @@ hipError_t mcpet_launch_selftest_ranecu(int seed, const long long* d_ids, int ns
   hipLaunchKernelGGL(k_selftest_ranecu, dim3(blocks), dim3(256), 0, stream, seed, d_ids, nstreams, n, d_out, d_out_d, as_double,
                      j1, j2);
   return hipGetLastError();
+}
+
+template <int FN>
+static hipError_t launch_selftest_fastmath(int fn, unsigned long long first, unsigned long long n, unsigned long long* d_res, hipStream_t stream)
+{
+  if constexpr (FN < FF_N) {
+    if (fn != FN) return launch_selftest_fastmath<FN + 1>(fn, first, n, d_res, stream);
+    const unsigned blocks = (unsigned)std::min<unsigned long long>(8192, (n + 255) / 256);
+    hipLaunchKernelGGL(k_selftest_fastmath<FN>, dim3(blocks), dim3(256), 0, stream, first, n, d_res);
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;
+}
+hipError_t mcpet_launch_selftest_fastmath(int fn, unsigned long long first, unsigned long long n, unsigned long long* d_res, hipStream_t stream)
+{
+  return launch_selftest_fastmath<0>(fn, first, n, d_res, stream);
 }
 
 hipError_t mcpet_launch_selftest_fmath(const double* d_x, const double* d_y, int n, double* d_od, float* d_of, hipStream_t stream)

@@ -181,6 +181,8 @@ hipError_t mcpet_launch_project(const KParams* d_params, const int* active_vox, 
 hipError_t mcpet_launch_scale_by_max(float* a, int n, unsigned* mx, hipStream_t stream);
 hipError_t mcpet_launch_selftest_ranecu(int seed, const long long* d_ids, int nstreams, int n, float* d_out, double* d_out_d,
                                         int as_double, const uint32_t* j1, const uint32_t* j2, hipStream_t stream);
+hipError_t mcpet_launch_selftest_fastmath(int fn, unsigned long long first, unsigned long long n, unsigned long long* d_res,
+                                          hipStream_t stream);
 hipError_t mcpet_launch_selftest_fmath(const double* d_x, const double* d_y, int n, double* d_od, float* d_of, hipStream_t stream);
 hipError_t mcpet_launch_copy(const uint4* src, uint4* dst, size_t n16, hipStream_t stream);
 int mcpet_transport_regs_hint();

@@ -1691,6 +1691,24 @@ extern "C" mcpet_status mcpet_selftest_fmath(const double* x, const double* y, i
   return rc;
 }
 
+extern "C" mcpet_status mcpet_selftest_fastmath(int32_t fn, uint64_t first, uint64_t n, uint64_t* res)
+{
+  if (!res || n < 1 || fn < 0) return set_err(nullptr, MCPET_E_ARG, "selftest_fastmath: bad args");
+  unsigned long long* d = nullptr;
+  unsigned long long h[3] = {0, ~0ull, 0};
+  hipError_t e = hipMalloc((void**)&d, sizeof h);
+  if (e == hipSuccess) e = hipMemcpy(d, h, sizeof h, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = mcpet_launch_selftest_fastmath(fn, first, n, d, 0);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (e == hipSuccess) e = hipMemcpy(h, d, sizeof h, hipMemcpyDeviceToHost);
+  if (d) (void)hipFree(d);
+  if (e != hipSuccess)
+    return set_err(nullptr, e == hipErrorInvalidValue ? MCPET_E_ARG : MCPET_E_HIP,
+                   std::string("selftest_fastmath: ") + hipGetErrorString(e));
+  for (int k = 0; k < 3; k++) res[k] = h[k];
+  return MCPET_OK;
+}
+
 extern "C" mcpet_status mcpet_selftest_sort(const uint64_t* keys, int64_t n, int32_t passes, uint32_t* perm)
 {
   if (!keys || !perm || n < 0 || n > 0x7fffffffLL || passes < 1 || passes > 8)

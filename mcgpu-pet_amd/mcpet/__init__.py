@@ -191,6 +191,7 @@ def lib():
     L.mcpet_selftest_ranecu.argtypes = [C.c_int32, P(C.c_int64), C.c_int32, C.c_int32, P(C.c_float), P(C.c_double),
                                         C.c_int32]
     L.mcpet_selftest_fmath.argtypes = [P(C.c_double), P(C.c_double), C.c_int32, P(C.c_double), P(C.c_float)]
+    L.mcpet_selftest_fastmath.argtypes = [C.c_int32, C.c_uint64, C.c_uint64, P(C.c_uint64)]
     L.mcpet_selftest_copy.argtypes = [C.c_size_t, C.c_int32, P(C.c_double)]
     L.mcpet_stream_seeds.argtypes = [C.c_int32, P(C.c_int64), C.c_int32, P(C.c_int32), P(C.c_int32)]
     L.mcpet_version.restype = C.c_char_p
@@ -854,6 +855,18 @@ def selftest_fmath(x, y):
     _check(lib().mcpet_selftest_fmath(x.ctypes.data_as(C.POINTER(C.c_double)), y.ctypes.data_as(C.POINTER(C.c_double)),
                                       n, od.ctypes.data_as(C.POINTER(C.c_double)), of.ctypes.data_as(C.POINTER(C.c_float))))
     return od, of
+
+
+FAST_FUNCTIONS = ("floor", "floor_nan", "sqrtf", "logf", "expf", "sincosf", "div_1000", "ranecu", "divf", "divf_r",
+                  "div", "sqrt", "log", "exp", "sincos")
+
+
+def selftest_fastmath(name, first, n):
+    """(on how many of n arguments the in-range function differs from the general one, the first of them, how many
+    arguments lie in its range): mcpet_selftest_fastmath."""
+    res = (C.c_uint64 * 3)()
+    _check(lib().mcpet_selftest_fastmath(FAST_FUNCTIONS.index(name), first, n, res))
+    return tuple(int(r) for r in res)
 
 
 def selftest_sort(keys, passes=8, noalloc=False):
