@@ -465,16 +465,16 @@ __device__ __forceinline__ bool gcoa_pz_trial(float E, int mat, Rng& r, CN& C, c
   }
   temp = rn(r, C) * gcoa_rnv(E, table, cs, ishell);
   const float fj = table[ishell].z;
-  // both halves of the profile through one logarithm and root; its argument is below 1, and zero
-  // (an infinite root) or subnormal only where the profile term underflows (lower half)
+  // both halves of the profile through one logarithm and root; its argument is below 1
   const bool low = temp < 0.5f;
-  const float y = low ? temp + temp : 2.0f - 2.0f * temp;
-  float root = sqrt_nz(0.5f - (y >= 0x1p-126f ? log_n(y) : mcf_logf(y)));
-  if (y == 0.0f) root = MCF_INFF;
-  const float dev = root - 0.70710678118654502f;
-  const float num = low ? -dev : dev, den = fj * 1.4142135623731f;
-  // a profile of zero width (the quotient is infinite) or nearly so takes the general division
-  const float pzomc = fabsf(den) >= 0x1p-80f && y != 0.0f ? div_n(num, den) : num / den;
+  const float y = low ? temp + temp : 2.0f - 2.0f * temp, den = fj * 1.4142135623731f;
+  const float dev = sqrt_nz(0.5f - log_n(y)) - 0.70710678118654502f;
+  float pzomc = div_n(low ? -dev : dev, den);
+  // y below 2^-126: the profile term underflows; no number: a profile of zero or hardly any width
+  if (!(y >= 0x1p-126f) || pzomc != pzomc) {
+    const float gdev = sqrtf(0.5f - mcf_logf(y)) - 0.70710678118654502f;
+    pzomc = (low ? -gdev : gdev) / den;
+  }
   cs.pzomc = pzomc;
   if (!(pzomc < -1.0f)) {
     float af;
