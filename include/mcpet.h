@@ -521,7 +521,8 @@ mcpet_status mcpet_batch_project_maps(mcpet_batch* b, int32_t k, int32_t D, int3
  * 2 width -> upsampling, concatenation with the width skip -> convolution to width -> 1^3
  * convolution; ReLU after every 3^3 convolution; the output is input channel 0 plus that
  * residual. Every convolution runs as an implicit GEMM on BF16 MFMA tiles with FP32
- * accumulation; parameters, activations and optimiser state are FP32. Parameter layout: per
+ * accumulation; parameters, gradients, optimiser state, input and output are FP32, the activations
+ * between the layers are held as the BF16 operands that the products read. Parameter layout: per
  * layer W[Cout][Cin][k^3] then b[Cout], layers in the order above. Created with He-normal
  * weights from `seed`, zero biases and a zero output layer (the identity on channel 0). Holds the
  * tensors of a group of samples (about 2^19 voxels, at most 1 GiB or one sample; what only the gradients
@@ -534,7 +535,8 @@ mcpet_status mcpet_surrogate_set_params(mcpet_surrogate* s, const float* in);
 /* x: batch x in_channels x D x H x W (host); y: batch x D x H x W (host). gflop: forward GFLOP per sample. */
 mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float* x, int32_t batch, float* y, double* gflop);
 /* Device time per sample (ms, HIP events on the network's stream) of the network proper in the last
- * mcpet_surrogate_forward call (its last samples that went through together; no host copies). */
+ * mcpet_surrogate_forward call (its last samples that went through together; without the copies from and to
+ * the host and the input's conversion, which is part of the copy). */
 mcpet_status mcpet_surrogate_forward_ms(mcpet_surrogate* s, double* ms);
 /* One estimate from the last run of ctx (a 2- or 4-input-channel network; same device), all on
  * the device: its scatter and trues rebinned onto the network's grid (mcpet_rebin_sinogram),

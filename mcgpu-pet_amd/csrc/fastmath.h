@@ -34,8 +34,9 @@ static __device__ __forceinline__ int floor_i32(float x)
 static __device__ __forceinline__ int floor_i32_nan(float x) { return x == x ? floor_i32(x) : INT32_MIN; }
 
 // sqrt(x), x normal and above 2^-100, or zero of either sign: one Newton step on the reciprocal
-// root and two on the root with exact residuals (the sequence of the compiler's own expansion of
-// a correctly rounded square root, without its scaling).
+// root and two on the root with exact residuals: Goldschmidt's coupled iteration for x^(1/2) and x^(-1/2)/2 and
+// Markstein's correction by the exact residual x - s s (P. Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", IBM J. Res. Dev. 34, 1990), without the scaling that arguments near the ends need.
 static __device__ __forceinline__ float sqrt_nz(float x)
 {
   const float r = __builtin_amdgcn_rsqf(fmaxf(x, 0x1p-126f));
@@ -46,8 +47,10 @@ static __device__ __forceinline__ float sqrt_nz(float x)
   return fmaf(fmaf(-s, s, x), h, s);
 }
 
-// a / b, b and a / b normal and a normal or zero, all far from the ends of the range: the steps
-// of the compiler's expansion, whose scaling and fix-up do nothing there. A zero quotient is +0.
+// a / b, b and a / b normal and a normal or zero, all far from the ends of the range: a Newton step on the
+// reciprocal and Markstein's corrections of the quotient by its exact residual a - b q (the same paper), without
+// the scaling and fix-up that do nothing there. A zero quotient is +0; b = 0, an infinite a or b and an overflow
+// of the steps give NaN.
 static __device__ __forceinline__ float div_n(float a, float b)
 {
   float r = __builtin_amdgcn_rcpf(b);

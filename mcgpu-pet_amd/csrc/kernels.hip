@@ -65,8 +65,9 @@
 #endif
 // Occupancy target of the persistent transport kernels: five waves per SIMD (96 registers, none spilled, up to
 // 32 KB of LDS a workgroup). Waves hide the dependent gathers until the vector ALUs' issue bounds the
-// kernel: head, 1e8 decays, 31.9 ms with four, 29.0 with five, 29.1 with six, whose 80 registers spill; 4e7
-// torso decays with singles, 4 / 5 / 6 waves: 38.1 / 36.3 / 36.8 ms.
+// kernel; six have 80 registers, which spill. With four / five / six, streams made ready by the wave and
+// pairs tallied from the queue: head, 1e8 decays, 29.7 / 26.9 / 28.2 ms; 4e7 torso decays with singles 35.7 /
+// 32.7 / 36.8; eight phantoms 7.05 / 6.58 / 7.08; 5e6 decays 1.49 / 1.46 / 1.51; 4e6 ragged 1.06 / 1.07 / 1.13.
 #ifndef MCPET_WAVES_PER_EU
 #define MCPET_WAVES_PER_EU 5
 #endif

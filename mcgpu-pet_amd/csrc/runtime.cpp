@@ -863,8 +863,10 @@ static mcpet_status clear_buffers(mcpet_ctx* c, hipStream_t stream, bool tallies
 // once, left the last waves too much: head, 1e8 decays, 27.7 -> 33.2 ms), down to chunks worth
 // about 64 decays, since a claim costs the device about 6 ns and one address serves them all, and to
 // what a wave makes ready together: 16-128 streams. own: the first claim is the wave's by its number,
-// without an atomic (only if every wave is resident from the start). 5e6 decays at 4 a stream: 1.44 ms;
-// with chunks of half the size 1.67-2.1, eight phantoms 6.7 -> 7.9.
+// without an atomic (only if every wave is resident from the start). Least chunks of half / this / twice the
+// size (16-128): scatter phantom of 1e6 decays 0.71 / 0.67 / 0.81 ms, 5e6 1.78 / 1.47 / 1.45, 2e7 4.65 / 4.67 /
+// 4.80; head of 1e7 3.62 / 3.21 / 3.22, of 1e8 27.4 / 26.9 / 26.8; ragged of 1e6 0.43 / 0.43 / 0.50, of 4e6
+// 1.28 / 1.07 / 1.03; 4e7 torso decays with singles 32.6 / 32.7 / 33.6; eight phantoms 6.66 / 6.58 / 6.64.
 static void set_claims(KParams& P, double expected_decays, long long n_waves, bool own)
 {
   P.n_claims = std::max(0LL, (P.n_streams - P.stream_base + P.stream_stride - 1) / std::max(1LL, P.stream_stride));
@@ -873,7 +875,9 @@ static void set_claims(KParams& P, double expected_decays, long long n_waves, bo
   P.chunk_shift = shift;
   const double per_stream = expected_decays / (double)std::max(1LL, P.n_streams);
   P.chunk_min = per_stream >= 4.0 ? 16 : per_stream >= 2.0 ? 64 : 128;
-  // at least 96, so that a wave fills its lanes at the start from what is its own (4e6 decays 1.15 -> 1.08 ms)
+  // at least 96, so that a wave fills its lanes at the start from what is its own: at least 1 / 48 / 96 / 192
+  // (where there are twice as many), scatter phantom of 5e6 decays 1.65 / 1.54 / 1.47 / 1.65 ms, of 1e7 2.73 / 2.60 /
+  // 2.51 / 2.75, ragged of 4e6 1.17 / 1.13 / 1.07 / 1.18; no difference for the head, the torso and 1e6 to 2.5e6 decays
   P.chunk0 = own ? (int)std::min(512LL, std::max<long long>(P.n_claims >= 192 * n_waves ? 96 : 1, P.n_claims >> shift)) : 0;
 }
 

@@ -5,9 +5,12 @@
 // Every convolution product (forward, input gradient, weight gradient) is an implicit GEMM
 //   C[m][n] (+)= sum_k A(m, k) * B(k, n)
 // on BF16 MFMA tiles (v_mfma_f32_16x16x32_bf16: 16x16 outputs, K = 32 per instruction, FP32
-// accumulation); operands are rounded to BF16, parameters, activations and gradients are kept
-// in FP32 (im2col is never materialised). k_conv holds the three products; k_gemm is a plain
-// GEMM on the same tiles, used by the self test of the MFMA operand layout.
+// accumulation); operands are rounded to BF16 (im2col is never materialised). Parameters, optimiser
+// state, the input, the output and all gradients are kept in FP32; the activations between the
+// layers exist only as the BF16 operands of the products that read them. k_conv_tiled, k_conv_planes,
+// k_conv_cols and k_conv_short hold the forward and input-gradient products, k_bwgt_tiled and
+// k_bwgt_point the weight gradients; k_gemm is a plain GEMM on the same tiles, used by the self test
+// of the MFMA operand layout.
 // MFMA lane layout (16x16x32 BF16): lane l holds A row (l % 16), k = 8 (l / 16) .. +7; B column
 // (l % 16), the same k; the accumulator's 4 values are rows 4 (l / 16) .. +3 of column (l % 16).
 #include <hip/hip_runtime.h>
@@ -104,15 +107,16 @@ hipError_t gemm(AOp A, BOp B, float* C, int M, int N, int K, int ldc, const floa
 // Each convolution product is one implicit GEMM with a tap-major reduction index
 // k = t * Cp + c (t: kernel tap, 27 for 3x3x3 or 1 for 1x1x1; c: channel, padded to
 // Cp = roundup(C, 8)), so a lane's 8 consecutive k share one tap: one address and bounds
-// computation, then 8 loads at channel stride.
+// computation, then one 16-byte load.
 //   FWD   : Y[co][p]        = act(sum_k Wf[co][k] X[c][s p + d_t] + b[co])    m = co, n = output voxel
 //   BDATA : dX[ci][p]      (+)= mask(sum_k Wb[ci][k] dY[c][q], s q + d_t = p)  m = ci, n = input voxel
-//   BWGT  : G[co][ci T + t] += sum_q dY[co][q] X[ci][s q + d_t]              m = co, n = t Cin + ci, k = q
+// and the weight gradient (k_bwgt_tiled, k_bwgt_point) is
+//           G[co][ci][t]    += sum_q dY[co][q] X[ci][s q + d_t]              m = co, n = ci, k = q
 // Wf, Wb: BF16 copies of the FP32 weights in those layouts (zero padded, in MFMA fragment order). FWD
 // and BDATA read their B tensor from a channels-last BF16 copy ([voxel][Cp], padding zero), so a
-// lane's 8 channels are one 16-byte load; their epilogues write such copies of what they produce
-// (for the next product) beside the FP32 channel-first tensor (which BWGT, the bias gradients and
-// the ReLU masks read). BWGT splits its (voxel) reduction over workgroups.
+// lane's 8 channels are one 16-byte load; their epilogues write such a copy of what they produce: FWD
+// nothing else (but the output layer, which writes FP32), as the next product, the weight gradient and, by its
+// sign, the ReLU mask read it; BDATA beside the FP32 gradient, which the bias gradient reads.
 
 // FWDUP: FWD of a concatenation whose first Cu channels are the nearest x2 upsampling of a tensor of
 // half the size, read where it is.
@@ -131,7 +135,7 @@ struct ConvK {
   const __bf16* Xu;    // FWDUP: channels 0 .. Cu - 1 at half size, [D/2][H/2][W/2][ldu]; Xl holds the others
   int ldx, ldu, Cu;
   ClOut o1;            // FWD, BDATA: channels-last copy of the output
-  float* C;            // FWD: Y [M][N]; BDATA: dX [M][N]; BWGT: weight gradient [Cout][Cin][T]
+  float* C;            // FWD: Y [M][N], may be null; BDATA: dX [M][N]
   const float* bias;   // FWD
   const __bf16* mask;  // BDATA: the layer input's channels from mask0 on, [N][ldm] (gradient zero where it is
   int ldm, mask0;      // not positive: the ReLU before it); may be null
@@ -139,7 +143,7 @@ struct ConvK {
   int relu, beta;      // FWD: ReLU on the output; BDATA: add to C
   int M, N, K, Kp;     // GEMM sizes; Kp: K padded to whole k-steps
   int nrb;             // 16-row blocks of A
-  int Cb, Cbp;         // channels of the B tensor (FWD, BWGT: Cin; BDATA: Cout) and Cb rounded up to 8
+  int Cb, Cbp;         // channels of the B tensor (FWD: Cin; BDATA: Cout) and Cb rounded up to 8
   int D, H, W, oD, oH, oW, ks, stride, T;
   size_t sX, sXu, sC, sR;   // from one sample to the next (blockIdx.z): B tensor(s); C; res
   int samples;
@@ -863,8 +867,13 @@ void launch_cols(const ConvK& a, int mt, hipStream_t st)
 // (two per CU), the smallest where none does.
 #define COLS_WGS 512
 // k_conv_planes takes a shape when its halo plane fits LDS beside a second workgroup's and its tiles
-// give PLANES_WGS workgroups: with fewer, k_conv_cols' smaller tiles end as soon (one sample of 32 x 56 x 56,
-// whose half resolution has 224: 0.157 -> 0.144 ms; thresholds of 100 and 48 no better on smaller volumes).
+// give PLANES_WGS workgroups: with fewer, k_conv_cols' smaller tiles end as soon. Forward at width 32, device
+// us a sample, with a threshold of 1 / 100 / 200 / 256 / 512 / never: one sample of 32 x 56 x 56 (its half
+// resolution has 224) 145 / 144 / 144 / 158 / 157 / 157, four 83 / 82 / 83 / 82 / 84 / 95; 24 x 40 x 40
+// one 117 / 109 / 102 / 102 / 101 / 114, four 51 / 51 / 51 / 51 / 56 / 65; 16 x 28 x 28 one 103 / 77 / 77 /
+// 77 / 77 / 77, eight 20 / 20 / 20 / 20 / 21 / 25; 12 x 20 x 36 four 29 / 27 / 25 / 25 / 25 / 28; 16 x 56 x 56
+// two 81 / 81 / 81 / 87 / 85 / 103; 64^3 one 210 / 212 / 209 / 209 / 209 / 244; width 16, one of
+// 32 x 56 x 56: 117 / 110 / 109 / 107 / 107 / 107.
 #define PLANES_WGS 200
 inline long long planes_tiles(const ConvK& a) { return (long long)((a.W + 15) / 16) * ((a.H + 3) / 4) * a.D; }
 inline size_t planes_lds(const ConvK& a, int mt) { return std::max<size_t>(16 * (size_t)(a.Cbp / 8) * FP_HP, 16 * 512 * (size_t)mt); }
@@ -940,13 +949,14 @@ hipError_t launch_conv(const ConvK& a, hipStream_t st)
 }
 
 // Stride-1 3x3x3 FWD / BDATA products with Cbp % 32 == 0 (k_conv_tiled); the row blocks as
-// k_conv's, so the A rows read stay inside the padded weight copy. Counted in 4-row tiles.
+// k_conv_cols', so the A rows read stay inside the padded weight copy. Counted in 4-row tiles.
 inline long long tiled_blocks(const ConvK& a)
 {
   return (long long)((a.W + FT_X - 1) / FT_X) * ((a.H + 3) / 4) * a.D * ((a.M + 16 * mt_for(a.M) - 1) / (16 * mt_for(a.M)));
 }
 // The tiled products on volumes with at least 1024 four-row tiles (the full-resolution level);
-// smaller volumes (the coarser U-Net levels) keep k_conv's 16-voxel tiles and in-workgroup k split.
+// smaller volumes (the coarser U-Net levels) take the 16-voxel tiles and in-workgroup k split of
+// k_conv_planes and k_conv_cols.
 #define TILED_MIN 1024
 inline bool use_tiled(const ConvK& a)
 {
@@ -1176,7 +1186,7 @@ constexpr size_t kBwPartFloats = (size_t)BW_WGS * 2 * 27 * 1024;   // half a wor
 
 // The input x and its gradient's copy gyl as in conv_bwd_weights; stride 1 (input and output volumes
 // equal) or 2 (output (D/2, H/2, W/2)). Output channels go in passes of as many 32-channel blocks as
-// the partial sums have room for (all of them up to 512 blocks of 32 x 32).
+// the partial sums have room for (all of them up to 256 blocks of 32 x 32: each workgroup writes two halves).
 hipError_t launch_bwgt_tiled(int samples, int stride, BwK b, const __bf16* gyl, float* G, hipStream_t st)
 {
   if (b.ldx % 8 != 0 || b.ldg % 8 != 0 || (stride != 1 && stride != 2)) return hipErrorInvalidValue;
@@ -2052,8 +2062,8 @@ extern "C" mcpet_status mcpet_surrogate_forward(mcpet_surrogate* s, const float*
 }
 
 // Device time per sample of the network in the last mcpet_surrogate_forward (its last samples that
-// went through together: every kernel from the input conversion to the output, HIP events on the
-// network's stream).
+// went through together: the layers from the converted input to the output, HIP events on the network's
+// stream; k_input, which converts the input while it reads it from pinned host memory, comes before).
 extern "C" mcpet_status mcpet_surrogate_forward_ms(mcpet_surrogate* s, double* ms)
 {
   if (!s || !ms) return serr(s, MCPET_E_ARG, "mcpet_surrogate_forward_ms: null argument");
